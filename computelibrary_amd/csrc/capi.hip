@@ -3,6 +3,7 @@
 #include "../../include/mi355_gemmlowp.h"
 #include "internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -170,7 +171,15 @@ struct GemmCore
     bool    has_narrow = false; // Bn holds the narrow kernel's image of B
     bool    pt_vectors = false; // streaming path, per-tensor requantisation: mult / shift hold the scalars, replicated
     std::string kname;
-    DevBuf  Bp, Bs, Bn, colsum, colvec, rowvec, mult, shift, bias, Ap, fill, qp, zeros, parts, zerocol;
+    DevBuf  Bp, Bs, Bn, colsum, colvec, colpart, rowvec, mult, shift, bias, Ap, fill, qp, zeros, parts, zerocol;
+    // A prepare that only enqueues (every operand in device memory, nothing left to set up): the stream it went to and an
+    // event behind it, which runs on other streams wait for
+    hipEvent_t  prep_done    = nullptr;
+    hipStream_t prep_stream  = nullptr;
+    bool        prep_pending = false;
+    int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not written yet)
+    bool        qp_scalar_set = false; // the per-tensor requantisation vectors hold qp_rq
+    mi355_requant qp_rq{};
     int     splitk = 1;      // K slices of the pipelined kernel
     int     splitk_plan = 1; // what the cost model chose with the tile shape (create()); prepare() checks it and allocates
     bool    conv_core = false; // the GEMM inside a convolution handle
@@ -204,7 +213,10 @@ struct GemmCore
 
     void release()
     {
-        Bp.release(), Bs.release(), Bn.release(), colsum.release(), colvec.release(), rowvec.release(), mult.release();
+        if (prep_done)
+            (void)hipEventDestroy(prep_done);
+        prep_done = nullptr, prep_pending = false;
+        Bp.release(), Bs.release(), Bn.release(), colsum.release(), colvec.release(), colpart.release(), rowvec.release(), mult.release();
         shift.release(), bias.release(), Ap.release(), fill.release(), qp.release(), zeros.release(), parts.release(), zerocol.release();
     }
 
@@ -320,15 +332,92 @@ struct GemmCore
         return 0;
     }
 
-    // after Bp / colsum have been written for every B: per-column vectors
-    int finish_prepare(const int32_t *bias_in, const int32_t *mult_in, const int32_t *shift_in, hipStream_t s)
+    ColumnFinish column_finish(const int32_t *bias_in) const
     {
-        has_bias = bias_in != nullptr;
+        return {colsum.as<int32_t>(), colvec.as<int32_t>(), bias_in, bias.as<int32_t>(), (uint32_t)a_off_eff(), (uint32_t)b_off_eff(),
+                (uint32_t)(k_const > 0 ? k_const : K), N};
+    }
+
+    // B (device memory; N rows of K elements when transposed) -> the packed image the chosen kernel reads, the columns' sums
+    // and the per-column terms of the epilogue. bias_in: device memory, or null
+    int pack(const void *B, int64_t ldb, int64_t b_bs, bool transposed, int kf, const int32_t *bias_in, hipStream_t s)
+    {
+        const bool   skinny = path == MI355_PATH_SKINNY;
+        DevBuf      &dst    = skinny ? Bs : Bp;
+        const size_t image  = (size_t)Np * Kp;
+        has_bias            = bias_in != nullptr;
+        TRY(dst.ensure(image * nb()));
+        TRY(colsum.ensure(sizeof(int32_t) * (size_t)Np * nb()));
+        TRY(colvec.ensure(sizeof(int32_t) * (size_t)Np * nb()));
         if (has_bias)
-        {
             TRY(bias.ensure(sizeof(int32_t) * (size_t)N));
-            HIP_TRY(hipMemcpyAsync(bias.p, bias_in, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s));
+        constexpr int MOST = 32768; // batch entries along a grid dimension
+        const int     splits = transposed ? 1 : pack_b_splits(Kp, Np, std::min(nb(), MOST));
+        if (splits > 1)
+            TRY(colpart.ensure(sizeof(int32_t) * (size_t)Np * nb() * splits));
+        for (int b = 0; b < nb(); b += MOST)
+        {
+            const int      n   = std::min(MOST, nb() - b);
+            const uint8_t *src = (const uint8_t *)B + (int64_t)b * b_bs;
+            int8_t        *out = dst.as<int8_t>() + (size_t)b * image;
+            ColumnFinish   f   = column_finish(epi == EPI_FIXEDPOINT ? bias_in : nullptr);
+            f.colsum += (int64_t)b * Np, f.colvec += (int64_t)b * Np;
+            if (transposed)
+                HIP_TRY(pack_bt_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, out, f, s));
+            else
+                HIP_TRY(pack_b_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, out, colpart.as<int32_t>(), f, s));
         }
+        return 0;
+    }
+
+    // Whether `s` is recording a graph (an error of the query counts as recording)
+    static bool capturing(hipStream_t s)
+    {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cap) == hipSuccess)
+            return cap != hipStreamCaptureStatusNone;
+        (void)hipGetLastError();
+        return true;
+    }
+
+    // behind a prepare whose work is left running on s
+    int prepare_enqueued(hipStream_t s)
+    {
+        prep_pending = false;
+        if (capturing(s))
+            return 0; // the graph's own order holds from here on
+        // (nothing on the host reads what the kernels wrote: without the system fence the event costs 0.9 us between the two
+        // kernels instead of 2.7)
+        if (prep_done == nullptr)
+            HIP_TRY(hipEventCreateWithFlags(&prep_done, hipEventDisableTiming | hipEventDisableSystemFence));
+        HIP_TRY(hipEventRecord(prep_done, s));
+        prep_stream = s, prep_pending = true;
+        return 0;
+    }
+
+    // in front of a run on s
+    int wait_for_prepare(hipStream_t s)
+    {
+        if (!prep_pending || (s == prep_stream && s != hipStreamPerThread))
+            return 0;
+        if (!capturing(s))
+        {
+            HIP_TRY(hipStreamWaitEvent(s, prep_done, 0));
+            return 0;
+        }
+        // a graph under construction cannot wait for work outside it: the host does
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        const hipError_t e = hipEventSynchronize(prep_done);
+        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        HIP_TRY(e);
+        prep_pending = false;
+        return 0;
+    }
+
+    // after pack(): everything else a run reads
+    int finish_prepare(const int32_t *mult_in, const int32_t *shift_in, hipStream_t s)
+    {
         has_pc = epi == EPI_FIXEDPOINT && rq.per_channel != 0;
         if (has_pc)
         {
@@ -342,12 +431,6 @@ struct GemmCore
             HIP_TRY(hipMemcpyAsync(mult.p, mult_in, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s));
             HIP_TRY(hipMemcpyAsync(shift.p, shift_in, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s));
         }
-        if (path == MI355_PATH_SKINNY)
-        {
-            TRY(Bs.ensure((size_t)nb() * Np * Kp));
-            for (int b = 0; b < nb(); ++b)
-                HIP_TRY(pack_b_skinny_launch(Bp.as<int8_t>() + (size_t)b * Np * Kp, Kp, Np, Bs.as<int8_t>() + (size_t)b * Np * Kp, s));
-        }
         // few output columns and a short K: the image of the B panel the narrow kernel copies into LDS
         has_narrow = path == MI355_PATH_MFMA && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192)) && narrow_panel_chunks(K) > 0;
         if (has_narrow)
@@ -357,9 +440,8 @@ struct GemmCore
             TRY(Bn.ensure((size_t)rows * (chunks + NARROW_PAD_PIECES) * 16));
             HIP_TRY(pack_b_narrow_launch(Bp.as<int8_t>(), Kp, Np, chunks, rows, Bn.as<int8_t>(), s));
         }
-        TRY(fill.ensure(16));
-        HIP_TRY(fill_i32_launch(fill.as<int32_t>(), (int32_t)(0x01010101u * fill_byte), 4, s));
-        if (path == MI355_PATH_SKINNY)
+        TRY(set_fill(s));
+        if (path == MI355_PATH_SKINNY && zeros.p == nullptr)
         {
             // the streaming kernel fetches its per-row vector without asking whether there is one
             TRY(zeros.ensure(sizeof(int32_t) * SKINNY_MAX_M));
@@ -376,23 +458,36 @@ struct GemmCore
         {
             const size_t ldp = ((size_t)N + 3) & ~(size_t)3;
             TRY(parts.ensure(sizeof(int32_t) * (size_t)splitk * M * ldp));
-            TRY(zerocol.ensure(sizeof(int32_t) * (size_t)Np));
-            HIP_TRY(fill_i32_launch(zerocol.as<int32_t>(), 0, Np, s));
+            if (zerocol.p == nullptr)
+            {
+                TRY(zerocol.ensure(sizeof(int32_t) * (size_t)Np));
+                HIP_TRY(fill_i32_launch(zerocol.as<int32_t>(), 0, Np, s));
+            }
         }
-        TRY(refresh_colvec(s));
         TRY(refresh_qparams(s));
         refresh_names();
         prepared = true;
         return 0;
     }
 
+    int set_fill(hipStream_t s)
+    {
+        TRY(fill.ensure(16));
+        if (fill_set != fill_byte)
+            HIP_TRY(fill_i32_launch(fill.as<int32_t>(), (int32_t)(0x01010101u * fill_byte), 4, s));
+        fill_set = fill_byte;
+        return 0;
+    }
+
     int refresh_colvec(hipStream_t s)
     {
-        TRY(colvec.ensure(sizeof(int32_t) * (size_t)Np * nb()));
-        for (int b = 0; b < nb(); ++b)
-            HIP_TRY(colvec_launch(colsum.as<int32_t>() + (size_t)b * Np,
-                                  (has_bias && epi == EPI_FIXEDPOINT) ? bias.as<int32_t>() : nullptr, a_off_eff(),
-                                  b_off_eff(), k_const > 0 ? k_const : K, N, colvec.as<int32_t>() + (size_t)b * Np, s));
+        constexpr int MOST = 32768;
+        for (int b = 0; b < nb(); b += MOST)
+        {
+            ColumnFinish f = column_finish((has_bias && epi == EPI_FIXEDPOINT) ? bias.as<int32_t>() : nullptr);
+            f.colsum += (int64_t)b * Np, f.colvec += (int64_t)b * Np;
+            HIP_TRY(colvec_launch(Np, std::min(MOST, nb() - b), f, s));
+        }
         return 0;
     }
 
@@ -401,6 +496,10 @@ struct GemmCore
     // nothing here waits for the device.
     int refresh_qparams(hipStream_t s)
     {
+        // per-tensor: what is there still holds unless the requantisation has changed
+        if (!has_pc && qp_scalar_set && memcmp(&qp_rq, &rq, sizeof(rq)) == 0)
+            return 0;
+        qp_scalar_set = !has_pc, qp_rq = rq;
         qp_on = false;
         if (path == MI355_PATH_SKINNY && epi == EPI_FIXEDPOINT && !has_pc)
         {
@@ -804,21 +903,16 @@ int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *b
     TRY(to_device(bias, sizeof(int32_t) * d.N, h->stageBias, s, &biasd));
     TRY(to_device(c.rq.per_channel ? mult : nullptr, sizeof(int32_t) * d.N, h->stageMult, s, &multd));
     TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * d.N, h->stageShift, s, &shiftd));
-    TRY(c.Bp.ensure((size_t)nb * c.Np * c.Kp));
-    TRY(c.colsum.ensure(sizeof(int32_t) * (size_t)nb * c.Np));
-    for (int b = 0; b < nb; ++b)
-    {
-        const uint8_t *src = (const uint8_t *)Bd + (size_t)b * d.b_batch_stride;
-        int8_t        *dst = c.Bp.as<int8_t>() + (size_t)b * c.Np * c.Kp;
-        int32_t       *cs  = c.colsum.as<int32_t>() + (size_t)b * c.Np;
-        if (d.b_transposed)
-            HIP_TRY(pack_bt_launch(src, d.ldb, d.K, d.N, c.Kp, c.Np, c.flip_b, d.b_k_interleave, dst, cs, s));
-        else
-            HIP_TRY(pack_b_launch(src, d.ldb, d.K, d.N, c.Kp, c.Np, c.flip_b, d.b_k_interleave, dst, cs, s));
-    }
-    TRY(c.finish_prepare((const int32_t *)biasd, (const int32_t *)multd, (const int32_t *)shiftd, s));
-    // staging buffers are reused by later calls: make sure the copies out of them have finished
+    // staging buffers are reused by later calls, so what was copied through them has to be read before this returns; and a
+    // first prepare ends with the handle's own set-up done. After that, preparing a new B only enqueues.
+    const bool wait = !c.prepared || Bd != B || biasd != bias || (multd != nullptr && multd != mult) || (shiftd != nullptr && shiftd != shift);
+    TRY(c.wait_for_prepare(s));
+    TRY(c.pack(Bd, d.ldb, nb > 1 ? d.b_batch_stride : 0, d.b_transposed != 0, d.b_k_interleave, (const int32_t *)biasd, s));
+    TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));
+    if (!wait)
+        return c.prepare_enqueued(s);
     HIP_TRY(hipStreamSynchronize(s));
+    c.prep_pending = false;
     return 0;
 }
 
@@ -901,6 +995,7 @@ int mi355_gemmlowp_run(mi355_gemm_handle *h, const void *A, const float *bias_f3
     const size_t a_bytes = (size_t)(d.batch - 1) * d.a_batch_stride + (size_t)a_span(d);
     const size_t d_elems = (size_t)(d.batch - 1) * d.d_batch_stride + (size_t)d_span(d);
     const void  *Ad, *bfd;
+    TRY(c.wait_for_prepare(s));
     TRY(to_device(A, a_bytes, h->stageA, s, &Ad, &h->kindA));
     TRY(to_device(bias_f32, sizeof(float) * d.N, h->stageBiasF, s, &bfd, &h->kindBiasF));
     const bool d_host = !h->kindD.is_device(D);
@@ -1026,13 +1121,7 @@ int mi355_gemmlowp_run_noalloc(mi355_gemm_handle *h, const void *A, const float 
     NoallocState               *st = nullptr;
     TRY(noalloc_state(&st));
     // (a stream under graph capture records no event and is not checked: the graph's own order is the caller's)
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess)
-    {
-        (void)hipGetLastError();
-        cap = hipStreamCaptureStatusActive;
-    }
-    const bool tracked = cap == hipStreamCaptureStatusNone;
+    const bool tracked = !GemmCore::capturing(s);
     if (tracked && st->recorded && st->last != s)
     {
         const hipError_t q = hipEventQuery(st->done);
@@ -1044,6 +1133,7 @@ int mi355_gemmlowp_run_noalloc(mi355_gemm_handle *h, const void *A, const float 
         else
             HIP_TRY(q);
     }
+    TRY(c.wait_for_prepare(s));
     c.ext_ws = st->ptr, c.ext_ws_bytes = MI355_NOALLOC_SCRATCH_BYTES, c.ext_ws_used = false;
     const int  rc   = c.run_dense((const int8_t *)A, d.lda, d.a_batch_stride, D, d.ldd, d.d_batch_stride, bias_f32, s);
     const bool used = c.ext_ws_used;
@@ -1369,12 +1459,10 @@ int mi355_conv_prepare(mi355_conv_handle *h, const void *weights, const void *bi
     TRY(to_device(bias, sizeof(int32_t) * c.N, h->stageBias, s, &biasd));
     TRY(to_device(c.rq.per_channel ? mult : nullptr, sizeof(int32_t) * c.N, h->stageMult, s, &multd));
     TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * c.N, h->stageShift, s, &shiftd));
-    TRY(c.Bp.ensure((size_t)c.Np * c.Kp));
-    TRY(c.colsum.ensure(sizeof(int32_t) * (size_t)c.Np));
     // weights [OFM][KH][KW][C] are already the K-contiguous layout with k = c + kx*C + ky*C*KW
     // (src/cpu/kernels/CpuWeightsReshapeKernel.cpp:150-166)
-    HIP_TRY(pack_bt_launch(wd, c.K, c.K, c.N, c.Kp, c.Np, c.flip_b, 0, c.Bp.as<int8_t>(), c.colsum.as<int32_t>(), s));
-    TRY(c.finish_prepare((const int32_t *)biasd, (const int32_t *)multd, (const int32_t *)shiftd, s));
+    TRY(c.pack(wd, c.K, 0, true, 0, (const int32_t *)biasd, s));
+    TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));
     HIP_TRY(hipStreamSynchronize(s));
     return 0;
 }
@@ -1410,7 +1498,7 @@ int mi355_conv_update_quant(mi355_conv_handle *h, int32_t src_offset, int32_t we
         HIP_TRY(hipMemcpyAsync(c.mult.p, multd, sizeof(int32_t) * (size_t)c.N, hipMemcpyDeviceToDevice, s));
         HIP_TRY(hipMemcpyAsync(c.shift.p, shiftd, sizeof(int32_t) * (size_t)c.N, hipMemcpyDeviceToDevice, s));
     }
-    HIP_TRY(fill_i32_launch(c.fill.as<int32_t>(), (int32_t)(0x01010101u * c.fill_byte), 4, s));
+    TRY(c.set_fill(s));
     TRY(c.refresh_colvec(s));
     TRY(c.refresh_qparams(s));
     HIP_TRY(hipStreamSynchronize(s));

@@ -122,19 +122,29 @@ constexpr int SKINNY_MAX_M = 64;
 int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStream_t s, const char **variant = nullptr);
 
 // kernels_aux.hip
-// B [K][ldb] (row-major, N contiguous) -> Bp [Np][Kp] int8 (flip: xor 0x80), colsum[Np] (sums of the packed int8 values)
-int pack_b_launch(const void *B, int64_t ldb, int K, int N, int Kp, int Np, bool flip, int kf, int8_t *Bp, int32_t *colsum,
-                  hipStream_t s);
-// B given as [N][ldk] with K contiguous (conv weights [OFM][KH*KW*C])
-int pack_bt_launch(const void *Bt, int64_t ldk, int K, int N, int Kp, int Np, bool flip, int kf, int8_t *Bp, int32_t *colsum,
-                   hipStream_t s);
-// Bp [Np][Kp] -> operand order for the skinny kernel: [Np/16][Kp/64][64 lanes][16 bytes]
-int pack_b_skinny_launch(const int8_t *Bp, int Kp, int Np, int8_t *Bs, hipStream_t s);
+// What the packing kernels make of a column's sum: colsum[b][Np] and colvec[b][j] = a_off*colsum + a_off*b_off*K (+ bias[j]);
+// bias (nullptr: none) is kept in bias_copy when that is another buffer
+struct ColumnFinish
+{
+    int32_t       *colsum, *colvec;
+    const int32_t *bias;
+    int32_t       *bias_copy;
+    uint32_t       a_off, b_off, K;
+    int32_t        N;
+};
+// nb matrices B [K][ldb] (row-major, N contiguous), b_bs bytes apart -> nb packed images of Np x Kp int8 (flip: xor 0x80)
+// and their columns' sums and terms. skinny: in matrix-core operand order, [Np/16][Kp/64][64 lanes][16 bytes]; else
+// [Np][Kp]. partial: nb * pack_b_splits() * Np words when that function returns more than 1.
+int pack_b_splits(int Kp, int Np, int nb);
+int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
+                  int8_t *out, int32_t *partial, const ColumnFinish &f, hipStream_t s);
+// the same from B given as [N][ldk] with K contiguous (conv weights [OFM][KH*KW*C])
+int pack_bt_launch(const void *Bt, int64_t ldk, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
+                   int8_t *out, const ColumnFinish &f, hipStream_t s);
 // rows 0..63 of Bp -> [64][chunks + 1] pieces of 16 bytes (the last one padding), zero beyond Kp
 int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows, int8_t *Bn, hipStream_t s);
-// colvec[j] = a_off*colsum[j] + a_off*b_off*K (+ bias[j])
-int colvec_launch(const int32_t *colsum, const int32_t *bias, int32_t a_off, int32_t b_off, int K, int N,
-                  int32_t *colvec, hipStream_t s);
+// the terms again from the sums in f.colsum
+int colvec_launch(int Np, int nb, const ColumnFinish &f, hipStream_t s);
 // (multiplier, shift) per column -> qp[QP_COUNT][Np]; *neg != 0 afterwards if any multiplier is negative
 int qparams_launch(const int32_t *mult, const int32_t *shift, int32_t mult_s, int32_t shift_s, int N, int Np,
                    int32_t *qp, int32_t *neg, hipStream_t s);

@@ -3,6 +3,8 @@
 // for cross-checking the matrix-core kernels.
 #include "internal.hpp"
 
+#include <algorithm>
+
 namespace mi355
 {
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -106,7 +108,7 @@ int splitk_finish_launch(int epi, const GemmArgs &g, const int32_t *parts, int64
     return launch_status();
 }
 
-// ---- P1: B[K][ldb] -> Bp[Np][Kp] (transpose to K-contiguous, optional sign flip, zero padding) + column sums ----------
+// ---- P1: B[K][ldb] -> packed B (K contiguous, optional sign flip, zero padding) + column sums + the per-column term -----
 // Replaces pretranspose_B_array (src/cpu/operators/internal/CpuGemmAssemblyDispatch.cpp:594-617) / CpuGemmTranspose1xWKernel and
 // CpuGemmLowpMatrixBReductionKernel (src/cpu/kernels/CpuGemmLowpMatrixReductionKernel.cpp:273-446) in one pass over B.
 // kf > 1 re-orders K on the way: packed row k = a*kf + b (b < kf) is source row b*(K/kf) + a, which is what
@@ -117,130 +119,208 @@ __device__ __forceinline__ int k_source(int k, int K, int kf)
     return kf > 1 ? (k % kf) * (K / kf) + k / kf : k;
 }
 
-__global__ __launch_bounds__(256) void pack_b_kernel(const uint8_t *__restrict__ B, int64_t ldb, int K, int N, int Kp,
-                                                     uint8_t flip, int kf, int8_t *__restrict__ Bp,
-                                                     int32_t *__restrict__ colsum)
+// colvec[j] = a_off*colsum[j] + a_off*b_off*K (+ bias[j]); the per-column part of the offset contribution, folded with the
+// bias like arm_gemm's col_bias (src/core/NEON/kernels/arm_gemm/quantized.cpp:963-968). bias_copy keeps the bias for a later
+// change of the offsets.
+__device__ __forceinline__ void finish_column(const ColumnFinish &f, int Np, int b, int j, int32_t sum)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t tile[64][64 + 16]; // [n][k]
-    const int          n0 = blockIdx.x * 64, k0 = blockIdx.y * 64;
-    const int          tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk)
+    f.colsum[(int64_t)b * Np + j] = sum;
+    if (j >= f.N)
+        return;
+    uint32_t v = f.a_off * (uint32_t)sum + f.a_off * f.b_off * f.K;
+    if (f.bias)
     {
-        const int k = k0 + ty * 16 + kk, n = n0 + tx;
-        uint8_t   v = 0;
-        if (k < K && n < N)
-            v = B[(int64_t)k_source(k, K, kf) * ldb + n] ^ flip;
-        tile[tx][ty * 16 + kk] = v;
+        const int32_t x = f.bias[j];
+        v += (uint32_t)x;
+        if (b == 0 && f.bias_copy != f.bias)
+            f.bias_copy[j] = x;
     }
-    __syncthreads();
-    const int n = threadIdx.x >> 2, kc = (threadIdx.x & 3) * 16;
-    const v4i v = *(const v4i *)&tile[n][kc];
-    *(v4i *)(Bp + (int64_t)(n0 + n) * Kp + k0 + kc) = v;
-    int32_t s = sum4_i8(v.x) + sum4_i8(v.y) + sum4_i8(v.z) + sum4_i8(v.w);
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    if ((threadIdx.x & 3) == 0 && s != 0)
-        atomicAdd(colsum + n0 + n, s);
+    f.colvec[(int64_t)b * Np + j] = (int32_t)v;
 }
 
-int pack_b_launch(const void *B, int64_t ldb, int K, int N, int Kp, int Np, bool flip, int kf, int8_t *Bp,
-                  int32_t *colsum, hipStream_t s)
+// Where piece kc / 16 (16 bytes along K) of column n goes: K-contiguous rows, or the 1 KiB blocks of 16 columns x 64 k in the
+// lane order in which the 16x16x64 matrix instruction reads its B operand (lane l: column l % 16, bytes 16 * (l / 16) ..
+// + 16 of the k block), one block after the other along K
+template <bool SKINNY>
+__device__ __forceinline__ int64_t packed_offset(int n, int kc, int Kp)
 {
-    if (Np % 64 || Kp % 64 || Np < N || Kp < K || (kf > 1 && K % kf != 0))
+    if (SKINNY)
+        return ((int64_t)(n >> 4) * (Kp >> 6) + (kc >> 6)) * 1024 + (((kc >> 4) & 3) * 16 + (n & 15)) * 16;
+    return (int64_t)n * Kp + kc;
+}
+
+// A workgroup packs 64 columns x a run of 128-deep K tiles of one batch entry. A thread fetches 8 columns of 4 rows (any
+// alignment: the hardware takes unaligned 8-byte loads), turns each 4 x 4 block of bytes round in registers (8 byte
+// permutes) and the tile leaves through LDS as whole 128-byte rows (piece c of column n lies at c ^ (n / 8), so that the
+// dword writes of a wave spread over the banks). All batch entries go out in one launch, and where a workgroup walks the
+// whole K (splits = 1) it finishes its columns' sums itself: packing a new B is one launch. Bound by HBM (1 byte read and
+// 1 written per element). One byte per lane and load, an LDS tile of bytes and one atomic per column and tile took 17.8 us
+// at 4096 x 4096, plus a second pass of 18 us into the streaming kernel's order; this form 11.5 + 6 us (sums) in either
+// order. 32 entries of 512 x 128, prepare and run together: 338 us as three launches per entry, 15.2 us now.
+template <bool SKINNY>
+__global__ __launch_bounds__(256) void pack_b_kernel(const uint8_t *__restrict__ B, int64_t ldb, int64_t b_bs, int K, int N, int Kp,
+                                                     int Np, uint32_t flip4, int kf, int tiles_per_split, int8_t *__restrict__ out,
+                                                     int32_t *__restrict__ partial, ColumnFinish f)
+{
+    __shared__ v4i     tile[64 * 8];
+    __shared__ int32_t csum[64];
+    const int          b = blockIdx.z, n0 = blockIdx.x * 64, tid = threadIdx.x;
+    const int          nq = tid & 7, kq = tid >> 3, n = n0 + nq * 8;
+    B += (int64_t)b * b_bs;
+    out += (int64_t)b * Np * Kp;
+    if (tid < 64)
+        csum[tid] = 0;
+    const int kt0 = blockIdx.y * tiles_per_split, kt1 = min(kt0 + tiles_per_split, Kp / 128);
+    int       row[2], piece[2];
+    int32_t   sum[2] = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+    {
+        const int idx = tid + 256 * j, blk = idx >> 6, lane = idx & 63;
+        row[j]   = SKINNY ? (blk >> 1) * 16 + (lane & 15) : idx >> 3;
+        piece[j] = SKINNY ? (blk & 1) * 4 + (lane >> 4) : idx & 7;
+    }
+    for (int kt = kt0; kt < kt1; ++kt)
+    {
+        const int k0 = kt * 128;
+        uint32_t  w[4][2];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            const int k = k0 + kq * 4 + r;
+            w[r][0] = 0, w[r][1] = 0;
+            if (k >= K || n >= N)
+                continue;
+            const uint8_t *p = B + (int64_t)k_source(k, K, kf) * ldb + n;
+            if (n + 8 <= N)
+            {
+                __builtin_memcpy(w[r], p, 8);
+                w[r][0] ^= flip4, w[r][1] ^= flip4;
+            }
+            else
+                for (int t = 0; t < N - n; ++t)
+                    w[r][t >> 2] |= (uint32_t)(uint8_t)(p[t] ^ (uint8_t)flip4) << (8 * (t & 3));
+        }
+        if (kt > kt0)
+            __syncthreads(); // the tile before this one has left LDS
+        uint32_t *lds = (uint32_t *)tile + (nq * 8) * 32 + (((kq >> 2) ^ nq) << 2) + (kq & 3);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+        {
+            const uint32_t lo01 = __builtin_amdgcn_perm(w[1][h], w[0][h], 0x05010400), hi01 = __builtin_amdgcn_perm(w[1][h], w[0][h], 0x07030602);
+            const uint32_t lo23 = __builtin_amdgcn_perm(w[3][h], w[2][h], 0x05010400), hi23 = __builtin_amdgcn_perm(w[3][h], w[2][h], 0x07030602);
+            lds[(h * 4 + 0) * 32] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100);
+            lds[(h * 4 + 1) * 32] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302);
+            lds[(h * 4 + 2) * 32] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100);
+            lds[(h * 4 + 3) * 32] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+        {
+            const v4i v = tile[row[j] * 8 + (piece[j] ^ ((row[j] >> 3) & 7))];
+            *(v4i *)(out + packed_offset<SKINNY>(n0 + row[j], k0 + piece[j] * 16, Kp)) = v;
+            sum[j] += sum4_i8(v.x) + sum4_i8(v.y) + sum4_i8(v.z) + sum4_i8(v.w);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        atomicAdd(&csum[row[j]], sum[j]);
+    __syncthreads();
+    if (tid >= 64)
+        return;
+    if (partial)
+        partial[((int64_t)b * gridDim.y + blockIdx.y) * Np + n0 + tid] = csum[tid];
+    else
+        finish_column(f, Np, b, n0 + tid, csum[tid]);
+}
+
+// sums the K runs of pack_b_kernel
+__global__ __launch_bounds__(256) void colsum_finish_kernel(const int32_t *__restrict__ partial, int splits, int Np, ColumnFinish f)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
+    if (j >= Np)
+        return;
+    int32_t sum = 0;
+    for (int i = 0; i < splits; ++i)
+        sum += partial[((int64_t)b * splits + i) * Np + j];
+    finish_column(f, Np, b, j, sum);
+}
+
+// K runs of a packing launch: about four workgroups per compute unit (4096 x 4096: 15 runs)
+int pack_b_splits(int Kp, int Np, int nb)
+{
+    const int64_t columns = (int64_t)(Np / 64) * nb, tiles = Kp / 128;
+    return (int)std::max<int64_t>(1, std::min<int64_t>(tiles, 1024 / columns));
+}
+
+int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
+                  int8_t *out, int32_t *partial, const ColumnFinish &f, hipStream_t s)
+{
+    if (Np % 64 || Kp % 128 || Np < N || Kp < K || nb < 1 || nb > 65535 || (kf > 1 && K % kf != 0))
         return (int)hipErrorInvalidValue;
-    int e = fill_i32_launch(colsum, 0, Np, s);
-    if (e)
-        return e;
-    pack_b_kernel<<<dim3(Np / 64, Kp / 64), dim3(256), 0, s>>>((const uint8_t *)B, ldb, K, N, Kp, flip ? 0x80 : 0, kf,
-                                                               Bp, colsum);
+    const int tiles = Kp / 128, want = pack_b_splits(Kp, Np, nb), per = (tiles + want - 1) / want, splits = (tiles + per - 1) / per;
+    if (splits > 1 && partial == nullptr)
+        return (int)hipErrorInvalidValue;
+    const dim3 grid(Np / 64, splits, nb), block(256);
+    int32_t   *pt = splits > 1 ? partial : nullptr;
+    if (skinny)
+        pack_b_kernel<true><<<grid, block, 0, s>>>((const uint8_t *)B, ldb, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, per, out, pt, f);
+    else
+        pack_b_kernel<false><<<grid, block, 0, s>>>((const uint8_t *)B, ldb, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, per, out, pt, f);
+    if (splits > 1)
+        colsum_finish_kernel<<<dim3((Np + 255) / 256, nb), dim3(256), 0, s>>>(partial, splits, Np, f);
     return launch_status();
 }
 
 // B already K-contiguous: Bt[N][ldk] (convolution weights [OFM][KH*KW*C], the layout CpuWeightsReshapeKernel
-// produces transposed: src/cpu/kernels/CpuWeightsReshapeKernel.cpp:150-166)
-__global__ __launch_bounds__(256) void pack_bt_kernel(const uint8_t *__restrict__ Bt, int64_t ldk, int K, int N, int Kp,
-                                                      int Np, uint8_t flip, int kf, int8_t *__restrict__ Bp,
-                                                      int32_t *__restrict__ colsum)
+// produces transposed: src/cpu/kernels/CpuWeightsReshapeKernel.cpp:150-166). One wave per packed row, so a row's sum needs
+// no other wave.
+template <bool SKINNY>
+__global__ __launch_bounds__(256) void pack_bt_kernel(const uint8_t *__restrict__ Bt, int64_t ldk, int64_t b_bs, int K, int N, int Kp,
+                                                      int Np, uint32_t flip4, int kf, int8_t *__restrict__ out, ColumnFinish f)
 {
-    const int     cpr = Kp / 16;
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)Np * cpr)
-        return;
-    const int n = (int)(idx / cpr), kc = (int)(idx % cpr) * 16;
-    union
-    {
-        v4i     v;
-        uint8_t b[16];
-    } u;
+    const int b = blockIdx.y, n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    out += (int64_t)b * Np * Kp;
+    const uint8_t *row = Bt + (int64_t)b * b_bs + (int64_t)n * ldk;
     int32_t        s   = 0;
-    const uint8_t *row = Bt + (int64_t)n * ldk + kc;
-    if (n < N && kc + 16 <= K && (((uintptr_t)row) & 15) == 0 && kf <= 1)
+    for (int kc = lane * 16; kc < Kp; kc += 64 * 16)
     {
-        // whole aligned 16-byte piece of a row
-        u.v = *(const v4i *)row;
-        const int f4 = (int)(flip * 0x01010101u);
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-            u.v[t] ^= f4;
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
-            s += (int8_t)u.b[t];
-    }
-    else
-    {
-#pragma unroll
-        for (int t = 0; t < 16; ++t)
+        uint32_t w[4] = {0, 0, 0, 0};
+        if (n < N && kc + 16 <= K && kf <= 1)
         {
-            uint8_t x = 0;
-            if (n < N && kc + t < K)
-                x = Bt[(int64_t)n * ldk + k_source(kc + t, K, kf)] ^ flip;
-            u.b[t] = x;
-            s += (int8_t)x;
+            __builtin_memcpy(w, row + kc, 16);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                w[t] ^= flip4;
         }
+        else if (n < N)
+        {
+#pragma unroll
+            for (int t = 0; t < 16; ++t)
+                if (kc + t < K)
+                    w[t >> 2] |= (uint32_t)(uint8_t)(row[k_source(kc + t, K, kf)] ^ (uint8_t)flip4) << (8 * (t & 3));
+        }
+        s += sum4_i8((int)w[0]) + sum4_i8((int)w[1]) + sum4_i8((int)w[2]) + sum4_i8((int)w[3]);
+        *(v4i *)(out + packed_offset<SKINNY>(n, kc, Kp)) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     }
-    *(v4i *)(Bp + (int64_t)n * Kp + kc) = u.v;
-    if (s != 0)
-        atomicAdd(colsum + n, s);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        s += __shfl_xor(s, o);
+    if (lane == 0)
+        finish_column(f, Np, b, n, s);
 }
 
-int pack_bt_launch(const void *Bt, int64_t ldk, int K, int N, int Kp, int Np, bool flip, int kf, int8_t *Bp,
-                   int32_t *colsum, hipStream_t s)
+int pack_bt_launch(const void *Bt, int64_t ldk, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
+                   int8_t *out, const ColumnFinish &f, hipStream_t s)
 {
-    if (Kp % 16 || Np < N || Kp < K || (kf > 1 && K % kf != 0))
+    if (Np % 4 || Kp % 64 || Np < N || Kp < K || nb < 1 || nb > 65535 || (kf > 1 && K % kf != 0))
         return (int)hipErrorInvalidValue;
-    int e = fill_i32_launch(colsum, 0, Np, s);
-    if (e)
-        return e;
-    const int64_t total = (int64_t)Np * (Kp / 16);
-    pack_bt_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s>>>((const uint8_t *)Bt, ldk, K, N, Kp, Np,
-                                                                               flip ? 0x80 : 0, kf, Bp, colsum);
-    return launch_status();
-}
-
-// Bp[Np][Kp] -> Bs[Np/16][Kp/64][64][16]: 1 KiB blocks holding 16 columns x 64 k in the lane order the 16x16x64 matrix
-// instruction reads its B operand (lane l: column l%16, bytes 16*(l/16) .. +16 of the k block)
-__global__ __launch_bounds__(256) void pack_b_skinny_kernel(const int8_t *__restrict__ Bp, int Kp, int Np,
-                                                            int8_t *__restrict__ Bs)
-{
-    const int64_t idx   = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t total = (int64_t)Np * Kp / 16;
-    if (idx >= total)
-        return;
-    const int     lane = (int)(idx & 63);
-    const int64_t blk  = idx >> 6;
-    const int     KB   = Kp / 64;
-    const int     kb = (int)(blk % KB), ng = (int)(blk / KB);
-    const int     col = lane & 15, kc = lane >> 4;
-    *(v4i *)(Bs + idx * 16) = *(const v4i *)(Bp + (int64_t)(ng * 16 + col) * Kp + kb * 64 + kc * 16);
-}
-
-int pack_b_skinny_launch(const int8_t *Bp, int Kp, int Np, int8_t *Bs, hipStream_t s)
-{
-    if (Kp % 64 || Np % 16)
-        return (int)hipErrorInvalidValue;
-    const int64_t total = (int64_t)Np * Kp / 16;
-    pack_b_skinny_kernel<<<dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s>>>(Bp, Kp, Np, Bs);
+    const dim3 grid(Np / 4, nb), block(256);
+    if (skinny)
+        pack_bt_kernel<true><<<grid, block, 0, s>>>((const uint8_t *)Bt, ldk, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, out, f);
+    else
+        pack_bt_kernel<false><<<grid, block, 0, s>>>((const uint8_t *)Bt, ldk, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, out, f);
     return launch_status();
 }
 
@@ -313,25 +393,19 @@ int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows,
     return launch_status();
 }
 
-// colvec[j] = a_off*colsum[j] + a_off*b_off*K (+ bias[j]); the per-column part of the offset contribution, folded with the
-// bias like arm_gemm's col_bias (src/core/NEON/kernels/arm_gemm/quantized.cpp:963-968)
-__global__ void colvec_kernel(const int32_t *__restrict__ colsum, const int32_t *__restrict__ bias, uint32_t a_off,
-                              uint32_t b_off, uint32_t K, int N, int32_t *__restrict__ colvec)
+// the per-column term again from the column sums that are there (new offsets), all batch entries in one launch
+__global__ __launch_bounds__(256) void colvec_kernel(int Np, ColumnFinish f)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N)
-        return;
-    uint32_t v = a_off * (uint32_t)colsum[j] + a_off * b_off * K;
-    if (bias)
-        v += (uint32_t)bias[j];
-    colvec[j] = (int32_t)v;
+    const int j = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
+    if (j < f.N)
+        finish_column(f, Np, b, j, f.colsum[(int64_t)b * Np + j]);
 }
 
-int colvec_launch(const int32_t *colsum, const int32_t *bias, int32_t a_off, int32_t b_off, int K, int N,
-                  int32_t *colvec, hipStream_t s)
+int colvec_launch(int Np, int nb, const ColumnFinish &f, hipStream_t s)
 {
-    colvec_kernel<<<dim3((N + 255) / 256), dim3(256), 0, s>>>(colsum, bias, (uint32_t)a_off, (uint32_t)b_off,
-                                                              (uint32_t)K, N, colvec);
+    if (nb < 1 || nb > 65535)
+        return (int)hipErrorInvalidValue;
+    colvec_kernel<<<dim3((f.N + 255) / 256, nb), dim3(256), 0, s>>>(Np, f);
     return launch_status();
 }
 
