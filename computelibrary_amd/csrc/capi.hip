@@ -182,7 +182,9 @@ struct GemmCore
     mi355_requant qp_rq{};
     int     splitk = 1;      // K slices of the pipelined kernel
     int     splitk_plan = 1; // what the cost model chose with the tile shape (create()); prepare() checks it and allocates
-    bool    conv_core = false; // the GEMM inside a convolution handle
+    int         patch_c = 0, patch_c_true = 0; // a convolution's channels in the kernels' K, and how many of them count (0: dense)
+    const void *rs_src = nullptr; // conv_row_terms
+    ConvGeom    rs_geom{};
     int     k_const = 0;       // > 0: the K of the constant term a_offset * b_offset * K, where the kernels' K counts padded channels
     bool    qp_on = false; // the digested requantisation vectors (and the flag word behind them) exist
     std::string kname_mfma, kname_dma, kprefix;
@@ -432,13 +434,13 @@ struct GemmCore
             HIP_TRY(hipMemcpyAsync(shift.p, shift_in, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s));
         }
         // few output columns and a short K: the image of the B panel the narrow kernel copies into LDS
-        has_narrow = path == MI355_PATH_MFMA && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192)) && narrow_panel_chunks(K) > 0;
+        has_narrow = path == MI355_PATH_MFMA && patch_c > 0 && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192)) && narrow_panel_chunks(K) > 0;
         if (has_narrow)
         {
             const int chunks = narrow_panel_chunks(K);
             const int rows = round_up(N, 64); // panels of 64 columns (Np, a multiple of 256, covers them)
             TRY(Bn.ensure((size_t)rows * (chunks + NARROW_PAD_PIECES) * 16));
-            HIP_TRY(pack_b_narrow_launch(Bp.as<int8_t>(), Kp, Np, chunks, rows, Bn.as<int8_t>(), s));
+            HIP_TRY(pack_b_narrow_launch(Bp.as<int8_t>(), Kp, Np, chunks, rows, K, patch_c, patch_c_true, Bn.as<int8_t>(), s));
         }
         TRY(set_fill(s));
         if (path == MI355_PATH_SKINNY && zeros.p == nullptr)
@@ -564,10 +566,11 @@ struct GemmCore
         const bool direct =
             path == MI355_PATH_SIMPLE || ((((uintptr_t)A | (uintptr_t)lda | (uintptr_t)a_bs) & 3) == 0);
         // the per-row term b_offset * rowsum(A): the pipelined kernels sum the rows of A themselves while its tiles pass
-        // through them (dword-aligned rows, K a whole number of 16-byte columns, one launch); otherwise one pass over A
+        // through them (dword-aligned rows, K a whole number of 16-byte columns; under K slices every slice its part, which
+        // the float epilogue could not take apart again); otherwise one pass over A
         // in front of the GEMM leaves the sums in a vector
         const bool rowsum_in_kernel = b_off_eff() != 0 && direct && path == MI355_PATH_MFMA && dma_idx >= 0 && K % 16 == 0 && K >= 16 &&
-                                      splitk == 1 && (int64_t)lda * 256 + K < ((int64_t)1 << 32);
+                                      (splitk == 1 || epi != EPI_F32) && (int64_t)lda * 256 + K < ((int64_t)1 << 32);
         const bool need_rowvec = b_off_eff() != 0 && !rowsum_in_kernel;
         // the two workspaces of a run: owned by the handle and grown on demand, or carved out of a buffer the caller of
         // this function brings (ext_ws != nullptr: nothing is allocated, sizes beyond ext_ws_bytes are an error)
@@ -626,6 +629,16 @@ struct GemmCore
         g.epi.vec_store16 = (esz == 1 && ((uintptr_t)g.D % 16) == 0 && g.ldd % 16 == 0 && g.d_batch_stride % 16 == 0) ? 1 : 0;
     }
 
+    // The row terms of a convolution by a pass over the source (rs_src, rs_geom: the caller's channel count), for the kernels
+    // that do not sum the patches themselves
+    int conv_row_terms(GemmArgs &g, hipStream_t s)
+    {
+        TRY(rowvec.ensure(sizeof(int32_t) * (size_t)M));
+        HIP_TRY(conv_rowsum_launch(rs_src, rs_geom, M, flip_a, g.epi.rowsum_mul, rowvec.as<int32_t>(), s));
+        g.epi.rowvec = rowvec.as<int32_t>(), g.epi.rowsum_mul = 0;
+        return 0;
+    }
+
     int launch(GemmArgs &g, bool flip_in_loader, bool conv, hipStream_t s)
     {
         if (path == MI355_PATH_SIMPLE)
@@ -669,12 +682,12 @@ struct GemmCore
                                       : (int64_t)g.lda * 256 + g.K;
             // few output columns and a short K: every wave for itself, weights resident in LDS (gemm_narrow.hip)
             if (has_narrow && batch == 1 && conv && !g.epi.accumulate && span < ((int64_t)1 << 31) &&
-                narrow_applies(g, conv))
+                narrow_applies(g))
             {
                 g.Bp            = Bn.as<int8_t>();
                 g.conv.pad_word = 0x01010101u * fill_byte; // as in the image: the kernel flips what it loads
                 bool band       = false;
-                HIP_TRY(narrow_launch(epi, flip_in_loader, conv, g, s, &band));
+                HIP_TRY(narrow_launch(epi, flip_in_loader, g, s, &band));
                 kname_run = band ? &kname_band : &kname_narrow;
             }
             else if (dma_idx >= 0 && aligned && g.K >= 16 && span < ((int64_t)1 << 32))
@@ -685,6 +698,9 @@ struct GemmCore
                 kname_run          = &kname_dma_full;
                 if (splitk > 1 && batch == 1 && g.K == K && K % (splitk * c.BK) == 0)
                 {
+                    // the float epilogue rounds the product and the offset terms apart: they must not meet in the planes
+                    if (conv && epi == EPI_F32 && g.epi.rowsum_mul != 0)
+                        TRY(conv_row_terms(g, s));
                     const int     ldp = (N + 3) & ~3;
                     const int64_t kc  = K / splitk;
                     GemmArgs      gp  = g;
@@ -692,6 +708,7 @@ struct GemmCore
                     gp.epi.colvec              = zerocol.as<int32_t>();
                     gp.epi.colvec_batch_stride = 0;
                     gp.epi.vec_store           = 1;
+                    gp.epi.rowsum_mul          = g.epi.rowsum_mul; // every slice adds its own part of the row terms
                     gp.D = parts.as<int32_t>(), gp.ldd = ldp, gp.d_batch_stride = (int64_t)M * ldp;
                     // (dense: a slice starts kc bytes into every row of A; convolution: kc values into every patch,
                     // which the loader adds to the k it decodes)
@@ -709,6 +726,8 @@ struct GemmCore
                 g.tiles_m          = (g.M + c.BM - 1) / c.BM;
                 g.tiles_n          = (g.N + c.BN - 1) / c.BN;
                 kname_run          = &kname_mfma_full;
+                if (conv && g.epi.rowsum_mul != 0)
+                    TRY(conv_row_terms(g, s));
                 if (conv)
                     g.conv.pad_word = (0x01010101u * fill_byte) ^ (flip_in_loader ? 0x80808080u : 0u);
                 HIP_TRY(mfma_launch(cfg_idx, epi, flip_in_loader, conv, g, batch, s));
@@ -1363,6 +1382,7 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
     // channel count: the row sums of the patches (needed under a weights offset) are taken from the unpadded source,
     // and the constant a_offset * b_offset * K uses the unpadded K.
     h->geom_true = h->geom;
+    h->geom.c_true = h->geom_true.c_true = d.C;
     {
         if (d.path == MI355_CONV_AUTO && d.C % 16 != 0)
         {
@@ -1371,7 +1391,7 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
             ConvGeom gp;
             conv_geom(dp, gp);
             if (conv_fast_div_ok(dp, gp) && conv_fast_div_ok(d, h->geom) && (int64_t)d.batch * d.H * d.W * dp.C < ((int64_t)1 << 31))
-                h->c_pad = dp.C, h->geom = gp;
+                h->c_pad = dp.C, gp.c_true = d.C, h->geom = gp;
         }
     }
     const int     c_eff = h->c_pad ? h->c_pad : d.C;
@@ -1382,8 +1402,9 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
         delete h;
         return fail("convolution too large");
     }
-    c.M = (int)M64, c.N = d.OFM, c.K = (int)K64, c.batch = 1, c.conv_core = true;
+    c.M = (int)M64, c.N = d.OFM, c.K = (int)K64, c.batch = 1;
     c.k_const = h->c_pad ? d.KH * d.KW * d.C : 0;
+    c.patch_c = h->geom.C, c.patch_c_true = h->geom.c_true;
     c.epi = f32 ? EPI_F32 : EPI_FIXEDPOINT, c.dst_dtype = d.dst_dtype;
     c.flip_a = d.src_dtype == MI355_U8, c.flip_b = d.weights_dtype == MI355_U8;
     c.a_offset = d.src_offset, c.b_offset = d.weights_offset;
@@ -1588,14 +1609,11 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
     {
         GemmArgs g{};
         c.fill_epi(g.epi, h->has_bias_f32 ? h->biasF.as<float>() : nullptr);
-        if (c.b_off_eff() != 0)
-        {
-            ConvGeom gr = h->c_pad ? h->geom_true : h->geom;
-            gr.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
-            TRY(c.rowvec.ensure(sizeof(int32_t) * (size_t)c.M));
-            HIP_TRY(conv_rowsum_launch(h->c_pad ? src_true : srcd, gr, c.M, c.flip_a, c.b_off_eff(), c.rowvec.as<int32_t>(), s));
-            g.epi.rowvec = c.rowvec.as<int32_t>();
-        }
+        // a weights offset: the kernels sum the patches as they pass (see conv_row_terms for those that do not)
+        g.epi.rowsum_mul   = c.b_off_eff();
+        c.rs_src           = h->c_pad ? src_true : srcd;
+        c.rs_geom          = h->c_pad ? h->geom_true : h->geom;
+        c.rs_geom.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
         g.A = (const int8_t *)srcd, g.lda = 0, g.a_batch_stride = 0;
         g.Bp = c.Bp.as<int8_t>(), g.Kp = c.Kp, g.bp_batch_stride = 0;
         g.D = Dd, g.ldd = c.N, g.d_batch_stride = 0;

@@ -1,4 +1,4 @@
-// K5: implicit-GEMM convolution (and dense GEMM) with few output columns: N <= 64, K <= 1152 - or, with K <= 192, up to
+// K5: implicit-GEMM convolution with few output columns: N <= 64, K <= 1152 - or, with K <= 192, up to
 // 256 columns as 2 to 4 panels of 64 (a 1 x 1 convolution that widens few channels: the patch of a wave stays in its
 // registers and goes against one panel after the other, every panel with its own epilogue).
 //
@@ -59,6 +59,16 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t x)
            (uint32_t)__builtin_amdgcn_readlane((int)x, 47) | (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
 }
 
+// k block kb of the row of ones that lies in the padding of the panel's rows (see pack_b_narrow_kernel), as a matrix
+// operand: every one of its 16 rows is the same, so the product with a block of A is that block's row sums - in every lane,
+// for the row the lane's accumulators belong to. Bytes of the patch that do not count are zeros in it.
+template <int PITCH, int KBLK>
+__device__ __forceinline__ v4i ones_block(const char *panel, int kb, int lh)
+{
+    static_assert(NARROW_PAD_PIECES == 2 && KBLK * 4 <= 64 * NARROW_PAD_PIECES, "two pieces of the row per row of the panel");
+    return *(const v4i *)(panel + (kb * 2 + (lh >> 1)) * PITCH + KBLK * 64 + (lh & 1) * 16);
+}
+
 constexpr int NARROW_WAVES  = 4;
 constexpr int NARROW_ROWS   = 32;  // per wave
 constexpr int NARROW_BN     = 64;
@@ -67,7 +77,9 @@ constexpr int NARROW_MAX_PANELS = 4; // panels of 64 columns with one batch (K <
                                      // workgroup's weights and measured slower than the tiled kernel)
 
 // UNI: C % 64 == 0 - a k block of 64 lies inside one tap, so the tap of a load is decoded with scalar arithmetic
-template <int EPI, bool FLIP_A, bool CONV, bool UNI, int NB>
+// ROWSUM: weights with an offset - the row sums of the patches come from one more matrix instruction per operand block,
+// against a block of ones (see ones_block)
+template <int EPI, bool FLIP_A, bool UNI, int NB, bool ROWSUM>
 // (4 waves per SIMD, i.e. 4 workgroups per compute unit: at most 128 registers per lane)
 __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_narrow_kernel(GemmArgs g)
 {
@@ -85,13 +97,13 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     uintptr_t u_a = (uintptr_t)g.A, u_b = (uintptr_t)g.Bp, u_cv = (uintptr_t)g.epi.colvec, u_qp = (uintptr_t)g.epi.qp,
               u_fl = (uintptr_t)g.epi.qp_flag;
     uint32_t  a_bytes = (uint32_t)(g.a_end - g.A); // bytes of A: what the range check of the A loads compares with
-    int32_t   a_M = g.M, a_K = g.K, a_lda = (int32_t)g.lda, a_kp = (int32_t)g.Kp, a_qps = (int32_t)g.epi.qp_stride;
+    int32_t   a_M = g.M, a_K = g.K, a_kp = (int32_t)g.Kp, a_qps = (int32_t)g.epi.qp_stride;
     int32_t   tail_start = g.tiles_m, tail_waves = g.tiles_n; // see narrow_launch
     int32_t   a_npan = g.nblocks;                             // panels of 64 columns (more than one only with NB == 1)
     asm volatile(""
                  : "+s"(cg.H), "+s"(cg.W), "+s"(cg.C), "+s"(cg.KW), "+s"(cg.OW), "+s"(cg.OH), "+s"(cg.stride_x), "+s"(cg.stride_y),
                    "+s"(cg.pad_left), "+s"(cg.pad_top), "+s"(cg.dil_x), "+s"(cg.dil_y), "+s"(cg.pad_word), "+s"(cg.magic_C),
-                   "+s"(cg.magic_KW), "+s"(cg.magic_OW), "+s"(cg.magic_OH), "+s"(a_M), "+s"(a_K), "+s"(a_lda), "+s"(a_kp),
+                   "+s"(cg.magic_KW), "+s"(cg.magic_OW), "+s"(cg.magic_OH), "+s"(a_M), "+s"(a_K), "+s"(a_kp),
                    "+s"(a_qps), "+s"(u_a), "+s"(u_b), "+s"(u_cv), "+s"(u_qp), "+s"(u_fl), "+s"(a_bytes), "+s"(tail_start), "+s"(tail_waves),
                    "+s"(a_npan));
     const int npan = NB == 1 ? a_npan : 1; // (a constant for the deeper forms: their code does not change)
@@ -188,21 +200,13 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     for (int rb = 0; rb < RS; ++rb)
     {
         const int gr = min(row0 + rb * 16 + lr, a_M - 1);
-        if (CONV)
-        {
-            const int t  = narrow_div(gr, cg.magic_OW);
-            const int ox = gr - t * cg.OW;
-            const int n  = narrow_div(t, cg.magic_OH);
-            const int oy = t - n * cg.OH;
-            iy0[rb]      = oy * cg.stride_y - cg.pad_top;
-            ix0[rb]      = ox * cg.stride_x - cg.pad_left;
-            pix[rb]      = n * (cg.H * cg.W * cg.C) + (iy0[rb] * cg.W + ix0[rb]) * cg.C;
-        }
-        else
-        {
-            iy0[rb] = ix0[rb] = 0;
-            pix[rb]           = gr * a_lda;
-        }
+        const int t  = narrow_div(gr, cg.magic_OW);
+        const int ox = gr - t * cg.OW;
+        const int n  = narrow_div(t, cg.magic_OH);
+        const int oy = t - n * cg.OH;
+        iy0[rb]      = oy * cg.stride_y - cg.pad_top;
+        ix0[rb]      = ox * cg.stride_x - cg.pad_left;
+        pix[rb]      = n * (cg.H * cg.W * cg.C) + (iy0[rb] * cg.W + ix0[rb]) * cg.C;
     }
     // A piece outside the image is replaced by the padding value when it is used; its load goes out all the same (inside
     // the tensor it reads a neighbouring pixel, outside it reads zero). Past K the value is irrelevant: B is zero there.
@@ -214,26 +218,22 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     auto tap_of = [&](int kb, int &dy, int &dx, int &off)
     {
         const int k = kb * 64 + lh * 16;
-        dy = 0, dx = 0, off = k;
-        if (CONV)
+        int       tap, c0;
+        if (UNI)
         {
-            int tap, c0;
-            if (UNI)
-            {
-                tap = narrow_div(kb * 64, cg.magic_C); // scalar
-                c0  = kb * 64 - tap * cg.C + lh * 16;
-            }
-            else
-            {
-                tap = narrow_div(k, cg.magic_C);
-                c0  = k - tap * cg.C;
-            }
-            const int ky = narrow_div(tap, cg.magic_KW);
-            const int kx = tap - ky * cg.KW;
-            dy           = ky * cg.dil_y;
-            dx           = kx * cg.dil_x;
-            off          = (dy * cg.W + dx) * cg.C + c0;
+            tap = narrow_div(kb * 64, cg.magic_C); // scalar
+            c0  = kb * 64 - tap * cg.C + lh * 16;
         }
+        else
+        {
+            tap = narrow_div(k, cg.magic_C);
+            c0  = k - tap * cg.C;
+        }
+        const int ky = narrow_div(tap, cg.magic_KW);
+        const int kx = tap - ky * cg.KW;
+        dy           = ky * cg.dil_y;
+        dx           = kx * cg.dil_x;
+        off          = (dy * cg.W + dx) * cg.C + c0;
     };
     auto load_a = [&](int slot, int batch)
     {
@@ -249,8 +249,6 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     };
     auto mask_a = [&](int slot, int batch)
     {
-        if (!CONV)
-            return;
         oob &= ~(((1u << (3 * RS)) - 1u) << (slot * 3 * RS));
 #pragma unroll
         for (int kk = 0; kk < 3; ++kk)
@@ -299,6 +297,11 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     // in fa[0]); every panel has its own accumulators and epilogue
     for (int np = 0; np < npan; ++np)
     {
+    int32_t rsum[RS];
+    v4i     asum[RS]; // the row sums: the same in all four registers of a lane
+#pragma unroll
+    for (int rb = 0; rb < RS; ++rb)
+        rsum[rb] = 0, asum[rb] = (v4i){0, 0, 0, 0};
     const int col0 = np * NARROW_BN;
     v4i       acc[RS][QS];
 #pragma unroll
@@ -317,6 +320,9 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
             // the panel - skip them, every panel would multiply them again)
             if (NB == 1 && kk > 0 && kk * 64 >= a_K)
                 continue;
+            v4i ones;
+            if constexpr (ROWSUM)
+                ones = ones_block<PITCH, KBLK>(smem, b * 3 + kk, lh);
             v4i fb[QS];
 #pragma unroll
             for (int q = 0; q < QS; ++q)
@@ -325,7 +331,7 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
             for (int rb = 0; rb < RS; ++rb)
             {
                 v4i a = fa[b & 1][kk][rb];
-                if (CONV && (oob_wave & (1u << (((b & 1) * 3 + kk) * RS + rb))))
+                if ((oob_wave & (1u << (((b & 1) * 3 + kk) * RS + rb))))
                 {
                     // (the asm keeps this a branch - as selects it would cost every wave four instructions per piece -
                     // and puts two idle cycles between the vector writes and the matrix instruction that reads them)
@@ -335,6 +341,8 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
                 }
                 if (FLIP_A)
                     a ^= (int)0x80808080;
+                if constexpr (ROWSUM)
+                    asum[rb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, a, asum[rb], 0, 0, 0);
 #pragma unroll
                 for (int q = 0; q < QS; ++q)
                     acc[rb][q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[q], a, acc[rb][q], 0, 0, 0);
@@ -348,13 +356,18 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     }
 
     __builtin_amdgcn_s_setprio(0);
+    if constexpr (ROWSUM)
+    {
+#pragma unroll
+        for (int rb = 0; rb < RS; ++rb)
+            rsum[rb] = (int32_t)((uint32_t)g.epi.rowsum_mul * (uint32_t)asum[rb][0]);
+    }
     if (fast && g.epi.qp_std && (qflag & 3) == 0 && g.epi.vec_store && (g.N & 3) == 0)
     {
         // every column has a normalised multiplier and a right shift of 2..31: the short form of the requantisation.
         // Lane l holds, for row rb * 16 + l % 16, the 4 consecutive columns q * 16 + 4 * (l / 16) + {0..3}: one dword
         // (N is a multiple of 4 here, so a lane's four columns exist together or not at all).
         const int32_t  off2p1 = 2 * g.epi.result_offset + 1, lo = g.epi.lo, hi = g.epi.hi;
-        const int32_t *rowvec = g.epi.rowvec;
         const int      a_N    = g.N;
         int32_t        rv[RS];
         char          *drow[RS]; // this lane's row of D at column 4 * (l / 16)
@@ -362,7 +375,7 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
         for (int rb = 0; rb < RS; ++rb)
         {
             const int i = row0 + rb * 16 + lr;
-            rv[rb]      = (rowvec && i < a_M) ? rowvec[i] : 0;
+            rv[rb]      = rsum[rb];
             drow[rb]    = (char *)g.D + (int64_t)i * g.ldd + col0 + 4 * lh;
         }
 #pragma unroll
@@ -391,9 +404,9 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
         }
     }
     else if (fast && npan == 1)
-        epilogue_store_fast<RS, QS, NARROW_BN>(acc, g, par, row0, 0, 0, lane, 0);
+        epilogue_store_fast<RS, QS, NARROW_BN>(acc, g, par, row0, 0, 0, lane, 0, rsum, ROWSUM);
     else
-        epilogue_store_t<EPI, RS, QS>(acc, g, row0, col0, lane, 0);
+        epilogue_store_t<EPI, RS, QS>(acc, g, row0, col0, lane, 0, rsum, ROWSUM);
     }
 #undef MI355_GLOBAL
 }
@@ -634,6 +647,43 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
     const int  qflag_u = __builtin_amdgcn_readfirstlane(par[NPAR * ncols]);
     const bool fast    = have_qp && (qflag_u & 1) == 0;
 
+    // Weights with an offset: the row sums of the tile's patches, by matrix instructions of their own against ones (here and
+    // not in the loop below, which a condition per k block makes slower). 56x56x64 -> 64, 3x3, batch 32, u8 weights with a
+    // zero point: 9.9 us against 8.0 without one; with a pass over the image in front of the kernel it was 43.3.
+    const bool rowsum = g.epi.rowsum_mul != 0;
+    int32_t    rsum[RS];
+#pragma unroll
+    for (int rb = 0; rb < RS; ++rb)
+        rsum[rb] = 0;
+    if (rowsum)
+    {
+        v4i asum[RS];
+#pragma unroll
+        for (int rb = 0; rb < RS; ++rb)
+            asum[rb] = (v4i){0, 0, 0, 0};
+        for (int kb = 0; kb * 64 < g.K; ++kb)
+        {
+            const int tap = narrow_div(kb * 64, cg.magic_C), c64 = kb * 64 - tap * cg.C;
+            const int ky = narrow_div(tap, cg.magic_KW), kx = tap - ky * cg.KW;
+            const int ds   = ((ky * cg.dil_y * Wp + kx * cg.dil_x) << lc) + c64;
+            const v4i ones = ones_block<PITCH, KBLK>(smem, kb, lh);
+#pragma unroll
+            for (int rb = 0; rb < RS; ++rb)
+            {
+                const int x = s0[rb] + ds;
+                v4i       a = *(const v4i *)(smem + (x ^ ((x >> sw_r) & sw_mask)));
+                if (FLIP_A)
+                    a ^= (int)0x80808080;
+                asum[rb] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, a, asum[rb], 0, 0, 0);
+            }
+        }
+        // (the issuing block is the loop's: see the note on wait states behind a taken branch)
+        asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+#pragma unroll
+        for (int rb = 0; rb < RS; ++rb)
+            rsum[rb] = (int32_t)((uint32_t)g.epi.rowsum_mul * (uint32_t)asum[rb][0]);
+    }
+
     // (Different priorities for the waves that share a SIMD - one at a time through the matrix instructions, its epilogue
     // beside the next wave's - paid while the loop carried twice the address arithmetic; with today's loop, equal
     // priorities measured 0.4 us faster on a 8.3 us kernel. Pinning the loop's order with scheduling barriers - all six
@@ -705,7 +755,6 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
             // consecutive columns pc0 + q * 16 + 4 * (l / 16) + {0..3}
             const int16_t  o16 = (int16_t)(2 * g.epi.result_offset + 1), lo16 = (int16_t)g.epi.lo, hi16 = (int16_t)g.epi.hi;
             const pk16_t   off2p1 = {o16, o16}, lo = {lo16, lo16}, hi = {hi16, hi16};
-            const int32_t *rowvec = g.epi.rowvec;
             const int      a_N    = g.N;
             int32_t        rv[RSX];
             char          *drow[RSX];
@@ -713,7 +762,7 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
             for (int rb = 0; rb < RSX; ++rb)
             {
                 const int i = row0 + rb * 16 + lr;
-                rv[rb]      = (rowvec && i < a_M) ? rowvec[i] : 0;
+                rv[rb]      = rsum[rb];
                 drow[rb]    = (char *)g.D + (int64_t)i * g.ldd + pc0 + 4 * lh;
             }
 #pragma unroll
@@ -743,13 +792,13 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
             gl.M        = a_M;
             // (the staged constants' form is built for rows of 64 constants: several panels take the general one)
             if constexpr (MULTI)
-                epilogue_store_t<EPI, RSX, QS>(acc, gl, row0, pc0, lane, 0);
+                epilogue_store_t<EPI, RSX, QS>(acc, gl, row0, pc0, lane, 0, rsum, rowsum);
             else
             {
                 if (fast)
-                    epilogue_store_fast<RSX, QS, NARROW_BN>(acc, gl, par, row0, 0, 0, lane, 0);
+                    epilogue_store_fast<RSX, QS, NARROW_BN>(acc, gl, par, row0, 0, 0, lane, 0, rsum, rowsum);
                 else
-                    epilogue_store_t<EPI, RSX, QS>(acc, gl, row0, 0, lane, 0);
+                    epilogue_store_t<EPI, RSX, QS>(acc, gl, row0, 0, lane, 0, rsum, rowsum);
             }
         }
     };
@@ -824,31 +873,27 @@ static bool halo_plan(const GemmArgs &a, int epi, int cus, int &rpw, int &wpi, s
     return true;
 }
 
-template <int EPI, bool FLIP_A, bool CONV, bool UNI>
+template <int EPI, bool FLIP_A, bool UNI, bool ROWSUM>
 static const void *narrow_fn(int nb)
 {
     switch (nb)
     {
-    case 1: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, CONV, UNI, 1>;
-    case 2: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, CONV, UNI, 2>;
-    case 3: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, CONV, UNI, 3>;
-    case 4: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, CONV, UNI, 4>;
-    case 5: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, CONV, UNI, 5>;
-    case 6: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, CONV, UNI, 6>;
+    case 1: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, UNI, 1, ROWSUM>;
+    case 2: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, UNI, 2, ROWSUM>;
+    case 3: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, UNI, 3, ROWSUM>;
+    case 4: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, UNI, 4, ROWSUM>;
+    case 5: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, UNI, 5, ROWSUM>;
+    case 6: return (const void *)gemm_narrow_kernel<EPI, FLIP_A, UNI, 6, ROWSUM>;
     }
     return nullptr;
 }
 
-template <int EPI>
-static const void *narrow_fn_e(bool flip_a, bool conv, bool uni, int nb)
+template <int EPI, bool ROWSUM>
+static const void *narrow_fn_e(bool flip_a, bool uni, int nb)
 {
-    if (conv)
-    {
-        if (uni)
-            return flip_a ? narrow_fn<EPI, true, true, true>(nb) : narrow_fn<EPI, false, true, true>(nb);
-        return flip_a ? narrow_fn<EPI, true, true, false>(nb) : narrow_fn<EPI, false, true, false>(nb);
-    }
-    return flip_a ? narrow_fn<EPI, true, false, false>(nb) : narrow_fn<EPI, false, false, false>(nb);
+    if (uni)
+        return flip_a ? narrow_fn<EPI, true, true, ROWSUM>(nb) : narrow_fn<EPI, false, true, ROWSUM>(nb);
+    return flip_a ? narrow_fn<EPI, true, false, ROWSUM>(nb) : narrow_fn<EPI, false, false, ROWSUM>(nb);
 }
 
 int narrow_panel_chunks(int K)
@@ -858,32 +903,26 @@ int narrow_panel_chunks(int K)
     return (K + 191) / 192 * 12;
 }
 
-bool narrow_applies(const GemmArgs &a, bool conv)
+bool narrow_applies(const GemmArgs &a)
 {
     if (a.N < 1 || a.N > NARROW_MAX_PANELS * NARROW_BN || a.K < 16 || a.K > NARROW_MAX_NB * 192 || a.K > a.Kp || a.Kp % 64 != 0 || a.M < 1)
         return false;
     if (a.N > NARROW_BN && a.K > 192) // several panels only while the whole patch stays in registers
         return false;
-    if (conv)
-    {
-        // whole 16-byte columns of one tap; the image batch within 31 bits of offset
-        const ConvGeom &c = a.conv;
-        const int64_t   images = ((int64_t)a.M + (int64_t)c.OH * c.OW - 1) / ((int64_t)c.OH * c.OW);
-        return c.C % 16 == 0 && ((uintptr_t)a.A & 15) == 0 && a.K % 16 == 0 && images * c.H * c.W * c.C < ((int64_t)1 << 31);
-    }
-    // dense: 16-byte aligned rows of whole 16-byte columns, offsets within 31 bits
-    return ((uintptr_t)a.A & 15) == 0 && a.lda % 16 == 0 && a.K % 16 == 0 && (int64_t)a.M * a.lda < ((int64_t)1 << 31);
+    // whole 16-byte columns of one tap; the image batch within 31 bits of offset
+    const ConvGeom &c = a.conv;
+    const int64_t   images = ((int64_t)a.M + (int64_t)c.OH * c.OW - 1) / ((int64_t)c.OH * c.OW);
+    return c.C % 16 == 0 && ((uintptr_t)a.A & 15) == 0 && a.K % 16 == 0 && images * c.H * c.W * c.C < ((int64_t)1 << 31);
 }
 
-int narrow_launch(int epi, bool flip_a, bool conv, const GemmArgs &args, hipStream_t s, bool *band)
+int narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, bool *band)
 {
     if (band)
         *band = false;
-    if (!narrow_applies(args, conv) || args.fill16 == nullptr || epi < 0 || epi > 2)
+    if (!narrow_applies(args) || args.fill16 == nullptr || (epi != EPI_FIXEDPOINT && epi != EPI_F32))
         return (int)hipErrorInvalidValue;
     const int   nb  = (args.K + 191) / 192;
-    const bool  uni = conv && args.conv.C % 64 == 0;
-    if (conv)
+    const bool  uni = args.conv.C % 64 == 0, rowsum = args.epi.rowsum_mul != 0;
     {
         int      rpw = 0, wpi = 0;
         size_t   hl  = 0;
@@ -919,9 +958,8 @@ int narrow_launch(int epi, bool flip_a, bool conv, const GemmArgs &args, hipStre
             return (int)hipLaunchKernel(hf, dim3((unsigned)(images * wpi)), dim3(HALO_WAVES * 64), kargs, hl, s);
         }
     }
-    const void *fn  = epi == EPI_S32 ? narrow_fn_e<EPI_S32>(flip_a, conv, uni, nb)
-                      : epi == EPI_FIXEDPOINT ? narrow_fn_e<EPI_FIXEDPOINT>(flip_a, conv, uni, nb)
-                                              : narrow_fn_e<EPI_F32>(flip_a, conv, uni, nb);
+    const void *fn = epi == EPI_FIXEDPOINT ? (rowsum ? narrow_fn_e<EPI_FIXEDPOINT, true>(flip_a, uni, nb) : narrow_fn_e<EPI_FIXEDPOINT, false>(flip_a, uni, nb))
+                                           : (rowsum ? narrow_fn_e<EPI_F32, true>(flip_a, uni, nb) : narrow_fn_e<EPI_F32, false>(flip_a, uni, nb));
     if (fn == nullptr)
         return (int)hipErrorInvalidValue;
     const int    npan = (args.N + NARROW_BN - 1) / NARROW_BN;
@@ -929,8 +967,8 @@ int narrow_launch(int epi, bool flip_a, bool conv, const GemmArgs &args, hipStre
     if (lds > 48 * 1024)
     {
         // once per kernel and device (for the largest panel count the kernel may meet)
-        static std::atomic<uint32_t> raised[3][2][2][2][NARROW_MAX_NB];
-        std::atomic<uint32_t>       &done = raised[epi][flip_a ? 1 : 0][conv ? 1 : 0][uni ? 1 : 0][nb - 1];
+        static std::atomic<uint32_t> raised[2][2][2][2][NARROW_MAX_NB];
+        std::atomic<uint32_t>       &done = raised[epi == EPI_F32 ? 1 : 0][flip_a ? 1 : 0][rowsum ? 1 : 0][uni ? 1 : 0][nb - 1];
         int                          dev  = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 32)
             return (int)hipErrorInvalidDevice;
@@ -946,14 +984,8 @@ int narrow_launch(int epi, bool flip_a, bool conv, const GemmArgs &args, hipStre
     GemmArgs a = args;
     a.nblocks  = npan;
     // what the A loads' range check compares with
-    if (conv)
-    {
-        const ConvGeom &c      = args.conv;
-        const int64_t   images = ((int64_t)args.M + (int64_t)c.OH * c.OW - 1) / ((int64_t)c.OH * c.OW);
-        a.a_end                = args.A + images * c.H * c.W * c.C;
-    }
-    else
-        a.a_end = args.A + (int64_t)(args.M - 1) * args.lda + args.K;
+    a.a_end = args.A + (((int64_t)args.M + (int64_t)args.conv.OH * args.conv.OW - 1) / ((int64_t)args.conv.OH * args.conv.OW)) * args.conv.H *
+                           args.conv.W * args.conv.C;
     // Workgroups of 4 waves x 32 rows, 4 to a compute unit. When the last round of workgroups would put a fourth
     // workgroup on only a few compute units (they finish last: the kernel's time is theirs), its rows go out in
     // workgroups with fewer working waves, to more compute units.

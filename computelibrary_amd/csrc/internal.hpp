@@ -22,6 +22,7 @@ struct ConvGeom
     int32_t H, W, C, KH, KW, OH, OW;
     int32_t stride_x, stride_y, pad_left, pad_top, dil_x, dil_y;
     uint32_t pad_word; // the padding byte (already sign-flipped if the loader flips) replicated into 4 bytes
+    int32_t  c_true; // channels of a pixel that count (C rounded up to whole 16-byte pieces may hold more)
     // floor(2^32 / d) + 1 for d = C, KW, OW, OH (0 when d == 1): x / d == mulhi(x, magic) exactly while x * d < 2^32
     uint32_t magic_C, magic_KW, magic_OW, magic_OH;
 };
@@ -104,7 +105,7 @@ MfmaConfig  dma_config(int idx);
 int         dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &args, int batch, hipStream_t s);
 
 // gemm_narrow.hip — N <= 64, K <= 1152, 16-byte aligned operands: A straight from global memory into the matrix cores'
-// operand layout, B resident in LDS; dense or implicit convolution (C % 16 == 0). needs args.fill16
+// operand layout, B resident in LDS; implicit convolution (C % 16 == 0). needs args.fill16
 // (args.Bp: the image written by pack_b_narrow_launch with narrow_panel_chunks(K) + NARROW_PAD_PIECES pieces per row)
 int  narrow_panel_chunks(int K); // 0: K outside the kernel's range
 // Pieces of padding after each row of that image. A ds_read_b128 goes through LDS in four batches of 16 lanes - lanes
@@ -112,9 +113,9 @@ int  narrow_panel_chunks(int K); // 0: K outside the kernel's range
 // conflicts when its 16 addresses differ modulo 256 bytes: with lane l at row l % 16, piece l / 16 that holds for a row
 // pitch of 32 modulo 64 bytes (measured: 2.8 clocks per instruction and compute unit against 4.6 with 16 modulo 64).
 constexpr int NARROW_PAD_PIECES = 2;
-bool narrow_applies(const GemmArgs &args, bool conv);
+bool narrow_applies(const GemmArgs &args);
 // *band (when given): whether the launch took the form that stages a band of input rows in LDS (large images)
-int  narrow_launch(int epi, bool flip_a, bool conv, const GemmArgs &args, hipStream_t s, bool *band = nullptr);
+int  narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, bool *band = nullptr);
 
 // gemm_skinny.hip — M <= 64, B packed in matrix-core operand order (see pack_b_skinny)
 constexpr int SKINNY_MAX_M = 64;
@@ -141,8 +142,9 @@ int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N
 // the same from B given as [N][ldk] with K contiguous (conv weights [OFM][KH*KW*C])
 int pack_bt_launch(const void *Bt, int64_t ldk, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
                    int8_t *out, const ColumnFinish &f, hipStream_t s);
-// rows 0..63 of Bp -> [64][chunks + 1] pieces of 16 bytes (the last one padding), zero beyond Kp
-int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows, int8_t *Bn, hipStream_t s);
+// the first rows of Bp -> [rows][chunks + NARROW_PAD_PIECES] pieces of 16 bytes, zero beyond Kp; the padding: a row of ones (zeros
+// for what does not count of a patch of K with c_true of C channels)
+int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows, int K, int C, int c_true, int8_t *Bn, hipStream_t s);
 // the terms again from the sums in f.colsum
 int colvec_launch(int Np, int nb, const ColumnFinish &f, hipStream_t s);
 // (multiplier, shift) per column -> qp[QP_COUNT][Np]; *neg != 0 afterwards if any multiplier is negative

@@ -370,9 +370,11 @@ int conv_rowsum_launch(const void *src, const ConvGeom &g, int M, bool flip, int
 }
 
 // The first `rows` (a multiple of 64) rows of Bp as the narrow kernel keeps them in LDS: rows of `chunks` 16-byte pieces of data plus
-// NARROW_PAD_PIECES of padding, zero beyond Kp - the workgroups copy this image into LDS with plain linear transfers
-__global__ __launch_bounds__(256) void pack_b_narrow_kernel(const int8_t *__restrict__ Bp, int Kp, int chunks, int rows,
-                                                            int8_t *__restrict__ Bn)
+// NARROW_PAD_PIECES of padding, zero beyond Kp - the workgroups copy this image into LDS with plain linear transfers. The
+// padding of a panel's 64 rows holds one more row of the patch, piece p in padding piece p % 2 of row p / 2: a one for
+// every byte that counts in the row sums of A, zeros for channels from c_true of C on and for k from K on.
+__global__ __launch_bounds__(256) void pack_b_narrow_kernel(const int8_t *__restrict__ Bp, int Kp, int chunks, int rows, int K, int C,
+                                                            int c_true, int8_t *__restrict__ Bn)
 {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     constexpr int PAD = NARROW_PAD_PIECES;
@@ -382,14 +384,22 @@ __global__ __launch_bounds__(256) void pack_b_narrow_kernel(const int8_t *__rest
     v4i       v = {0, 0, 0, 0};
     if (c < chunks && c * 16 < Kp)
         v = *(const v4i *)(Bp + (int64_t)r * Kp + c * 16);
+    else if (c >= chunks)
+    {
+        const int k0 = ((r & 63) * PAD + c - chunks) * 16;
+#pragma unroll
+        for (int t = 0; t < 16; ++t)
+            if (k0 + t < K && (k0 + t) % C < c_true)
+                v[t >> 2] |= 1 << (8 * (t & 3));
+    }
     *(v4i *)(Bn + (int64_t)idx * 16) = v;
 }
 
-int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows, int8_t *Bn, hipStream_t s)
+int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows, int K, int C, int c_true, int8_t *Bn, hipStream_t s)
 {
-    if (Kp % 16 || rows < 64 || rows % 64 != 0 || Np < rows || chunks < 1)
+    if (Kp % 16 || rows < 64 || rows % 64 != 0 || Np < rows || chunks < 1 || C < 1)
         return (int)hipErrorInvalidValue;
-    pack_b_narrow_kernel<<<dim3((rows * (chunks + NARROW_PAD_PIECES) + 255) / 256), dim3(256), 0, s>>>(Bp, Kp, chunks, rows, Bn);
+    pack_b_narrow_kernel<<<dim3((rows * (chunks + NARROW_PAD_PIECES) + 255) / 256), dim3(256), 0, s>>>(Bp, Kp, chunks, rows, K, C, c_true, Bn);
     return launch_status();
 }
 

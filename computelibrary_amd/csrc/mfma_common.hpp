@@ -95,12 +95,33 @@ __device__ __forceinline__ void finish_row_sums(int32_t (&sums)[RS], int32_t mul
         sums[f] = (int32_t)((uint32_t)mul * (uint32_t)(v + 128 * flipped_pad_bytes));
     }
 }
-__device__ __forceinline__ int32_t sum_bytes(v4i x, int32_t acc)
+constexpr int32_t ONES4 = 0x01010101;
+__device__ __forceinline__ int32_t sum_bytes(v4i x, int32_t acc, v4i ones = (v4i){ONES4, ONES4, ONES4, ONES4})
 {
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-        acc = __builtin_amdgcn_sdot4(x[t], 0x01010101, acc, false);
+        acc = __builtin_amdgcn_sdot4(x[t], ones[t], acc, false);
     return acc;
+}
+// a one in each of the first n of 16 bytes (n of any sign and size): what sum_bytes counts of a piece that is partly
+// padding
+__device__ __forceinline__ v4i first_bytes(int n)
+{
+    v4i m;
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+    {
+        const int r = min(max(n - 4 * t, 0), 4);
+        m[t]        = r == 0 ? 0 : (int)((uint32_t)ONES4 >> (8 * (4 - r)));
+    }
+    return m;
+}
+// The same for the 16 bytes at k of a convolution's patch (k < K): a pixel's channels beyond c_true are padding of the
+// channel count, and k from K on is nothing. Padded taps count: they hold the padding value, as in the patch matrix.
+__device__ __forceinline__ v4i patch_bytes(const ConvGeom &c, int k, int K)
+{
+    const int c0 = k - fast_div(k, c.magic_C) * c.C;
+    return first_bytes(k < K ? c.c_true - c0 : 0);
 }
 
 // Accumulator (fm, fn, r) of lane l holds row 8*(r/4) + 4*(l/32) + r%4, column l%32 of its 32 x 32 block.
