@@ -222,6 +222,8 @@ struct GemmCore
         shift.release(), bias.release(), Ap.release(), fill.release(), qp.release(), zeros.release(), parts.release(), zerocol.release();
     }
 
+    static constexpr int MOST_SLICES = 32;
+
     int choose_kernel()
     {
         Kp = round_up(K, PACK_K_ALIGN);
@@ -270,18 +272,19 @@ struct GemmCore
                 (void)env;
                 return best;
             };
-            // The pipelined kernel's tile is chosen with a small cost model in clocks per compute unit, from what was
-            // measured on the device: a K step costs the largest of its direct-to-LDS stream (about 44 bytes per
-            // clock and compute unit), its matrix instructions (4096 multiply-accumulates per clock) and the two
-            // barrier-separated slots of the consumer groups (about 1000 clocks per 128 bytes of K, whatever the tile);
-            // every tile adds a fixed start-up plus an epilogue proportional to its outputs, which co-resident
-            // workgroups overlap. Ties go to the deeper ring (more loads in flight when B comes from HBM).
-            // A single dense GEMM may also run its K range as 2, 4 or 8 slices (see prepare()): the tiles of all slices
-            // share the chip, every slice has 1/S of the K steps, and a second kernel reads the S planes of partial
-            // sums back (measured: about 2.5 bytes per clock and compute unit of the whole chip, plus a launch).
+            // The pipelined kernel's tile is chosen with a small cost model in microseconds, fitted to sweeps of every tile
+            // shape and slice count over 33 shapes (M 65-2048, N 24-12288, K 512-11008, B hot and rotated through HBM): a tile
+            // costs MfmaConfig::us_tile for its start-up and epilogue, shared by the workgroups that fit a compute unit
+            // together, plus us_step for every K step, which a full chip slows down by a share us_load of it (L2, HBM and
+            // the power limit are shared by all compute units).
+            // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
+            // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.8 us for the launch
+            // and its latency, 0.12 us per plane one thread walks over and 0.25 us per MB. (254 x 33 x 10588: 39.0 us whole,
+            // 11.4 as 21 slices, 11.3 as 12; 640 x 480 x 2048: 10.4 whole, 11.0 as 3.) Slices have to promise an eighth:
+            // below that the model's error decides, and they need a workspace.
             auto pick_dma = [&]() -> int
             {
-                int    best = -1, best_lds = 0;
+                int    best = -1;
                 double best_cost = 0;
                 for (int i = 0; i < dma_num_configs(); ++i)
                 {
@@ -291,19 +294,23 @@ struct GemmCore
                     const double tiles   = (double)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN) * batch;
                     const int    occ_lds = (160 * 1024) / c.lds_bytes, occ_wav = 32 / c.waves;
                     const double occ     = std::max(1, std::min(occ_lds, occ_wav));
-                    const double nk      = (double)((K + c.BK - 1) / c.BK);
-                    const double step    = std::max({(double)(c.BM + c.BN) * c.BK / 44.0, (double)c.BM * c.BN * c.BK / 4096.0,
-                                                     1000.0 * c.BK / 128.0});
-                    const double fixed   = 6000.0 + (double)c.BM * c.BN / 4.4;
-                    for (int sl = 1; sl <= 8; sl *= 2)
+                    const int    nk      = (K + c.BK - 1) / c.BK;
+                    // (the loader of a convolution decodes taps: 6272 x 256 x 2304 and 25088 x 128 x 1152, 1.15 of the dense)
+                    const double us_step = patch_c > 0 ? 1.15 * c.us_step : c.us_step;
+                    for (int want = 1; want <= MOST_SLICES; ++want)
                     {
-                        if (sl > 1 && (batch != 1 || K % (sl * c.BK) != 0 || K / sl < 1024))
+                        // (slices of equal whole K steps but the last, none of them empty)
+                        const int per = (nk + want - 1) / want, sl = (nk + per - 1) / per;
+                        if (want > 1 && (batch != 1 || per * c.BK < 512))
                             break;
-                        const double per_cu = std::ceil(tiles * sl / cus);
-                        const double finish = sl > 1 ? 4000.0 + (double)sl * M * N * 4.0 / (2.5 * cus) : 0.0;
-                        const double cost   = per_cu * (nk / sl) * step + std::ceil(per_cu / occ) * fixed + finish;
-                        if (best < 0 || cost < best_cost || (cost == best_cost && sl == 1 && c.lds_bytes > best_lds))
-                            best = i, best_cost = cost, best_lds = c.lds_bytes, splitk_plan = sl;
+                        if (sl != want)
+                            continue;
+                        const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
+                        const double finish = sl > 1 ? 2.8 + 0.12 * sl + (double)sl * M * N * 1e-6 : 0.0;
+                        const double cost   = (std::ceil(per_cu / occ) * c.us_tile + per_cu * per * us_step * (1.0 + c.us_load * load) + finish) *
+                                            (sl > 1 ? 1.125 : 1.0);
+                        if (best < 0 || cost < best_cost)
+                            best = i, best_cost = cost, splitk_plan = sl;
                     }
                 }
                 return best;
@@ -318,10 +325,9 @@ struct GemmCore
                 const int64_t    tiles = (int64_t)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN);
                 if (batch == 1 && tiles * 2 <= cus && K >= 2048)
                 {
-                    int sl = (int)std::min<int64_t>(std::min<int64_t>(cus / tiles, K / 1024), 8);
-                    while (sl > 1 && K % (sl * c.BK) != 0)
-                        --sl;
-                    splitk_plan = sl;
+                    const int nk = (K + c.BK - 1) / c.BK, want = (int)std::min<int64_t>(std::min<int64_t>(cus / tiles, K / 1024), 8);
+                    const int per = (nk + want - 1) / want;
+                    splitk_plan   = (nk + per - 1) / per;
                 }
             }
             if (K < 16)
@@ -452,9 +458,9 @@ struct GemmCore
         // A deep K under few output tiles: the pipelined kernel would leave most compute units idle, each of the others
         // walking the whole K. The K range is cut into slices that run as the batch entries of one S32 launch (the slice
         // offset is the batch stride of A and of the packed B alike), and a second kernel sums the planes and applies the
-        // epilogue. Slices are whole k steps of the tile shape, so no slice but the matrix' own end has a tail.
+        // epilogue. Slices are whole K steps of the tile shape, the last one as many as are left.
         splitk = 1;
-        if (path == MI355_PATH_MFMA && dma_idx >= 0 && batch == 1 && splitk_plan > 1 && K % (splitk_plan * dma_config(dma_idx).BK) == 0)
+        if (path == MI355_PATH_MFMA && dma_idx >= 0 && batch == 1)
             splitk = splitk_plan;
         if (splitk > 1)
         {
@@ -696,13 +702,13 @@ struct GemmCore
                 g.tiles_m          = (g.M + c.BM - 1) / c.BM;
                 g.tiles_n          = (g.N + c.BN - 1) / c.BN;
                 kname_run          = &kname_dma_full;
-                if (splitk > 1 && batch == 1 && g.K == K && K % (splitk * c.BK) == 0)
+                if (splitk > 1 && batch == 1)
                 {
                     // the float epilogue rounds the product and the offset terms apart: they must not meet in the planes
                     if (conv && epi == EPI_F32 && g.epi.rowsum_mul != 0)
                         TRY(conv_row_terms(g, s));
                     const int     ldp = (N + 3) & ~3;
-                    const int64_t kc  = K / splitk;
+                    const int64_t kc  = (int64_t)(((K + c.BK - 1) / c.BK + splitk - 1) / splitk) * c.BK;
                     GemmArgs      gp  = g;
                     gp.epi                     = EpiParams{};
                     gp.epi.colvec              = zerocol.as<int32_t>();
@@ -712,7 +718,8 @@ struct GemmCore
                     gp.D = parts.as<int32_t>(), gp.ldd = ldp, gp.d_batch_stride = (int64_t)M * ldp;
                     // (dense: a slice starts kc bytes into every row of A; convolution: kc values into every patch,
                     // which the loader adds to the k it decodes)
-                    gp.K = (int)kc, gp.a_batch_stride = conv ? 0 : kc, gp.bp_batch_stride = kc, gp.k_slice = conv ? (int32_t)kc : 0;
+                    // (g.K: K, or K padded to whole steps where the rows of A were copied)
+                    gp.a_batch_stride = conv ? 0 : kc, gp.bp_batch_stride = kc, gp.k_slice = (int32_t)kc;
                     kname_run = &kname_splitk;
                     HIP_TRY(dma_launch(dma_idx, EPI_S32, flip_in_loader, conv, gp, splitk, s));
                     HIP_TRY(splitk_finish_launch(epi, g, parts.as<int32_t>(), (int64_t)M * ldp, ldp, splitk, s));

@@ -267,7 +267,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     asm volatile(""
                  : "+s"(g.tiles_m), "+s"(g.tiles_n), "+s"(g.magic_tiles), "+s"(g.magic_group), "+s"(g.tile_magic_ok), "+s"(g.lda),
                    "+s"(g.a_batch_stride), "+s"(g.Kp), "+s"(g.bp_batch_stride), "+s"(g.M), "+s"(g.N), "+s"(g.K),
-                   "+s"(g.epi.qp_stride), "+s"(g.epi.colvec_batch_stride), "+s"(g.nblocks));
+                   "+s"(g.epi.qp_stride), "+s"(g.epi.colvec_batch_stride), "+s"(g.nblocks), "+s"(g.k_slice));
     typedef const __attribute__((address_space(1))) int32_t *global_i32;
     uintptr_t u_cv = (uintptr_t)g.epi.colvec, u_qp = (uintptr_t)g.epi.qp, u_fl = (uintptr_t)g.epi.qp_flag;
     asm volatile("" : "+s"(u_cv), "+s"(u_qp), "+s"(u_fl));
@@ -327,6 +327,8 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     else
         tile_coords_batched(blockIdx.x, g.nblocks, g.tiles_m, g.tiles_n, bz, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
+    if (g.k_slice != 0) // K slices: this entry's part of K (the last one ends where K does)
+        g.K = min(g.k_slice, g.K - bz * g.k_slice);
     const int nk = (g.K + BK - 1) / BK;
     // which requantisation formula applies was decided on the device when the per-column constants were digested
     // (a scalar load: as a vector load its wait would also wait for every direct-to-LDS load issued before it)
@@ -615,7 +617,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
     asm volatile(""
                  : "+s"(g.tiles_m), "+s"(g.tiles_n), "+s"(g.magic_tiles), "+s"(g.magic_group), "+s"(g.tile_magic_ok), "+s"(g.lda),
                    "+s"(g.a_batch_stride), "+s"(g.Kp), "+s"(g.bp_batch_stride), "+s"(g.M), "+s"(g.N), "+s"(g.K),
-                   "+s"(g.epi.qp_stride), "+s"(g.epi.colvec_batch_stride), "+s"(g.nblocks));
+                   "+s"(g.epi.qp_stride), "+s"(g.epi.colvec_batch_stride), "+s"(g.nblocks), "+s"(g.k_slice));
     typedef const __attribute__((address_space(1))) int32_t *global_i32;
     uintptr_t u_cv = (uintptr_t)g.epi.colvec, u_qp = (uintptr_t)g.epi.qp, u_fl = (uintptr_t)g.epi.qp_flag;
     asm volatile("" : "+s"(u_cv), "+s"(u_qp), "+s"(u_fl));
@@ -653,6 +655,8 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
     else
         tile_coords_batched(blockIdx.x, g.nblocks, g.tiles_m, g.tiles_n, bz, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
+    if (g.k_slice != 0) // K slices: this entry's part of K (the last one ends where K does)
+        g.K = min(g.k_slice, g.K - bz * g.k_slice);
     const int nk = (g.K + BK - 1) / BK;
     const bool inside = m0 + BM <= g.M; // no row of this tile lies beyond the matrix
     // which requantisation formula applies was decided on the device when the per-column constants were digested; the
@@ -949,6 +953,17 @@ static const void *const g_rowsum_256x128x128[3][2] = {
     {MI355_DFN(256, 128, 128, 2, 2, 3, 1, false, false), MI355_DFN(256, 128, 128, 2, 2, 3, 1, true, false)},
     {MI355_DFN(256, 128, 128, 2, 2, 3, 2, false, false), MI355_DFN(256, 128, 128, 2, 2, 3, 2, true, false)}};
 
+// What a tile and a K step of each configuration cost, in microseconds, and by what share a K step gets slower as the chip
+// fills: read off sweeps over the depth of K (64 x 64, 3 stages: 5.75 us at K = 512, 7.27 at 1024, 10.0 at 2048) and over the
+// number of tiles. The 6-stage ring never was the faster one of its tile in them, by 0.5 us, with B from HBM or not.
+struct DmaCost
+{
+    double us_tile, us_step, us_load;
+};
+static const DmaCost g_dma_cost[] = {
+    {5.6, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.5, 0.385, 0.35}, {2.7, 0.354, 0.35}, {3.2, 0.354, 0.35}, {4.1, 0.618, 0.35},
+};
+
 static const DmaEntry g_dma[] = {
     MI355_WCFG("pp_256x128x128_s3", 256, 128, 128, 2, 2, 3),
     MI355_DCFG("pp_128x128x128_s3", 128, 128, 128, 2, 2, 3),
@@ -967,6 +982,8 @@ MfmaConfig dma_config(int idx)
     MfmaConfig c = g_dma[idx].cfg;
     c.waves      = g_dma[idx].threads / 64;
     c.lds_bytes  = g_dma[idx].lds_bytes;
+    static_assert(sizeof(g_dma_cost) / sizeof(g_dma_cost[0]) == sizeof(g_dma) / sizeof(g_dma[0]), "one price per configuration");
+    c.us_tile = g_dma_cost[idx].us_tile, c.us_step = g_dma_cost[idx].us_step, c.us_load = g_dma_cost[idx].us_load;
     return c;
 }
 
@@ -986,8 +1003,9 @@ int dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &arg
     }
     if (fn == nullptr || args.fill16 == nullptr)
         return (int)hipErrorInvalidValue;
-    // K slices of a convolution: whole K steps, and K names one slice
-    if (args.k_slice != 0 && (!conv || args.K != args.k_slice || args.k_slice % c.cfg.BK != 0 || (int64_t)args.k_slice * batch > args.Kp))
+    // K slices: whole K steps, the last slice not empty
+    if (args.k_slice != 0 && (args.k_slice < 0 || args.k_slice % c.cfg.BK != 0 || (int64_t)args.k_slice * (batch - 1) >= args.K ||
+                              (int64_t)args.k_slice * batch < args.K))
         return (int)hipErrorInvalidValue;
     // shapes the kernel assumes: dword-aligned rows of at least one 16-byte column (whole columns of one tap for the
     // convolution), tiles that cover the output and stay inside the packed B panel

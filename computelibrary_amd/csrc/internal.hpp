@@ -52,8 +52,8 @@ struct GemmArgs
     uint32_t magic_tiles, magic_group;
     int32_t  tile_magic_ok;
     int32_t  nblocks; // workgroups of the launch (gridDim.x is a hidden argument behind this block: one more fetch)
-    // implicit convolution whose K range runs as slices (the batch entries of one launch): K values per slice, a whole
-    // number of K steps; entry z covers k in [z * k_slice, (z + 1) * k_slice) of the patch and K holds k_slice. 0: no slices
+    // a K range that runs as slices (the batch entries of one launch): K values per slice, a whole number of K steps; entry z
+    // covers k in [z * k_slice, min((z + 1) * k_slice, K)). 0: no slices
     int32_t  k_slice;
     // dense A whose K ends inside the last K step, set by dma_launch: the batch entry in whose last row tile a 16-byte
     // column of that step could reach beyond a_end. Every other tile may fetch the step whole - the columns at and
@@ -66,6 +66,7 @@ struct MfmaConfig
     const char *name;
     int         BM, BN, BK;
     int         waves = 0, lds_bytes = 0; // per workgroup (filled in for the pipelined kernel's configurations)
+    double      us_tile = 0, us_step = 0, us_load = 0; // ... and what the cost model prices them at (see GemmCore::choose_kernel)
 };
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));

@@ -51,8 +51,18 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__res
         return;
     const int i = (int)(t / n4), j0 = (int)(t % n4) * 4;
     v4i       acc = {0, 0, 0, 0};
-    for (int sl = 0; sl < splits; ++sl) // (columns from N on hold whatever the allocation held: never used below)
-        acc += *(const v4i *)(parts + (int64_t)sl * plane + (int64_t)i * ldp + j0);
+    // (columns from N on hold whatever the allocation held: never used below. Four loads at a time: few threads read many
+    // planes, and one load after the other is all latency)
+    const int32_t *from = parts + (int64_t)i * ldp + j0;
+    int            sl   = 0;
+    for (; sl + 4 <= splits; sl += 4, from += 4 * plane)
+    {
+        const v4i p0 = *(const v4i *)from, p1 = *(const v4i *)(from + plane), p2 = *(const v4i *)(from + 2 * plane),
+                  p3 = *(const v4i *)(from + 3 * plane);
+        acc += (p0 + p1) + (p2 + p3);
+    }
+    for (; sl < splits; ++sl, from += plane)
+        acc += *(const v4i *)from;
     const int32_t rv  = p.rowvec ? p.rowvec[i] : 0;
     const int64_t idx = (int64_t)i * g.ldd + j0;
     const bool    vec = p.vec_store && j0 + 3 < g.N;
