@@ -168,6 +168,9 @@ int transpose_bytes_launch(const void *src, void *dst, int batch, int R, int C, 
 int transpose_words_launch(const void *src, void *dst, int batch, int R, int C, hipStream_t s);
 // `runs` runs of C bytes -> runs of Cp bytes (Cp a multiple of 16): the first C copied, the rest set to `fill`
 int channel_pad_launch(const void *src, void *dst, int64_t runs, int C, int Cp, uint8_t fill, hipStream_t s);
+// `rows` image rows of W pixels of C bytes -> per row OW runs of Cr bytes (a multiple of 16), run ox starting stride_x * ox - pad_left
+// pixels into the row, `fill` where that lies outside
+int patch_rows_launch(const void *src, void *dst, int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr, uint8_t fill, hipStream_t s);
 // dst[s * dst_stride + c] = src[s * src_stride + c] for s < segments, c < seg (bytes)
 // dense F32 [batch][M][N] -> F16 destination (row stride ldh, batch stride, in elements), optionally added to its
 // previous contents in half arithmetic and clamped

@@ -744,7 +744,7 @@ __global__ __launch_bounds__(256) void transpose_kernel(const T *__restrict__ sr
 // 4 x 4 blocks turned round in registers, so that nothing moves byte by byte. A thread owns 16 rows x 4 columns between
 // LDS and the stores; TR / 16 threads of neighbouring row blocks write up to TR contiguous bytes. The 16-byte pieces of LDS rows
 // are swizzled with the row's 16-block (a read takes several blocks at once). Bounded by latency at the sizes of one layer.
-// 32 x (128 x 784): @TR@.
+// 32 x (128 x 784): 2.4 to 4 us each way, byte by byte 7 to 10.
 template <int TR, int TC>
 __global__ __launch_bounds__(256) void transpose_bytes_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int R, int C)
 {
@@ -1027,6 +1027,71 @@ int channel_pad_launch(const void *src, void *dst, int64_t runs, int C, int Cp, 
     if ((n + 255) / 256 > 0x7fffffff)
         return (int)hipErrorInvalidValue;
     channel_pad_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s>>>((const uint8_t *)src, (uint8_t *)dst, runs, C, Cp, fill);
+    return launch_status();
+}
+
+// ---- an NHWC image as patch rows: for every image row and output column the KW taps of C channels that lie side by side
+// under the kernel window, Cr >= KW * C bytes (a multiple of 16) apart. A KH x KW convolution of C channels becomes one of
+// KH x 1 over OW columns of KW * C channels. Bounded by the image it writes. One thread per 16 bytes: inside a row they are
+// one unaligned load; at its ends the load is moved into the row and its bytes shifted back, `fill` where the row has none.
+// Bytes from KW * C on hold whatever follows in the row and meet zero weights.
+// 32 x 224 x 224 x 3 under 7 x 7, stride 2 (25.7 MB written): 9 us, as long as the copy of single pixels took that it replaces; the
+// convolution behind it 44 -> 28 us.
+__global__ __launch_bounds__(256) void patch_rows_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst, int row_bytes, int step,
+                                                         int left, int per, uint32_t magic_per, int units, uint32_t blocks_per_row, uint32_t fill)
+{
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    typedef v4i v4i_any __attribute__((aligned(1)));
+    const uint32_t row = blockIdx.x / blocks_per_row;
+    const int      u   = (int)((blockIdx.x - row * blocks_per_row) * 256 + threadIdx.x);
+    if (u >= units)
+        return;
+    const int      ox = fast_div(u, magic_per);
+    const int      b  = ox * step - left + (u - ox * per) * 16; // first byte in the row
+    const uint8_t *in = src + (int64_t)row * row_bytes;
+    v4i            v;
+    if (b >= 0 && b + 16 <= row_bytes)
+        v = *(const v4i_any *)(in + b);
+    else if (row_bytes >= 16)
+    {
+        const int               at = min(max(b, 0), row_bytes - 16), sh = b - at;
+        const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, (v4i)(*(const v4i_any *)(in + at))), ones = ~(unsigned __int128)0;
+        const unsigned __int128 f = __builtin_bit_cast(unsigned __int128, (v4i){(int)fill, (int)fill, (int)fill, (int)fill});
+        unsigned __int128       y = f;
+        if (sh > 0 && sh < 16)
+            y = (x >> (8 * sh)) | (f & ~(ones >> (8 * sh)));
+        else if (sh < 0 && sh > -16)
+            y = (x << (-8 * sh)) | (f & ~(ones << (-8 * sh)));
+        v = __builtin_bit_cast(v4i, y);
+    }
+    else
+    {
+        uint32_t w[4];
+        for (int q = 0; q < 4; ++q)
+        {
+            w[q] = 0;
+            for (int t = 0; t < 4; ++t)
+            {
+                const int at = b + q * 4 + t;
+                w[q] |= (at >= 0 && at < row_bytes ? (uint32_t)in[at] : (fill & 0xFFu)) << (8 * t);
+            }
+        }
+        v = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    }
+    *(v4i *)(dst + ((int64_t)row * units + u) * 16) = v;
+}
+int patch_rows_launch(const void *src, void *dst, int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr, uint8_t fill, hipStream_t s)
+{
+    const int64_t units = (int64_t)OW * (Cr / 16), bpr = (units + 255) / 256;
+    if (rows < 1 || W < 1 || C < 1 || OW < 1 || Cr < 16 || Cr % 16 != 0 || ((uintptr_t)dst & 15) != 0 || rows * bpr > 0x7fffffff ||
+        units * 16 > 0x7fffffff || (int64_t)W * C > 0x7fffffff || ((int64_t)OW * stride_x + pad_left) * C + Cr > 0x7fffffff)
+        return (int)hipErrorInvalidValue;
+    const int      per   = Cr / 16;
+    const uint32_t magic = per == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)per) + 1u; // exact while units * per < 2^32
+    if (units * per >= ((int64_t)1 << 32))
+        return (int)hipErrorInvalidValue;
+    patch_rows_kernel<<<dim3((unsigned)(rows * bpr)), dim3(256), 0, s>>>((const uint8_t *)src, (uint8_t *)dst, W * C, stride_x * C, pad_left * C, per,
+                                                                         magic, (int)units, (uint32_t)bpr, 0x01010101u * fill);
     return launch_status();
 }
 
