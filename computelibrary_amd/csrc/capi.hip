@@ -1387,7 +1387,7 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
     // allow. Channels can be added for nothing: source pixels and weight taps are copied into buffers with the channels
     // padded to the next multiple of 16, the added weights are zero in the kernels' signed form, so no dot product
     // changes and neither do the column sums of the weights. The two other offset terms are kept on the caller's
-    // channel count: the row sums of the patches (needed under a weights offset) are taken from the unpadded source,
+    // channel count: the row sums of the patches (needed under a weights offset) count only those,
     // and the constant a_offset * b_offset * K uses the unpadded K.
     h->geom_true = h->geom;
     h->geom.c_true = h->geom_true.c_true = d.C;
