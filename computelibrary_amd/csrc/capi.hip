@@ -388,7 +388,7 @@ struct GemmCore
         return true;
     }
 
-    // behind a prepare whose work is left running on s
+    // behind a prepare (or an update behind one) whose work is left running on s
     int prepare_enqueued(hipStream_t s)
     {
         prep_pending = false;
@@ -403,7 +403,7 @@ struct GemmCore
         return 0;
     }
 
-    // in front of a run on s
+    // in front of whatever reads or writes on s what a prepare writes
     int wait_for_prepare(hipStream_t s)
     {
         if (!prep_pending || (s == prep_stream && s != hipStreamPerThread))
@@ -959,12 +959,15 @@ int mi355_gemmlowp_update_quant(mi355_gemm_handle *h, int32_t a_offset, int32_t 
     }
     c.a_offset = a_offset, c.b_offset = b_offset, c.scale = scale;
     h->d.a_offset = a_offset, h->d.b_offset = b_offset, h->d.scale = scale;
-    if (c.prepared)
-    {
-        TRY(c.refresh_colvec((hipStream_t)stream));
-        TRY(c.refresh_qparams((hipStream_t)stream));
-    }
-    return 0;
+    if (!c.prepared)
+        return 0;
+    // behind a prepare that is still running elsewhere: it writes the column sums that are read here, and terms of its own
+    // (with the offsets from before) over the ones that are written here
+    hipStream_t s = (hipStream_t)stream;
+    TRY(c.wait_for_prepare(s));
+    TRY(c.refresh_colvec(s));
+    TRY(c.refresh_qparams(s));
+    return c.prep_pending ? c.prepare_enqueued(s) : 0; // a run on a third stream comes behind both
 }
 
 static int set_gemm_strides(mi355_gemm_handle *h, int64_t lda, int64_t ldb, int64_t ldd, int64_t a_batch_stride,
