@@ -172,10 +172,9 @@ struct GemmCore
     bool    pt_vectors = false; // streaming path, per-tensor requantisation: mult / shift hold the scalars, replicated
     std::string kname;
     DevBuf  Bp, Bs, Bn, colsum, colvec, colpart, rowvec, mult, shift, bias, Ap, fill, qp, zeros, parts, zerocol;
-    // A prepare that only enqueues (every operand in device memory, nothing left to set up): the stream it went to and an
+    // A prepare that only enqueues (on the legacy default stream, every operand in device memory, nothing left to set up): an
     // event behind it, which runs on other streams wait for
     hipEvent_t  prep_done    = nullptr;
-    hipStream_t prep_stream  = nullptr;
     bool        prep_pending = false;
     int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not written yet)
     bool        qp_scalar_set = false; // the per-tensor requantisation vectors hold qp_rq
@@ -388,32 +387,42 @@ struct GemmCore
         return true;
     }
 
-    // behind a prepare (or an update behind one) whose work is left running on s
-    int prepare_enqueued(hipStream_t s)
+    // Behind a prepare (or an update behind one) whose work is left running on the legacy default stream. Only there: a stream
+    // that can be captured may be recording the run that follows, and then neither the host nor another stream is allowed to
+    // wait for an event that was recorded in it.
+    int prepare_enqueued()
     {
         prep_pending = false;
-        if (capturing(s))
-            return 0; // the graph's own order holds from here on
+        if (capturing(nullptr))
+        {
+            HIP_TRY(hipStreamSynchronize(nullptr));
+            return 0;
+        }
         // (nothing on the host reads what the kernels wrote: without the system fence the event costs 0.9 us between the two
         // kernels instead of 2.7)
         if (prep_done == nullptr)
             HIP_TRY(hipEventCreateWithFlags(&prep_done, hipEventDisableTiming | hipEventDisableSystemFence));
-        HIP_TRY(hipEventRecord(prep_done, s));
-        prep_stream = s, prep_pending = true;
+        HIP_TRY(hipEventRecord(prep_done, nullptr));
+        prep_pending = true;
         return 0;
     }
 
     // in front of whatever reads or writes on s what a prepare writes
     int wait_for_prepare(hipStream_t s)
     {
-        if (!prep_pending || (s == prep_stream && s != hipStreamPerThread))
+        if (!prep_pending || s == nullptr)
             return 0;
-        if (!capturing(s))
-        {
-            HIP_TRY(hipStreamWaitEvent(s, prep_done, 0));
+        if (capturing(s)) // a graph under construction cannot wait for work outside it, and may be launched on any stream
+            return prepare_over();
+        HIP_TRY(hipStreamWaitEvent(s, prep_done, 0));
+        return 0;
+    }
+
+    // the host waits, whatever the thread is recording
+    int prepare_over()
+    {
+        if (!prep_pending)
             return 0;
-        }
-        // a graph under construction cannot wait for work outside it: the host does
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
         const hipError_t e = hipEventSynchronize(prep_done);
@@ -931,13 +940,14 @@ int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *b
     TRY(to_device(c.rq.per_channel ? mult : nullptr, sizeof(int32_t) * d.N, h->stageMult, s, &multd));
     TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * d.N, h->stageShift, s, &shiftd));
     // staging buffers are reused by later calls, so what was copied through them has to be read before this returns; and a
-    // first prepare ends with the handle's own set-up done. After that, preparing a new B only enqueues.
-    const bool wait = !c.prepared || Bd != B || biasd != bias || (multd != nullptr && multd != mult) || (shiftd != nullptr && shiftd != shift);
+    // first prepare ends with the handle's own set-up done. After that, preparing a new B on the legacy default stream only
+    // enqueues (see prepare_enqueued).
+    const bool wait = s != nullptr || !c.prepared || Bd != B || biasd != bias || (multd != nullptr && multd != mult) || (shiftd != nullptr && shiftd != shift);
     TRY(c.wait_for_prepare(s));
     TRY(c.pack(Bd, d.ldb, nb > 1 ? d.b_batch_stride : 0, d.b_transposed != 0, d.b_k_interleave, (const int32_t *)biasd, s));
     TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));
     if (!wait)
-        return c.prepare_enqueued(s);
+        return c.prepare_enqueued();
     HIP_TRY(hipStreamSynchronize(s));
     c.prep_pending = false;
     return 0;
@@ -964,10 +974,11 @@ int mi355_gemmlowp_update_quant(mi355_gemm_handle *h, int32_t a_offset, int32_t 
     // behind a prepare that is still running elsewhere: it writes the column sums that are read here, and terms of its own
     // (with the offsets from before) over the ones that are written here
     hipStream_t s = (hipStream_t)stream;
-    TRY(c.wait_for_prepare(s));
+    if (s != nullptr)
+        TRY(c.prepare_over());
     TRY(c.refresh_colvec(s));
     TRY(c.refresh_qparams(s));
-    return c.prep_pending ? c.prepare_enqueued(s) : 0; // a run on a third stream comes behind both
+    return c.prep_pending ? c.prepare_enqueued() : 0; // a run on another stream comes behind both
 }
 
 static int set_gemm_strides(mi355_gemm_handle *h, int64_t lda, int64_t ldb, int64_t ldd, int64_t a_batch_stride,

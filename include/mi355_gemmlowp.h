@@ -167,9 +167,9 @@ int mi355_gemmlowp_create(const mi355_gemm_desc *desc, mi355_gemm_handle **out);
  * + set_quantized_bias (:963-968 of src/core/NEON/kernels/arm_gemm/quantized.cpp): re-lays B out for the
  * matrix cores, reduces its columns, and folds a_offset*colsum + a_offset*b_offset*K + bias into one per-column
  * int32 vector. bias (N int32) may be NULL; mult / shift (N int32 each) are read only when requant.per_channel.
- * Call again whenever B, bias or the per-channel vectors change (a non-constant B: before every run). The first call on a
- * handle returns when its work is done; later ones with device memory only enqueue, and runs on other streams wait for
- * them by themselves. */
+ * Call again whenever B, bias or the per-channel vectors change (a non-constant B: before every run). The call returns
+ * when its work is done - except that, after the first call on a handle, one on the default stream (NULL) with every
+ * operand in device memory only enqueues; runs on other streams wait for it by themselves. */
 int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *bias, const int32_t *mult,
                            const int32_t *shift, void *stream);
 
