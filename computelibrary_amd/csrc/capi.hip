@@ -176,6 +176,7 @@ struct GemmCore
     // event behind it, which runs on other streams wait for
     hipEvent_t  prep_done    = nullptr;
     bool        prep_pending = false;
+    bool        recorded = false; // a run was recorded into a graph, which may be launched at any time
     int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not written yet)
     bool        qp_scalar_set = false; // the per-tensor requantisation vectors hold qp_rq
     mi355_requant qp_rq{};
@@ -410,10 +411,16 @@ struct GemmCore
     // in front of whatever reads or writes on s what a prepare writes
     int wait_for_prepare(hipStream_t s)
     {
-        if (!prep_pending || s == nullptr)
+        if (s == nullptr)
             return 0;
-        if (capturing(s)) // a graph under construction cannot wait for work outside it, and may be launched on any stream
+        if (recorded ? prep_pending && capturing(s) : capturing(s))
+        {
+            // a graph under construction cannot wait for work outside it, and may be launched on any stream
+            recorded = true;
             return prepare_over();
+        }
+        if (!prep_pending)
+            return 0;
         HIP_TRY(hipStreamWaitEvent(s, prep_done, 0));
         return 0;
     }
@@ -941,8 +948,9 @@ int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *b
     TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * d.N, h->stageShift, s, &shiftd));
     // staging buffers are reused by later calls, so what was copied through them has to be read before this returns; and a
     // first prepare ends with the handle's own set-up done. After that, preparing a new B on the legacy default stream only
-    // enqueues (see prepare_enqueued).
-    const bool wait = s != nullptr || !c.prepared || Bd != B || biasd != bias || (multd != nullptr && multd != mult) || (shiftd != nullptr && shiftd != shift);
+    // enqueues (see prepare_enqueued) - unless there may be a graph with a run in it: nothing of this library is called when
+    // it is launched, so nothing could wait.
+    const bool wait = s != nullptr || !c.prepared || c.recorded || Bd != B || biasd != bias || (multd != nullptr && multd != mult) || (shiftd != nullptr && shiftd != shift);
     TRY(c.wait_for_prepare(s));
     TRY(c.pack(Bd, d.ldb, nb > 1 ? d.b_batch_stride : 0, d.b_transposed != 0, d.b_k_interleave, (const int32_t *)biasd, s));
     TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));

@@ -103,3 +103,18 @@ def test_run_recorded_behind_a_prepare(side, captured_on):
         c.Dd.zero_()
     graph.close()
     c.g.close()
+
+
+def test_graph_recorded_before_a_prepare():
+    """Nothing of the library is called when a graph is launched: a prepare behind a recorded run is over when it returns."""
+    c = _Changing(23)
+    announce("graph recorded before a prepare")
+    graph = _Graph(lambda s: c.g.run(c.Ad, c.Dd, None, s), c.other)
+    for which in (1, 0, 1):
+        c.prepare_held_up(which)
+        graph.launch(c.third)
+        c.third.synchronize()
+        c.check(which)
+        c.Dd.zero_()
+    graph.close()
+    c.g.close()
