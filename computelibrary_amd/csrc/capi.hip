@@ -49,8 +49,10 @@ int fail(const char *fmt, ...)
             return 1;        \
     } while (0)
 
-bool is_device_ptr(const void *p)
+bool is_device_ptr(const void *p, bool *managed = nullptr)
 {
+    if (managed)
+        *managed = false;
     if (p == nullptr)
         return false;
     hipPointerAttribute_t attr;
@@ -60,6 +62,8 @@ bool is_device_ptr(const void *p)
         (void)hipGetLastError(); // plain host memory: clear the sticky error
         return false;
     }
+    if (managed)
+        *managed = attr.type == hipMemoryTypeManaged || (attr.type == hipMemoryTypeDevice && attr.isManaged);
     return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
 }
 
@@ -112,19 +116,26 @@ struct DevBuf
     }
 };
 
-// brings `bytes` at `src` to the device if it is host memory; returns the device pointer to use
-int to_device(const void *src, size_t bytes, DevBuf &stage, hipStream_t s, const void **out, PtrKind *kind = nullptr)
+// brings `bytes` at `src` to the device if it is host memory; returns the device pointer to use. *host_may_write (when
+// given) is set, never cleared, if the host may write the memory that is read: the staging buffer or managed memory.
+int to_device(const void *src, size_t bytes, DevBuf &stage, hipStream_t s, const void **out, PtrKind *kind = nullptr,
+              bool *host_may_write = nullptr)
 {
     if (src == nullptr)
     {
         *out = nullptr;
         return 0;
     }
-    if (kind ? kind->is_device(src) : is_device_ptr(src))
+    bool managed = false;
+    if (kind ? kind->is_device(src) : is_device_ptr(src, &managed))
     {
+        if (host_may_write && managed)
+            *host_may_write = true;
         *out = src;
         return 0;
     }
+    if (host_may_write)
+        *host_may_write = true;
     TRY(stage.ensure(bytes));
     HIP_TRY(hipMemcpyAsync(stage.p, src, bytes, hipMemcpyHostToDevice, s));
     *out = stage.p;
@@ -942,15 +953,15 @@ int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *b
     const size_t           b_bytes = (size_t)(nb - 1) * d.b_batch_stride +
                            (d.b_transposed ? (size_t)(d.N - 1) * d.ldb + d.K : (size_t)(d.K - 1) * d.ldb + d.N);
     const void            *Bd, *biasd, *multd, *shiftd;
-    TRY(to_device(B, b_bytes, h->stageB, s, &Bd));
-    TRY(to_device(bias, sizeof(int32_t) * d.N, h->stageBias, s, &biasd));
-    TRY(to_device(c.rq.per_channel ? mult : nullptr, sizeof(int32_t) * d.N, h->stageMult, s, &multd));
-    TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * d.N, h->stageShift, s, &shiftd));
-    // staging buffers are reused by later calls, so what was copied through them has to be read before this returns; and a
-    // first prepare ends with the handle's own set-up done. After that, preparing a new B on the legacy default stream only
-    // enqueues (see prepare_enqueued) - unless there may be a graph with a run in it: nothing of this library is called when
-    // it is launched, so nothing could wait.
-    const bool wait = s != nullptr || !c.prepared || c.recorded || Bd != B || biasd != bias || (multd != nullptr && multd != mult) || (shiftd != nullptr && shiftd != shift);
+    // Staging buffers are reused by later calls and managed memory is written by the host, so what was read from them has to
+    // be read before this returns; and a first prepare ends with the handle's own set-up done. After that, preparing a new B
+    // on the legacy default stream only enqueues (see prepare_enqueued) - unless there may be a graph with a run in it:
+    // nothing of this library is called when it is launched, so nothing could wait.
+    bool wait = s != nullptr || !c.prepared || c.recorded;
+    TRY(to_device(B, b_bytes, h->stageB, s, &Bd, nullptr, &wait));
+    TRY(to_device(bias, sizeof(int32_t) * d.N, h->stageBias, s, &biasd, nullptr, &wait));
+    TRY(to_device(c.rq.per_channel ? mult : nullptr, sizeof(int32_t) * d.N, h->stageMult, s, &multd, nullptr, &wait));
+    TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * d.N, h->stageShift, s, &shiftd, nullptr, &wait));
     TRY(c.wait_for_prepare(s));
     TRY(c.pack(Bd, d.ldb, nb > 1 ? d.b_batch_stride : 0, d.b_transposed != 0, d.b_k_interleave, (const int32_t *)biasd, s));
     TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));

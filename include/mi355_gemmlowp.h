@@ -169,8 +169,10 @@ int mi355_gemmlowp_create(const mi355_gemm_desc *desc, mi355_gemm_handle **out);
  * int32 vector. bias (N int32) may be NULL; mult / shift (N int32 each) are read only when requant.per_channel.
  * Call again whenever B, bias or the per-channel vectors change (a non-constant B: before every run). The call returns
  * when its work is done - except that, after the first call on a handle, one on the default stream (NULL) with every
- * operand in device memory only enqueues, if no run of the handle has been recorded into a graph; runs on other streams
- * wait for it by themselves. */
+ * operand in device memory (not managed memory, which the host may write) only enqueues, if no run of the handle has been
+ * recorded into a graph; runs on other streams wait for it by themselves. The operands of such a call belong to the
+ * default stream's work until it is done, like A and D of a run: what overwrites or frees them from a stream that does not
+ * wait for the default stream (hipStreamNonBlocking) has to be ordered behind it. */
 int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *bias, const int32_t *mult,
                            const int32_t *shift, void *stream);
 
