@@ -188,8 +188,11 @@ struct GemmCore
     hipEvent_t  prep_done    = nullptr;
     bool        prep_pending = false;
     bool        recorded = false; // a run was recorded into a graph, which may be launched at any time
-    int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not written yet)
+    // What is known of buffers that are written once and then kept (see keep_flags)
+    int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not known)
+    bool        zeros_set = false, zerocol_set = false;
     bool        qp_scalar_set = false; // the per-tensor requantisation vectors hold qp_rq
+    bool        writes_recorded = false;
     mi355_requant qp_rq{};
     int     splitk = 1;      // K slices of the pipelined kernel
     int     splitk_plan = 1; // what the cost model chose with the tile shape (create()); prepare() checks it and allocates
@@ -453,6 +456,7 @@ struct GemmCore
     // after pack(): everything else a run reads
     int finish_prepare(const int32_t *mult_in, const int32_t *shift_in, hipStream_t s)
     {
+        keep_flags(s);
         has_pc = epi == EPI_FIXEDPOINT && rq.per_channel != 0;
         if (has_pc)
         {
@@ -476,11 +480,12 @@ struct GemmCore
             HIP_TRY(pack_b_narrow_launch(Bp.as<int8_t>(), Kp, Np, chunks, rows, K, patch_c, patch_c_true, Bn.as<int8_t>(), s));
         }
         TRY(set_fill(s));
-        if (path == MI355_PATH_SKINNY && zeros.p == nullptr)
+        if (path == MI355_PATH_SKINNY && !zeros_set)
         {
             // the streaming kernel fetches its per-row vector without asking whether there is one
             TRY(zeros.ensure(sizeof(int32_t) * SKINNY_MAX_M));
             HIP_TRY(fill_i32_launch(zeros.as<int32_t>(), 0, SKINNY_MAX_M, s));
+            zeros_set = true;
         }
         // A deep K under few output tiles: the pipelined kernel would leave most compute units idle, each of the others
         // walking the whole K. The K range is cut into slices that run as the batch entries of one S32 launch (the slice
@@ -493,23 +498,37 @@ struct GemmCore
         {
             const size_t ldp = ((size_t)N + 3) & ~(size_t)3;
             TRY(parts.ensure(sizeof(int32_t) * (size_t)splitk * M * ldp));
-            if (zerocol.p == nullptr)
+            if (!zerocol_set)
             {
                 TRY(zerocol.ensure(sizeof(int32_t) * (size_t)Np));
                 HIP_TRY(fill_i32_launch(zerocol.as<int32_t>(), 0, Np, s));
+                zerocol_set = true;
             }
         }
         TRY(refresh_qparams(s));
         refresh_names();
-        prepared = true;
+        keep_flags(s); // (what was set on the way here may only have been recorded)
         return 0;
+    }
+
+    // In front of what the flags decide and behind what sets them. Under capture a write only goes into a graph: it has not
+    // happened, and launching the graph repeats it whatever came after. From the first one on nothing is taken as known, and
+    // every prepare and update writes all of it.
+    void keep_flags(hipStream_t s)
+    {
+        if (!writes_recorded && s != nullptr && capturing(s))
+            writes_recorded = true;
+        if (writes_recorded)
+            fill_set = -1, zeros_set = zerocol_set = qp_scalar_set = false;
     }
 
     int set_fill(hipStream_t s)
     {
         TRY(fill.ensure(16));
-        if (fill_set != fill_byte)
-            HIP_TRY(fill_i32_launch(fill.as<int32_t>(), (int32_t)(0x01010101u * fill_byte), 4, s));
+        if (fill_set == fill_byte)
+            return 0;
+        fill_set = -1;
+        HIP_TRY(fill_i32_launch(fill.as<int32_t>(), (int32_t)(0x01010101u * fill_byte), 4, s));
         fill_set = fill_byte;
         return 0;
     }
@@ -534,7 +553,14 @@ struct GemmCore
         // per-tensor: what is there still holds unless the requantisation has changed
         if (!has_pc && qp_scalar_set && memcmp(&qp_rq, &rq, sizeof(rq)) == 0)
             return 0;
+        qp_scalar_set = false;
+        TRY(write_qparams(s));
         qp_scalar_set = !has_pc, qp_rq = rq;
+        return 0;
+    }
+
+    int write_qparams(hipStream_t s)
+    {
         qp_on = false;
         if (path == MI355_PATH_SKINNY && epi == EPI_FIXEDPOINT && !has_pc)
         {
@@ -968,7 +994,7 @@ int mi355_gemmlowp_prepare(mi355_gemm_handle *h, const void *B, const int32_t *b
     if (!wait)
         return c.prepare_enqueued();
     HIP_TRY(hipStreamSynchronize(s));
-    c.prep_pending = false;
+    c.prep_pending = false, c.prepared = true;
     return 0;
 }
 
@@ -995,8 +1021,10 @@ int mi355_gemmlowp_update_quant(mi355_gemm_handle *h, int32_t a_offset, int32_t 
     hipStream_t s = (hipStream_t)stream;
     if (s != nullptr)
         TRY(c.prepare_over());
+    c.keep_flags(s);
     TRY(c.refresh_colvec(s));
     TRY(c.refresh_qparams(s));
+    c.keep_flags(s);
     return c.prep_pending ? c.prepare_enqueued() : 0; // a run on another stream comes behind both
 }
 
@@ -1544,6 +1572,7 @@ int mi355_conv_prepare(mi355_conv_handle *h, const void *weights, const void *bi
     TRY(c.pack(wd, c.K, 0, true, 0, (const int32_t *)biasd, s));
     TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));
     HIP_TRY(hipStreamSynchronize(s));
+    c.prepared = true;
     return 0;
 }
 
@@ -1578,9 +1607,11 @@ int mi355_conv_update_quant(mi355_conv_handle *h, int32_t src_offset, int32_t we
         HIP_TRY(hipMemcpyAsync(c.mult.p, multd, sizeof(int32_t) * (size_t)c.N, hipMemcpyDeviceToDevice, s));
         HIP_TRY(hipMemcpyAsync(c.shift.p, shiftd, sizeof(int32_t) * (size_t)c.N, hipMemcpyDeviceToDevice, s));
     }
+    c.keep_flags(s);
     TRY(c.set_fill(s));
     TRY(c.refresh_colvec(s));
     TRY(c.refresh_qparams(s));
+    c.keep_flags(s);
     HIP_TRY(hipStreamSynchronize(s));
     return 0;
 }
