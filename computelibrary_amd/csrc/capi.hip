@@ -374,6 +374,7 @@ struct GemmCore
         if (has_bias)
             TRY(bias.ensure(sizeof(int32_t) * (size_t)N));
         constexpr int MOST = 32768; // batch entries along a grid dimension
+        // (one count for all parts, the last of which may be small: the workspace is sized by it)
         const int     splits = transposed ? 1 : pack_b_splits(Kp, Np, std::min(nb(), MOST));
         if (splits > 1)
             TRY(colpart.ensure(sizeof(int32_t) * (size_t)Np * nb() * splits));
@@ -387,7 +388,7 @@ struct GemmCore
             if (transposed)
                 HIP_TRY(pack_bt_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, out, f, s));
             else
-                HIP_TRY(pack_b_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, out, colpart.as<int32_t>(), f, s));
+                HIP_TRY(pack_b_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, splits, out, colpart.as<int32_t>(), f, s));
         }
         return 0;
     }

@@ -136,9 +136,10 @@ struct ColumnFinish
 };
 // nb matrices B [K][ldb] (row-major, N contiguous), b_bs bytes apart -> nb packed images of Np x Kp int8 (flip: xor 0x80)
 // and their columns' sums and terms. skinny: in matrix-core operand order, [Np/16][Kp/64][64 lanes][16 bytes]; else
-// [Np][Kp]. partial: nb * pack_b_splits() * Np words when that function returns more than 1.
+// [Np][Kp]. splits: the runs that K is packed in (pack_b_splits() of this or of a larger nb); partial: nb * splits * Np words
+// if there are several.
 int pack_b_splits(int Kp, int Np, int nb);
-int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
+int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny, int splits,
                   int8_t *out, int32_t *partial, const ColumnFinish &f, hipStream_t s);
 // the same from B given as [N][ldk] with K contiguous (conv weights [OFM][KH*KW*C])
 int pack_bt_launch(const void *Bt, int64_t ldk, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,

@@ -257,21 +257,23 @@ __global__ __launch_bounds__(256) void colsum_finish_kernel(const int32_t *__res
     finish_column(f, Np, b, j, sum);
 }
 
-// K runs of a packing launch: about four workgroups per compute unit (4096 x 4096: 15 runs)
+// K runs of a packing launch: about four workgroups per compute unit (4096 x 4096: 16 runs of 2 tiles), none of them empty
 int pack_b_splits(int Kp, int Np, int nb)
 {
     const int64_t columns = (int64_t)(Np / 64) * nb, tiles = Kp / 128;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(tiles, 1024 / columns));
+    const int64_t want = std::max<int64_t>(1, std::min<int64_t>(tiles, 1024 / columns)), per = (tiles + want - 1) / want;
+    return (int)((tiles + per - 1) / per);
 }
 
-int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
+int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny, int splits,
                   int8_t *out, int32_t *partial, const ColumnFinish &f, hipStream_t s)
 {
     if (Np % 64 || Kp % 128 || Np < N || Kp < K || nb < 1 || nb > 65535 || (kf > 1 && K % kf != 0))
         return (int)hipErrorInvalidValue;
-    const int tiles = Kp / 128, want = pack_b_splits(Kp, Np, nb), per = (tiles + want - 1) / want, splits = (tiles + per - 1) / per;
-    if (splits > 1 && partial == nullptr)
+    const int tiles = Kp / 128;
+    if (splits < 1 || splits > tiles || (splits > 1 && partial == nullptr))
         return (int)hipErrorInvalidValue;
+    const int  per = (tiles + splits - 1) / splits; // (a run that is left empty sums to zero)
     const dim3 grid(Np / 64, splits, nb), block(256);
     int32_t   *pt = splits > 1 ? partial : nullptr;
     if (skinny)

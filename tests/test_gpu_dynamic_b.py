@@ -100,3 +100,21 @@ def test_run_on_another_stream_waits_for_the_prepare(captured):
     want = A.astype(np.float64) @ Bs[1].astype(np.float64)
     np.testing.assert_array_equal(Dd.cpu().numpy(), want.astype(np.int32))
     g.close()
+
+
+def test_more_batch_entries_than_one_packing_launch_takes():
+    """32768 entries are packed at a time. What is left over is one entry, which alone would be packed in several runs of K: the
+    workspace of the column sums belongs to the count of the large parts."""
+    batch, M, N, K = 32769, 2, 16, 200
+    rng = np.random.default_rng(12)
+    A = rng.integers(-128, 128, size=(batch, M, K)).astype(np.int8)
+    B = rng.integers(-128, 128, size=(batch, K, N)).astype(np.int8)
+    announce("many batch entries", batch)
+    g = capi.Gemm(M, N, K, capi.S8, capi.S8, capi.S32, capi.EPI_S32, 3, 0, batch=batch, b_batched=True)
+    Ad, Bd = to_dev(A), to_dev(B)
+    for _ in range(2):
+        Dd = to_dev(np.full((batch, M, N), 77, np.int32))
+        g.prepare(Bd)
+        g.run(Ad, Dd)
+        np.testing.assert_array_equal(Dd.cpu().numpy(), np.matmul(A.astype(np.float32) + 3, B.astype(np.float32)).astype(np.int32))
+    g.close()
