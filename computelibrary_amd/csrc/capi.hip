@@ -197,6 +197,7 @@ struct GemmCore
     int     splitk = 1;      // K slices of the pipelined kernel
     int     splitk_plan = 1; // what the cost model chose with the tile shape (create()); prepare() checks it and allocates
     int         patch_c = 0, patch_c_true = 0; // a convolution's channels in the kernels' K, and how many of them count (0: dense)
+    int         panels_from = 0; // rows of the output from which the narrow kernel takes several panels of columns
     const void *rs_src = nullptr; // conv_row_terms
     ConvGeom    rs_geom{};
     int     k_const = 0;       // > 0: the K of the constant term a_offset * b_offset * K, where the kernels' K counts padded channels
@@ -472,7 +473,7 @@ struct GemmCore
             HIP_TRY(hipMemcpyAsync(shift.p, shift_in, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s));
         }
         // few output columns and a short K: the image of the B panel the narrow kernel copies into LDS
-        has_narrow = path == MI355_PATH_MFMA && patch_c > 0 && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192)) && narrow_panel_chunks(K) > 0;
+        has_narrow = path == MI355_PATH_MFMA && patch_c > 0 && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192 && M >= panels_from)) && narrow_panel_chunks(K) > 0;
         if (has_narrow)
         {
             const int chunks = narrow_panel_chunks(K);
@@ -1470,10 +1471,14 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
             // 112 x 112 x 24 -> 32, 3 x 3, stride 2: 12.2 -> 11.1. Not: 112 x 112 x 8 -> 64, 3 x 3: 30.9 -> 31.8, 5 x 5: 32.7 ->
             // 34.3; 56 x 56 x 24, 3 x 3: 14.3 -> 15.0. Less than 8 bytes of a row save nothing where the padded K fits one batch of
             // the narrow kernel's k blocks (192) either way: 224 x 224 x 1 -> 64, 3 x 3: 91.4 -> 96.1.
+            // Not either where the row's K just fits that one batch and the padded taps fit two, under few output rows: the form
+            // for one batch, which knows several panels, starts half a microsecond later (6272 rows of 20 -> 32 channels, 3 x 3,
+            // stride 2, channels padded 6.2, rows 6.5; 12544 rows: 7.1, 6.9).
             mi355_conv_desc dr = d;
             dr.C = round_up(d.KW * d.C, 16), dr.W = h->geom_true.OW, dr.KW = dr.stride_x = dr.dilation_x = 1, dr.pad_left = dr.pad_right = 0;
             const int64_t row_bytes = (int64_t)dr.W * dr.C, pad_bytes = (int64_t)d.W * dp.C, k_row = (int64_t)d.KH * dr.C, k_pad = (int64_t)d.KH * d.KW * dp.C;
-            if (h->c_pad && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
+            const bool    one_batch_late = d.OFM <= 64 && k_row <= 192 && k_pad > 192 && k_pad <= 384 && (int64_t)d.batch * gp.OH * gp.OW < 8192;
+            if (h->c_pad && !one_batch_late && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
                 (d.KW * d.C >= 8 || k_pad > 192) &&
                 (int64_t)d.batch * d.H * row_bytes < ((int64_t)1 << 31))
             {
@@ -1493,6 +1498,11 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
     c.M = (int)M64, c.N = d.OFM, c.K = (int)K64, c.batch = 1;
     c.k_const = h->c_pad ? d.KH * d.KW * d.C : 0;
     c.patch_c = h->geom.C, c.patch_c_true = h->geom.c_true;
+    // Patch rows bring a short K to convolutions of few channels whatever their size; one panel after the other pays from some
+    // rows per compute unit on (us, panels against the pipelined kernel, 128 and 256 columns, 3 channels, 5 x 5, stride 2: 1568
+    // rows 8.0 / 5.9 and 11.1 / 5.9; 12544: 8.3 / 6.9 and 11.7 / 8.4; 25088: 9.0 / 8.7 and 12.5 / 10.6; 18 channels, 3 x 3, 12544: 8.7 / 8.5
+    // and 11.9 / 9.8; 25088: 9.9 / 9.9 and 13.3 / 13.6)
+    c.panels_from = h->patch_rows ? 16384 : 0;
     c.epi = f32 ? EPI_F32 : EPI_FIXEDPOINT, c.dst_dtype = d.dst_dtype;
     c.flip_a = d.src_dtype == MI355_U8, c.flip_b = d.weights_dtype == MI355_U8;
     c.a_offset = d.src_offset, c.b_offset = d.weights_offset;

@@ -36,6 +36,20 @@ def test_layout_conversion(C, H, W, OFM):
     _check(C + W + OFM, (3, H, W, C), (OFM, 1, 1, C), (1, 1), (0, 0, 0, 0), (1, 1), np.int8, np.int8, capi.NCHW)
 
 
+@pytest.mark.parametrize("shape,wshape,kernel", [
+    ((1, 255, 253, 3), (96, 5, 5, 3), "implicit_pp"),       # 16256 output rows: one column panel after the other does not pay yet
+    ((1, 255, 255, 3), (96, 5, 5, 3), "implicit_narrow"),   # 16384
+    ((2, 7, 9, 4), (256, 5, 5, 4), "implicit_pp"),
+    ((2, 9, 9, 20), (64, 3, 3, 20), "implicit_narrow"),     # K = 192 by rows, 288 by taps: taps
+    ((1, 181, 181, 20), (32, 3, 3, 20), "implicit_"),       # 8281 rows: rows
+])
+@pytest.mark.parametrize("dt,w_dt", [(np.int8, np.int8), (np.uint8, np.uint8)])
+def test_patch_rows_follow_the_size(shape, wshape, kernel, dt, w_dt):
+    k = wshape[1]
+    name = _check(800 + shape[1], shape, wshape, (2, 2), (k // 2,) * 4, (1, 1), dt, w_dt, capi.NHWC)
+    assert name.startswith(kernel), name
+
+
 def _check(seed, shape, wshape, stride, pad, dil, dt, w_dt, layout):
     rng = np.random.default_rng(seed)
     info, w_info = np.iinfo(dt), np.iinfo(w_dt)
@@ -46,6 +60,7 @@ def _check(seed, shape, wshape, stride, pad, dil, dt, w_dt, layout):
     scales = rng.uniform(0.5, 2.0, size=wshape[0]) * 40.0 / ((wshape[1] * wshape[2] * wshape[3]) ** 0.5 * 74.0 * 74.0)
     mult, shift = oracle.calculate_quantized_multipliers(1.0, scales, 1.0)
     announce("conv few channels / layouts", shape, wshape, stride, pad, dil, dt.__name__, w_dt.__name__, layout)
-    got, _ = run_conv(src, w, bias, zp, w_zp, mult, shift, ozp, info.min, info.max, stride, pad, dil, layout=layout)
+    got, name = run_conv(src, w, bias, zp, w_zp, mult, shift, ozp, info.min, info.max, stride, pad, dil, layout=layout)
     want = oracle.conv_nhwc_direct(src, w, bias, zp, w_zp, mult, shift, ozp, info.min, info.max, stride, pad, dil)
     np.testing.assert_array_equal(got, want)
+    return name
