@@ -303,15 +303,13 @@ struct GemmCore
                 double best_cost = 0;
                 for (int i = 0; i < dma_num_configs(); ++i)
                 {
-                    const MfmaConfig c = dma_config(i);
+                    const MfmaConfig c = dma_config(i, patch_c > 0);
                     if ((N <= 64 && c.BN > 64) || Kp % c.BK != 0)
                         continue;
                     const double tiles   = (double)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN) * batch;
                     const int    occ_lds = (160 * 1024) / c.lds_bytes, occ_wav = 32 / c.waves;
                     const double occ     = std::max(1, std::min(occ_lds, occ_wav));
                     const int    nk      = (K + c.BK - 1) / c.BK;
-                    // (the loader of a convolution decodes taps: 6272 x 256 x 2304 and 25088 x 128 x 1152, 1.15 of the dense)
-                    const double us_step = patch_c > 0 ? 1.15 * c.us_step : c.us_step;
                     for (int want = 1; want <= MOST_SLICES; ++want)
                     {
                         // (slices of equal whole K steps but the last, none of them empty)
@@ -322,7 +320,7 @@ struct GemmCore
                             continue;
                         const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
                         const double finish = sl > 1 ? 2.8 + 0.12 * sl + (double)sl * M * N * 1e-6 : 0.0;
-                        const double cost   = (std::ceil(per_cu / occ) * c.us_tile + per_cu * per * us_step * (1.0 + c.us_load * load) + finish) *
+                        const double cost   = (std::ceil(per_cu / occ) * c.us_tile + per_cu * per * c.us_step * (1.0 + c.us_load * load) + finish) *
                                             (sl > 1 ? 1.125 : 1.0);
                         if (best < 0 || cost < best_cost)
                             best = i, best_cost = cost, splitk_plan = sl;
@@ -1519,8 +1517,9 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
         return 1;
     }
     // The patch matrix is only materialised on request (path 1) or where the loaders' reciprocal divisions would not be
-    // exact. Channel counts that are not a multiple of 16 take the register-staged kernel, whose loader then looks up
-    // every byte; a weights offset adds a pass over the source for the patches' row sums.
+    // exact. Channel counts that are not a multiple of 16 and are not padded (see above: a request for the caller's tensor as
+    // it is, or sizes beyond 31 bits) take the register-staged kernel, whose loader looks up every byte; there, and in K slices to
+    // a float destination, a weights offset costs a pass over the source for the patches' row sums.
     h->implicit      = d.path != MI355_CONV_EXPLICIT && (h->c_pad > 0 || conv_fast_div_ok(d, h->geom));
     h->geom.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
     if (h->implicit)

@@ -956,12 +956,17 @@ static const void *const g_rowsum_256x128x128[3][2] = {
 // What a tile and a K step of each configuration cost, in microseconds, and by what share a K step gets slower as the chip
 // fills: read off sweeps over the depth of K (64 x 64, 3 stages: 5.75 us at K = 512, 7.27 at 1024, 10.0 at 2048) and over the
 // number of tiles. The 6-stage ring never was the faster one of its tile in them, by 0.5 us, with B from HBM or not.
+// The loader of a convolution has its own prices, from a sweep of every tile and slice count over 172 convolutions (16 to 2048 channels,
+// 64 to 103k rows, 16 to 512 columns): it works at the decoding of taps and at per-lane addresses whether the chip is full or
+// not, so few tiles save little: on an idle chip a step costs 1.4 (64 x 64) to 2.3 times (256 x 128) the dense one. (The dense prices times
+// 1.15 took 34300 x 24 x 3024 to the 256-deep tile: 33.2 us, 128 x 64 24.8; and 392 x 512 x 2304 whole: 12.5 us, 4 slices 9.9.)
 struct DmaCost
 {
     double us_tile, us_step, us_load;
 };
-static const DmaCost g_dma_cost[] = {
-    {5.6, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.5, 0.385, 0.35}, {2.7, 0.354, 0.35}, {3.2, 0.354, 0.35}, {4.1, 0.618, 0.35},
+static const DmaCost g_dma_cost[2][6] = {
+    {{5.6, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.5, 0.385, 0.35}, {2.7, 0.354, 0.35}, {3.2, 0.354, 0.35}, {4.1, 0.618, 0.35}},
+    {{5.8, 1.07, 0.25}, {4.1, 0.81, 0.13}, {3.4, 0.585, 0.10}, {3.0, 0.50, 0.0}, {3.5, 0.50, 0.0}, {3.4, 1.03, 0.18}},
 };
 
 static const DmaEntry g_dma[] = {
@@ -977,13 +982,14 @@ int dma_num_configs()
 {
     return (int)(sizeof(g_dma) / sizeof(g_dma[0]));
 }
-MfmaConfig dma_config(int idx)
+MfmaConfig dma_config(int idx, bool conv)
 {
     MfmaConfig c = g_dma[idx].cfg;
     c.waves      = g_dma[idx].threads / 64;
     c.lds_bytes  = g_dma[idx].lds_bytes;
-    static_assert(sizeof(g_dma_cost) / sizeof(g_dma_cost[0]) == sizeof(g_dma) / sizeof(g_dma[0]), "one price per configuration");
-    c.us_tile = g_dma_cost[idx].us_tile, c.us_step = g_dma_cost[idx].us_step, c.us_load = g_dma_cost[idx].us_load;
+    static_assert(sizeof(g_dma_cost[0]) / sizeof(g_dma_cost[0][0]) == sizeof(g_dma) / sizeof(g_dma[0]), "one price per configuration");
+    const DmaCost &cost = g_dma_cost[conv ? 1 : 0][idx];
+    c.us_tile = cost.us_tile, c.us_step = cost.us_step, c.us_load = cost.us_load;
     return c;
 }
 

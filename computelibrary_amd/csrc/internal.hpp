@@ -102,7 +102,7 @@ int         mfma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const Gemm
 
 // gemm_dma.hip — same contract as mfma_launch; additionally needs 16-byte aligned A rows, K % 16 == 0 and args.fill16
 int         dma_num_configs();
-MfmaConfig  dma_config(int idx);
+MfmaConfig  dma_config(int idx, bool conv = false); // conv: priced for the implicit convolution's loader
 int         dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &args, int batch, hipStream_t s);
 
 // gemm_narrow.hip — N <= 64, K <= 1152, 16-byte aligned operands: A straight from global memory into the matrix cores'
