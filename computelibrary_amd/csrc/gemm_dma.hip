@@ -966,7 +966,7 @@ struct DmaCost
 };
 static const DmaCost g_dma_cost[2][6] = {
     {{5.6, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.5, 0.385, 0.35}, {2.7, 0.354, 0.35}, {3.2, 0.354, 0.35}, {4.1, 0.618, 0.35}},
-    {{5.8, 1.07, 0.25}, {4.1, 0.81, 0.13}, {3.4, 0.585, 0.10}, {3.0, 0.50, 0.0}, {3.5, 0.50, 0.0}, {3.4, 1.03, 0.18}},
+    {{6.0, 1.07, 0.25}, {4.1, 0.81, 0.13}, {3.4, 0.585, 0.10}, {3.0, 0.50, 0.0}, {3.5, 0.50, 0.0}, {3.4, 1.03, 0.18}},
 };
 
 static const DmaEntry g_dma[] = {
