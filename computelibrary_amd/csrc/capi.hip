@@ -289,8 +289,8 @@ struct GemmCore
             };
             // The pipelined kernel's tile is chosen with a small cost model in microseconds, fitted to sweeps of every tile
             // shape and slice count over 33 shapes (M 65-2048, N 24-12288, K 512-11008, B hot and rotated through HBM): a tile
-            // costs MfmaConfig::us_tile for its start-up and epilogue, shared by the workgroups that fit a compute unit
-            // together, plus us_step for every K step, which a full chip slows down by a share us_load of it (L2, HBM and
+            // costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that fit a compute unit
+            // together share all but us_more, plus us_step for every K step, which a full chip slows down by a share us_load of it (L2, HBM and
             // the power limit are shared by all compute units).
             // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
             // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.8 us for the launch
@@ -320,8 +320,8 @@ struct GemmCore
                             continue;
                         const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
                         const double finish = sl > 1 ? 2.8 + 0.12 * sl + (double)sl * M * N * 1e-6 : 0.0;
-                        const double cost   = (std::ceil(per_cu / occ) * c.us_tile + per_cu * per * c.us_step * (1.0 + c.us_load * load) + finish) *
-                                            (sl > 1 ? 1.125 : 1.0);
+                        const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load);
+                        const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 1.125 : 1.0);
                         if (best < 0 || cost < best_cost)
                             best = i, best_cost = cost, splitk_plan = sl;
                     }
