@@ -435,22 +435,39 @@ struct GemmCore
         }
         if (!prep_pending)
             return 0;
-        HIP_TRY(hipStreamWaitEvent(s, prep_done, 0));
+        // (once it is over no later run waits again: 0.1 us of host time each)
+        const hipError_t e = event_call(hipEventQuery);
+        if (e == hipSuccess)
+            prep_pending = false;
+        else if (e == hipErrorNotReady)
+            HIP_TRY(hipStreamWaitEvent(s, prep_done, 0));
+        else
+            HIP_TRY(e);
         return 0;
     }
 
-    // the host waits, whatever the thread is recording
+    // the host waits
     int prepare_over()
     {
         if (!prep_pending)
             return 0;
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-        const hipError_t e = hipEventSynchronize(prep_done);
-        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-        HIP_TRY(e);
+        HIP_TRY(event_call(hipEventSynchronize));
         prep_pending = false;
         return 0;
+    }
+
+    // `call` on the prepare's event, whatever the thread is recording
+    hipError_t event_call(hipError_t (*call)(hipEvent_t))
+    {
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        hipError_t           e    = hipThreadExchangeStreamCaptureMode(&mode);
+        if (e != hipSuccess)
+            return e;
+        const hipError_t got = call(prep_done);
+        if (got == hipErrorNotReady)
+            (void)hipGetLastError(); // not an error: the launches behind it ask for the last one
+        e = hipThreadExchangeStreamCaptureMode(&mode);
+        return e != hipSuccess ? e : got;
     }
 
     // after pack(): everything else a run reads
