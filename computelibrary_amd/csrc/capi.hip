@@ -515,6 +515,8 @@ struct GemmCore
         {
             const size_t ldp = ((size_t)N + 3) & ~(size_t)3;
             TRY(parts.ensure(sizeof(int32_t) * (size_t)splitk * M * ldp));
+            if (own_row_terms())
+                TRY(rowvec.ensure(sizeof(int32_t) * (size_t)M));
             if (!zerocol_set)
             {
                 TRY(zerocol.ensure(sizeof(int32_t) * (size_t)Np));
@@ -629,6 +631,10 @@ struct GemmCore
         p.act_twice           = act_twice ? 1 : 0;
     }
 
+    // K slices to a float destination take the row terms from a pass (see run_dense) that the same product whole would not
+    // need: the vector is there from prepare on, so that a first run can be recorded and a run_noalloc needs no workspace
+    bool own_row_terms() const { return splitk > 1 && epi == EPI_F32; }
+
     // A, D and bias_f32 are device pointers here
     int run_dense(const int8_t *A, int64_t lda, int64_t a_bs, void *D, int64_t ldd, int64_t d_bs,
                   const float *bias_f32, hipStream_t s)
@@ -650,7 +656,7 @@ struct GemmCore
         const bool need_rowvec = b_off_eff() != 0 && !rowsum_in_kernel;
         // the two workspaces of a run: owned by the handle and grown on demand, or carved out of a buffer the caller of
         // this function brings (ext_ws != nullptr: nothing is allocated, sizes beyond ext_ws_bytes are an error)
-        const size_t rv_bytes = need_rowvec ? ((sizeof(int32_t) * (size_t)M * batch + 255) & ~(size_t)255) : 0;
+        const size_t rv_bytes = need_rowvec && !own_row_terms() ? ((sizeof(int32_t) * (size_t)M * batch + 255) & ~(size_t)255) : 0;
         const size_t ap_bytes = direct ? 0 : (size_t)batch * M * Kp;
         int32_t     *rv       = nullptr;
         int8_t      *ap       = nullptr;
@@ -667,12 +673,14 @@ struct GemmCore
         }
         else
         {
-            if (need_rowvec)
+            if (rv_bytes > 0)
                 TRY(rowvec.ensure(rv_bytes));
             if (!direct)
                 TRY(Ap.ensure(ap_bytes));
             rv = rowvec.as<int32_t>(), ap = Ap.as<int8_t>();
         }
+        if (own_row_terms())
+            rv = rowvec.as<int32_t>();
         if (!direct)
         {
             // rows not dword aligned: padded, sign-normalised copy (and the row sums in the same pass)

@@ -5,8 +5,9 @@ import pytest
 
 import oracle
 from computelibrary_amd import capi
-from gpu_util import announce, run_gemm
+from gpu_util import announce, run_gemm, to_dev, torch_dev
 from test_gpu_conv import run_conv
+from test_gpu_prepare_order import _Graph
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +53,41 @@ def test_convolution(shape, OFM, k, dt, w_dt):
     got, name = run_conv(src, w, bias, zp, w_zp, mult, shift, 5, info.min, info.max, (1, 1), (p, p, p, p))
     assert "_splitk" in name, name
     np.testing.assert_array_equal(got, oracle.conv_nhwc_direct(src, w, bias, zp, w_zp, mult, shift, 5, info.min, info.max, (1, 1), (p, p, p, p)))
+
+
+def test_float_slices_with_an_offset_need_no_workspace_in_the_run():
+    """Their row terms come from a pass over A (the planes must not mix them into the product), into a vector that prepare has
+    made: a first run is recorded, and run_noalloc is not refused while the workspace is in use on another stream."""
+    torch = torch_dev()
+    M, N, K = 190, 130, 3008
+    rng = np.random.default_rng(40)
+    A, B = (rng.integers(-128, 128, size=s).astype(np.int8) for s in ((M, K), (K, N)))
+    want = np.asarray(oracle.gemmlowp_f32(A, B, None, -5, 9, 1e-4)).view(np.uint32)
+    busy = capi.Gemm(1024, 1024, 4000, capi.S8, capi.S8, capi.S32, capi.EPI_S32, 3, 4, lda=4003)  # (a padded copy of A)
+    A_busy, B_busy = (torch.zeros(s, dtype=torch.int8, device="cuda") for s in ((1024, 4003), (4000, 1024)))
+    D_busy = torch.zeros((1024, 1024), dtype=torch.int32, device="cuda")
+    busy.prepare(B_busy)
+    g = capi.Gemm(M, N, K, capi.S8, capi.S8, capi.F32, capi.EPI_F32, -5, 9, scale=1e-4)
+    Ad, Bd = to_dev(A), to_dev(B)
+    Dd = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    g.prepare(Bd)
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    announce("float slices, workspace")
+    graph = _Graph(lambda s: g.run(Ad, Dd, None, s), s2)
+    assert "_splitk" in g.kernel_name, g.kernel_name
+    for _ in range(2):
+        graph.launch(s2)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(Dd.cpu().numpy().view(np.uint32), want)
+        Dd.zero_()
+        torch.cuda.synchronize()
+    with torch.cuda.stream(s1):
+        torch.cuda._sleep(50_000_000)
+    busy.run_noalloc(A_busy, D_busy, stream=s1.cuda_stream)
+    g.run_noalloc(Ad, Dd, stream=s2.cuda_stream)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(Dd.cpu().numpy().view(np.uint32), want)
+    graph.close()
+    g.close()
+    busy.close()
