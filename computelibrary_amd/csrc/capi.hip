@@ -1503,7 +1503,8 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
             const bool    one_batch_late = d.OFM <= 64 && k_row <= 192 && k_pad > 192 && k_pad <= 384 && (int64_t)d.batch * gp.OH * gp.OW < 8192;
             if (h->c_pad && !one_batch_late && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
                 (d.KW * d.C >= 8 || k_pad > 192) &&
-                (int64_t)d.batch * d.H * row_bytes < ((int64_t)1 << 31))
+                (int64_t)d.batch * d.H * row_bytes < ((int64_t)1 << 31) &&
+                patch_rows_fit((int64_t)d.batch * d.H, d.W, d.C, dr.W, d.stride_x, d.pad_left, dr.C))
             {
                 conv_geom(dr, gp);
                 if (conv_fast_div_ok(dr, gp))

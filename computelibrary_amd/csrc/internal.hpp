@@ -171,6 +171,8 @@ int transpose_words_launch(const void *src, void *dst, int batch, int R, int C, 
 int channel_pad_launch(const void *src, void *dst, int64_t runs, int C, int Cp, uint8_t fill, hipStream_t s);
 // `rows` image rows of W pixels of C bytes -> per row OW runs of Cr bytes (a multiple of 16), run ox starting stride_x * ox - pad_left
 // pixels into the row, `fill` where that lies outside
+// (patch_rows_fit: whether the kernel's arithmetic takes these sizes)
+bool patch_rows_fit(int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr);
 int patch_rows_launch(const void *src, void *dst, int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr, uint8_t fill, hipStream_t s);
 // dst[s * dst_stride + c] = src[s * src_stride + c] for s < segments, c < seg (bytes)
 // dense F32 [batch][M][N] -> F16 destination (row stride ldh, batch stride, in elements), optionally added to its

@@ -1140,16 +1140,22 @@ __global__ __launch_bounds__(256) void patch_rows_kernel(const uint8_t *__restri
     }
     *(v4i *)(dst + ((int64_t)row * units + u) * 16) = v;
 }
-int patch_rows_launch(const void *src, void *dst, int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr, uint8_t fill, hipStream_t s)
+// what the kernel's 32-bit arithmetic takes
+bool patch_rows_fit(int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr)
 {
     const int64_t units = (int64_t)OW * (Cr / 16), bpr = (units + 255) / 256;
-    if (rows < 1 || W < 1 || C < 1 || OW < 1 || Cr < 16 || Cr % 16 != 0 || ((uintptr_t)dst & 15) != 0 || rows * bpr > 0x7fffffff ||
-        units * 16 > 0x7fffffff || (int64_t)W * C > 0x7fffffff || ((int64_t)OW * stride_x + pad_left) * C + Cr > 0x7fffffff)
+    return rows >= 1 && W >= 1 && C >= 1 && OW >= 1 && Cr >= 16 && Cr % 16 == 0 && rows * bpr <= 0x7fffffff && units * 16 <= 0x7fffffff &&
+           (int64_t)W * C <= 0x7fffffff && ((int64_t)OW * stride_x + pad_left) * C + Cr <= 0x7fffffff &&
+           units * (Cr / 16) < ((int64_t)1 << 32);
+}
+
+int patch_rows_launch(const void *src, void *dst, int64_t rows, int W, int C, int OW, int stride_x, int pad_left, int Cr, uint8_t fill, hipStream_t s)
+{
+    if (!patch_rows_fit(rows, W, C, OW, stride_x, pad_left, Cr) || ((uintptr_t)dst & 15) != 0)
         return (int)hipErrorInvalidValue;
+    const int64_t  units = (int64_t)OW * (Cr / 16), bpr = (units + 255) / 256;
     const int      per   = Cr / 16;
     const uint32_t magic = per == 1 ? 0u : (uint32_t)(((uint64_t)1 << 32) / (uint64_t)per) + 1u; // exact while units * per < 2^32
-    if (units * per >= ((int64_t)1 << 32))
-        return (int)hipErrorInvalidValue;
     patch_rows_kernel<<<dim3((unsigned)(rows * bpr)), dim3(256), 0, s>>>((const uint8_t *)src, (uint8_t *)dst, W * C, stride_x * C, pad_left * C, per,
                                                                          magic, (int)units, (uint32_t)bpr, 0x01010101u * fill);
     return launch_status();

@@ -50,6 +50,11 @@ def test_patch_rows_follow_the_size(shape, wshape, kernel, dt, w_dt):
     assert name.startswith(kernel), name
 
 
+def test_a_step_too_long_for_patch_rows():
+    """One output column and a step whose bytes pass 31 bits: the channels are padded instead"""
+    _check(900, (2, 5, 6, 3), (24, 3, 3, 3), (800_000_000, 1), (1, 1, 1, 1), (1, 1), np.int8, np.int8, capi.NHWC)
+
+
 def _check(seed, shape, wshape, stride, pad, dil, dt, w_dt, layout):
     rng = np.random.default_rng(seed)
     info, w_info = np.iinfo(dt), np.iinfo(w_dt)
