@@ -15,10 +15,10 @@ pytestmark = pytest.mark.gpu
 CASES = [
     ((2, 9, 11, 16), (24, 3, 3, 16), (1, 1), (1, 1, 1, 1), (1, 1), "implicit_narrow"),     # K = 144 of 192
     ((3, 12, 10, 24), (40, 3, 3, 24), (2, 1), (1, 0, 1, 2), (1, 1), "implicit_narrow"),    # 24 channels in 32, K = 288
-    ((1, 17, 15, 40), (64, 5, 5, 40), (1, 2), (2, 2, 2, 2), (1, 1), "implicit_"),          # 40 in 48, K = 1200: past the narrow kernel
+    ((1, 17, 15, 40), (64, 5, 5, 40), (1, 2), (2, 2, 2, 2), (1, 1), "implicit_pp"),        # 40 in 48, K = 1200: past the narrow kernel
     ((2, 20, 20, 64), (200, 1, 1, 64), (1, 1), (0, 0, 0, 0), (1, 1), "implicit_narrow"),   # 4 panels
     ((2, 8, 8, 128), (64, 3, 3, 128), (1, 1), (1, 1, 1, 1), (1, 1), "implicit_narrow"),    # 6 batches of k blocks
-    ((4, 56, 57, 64), (48, 3, 3, 64), (1, 1), (1, 1, 1, 1), (1, 1), "implicit_"),          # tiles for the narrow kernel or the band
+    ((4, 56, 57, 64), (48, 3, 3, 64), (1, 1), (1, 1, 1, 1), (1, 1), "implicit_narrow"),    # images below the band form's
     ((32, 56, 56, 60), (33, 3, 3, 60), (1, 1), (1, 1, 1, 1), (1, 1), "implicit_band"),     # band, 60 channels in 64
     ((32, 56, 56, 64), (130, 1, 1, 64), (1, 1), (0, 0, 0, 0), (1, 1), "implicit_band"),    # band, 3 panels
     ((5, 13, 12, 32), (70, 3, 3, 32), (1, 1), (1, 1, 1, 1), (2, 1), "implicit_pp"),        # pipelined, K = 288 of 3 steps

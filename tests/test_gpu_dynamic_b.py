@@ -1,5 +1,5 @@
-"""B that changes between runs: prepare() on a handle that is already prepared packs all batch entries in one launch and only
-enqueues. Sizes around the packing kernel's tile (64 columns x 128 of K) and its K runs, both operand orders, both packed
+"""B that changes between runs: prepare() on a handle that is already prepared packs all batch entries in one launch and, on the
+default stream, only enqueues. Sizes around the packing kernel's tile (64 columns x 128 of K) and its K runs, both operand orders, both packed
 layouts; and a run on another stream, plain and under graph capture, behind a prepare that has not been waited for."""
 import numpy as np
 import pytest
@@ -7,6 +7,7 @@ import pytest
 import oracle
 from computelibrary_amd import capi
 from gpu_util import announce, to_dev, torch_dev
+from test_gpu_prepare_order import _Graph
 
 pytestmark = pytest.mark.gpu
 
@@ -78,7 +79,7 @@ def test_run_on_another_stream_waits_for_the_prepare(captured):
     g = capi.Gemm(M, N, K, capi.S8, capi.S8, capi.S32, capi.EPI_S32)
     Ad, Bd = to_dev(A), [to_dev(b) for b in Bs]
     Dd = torch.zeros((M, N), dtype=torch.int32, device="cuda")
-    here, other = torch.cuda.Stream(), torch.cuda.Stream()
+    here, other, third = torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()
     torch.cuda.synchronize()
     g.prepare(Bd[0], stream=here.cuda_stream)
     g.run(Ad, Dd, None, other.cuda_stream)
@@ -86,19 +87,20 @@ def test_run_on_another_stream_waits_for_the_prepare(captured):
     want = A.astype(np.float64) @ Bs[0].astype(np.float64)
     np.testing.assert_array_equal(Dd.cpu().numpy(), want.astype(np.int32))
     announce("another stream, captured", captured)
-    graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(here):
         torch.cuda._sleep(20_000_000)  # what is in front of the prepare takes some milliseconds
     g.prepare(Bd[1], stream=here.cuda_stream)
     if captured:
-        with torch.cuda.graph(graph, stream=other):
-            g.run(Ad, Dd, None, torch.cuda.current_stream().cuda_stream)
-        graph.replay()
+        # (not torch.cuda.graph, which synchronises the device first: the prepare would be over)
+        graph = _Graph(lambda s: g.run(Ad, Dd, None, s), other)
+        graph.launch(third)
     else:
         g.run(Ad, Dd, None, other.cuda_stream)
     torch.cuda.synchronize()
     want = A.astype(np.float64) @ Bs[1].astype(np.float64)
     np.testing.assert_array_equal(Dd.cpu().numpy(), want.astype(np.int32))
+    if captured:
+        graph.close()
     g.close()
 
 

@@ -38,7 +38,8 @@ def test_dense(M, N, K, dt):
         np.testing.assert_array_equal(got.view(np.uint32), np.asarray(oracle.gemmlowp_f32(A, B, None, ao, bo, 1e-4)).view(np.uint32))
 
 
-@pytest.mark.parametrize("shape,OFM,k", [((2, 9, 10, 304), 24, 5), ((1, 14, 14, 336), 130, 3), ((3, 7, 7, 432), 56, 5)])
+@pytest.mark.parametrize("shape,OFM,k", [((2, 9, 10, 304), 24, 5), ((1, 14, 14, 336), 130, 3), ((3, 7, 7, 432), 56, 5),
+                                         ((2, 9, 10, 300), 24, 5), ((1, 14, 14, 330), 130, 3)])  # channels padded to 304 and 336
 @pytest.mark.parametrize("dt,w_dt", [(np.int8, np.int8), (np.uint8, np.uint8)])
 def test_convolution(shape, OFM, k, dt, w_dt):
     rng = np.random.default_rng(sum(shape) + OFM)
