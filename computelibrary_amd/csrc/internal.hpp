@@ -118,7 +118,7 @@ bool narrow_applies(const GemmArgs &args);
 // *band (when given): whether the launch took the form that stages a band of input rows in LDS (large images)
 int  narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, bool *band = nullptr);
 
-// gemm_skinny.hip — M <= 64, B packed in matrix-core operand order (see pack_b_skinny)
+// gemm_skinny.hip — M <= 64, B packed in matrix-core operand order (see pack_b_launch)
 constexpr int SKINNY_MAX_M = 64;
 // *variant (when given): a static string naming the form of the kernel that ran
 int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStream_t s, const char **variant = nullptr);

@@ -988,7 +988,7 @@ __global__ __launch_bounds__(256) void f32_to_f16_kernel(const float *__restrict
 int f32_to_f16_launch(const float *dense_f32, void *half_matrix, int batch, int M, int N, int64_t ldh,
                       int64_t h_batch_stride, bool accumulate, float act_min, float act_max, hipStream_t s)
 {
-        const int64_t rows = (int64_t)batch * M;
+    const int64_t rows = (int64_t)batch * M;
     if (rows <= 0 || N <= 0)
         return 0;
     // 8 elements per thread from two waves per compute unit on. GEMM and rounding, us, 1 element -> 8: 2048 x 8192 106.9 -> 82.2,

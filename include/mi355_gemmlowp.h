@@ -28,8 +28,10 @@
  *    between two runs of one handle, pass a different address first or use a new handle.
  *  - All functions return 0 on success, non-zero on failure; mi355_last_error() then returns
  *    a thread-local message. No exception crosses this boundary.
- *  - A handle is single-caller: one call at a time per handle. Distinct handles may be used
- *    from distinct threads / streams.
+ *  - A handle is single-caller: one call at a time per handle, and its runs share workspaces that the
+ *    handle owns (planes of K slices, row sums, padded and converted copies), so the work of two runs
+ *    of one handle must not overlap on the device either: on two streams, order the second behind the
+ *    first. Distinct handles may be used from distinct threads / streams.
  */
 #ifndef MI355_GEMMLOWP_H
 #define MI355_GEMMLOWP_H
