@@ -959,7 +959,7 @@ static const void *const g_rowsum_256x128x128[3][2] = {
 // (nor in convolutions of 98 to 490 rows, K 720 to 1440: 0.998 to 1.014 of the 3 stages' time).
 // us_more: what of the start-up and the epilogue a tile does not share with the tile beside it on its compute unit. It decides
 // under one or two K steps (us, two 64 x 64 per compute unit against one 128 x 64: 3000 x 512 x 64 4.8 and 4.5; two 128 x 64
-// against one 128 x 128: 1000 x 4096 x 200 7.5 and 6.5).
+// against one 128 x 128: 1000 x 4096 x 200 7.5 and 6.5; 25 x 320 x 977 x 23 to F32, 400 tiles of 256 x 128 38.6, 64 x 64 27.2).
 // The loader of a convolution has its own prices, from a sweep of every tile and slice count over 172 convolutions (16 to 2048 channels,
 // 64 to 103k rows, 16 to 512 columns): it works at the decoding of taps and at per-lane addresses whether the chip is full or
 // not, so few tiles save little: on an idle chip a step costs 1.4 (64 x 64) to 2.3 times (256 x 128) the dense one. (The dense prices times
@@ -969,7 +969,7 @@ struct DmaCost
     double us_tile, us_step, us_load, us_more = 0;
 };
 static const DmaCost g_dma_cost[2][6] = {
-    {{5.6, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.3, 0.385, 0.35, 0.8}, {2.7, 0.365, 0.35, 0.2}, {3.2, 0.365, 0.35}, {4.1, 0.618, 0.35}},
+    {{6.2, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.3, 0.385, 0.35, 0.8}, {2.7, 0.365, 0.35, 0.2}, {3.2, 0.365, 0.35}, {4.1, 0.618, 0.35}},
     {{6.0, 1.07, 0.25}, {4.1, 0.81, 0.13}, {3.4, 0.585, 0.10}, {3.0, 0.50, 0.0}, {3.5, 0.50, 0.0}, {3.4, 1.03, 0.18}},
 };
 
