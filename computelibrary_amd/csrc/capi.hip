@@ -1497,12 +1497,15 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
             // the narrow kernel's k blocks (192) either way: 224 x 224 x 1 -> 64, 3 x 3: 91.4 -> 96.1.
             // Not either where the row's K just fits that one batch and the padded taps fit two, under few output rows: the form
             // for one batch, which knows several panels, starts half a microsecond later (6272 rows of 20 -> 32 channels, 3 x 3,
-            // stride 2, channels padded 6.2, rows 6.5; 12544 rows: 7.1, 6.9).
+            // stride 2, channels padded 6.2, rows 6.5; 12544 rows: 7.1, 6.9). And up to 64 output channels, where the narrow kernel
+            // runs either way, a K of 400 (5 x 5) or 576 saves less than a copy costs that is more than half again as large: 16 of 128 x
+            // 128 x 4 -> 64, 5 x 5: 24.4 -> 28.3; -> 32: 21.9 -> 23.9 (7 x 7 saves more: see above).
             mi355_conv_desc dr = d;
             dr.C = round_up(d.KW * d.C, 16), dr.W = h->geom_true.OW, dr.KW = dr.stride_x = dr.dilation_x = 1, dr.pad_left = dr.pad_right = 0;
             const int64_t row_bytes = (int64_t)dr.W * dr.C, pad_bytes = (int64_t)d.W * dp.C, k_row = (int64_t)d.KH * dr.C, k_pad = (int64_t)d.KH * d.KW * dp.C;
             const bool    one_batch_late = d.OFM <= 64 && k_row <= 192 && k_pad > 192 && k_pad <= 384 && (int64_t)d.batch * gp.OH * gp.OW < 8192;
-            if (h->c_pad && !one_batch_late && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
+            const bool    large_copy = d.OFM <= 64 && 2 * row_bytes > 3 * pad_bytes && k_pad <= 576;
+            if (h->c_pad && !one_batch_late && !large_copy && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
                 (d.KW * d.C >= 8 || k_pad > 192) &&
                 (int64_t)d.batch * d.H * row_bytes < ((int64_t)1 << 31) &&
                 patch_rows_fit((int64_t)d.batch * d.H, d.W, d.C, dr.W, d.stride_x, d.pad_left, dr.C))

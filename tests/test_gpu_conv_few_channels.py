@@ -21,6 +21,8 @@ FEW = [
     ((3, 33, 31, 3), (64, 7, 7, 3), (2, 2), (3, 3, 3, 3), (1, 1)),
     ((1, 12, 20, 5), (96, 5, 5, 5), (4, 1), (2, 2, 2, 2), (1, 2)),    # dilated down the image
     ((2, 8, 150, 8), (24, 3, 5, 8), (2, 2), (2, 1, 2, 1), (1, 1)),    # several workgroups per row
+    ((2, 14, 15, 4), (64, 5, 5, 4), (1, 1), (2, 2, 2, 2), (1, 1)),    # the copy would double: channels padded
+    ((2, 14, 15, 4), (65, 5, 5, 4), (1, 1), (2, 2, 2, 2), (1, 1)),    # ... and does, where it saves the pipelined kernel K steps
 ]
 
 
