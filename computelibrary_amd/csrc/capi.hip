@@ -288,7 +288,7 @@ struct GemmCore
                 return best;
             };
             // The pipelined kernel's tile is chosen with a small cost model in microseconds, fitted to sweeps of every tile
-            // shape and slice count over 33 shapes (M 65-2048, N 24-12288, K 512-11008, B hot and rotated through HBM), later 279
+            // shape and slice count over 33 shapes (M 65-2048, N 24-12288, K 512-11008, B hot and rotated through HBM), later 352
             // dense products (K from 16) and 172 convolutions: a tile
             // costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that fit a compute unit
             // together share all but us_more, plus us_step for every K step, which a full chip slows down by a share us_load of it (L2, HBM and
