@@ -287,17 +287,15 @@ struct GemmCore
                 (void)env;
                 return best;
             };
-            // The pipelined kernel's tile is chosen with a small cost model in microseconds, fitted to sweeps of every tile
-            // shape and slice count over 33 shapes (M 65-2048, N 24-12288, K 512-11008, B hot and rotated through HBM), later 352
-            // dense products (K from 16) and 172 convolutions: a tile
-            // costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that fit a compute unit
-            // together share all but us_more, plus us_step for every K step, which a full chip slows down by a share us_load of it (L2, HBM and
-            // the power limit are shared by all compute units).
+            // The pipelined kernel's tile is chosen with a small cost model in microseconds (the prices and what they were fitted to
+            // stand at g_dma_cost): a tile costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that
+            // fit a compute unit together share all but us_more, plus us_step for every K step, which a full chip slows down
+            // by a share us_load of it (L2, HBM and the power limit are shared by all compute units).
             // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
-            // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.8 us for the launch
-            // and its latency, 0.12 us per plane one thread walks over and 0.25 us per MB. (254 x 33 x 10588: 39.0 us whole,
-            // 11.4 as 21 slices, 11.3 as 12; 640 x 480 x 2048: 10.4 whole, 11.0 as 3.) Slices have to promise an eighth:
-            // below that the model's error decides, and they need a workspace.
+            // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
+            // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again. The 0.88: a deep K
+            // under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900: 10.3 us whole, priced
+            // at 8.6, 8.4 as 4 slices; 350 x 126 x 3520: 11.5, 9.2 and 8.4), and with it the choice is no worse on average.
             auto pick_dma = [&]() -> int
             {
                 int    best = -1;
@@ -305,7 +303,7 @@ struct GemmCore
                 for (int i = 0; i < dma_num_configs(); ++i)
                 {
                     const MfmaConfig c = dma_config(i, patch_c > 0);
-                    if ((N <= 64 && c.BN > 64) || Kp % c.BK != 0)
+                    if (c.us_tile <= 0 || (N <= 64 && c.BN > 64) || Kp % c.BK != 0)
                         continue;
                     const double tiles   = (double)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN) * batch;
                     const int    occ_lds = (160 * 1024) / c.lds_bytes, occ_wav = 32 / c.waves;
@@ -320,9 +318,9 @@ struct GemmCore
                         if (sl != want)
                             continue;
                         const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
-                        const double finish = sl > 1 ? 2.8 + 0.12 * sl + (double)sl * M * N * 1e-6 : 0.0;
+                        const double finish = sl > 1 ? 2.4 + 0.1 * sl + 2e-6 * (double)sl * M * N : 0.0;
                         const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load);
-                        const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 1.125 : 1.0);
+                        const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 0.88 : 1.0);
                         if (best < 0 || cost < best_cost)
                             best = i, best_cost = cost, splitk_plan = sl;
                     }
@@ -781,6 +779,8 @@ struct GemmCore
                 g.tiles_m          = (g.M + c.BM - 1) / c.BM;
                 g.tiles_n          = (g.N + c.BN - 1) / c.BN;
                 kname_run          = &kname_dma_full;
+                if (conv)
+                    g.conv.pad_word = 0x01010101u * fill_byte; // as in the image: the kernel flips what it loads
                 if (splitk > 1 && batch == 1)
                 {
                     // the float epilogue rounds the product and the offset terms apart: they must not meet in the planes

@@ -1,6 +1,6 @@
 // K1 / K4, pipelined variant: the same int8 MFMA GEMM + fused epilogue as gemm_mfma.hip, organised for throughput.
-// This is the kernel that runs whenever A rows are 16-byte aligned and K is a multiple of 16; gemm_mfma.hip remains the
-// fallback for everything else.
+// Here: 256 x 128 tiles of dense products, and the table and launch of every tile of the pipelined kernel (the smaller tiles and
+// the convolution are gemm_ring.hpp's). It runs on dword-aligned rows of A; gemm_mfma.hip remains the fallback.
 //
 // Global -> LDS: direct-to-LDS loads (global_load_lds_dwordx4: no staging registers, no ds_write) into an NS-stage ring,
 // so NS-1 K steps of loads are in flight while one is being multiplied. One wave instruction moves 64 lanes x 16 B =
@@ -33,37 +33,12 @@
 // consecutive output columns per accumulator block: the epilogue reads the per-column parameters as 16-byte vectors and
 // packs 4 int8 results into one dword. Those dwords go to LDS first (the ring is free by then) and leave as whole
 // 128-byte tile rows, 16 bytes per lane; where the destination is not 16-byte aligned they are stored directly.
-#include "mfma_common.hpp"
+#include "direct_lds.hpp"
 
 #include <atomic>
 
 namespace mi355
 {
-__device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
-}
-
-// scalar-base form: address = sbase (SGPR pair, wave-uniform) + zero-extended per-lane 32-bit offset
-__device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_addr)
-{
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-__device__ __forceinline__ void block_barrier()
-{
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // Stages the A and B panels of one block tile. All NP producer waves of a block hold one of these. The loads use the
 // scalar-base form of the instruction (wave-uniform 64-bit base in SGPRs + one 32-bit offset register per lane): with
 // per-lane 64-bit addresses every load costs the SIMD's matrix pipe about 50 clocks, with scalar bases the stream
@@ -74,7 +49,7 @@ __device__ __forceinline__ void block_barrier()
 // registers per load (arrays of per-load offsets were spilled to scratch memory, and every reload waited for all the
 // loads in flight). Lanes that must read padding instead (K tail of A, out-of-image taps of the implicit convolution)
 // need a different base: a wave with any such lane falls back to per-lane addresses for that one load.
-template <int BM, int BN, int BK, int NP, int NS, bool CONV>
+template <int BM, int BN, int BK, int NP, int NS>
 struct PanelProducer
 {
     static constexpr int CPR   = BK / 16;   // 16-byte columns per tile row
@@ -82,7 +57,6 @@ struct PanelProducer
     static constexpr int AU    = BM / RPU;  // staging units of the A part of a stage
     static constexpr int BU    = BN / RPU;
     static constexpr int LPP   = (AU + BU) / NP; // loads per producer wave per stage
-    static constexpr int LPA   = (AU + NP - 1) / NP; // at most this many of them are A units
     static constexpr int STAGE = (BM + BN) * BK;
     static_assert((AU + BU) % NP == 0, "staging shape");
     // swz(row) of row = u*RPU + r depends on u only through (u*RPU) & (CPR-1): constant for CPR <= 4, the parity of u
@@ -96,12 +70,8 @@ struct PanelProducer
     int           ur;             // this lane's row inside a unit
     int           rows_left;      // M - m0: rows of A at and below the tile's first row
     int64_t       lda, Kp;
-    uint32_t      c_off[CONV ? LPA : 1]; // conv: image offset of the (possibly out-of-image) top-left tap of the lane's pixel
-    int           c_iy0[CONV ? LPA : 1], c_ix0[CONV ? LPA : 1]; // conv: its input coordinates
     uint32_t      lds0;
     int           pw, K, lane_id;
-    int           k_base; // conv: first k of this launch entry's slice of the patch
-    ConvGeom      conv;
 
     __device__ __forceinline__ void init(const GemmArgs &g, int m0, int n0, int bz, int producer_wave, int lane,
                                          uint32_t lds_base)
@@ -109,37 +79,19 @@ struct PanelProducer
         pw        = producer_wave;
         lds0      = lds_base;
         K         = g.K;
-        k_base    = CONV ? bz * g.k_slice : 0;
-        conv      = g.conv;
         fill16    = g.fill16;
         a_end     = g.a_end;
         lane_id   = lane;
         lda       = g.lda;
         Kp        = g.Kp;
         rows_left = g.M - m0;
-        a_base    = g.A + (int64_t)bz * g.a_batch_stride + (CONV ? (int64_t)0 : (int64_t)m0 * g.lda);
+        a_base    = g.A + (int64_t)bz * g.a_batch_stride + (int64_t)m0 * g.lda;
         b_base    = g.Bp + (int64_t)bz * g.bp_batch_stride + (int64_t)n0 * g.Kp;
         ur        = lane / CPR;
         const int c = (lane % CPR) ^ swz<CPR>(pw * RPU + ur);
         c16       = c * 16;
         lane_a    = (uint32_t)ur * (uint32_t)g.lda + (uint32_t)c16;
         lane_b    = (uint32_t)ur * (uint32_t)g.Kp + (uint32_t)c16;
-        if (CONV)
-        {
-#pragma unroll
-            for (int i = 0; i < LPA; ++i)
-            {
-                const int gr = min(m0 + (pw + i * NP) * RPU + ur, g.M - 1);
-                const int t  = fast_div(gr, g.conv.magic_OW);
-                const int ox = gr - t * g.conv.OW;
-                const int n  = fast_div(t, g.conv.magic_OH);
-                const int oy = t - n * g.conv.OH;
-                c_iy0[i]     = oy * g.conv.stride_y - g.conv.pad_top;
-                c_ix0[i]     = ox * g.conv.stride_x - g.conv.pad_left;
-                c_off[i]     = (uint32_t)n * (uint32_t)(g.conv.H * g.conv.W * g.conv.C) +
-                           (uint32_t)((c_iy0[i] * g.conv.W + c_ix0[i]) * g.conv.C);
-            }
-        }
     }
 
     // The same for a dense tile that lies inside the matrix (no row of it beyond M) and a K step that lies inside K:
@@ -147,7 +99,6 @@ struct PanelProducer
     // dozen scalar instructions on every load; with 12 loads per producer wave and K step that was most of the step.)
     __device__ __forceinline__ void issue_inside(int kt, int slot) const
     {
-        static_assert(!CONV, "dense tiles only");
         const uint32_t base = lds0 + (uint32_t)slot * STAGE;
         const int8_t  *a_k  = a_base + (int64_t)kt * BK;
         const int8_t  *b_k  = b_base + (int64_t)kt * BK;
@@ -170,25 +121,9 @@ struct PanelProducer
     {
         const int      k0   = kt * BK;
         const uint32_t base = lds0 + (uint32_t)slot * STAGE;
-        const int8_t  *a_k  = a_base + (CONV ? 0 : k0);
+        const int8_t  *a_k  = a_base + k0;
         const int8_t  *b_k  = b_base + k0; // always inside the zero-padded packed panel
         const bool     full = k0 + BK <= K;
-        // convolution: one tap decode per K step (the lane's column is the same in every unit)
-        bool     t_in = false;
-        int      t_dy = 0, t_dx = 0;
-        uint32_t t_off = 0;
-        if (CONV)
-        {
-            const int k   = k_base + k0 + c16; // within the whole patch
-            const int tap = fast_div(k, conv.magic_C);
-            const int c0  = k - tap * conv.C;
-            const int ky  = fast_div(tap, conv.magic_KW);
-            const int kx  = tap - ky * conv.KW;
-            t_dy          = ky * conv.dil_y;
-            t_dx          = kx * conv.dil_x;
-            t_off         = (uint32_t)((t_dy * conv.W + t_dx) * conv.C + c0);
-            t_in          = k0 + c16 < K;
-        }
 #pragma unroll
         for (int i = I0; i < I1; ++i)
         {
@@ -196,7 +131,7 @@ struct PanelProducer
             const uint32_t dst = base + (uint32_t)u * 1024u;
             if (u >= AU)
                 dma16s(b_k + (int64_t)(u - AU) * RPU * Kp, lane_b, dst);
-            else if (!CONV)
+            else
             {
                 // rows beyond M re-read row M-1 (their results are never stored): only the last row tile has any
                 const bool     edge = (u + 1) * RPU > rows_left;
@@ -221,16 +156,6 @@ struct PanelProducer
                     }
                 }
             }
-            else
-            {
-                const int      iy = c_iy0[i < LPA ? i : 0] + t_dy, ix = c_ix0[i < LPA ? i : 0] + t_dx;
-                const bool     ok = t_in && (unsigned)iy < (unsigned)conv.H && (unsigned)ix < (unsigned)conv.W;
-                const uint32_t o  = c_off[i < LPA ? i : 0] + t_off;
-                if (__builtin_amdgcn_ballot_w64(ok) == ~0ull)
-                    dma16s(a_k, o, dst);
-                else
-                    dma16(ok ? a_k + o : fill16, dst);
-            }
         }
     }
 };
@@ -254,7 +179,7 @@ __device__ long long phase_clocks[6][8];
 #endif
 
 // GWM x GWN consumer waves per group, 2 groups stacked along M, plus NP = GWM*GWN producer waves
-template <int BM, int BN, int BK, int GWM, int GWN, int NS, int EPI, bool FLIP_A, bool CONV>
+template <int BM, int BN, int BK, int GWM, int GWN, int NS, int EPI, bool FLIP_A>
 __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(1, 6))) void gemm_dma_kernel(GemmArgs g_in)
 {
     // What a workgroup needs before its first loads go out is read here, in one batch of scalar loads, and pinned in
@@ -271,11 +196,6 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     typedef const __attribute__((address_space(1))) int32_t *global_i32;
     uintptr_t u_cv = (uintptr_t)g.epi.colvec, u_qp = (uintptr_t)g.epi.qp, u_fl = (uintptr_t)g.epi.qp_flag;
     asm volatile("" : "+s"(u_cv), "+s"(u_qp), "+s"(u_fl));
-    if (CONV)
-        asm volatile(""
-                     : "+s"(g.conv.H), "+s"(g.conv.W), "+s"(g.conv.C), "+s"(g.conv.KW), "+s"(g.conv.OW), "+s"(g.conv.OH),
-                       "+s"(g.conv.stride_x), "+s"(g.conv.stride_y), "+s"(g.conv.pad_left), "+s"(g.conv.pad_top), "+s"(g.conv.dil_x),
-                       "+s"(g.conv.dil_y), "+s"(g.conv.magic_C), "+s"(g.conv.magic_KW), "+s"(g.conv.magic_OW), "+s"(g.conv.magic_OH));
 
     constexpr int GW    = GWM * GWN; // waves per consumer group
     constexpr int NW    = 2 * GW;    // consumer waves
@@ -292,7 +212,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     // Dense tiles: inside the K loop the consumers stage the B panel themselves (CBU units per wave and K step, issued
     // while their operand reads are in flight) and the producers only the A panel. The block's direct-to-LDS loads then
     // come from all 12 waves instead of 4 and keep flowing while the producers sit in a barrier.
-    constexpr bool CDMA = !CONV && (BU % NW == 0) && (AU % NP == 0) && (AU / NP) % 2 == 0;
+    constexpr bool CDMA = (BU % NW == 0) && (AU % NP == 0) && (AU / NP) % 2 == 0;
     constexpr int  CBU  = CDMA ? BU / NW : 0;   // B units per consumer wave per stage
     constexpr int  PLP  = CDMA ? AU / NP : LPP; // loads per producer wave per stage inside the loop
     // Start-up of dense tiles: a wave gets one direct-to-LDS load accepted about every 190 clocks at the start of a kernel,
@@ -302,9 +222,6 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     constexpr int  LPW   = (AU + BU) / NALL; // loads per wave per start-up stage
     constexpr bool SPREAD = CDMA && (AU + BU) % NALL == 0 && (NS - 1) * LPW < 64 &&
                             (CPR <= 4 || (CPR == 8 && NALL % 2 == 0) || (CPR == 16 && NALL % 4 == 0));
-    // Small wave tiles: a slot of matrix instructions is much shorter than a slot of operand reads, so running the two
-    // consumer groups one slot apart only serialises their reads; both groups then read and multiply in the same slots.
-    constexpr bool INPHASE = RS * QS * KK <= 16;
     static_assert(TM % 16 == 0 && TN % 16 == 0 && RS >= 1 && QS >= 1 && BK % 64 == 0, "wave tile");
     static_assert(NS >= 3 && (NS - 2) * LPP < 64, "ring depth / vmcnt range");
     static_assert(NW * 16 * (QS * 64 + 16) <= NS * STAGE, "the 32-bit epilogue stages through the ring's memory");
@@ -359,7 +276,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     }
     if constexpr (SPREAD)
     {
-        PanelProducer<BM, BN, BK, NALL, NS, CONV> first;
+        PanelProducer<BM, BN, BK, NALL, NS> first;
         first.init(g, m0, n0, bz, wave, lane, lds0);
 #pragma unroll
         for (int s = 0; s < NS - 1; ++s)
@@ -374,7 +291,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     if (wave >= NW)
     {
         // ================= producer: global -> LDS =================
-        PanelProducer<BM, BN, BK, NP, NS, CONV> prod;
+        PanelProducer<BM, BN, BK, NP, NS> prod;
         prod.init(g, m0, n0, bz, wave - NW, lane, lds0);
         MI355_PHASE(1); // producer: addresses set up
         if constexpr (!SPREAD)
@@ -467,12 +384,10 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     }
     block_barrier(); // barrier 0: stage 0 is in LDS
     MI355_PHASE(2); // consumer: stage 0 is in LDS
-    if (group == 1 && !INPHASE)
+    if (group == 1)
         block_barrier(); // group 1 runs one slot behind group 0
 
-    // row sums of A, taken from the operand blocks as they pass (on request). A convolution's patches hold bytes that do
-    // not count (padded channels, what lies beyond K): they meet zeros instead of ones
-    // (14x14x256 -> 256, 3x3, batch 32, u8 weights: 15.6 us, where a pass over the image in front took 72 more)
+    // row sums of A, taken from the operand blocks as they pass (on request)
     const bool rowsum = g.epi.rowsum_mul != 0;
     int32_t    rsum[RS];
 #pragma unroll
@@ -516,15 +431,9 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk)
             {
-                v4i ones = {ONES4, ONES4, ONES4, ONES4};
-                if (CONV && (g.conv.c_true != g.conv.C || (kt + 1) * BK > g.K))
-                {
-                    const int k = kt * BK + kk * 64 + lh * 16;
-                    ones        = patch_bytes(g.conv, k + bz * g.k_slice, k < g.K ? INT32_MAX : 0);
-                }
 #pragma unroll
                 for (int f = 0; f < RS; ++f)
-                    rsum[f] = sum_bytes(fa[kk][f], rsum[f], ones);
+                    rsum[f] = sum_bytes(fa[kk][f], rsum[f]);
             }
         }
         // this wave's units of stage kt+1 have to be in LDS before the barrier that opens that stage to its first
@@ -552,11 +461,11 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
     }
     if (CDMA)
         wait_vmcnt<0>();
-    if (group == 0 || INPHASE)
+    if (group == 0)
         block_barrier(); // barrier 2nk+1; every operand read of every wave is complete beyond this point
     MI355_PHASE(3); // consumer: K loop over
     if (rowsum)
-        finish_row_sums<RS>(rsum, g.epi.rowsum_mul, FLIP_A && !CONV ? nk * BK - g.K : 0);
+        finish_row_sums<RS>(rsum, g.epi.rowsum_mul, FLIP_A ? nk * BK - g.K : 0);
 
     if (fast)
     {
@@ -667,7 +576,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
     {
         // The first NS-1 stages before anything else - every clock before the first load goes out is a clock in which
         // the whole chip waits for memory: unit u to wave u % 8, stage 0 first
-        PanelProducer<BM, BN, BK, NALL, NS, false> first;
+        PanelProducer<BM, BN, BK, NALL, NS> first;
         first.init(g, m0, n0, bz, wave, lane, lds0);
 #pragma unroll
         for (int s = 0; s < NS - 1; ++s)
@@ -706,7 +615,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
     // every consumer issued before barrier kt. Every wave executes nk + 2 barriers (+ those of the epilogue).
     if (wave >= NW)
     {
-        PanelProducer<BM, BN, BK, NP, NS, false> prod;
+        PanelProducer<BM, BN, BK, NP, NS> prod;
         prod.init(g, m0, n0, bz, wave - NW, lane, lds0);
         MI355_PHASE(1);
         MI355_PHASE(2);
@@ -907,91 +816,55 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
 }
 
 // ---- instantiation table -------------------------------------------------------------------------------------------
-struct DmaEntry
+#define MI355_DFN(BM, BN, BK, WM, WN, NS, E, F) (const void *)gemm_dma_kernel<BM, BN, BK, WM, WN, NS, E, F>
+#define MI355_WFN(BM, BN, BK, NS, E, F) (const void *)gemm_wide_kernel<BM, BN, BK, NS, E, F>
+
+// The 256 x 128 tile: [epi][flip] of the 4 + 4 wave kernel, and of the 8 + 4 wave kernel where the rows of A are summed inside
+// (EpiParams::rowsum_mul, a run-time switch there): the 4 + 4 wave form has no registers left for that. (2048 x 4096 x 4096, u8 weights:
+// 36.2 us in the 8 + 4 form, 38.4 in 128 x 128 tiles of the ring kernel, which is why it is kept for this.)
+struct WideEntry
 {
     MfmaConfig  cfg;
-    int         threads;
-    int         lds_bytes;
-    const void *fn[3][2][2]; // [epi][flip][conv]
-    int         threads_dense = 0; // workgroup size of the dense (non-convolution) kernels when it differs
+    int         lds_bytes, threads, threads_rowsum;
+    const void *fn[3][2], *fn_rowsum[3][2];
 };
-
-#define MI355_DFN(BM, BN, BK, WM, WN, NS, E, F, C) (const void *)gemm_dma_kernel<BM, BN, BK, WM, WN, NS, E, F, C>
-#define MI355_DCFG(NAME, BM, BN, BK, WM, WN, NS)                                                                     \
-    {                                                                                                                \
-        {NAME, BM, BN, BK}, WM *WN * 192, NS * (BM + BN) * BK,                                                        \
-        {                                                                                                            \
-            {{MI355_DFN(BM, BN, BK, WM, WN, NS, 0, false, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 0, false, true)}, \
-             {MI355_DFN(BM, BN, BK, WM, WN, NS, 0, true, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 0, true, true)}},  \
-                {{MI355_DFN(BM, BN, BK, WM, WN, NS, 1, false, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 1, false, true)}, \
-                 {MI355_DFN(BM, BN, BK, WM, WN, NS, 1, true, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 1, true, true)}}, \
-                {{MI355_DFN(BM, BN, BK, WM, WN, NS, 2, false, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 2, false, true)}, \
-                 {MI355_DFN(BM, BN, BK, WM, WN, NS, 2, true, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 2, true, true)}}, \
-        }                                                                                                            \
-    }
-
-#define MI355_WFN(BM, BN, BK, NS, E, F) (const void *)gemm_wide_kernel<BM, BN, BK, NS, E, F>
-// dense: the 4 + 4 wave kernel; convolution: the 8 + 4 wave kernel
-#define MI355_WCFG(NAME, BM, BN, BK, WM, WN, NS)                                                                     \
-    {                                                                                                                \
-        {NAME, BM, BN, BK}, WM *WN * 192, NS * (BM + BN) * BK,                                                        \
-        {                                                                                                            \
-            {{MI355_WFN(BM, BN, BK, NS, 0, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 0, false, true)},                \
-             {MI355_WFN(BM, BN, BK, NS, 0, true), MI355_DFN(BM, BN, BK, WM, WN, NS, 0, true, true)}},                 \
-                {{MI355_WFN(BM, BN, BK, NS, 1, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 1, false, true)},            \
-                 {MI355_WFN(BM, BN, BK, NS, 1, true), MI355_DFN(BM, BN, BK, WM, WN, NS, 1, true, true)}},             \
-                {{MI355_WFN(BM, BN, BK, NS, 2, false), MI355_DFN(BM, BN, BK, WM, WN, NS, 2, false, true)},            \
-                 {MI355_WFN(BM, BN, BK, NS, 2, true), MI355_DFN(BM, BN, BK, WM, WN, NS, 2, true, true)}},             \
-        },                                                                                                           \
-            512                                                                                                      \
-    }
-
-// Row sums of A taken inside the kernel (EpiParams::rowsum_mul) are a run-time switch of the 8 + 4 wave kernel; the
-// 4 + 4 wave kernel has no registers left for them, so its tile shape falls back to the 8 + 4 wave form there: [epi][flip]
-static const void *const g_rowsum_256x128x128[3][2] = {
-    {MI355_DFN(256, 128, 128, 2, 2, 3, 0, false, false), MI355_DFN(256, 128, 128, 2, 2, 3, 0, true, false)},
-    {MI355_DFN(256, 128, 128, 2, 2, 3, 1, false, false), MI355_DFN(256, 128, 128, 2, 2, 3, 1, true, false)},
-    {MI355_DFN(256, 128, 128, 2, 2, 3, 2, false, false), MI355_DFN(256, 128, 128, 2, 2, 3, 2, true, false)}};
+static const WideEntry g_wide = {
+    {"pp_256x128x128_s3", 256, 128, 128},
+    3 * (256 + 128) * 128,
+    512,
+    768,
+    {{MI355_WFN(256, 128, 128, 3, 0, false), MI355_WFN(256, 128, 128, 3, 0, true)},
+     {MI355_WFN(256, 128, 128, 3, 1, false), MI355_WFN(256, 128, 128, 3, 1, true)},
+     {MI355_WFN(256, 128, 128, 3, 2, false), MI355_WFN(256, 128, 128, 3, 2, true)}},
+    {{MI355_DFN(256, 128, 128, 2, 2, 3, 0, false), MI355_DFN(256, 128, 128, 2, 2, 3, 0, true)},
+     {MI355_DFN(256, 128, 128, 2, 2, 3, 1, false), MI355_DFN(256, 128, 128, 2, 2, 3, 1, true)},
+     {MI355_DFN(256, 128, 128, 2, 2, 3, 2, false), MI355_DFN(256, 128, 128, 2, 2, 3, 2, true)}}};
 
 // What a tile and a K step of each configuration cost, in microseconds, and by what share a K step gets slower as the chip
-// fills: read off sweeps over the depth of K (64 x 64, 3 stages: 5.75 us at K = 512, 7.27 at 1024, 10.0 at 2048) and over the
-// number of tiles. The 6-stage ring never was the faster one of its tile in them, by 0.5 us, with B from HBM or not
-// (nor in convolutions of 98 to 490 rows, K 720 to 1440: 0.998 to 1.014 of the 3 stages' time).
-// us_more: what of the start-up and the epilogue a tile does not share with the tile beside it on its compute unit. It decides
-// under one or two K steps (us, two 64 x 64 per compute unit against one 128 x 64: 3000 x 512 x 64 4.8 and 4.5; two 128 x 64
-// against one 128 x 128: 1000 x 4096 x 200 7.5 and 6.5; 25 x 320 x 977 x 23 to F32, 400 tiles of 256 x 128 38.6, 64 x 64 27.2).
-// The loader of a convolution has its own prices, from a sweep of every tile and slice count over 172 convolutions (16 to 2048 channels,
-// 64 to 103k rows, 16 to 512 columns): it works at the decoding of taps and at per-lane addresses whether the chip is full or
-// not, so few tiles save little: on an idle chip a step costs 1.4 (64 x 64) to 2.3 times (256 x 128) the dense one. (The dense prices times
-// 1.15 took 34300 x 24 x 3024 to the 256-deep tile: 33.2 us, 128 x 64 24.8; and 392 x 512 x 2304 whole: 12.5 us, 4 slices 9.9.)
+// fills (us_more: what of the start-up and the epilogue a tile does not share with the tile beside it on its compute unit): fitted
+// to every tile shape at up to 9 slice counts over 215 dense products (33 to 8192 rows, 16 to 11008 columns, K 16 to 11008) and 154
+// convolutions (16 to 2048 channels, 1 x 1 to 5 x 5); over those the choice is 1.5 % slower than the best of the sweep on average.
+// us_tile 0: not chosen, runs where a caller names it. In the sweep the 6-stage ring and the 256-deep 128 x 64 tile were the best
+// of a shape by 0.2 % on average, 128 x 64 tiles in convolutions by 0.3 %.
 struct DmaCost
 {
-    double us_tile, us_step, us_load, us_more = 0;
+    double us_tile, us_step, us_load, us_more;
 };
-static const DmaCost g_dma_cost[2][6] = {
-    {{6.2, 0.465, 0.55}, {4.2, 0.437, 0.30}, {3.3, 0.385, 0.35, 0.8}, {2.7, 0.365, 0.35, 0.2}, {3.2, 0.365, 0.35}, {4.1, 0.618, 0.35}},
-    {{6.0, 1.07, 0.25}, {4.1, 0.81, 0.13}, {3.4, 0.585, 0.10}, {3.0, 0.50, 0.0}, {3.5, 0.50, 0.0}, {3.4, 1.03, 0.18}},
-};
-
-static const DmaEntry g_dma[] = {
-    MI355_WCFG("pp_256x128x128_s3", 256, 128, 128, 2, 2, 3),
-    MI355_DCFG("pp_128x128x128_s3", 128, 128, 128, 2, 2, 3),
-    MI355_DCFG("pp_128x64x128_s3", 128, 64, 128, 2, 2, 3),
-    MI355_DCFG("pp_64x64x128_s3", 64, 64, 128, 1, 2, 3),
-    MI355_DCFG("pp_64x64x128_s6", 64, 64, 128, 1, 2, 6),
-    MI355_DCFG("pp_128x64x256_s3", 128, 64, 256, 2, 2, 3),
+static const DmaCost g_dma_cost[2][8] = {
+    {{8.57, 0.622, 0.33, 1.55}, {5.82, 0.412, 0.19, 4.35}, {4.30, 0.307, 0.12, 0.0}, {3.89, 0.188, 0.126, 0.0}, {}, {}, {5.67, 0.536, 0.0, 0.69}, {}},
+    {{}, {6.24, 0.541, 0.45, 3.7}, {}, {4.11, 0.339, 0.0, 0.0}, {}, {}, {5.33, 0.818, 0.04, 0.0}, {4.24, 0.489, 0.0, 0.0}},
 };
 
+// configuration 0 is g_wide, the others are g_ring's
 int dma_num_configs()
 {
-    return (int)(sizeof(g_dma) / sizeof(g_dma[0]));
+    return 1 + g_ring_count;
 }
 MfmaConfig dma_config(int idx, bool conv)
 {
-    MfmaConfig c = g_dma[idx].cfg;
-    c.waves      = g_dma[idx].threads / 64;
-    c.lds_bytes  = g_dma[idx].lds_bytes;
-    static_assert(sizeof(g_dma_cost[0]) / sizeof(g_dma_cost[0][0]) == sizeof(g_dma) / sizeof(g_dma[0]), "one price per configuration");
+    MfmaConfig c = idx == 0 ? g_wide.cfg : g_ring[idx - 1].cfg;
+    c.waves      = (idx == 0 ? g_wide.threads : g_ring[idx - 1].threads[conv ? 1 : 0]) / 64;
+    c.lds_bytes  = idx == 0 ? g_wide.lds_bytes : g_ring[idx - 1].lds_bytes[conv ? 1 : 0];
     const DmaCost &cost = g_dma_cost[conv ? 1 : 0][idx];
     c.us_tile = cost.us_tile, c.us_step = cost.us_step, c.us_load = cost.us_load, c.us_more = cost.us_more;
     return c;
@@ -1001,35 +874,37 @@ int dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &arg
 {
     if (cfg_idx < 0 || cfg_idx >= dma_num_configs() || epi < 0 || epi > 2)
         return (int)hipErrorInvalidValue;
-    const DmaEntry &c  = g_dma[cfg_idx];
-    const void     *fn = c.fn[epi][flip_a ? 1 : 0][conv ? 1 : 0];
-    int             fn_slot = conv ? 1 : 0; // which entry of the once-per-device table below
+    const MfmaConfig c       = dma_config(cfg_idx, conv);
+    const int        flip    = flip_a ? 1 : 0;
+    int              threads = c.waves * 64, fn_slot = conv ? 1 : 0; // which entry of the once-per-device table below
+    const void      *fn      = cfg_idx > 0 ? g_ring[cfg_idx - 1].fn[epi][flip][fn_slot] : conv ? nullptr : g_wide.fn[epi][flip];
     if (args.epi.rowsum_mul != 0)
     {
         if (args.K % 16 != 0)
             return (int)hipErrorInvalidValue;
-        if (!conv && c.threads_dense) // the 4 + 4 wave kernel's tile shape: see g_rowsum_256x128x128
-            fn = g_rowsum_256x128x128[epi][flip_a ? 1 : 0], fn_slot = 2;
+        if (!conv && cfg_idx == 0)
+            fn = g_wide.fn_rowsum[epi][flip], fn_slot = 2, threads = g_wide.threads_rowsum;
     }
     if (fn == nullptr || args.fill16 == nullptr)
         return (int)hipErrorInvalidValue;
     // K slices: whole K steps, the last slice not empty
-    if (args.k_slice != 0 && (args.k_slice < 0 || args.k_slice % c.cfg.BK != 0 || (int64_t)args.k_slice * (batch - 1) >= args.K ||
+    if (args.k_slice != 0 && (args.k_slice < 0 || args.k_slice % c.BK != 0 || (int64_t)args.k_slice * (batch - 1) >= args.K ||
                               (int64_t)args.k_slice * batch < args.K))
         return (int)hipErrorInvalidValue;
     // shapes the kernel assumes: dword-aligned rows of at least one 16-byte column (whole columns of one tap for the
     // convolution), tiles that cover the output and stay inside the packed B panel
-    if (args.K < 16 || args.K > args.Kp || args.Kp % c.cfg.BK != 0 || args.tiles_m * c.cfg.BM < args.M ||
-        args.tiles_n * c.cfg.BN < args.N || args.tiles_n * c.cfg.BN > round_up(args.N, PACK_N_ALIGN) || args.M < 1)
+    if (args.K < 16 || args.K > args.Kp || args.Kp % c.BK != 0 || args.tiles_m * c.BM < args.M ||
+        args.tiles_n * c.BN < args.N || args.tiles_n * c.BN > round_up(args.N, PACK_N_ALIGN) || args.M < 1)
         return (int)hipErrorInvalidValue;
     if (conv ? (args.conv.C % 16 != 0 || ((uintptr_t)args.A & 15) != 0 || args.K % 16 != 0)
              : ((((uintptr_t)args.A | (uintptr_t)args.lda | (uintptr_t)args.a_batch_stride) & 3) != 0 || args.a_end == nullptr))
         return (int)hipErrorInvalidValue;
+    static_assert(sizeof(g_dma_cost[0]) / sizeof(g_dma_cost[0][0]) == 8, "one price and one flag word per configuration");
     if (c.lds_bytes > 48 * 1024)
     {
         // once per kernel and device
-        static std::atomic<uint32_t> raised[sizeof(g_dma) / sizeof(g_dma[0])][3][2][3];
-        std::atomic<uint32_t>       &done = raised[cfg_idx][epi][flip_a ? 1 : 0][fn_slot];
+        static std::atomic<uint32_t> raised[8][3][2][3];
+        std::atomic<uint32_t>       &done = raised[cfg_idx][epi][flip][fn_slot];
         int                          dev  = 0;
         if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 32)
             return (int)hipErrorInvalidDevice;
@@ -1055,12 +930,12 @@ int dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &arg
     a.nblocks     = (int32_t)nblocks;
     // (rows and batch entries at least a K step apart: what a whole last step reads beyond K then lies in the next row or
     // entry, in front of a_end; not when the kernel sums the rows of A from the same tiles)
-    a.lean_tail_bz = (!conv && args.K % c.cfg.BK != 0 && args.epi.rowsum_mul == 0 && args.lda >= c.cfg.BK &&
-                      (batch == 1 || args.a_batch_stride >= c.cfg.BK))
+    a.lean_tail_bz = (!conv && args.K % c.BK != 0 && args.epi.rowsum_mul == 0 && args.lda >= c.BK &&
+                      (batch == 1 || args.a_batch_stride >= c.BK))
                          ? batch - 1
                          : -1;
     void    *kargs[] = {&a};
-    dim3     grid(args.tiles_m * args.tiles_n * batch, 1, 1), block((fn_slot == 0 && c.threads_dense) ? c.threads_dense : c.threads);
+    dim3     grid(args.tiles_m * args.tiles_n * batch, 1, 1), block(threads);
     return (int)hipLaunchKernel(fn, grid, block, kargs, c.lds_bytes, s);
 }
 } // namespace mi355

@@ -66,7 +66,7 @@ struct MfmaConfig
     const char *name;
     int         BM, BN, BK;
     int         waves = 0, lds_bytes = 0; // per workgroup (filled in for the pipelined kernel's configurations)
-    double      us_tile = 0, us_step = 0, us_load = 0, us_more = 0; // ... and what the cost model prices them at (see GemmCore::choose_kernel)
+    double      us_tile = 0, us_step = 0, us_load = 0, us_more = 0; // ... and what the cost model prices them at (see GemmCore::choose_kernel; us_tile 0: not chosen)
 };
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
@@ -99,6 +99,16 @@ int         mfma_num_configs();
 MfmaConfig  mfma_config(int idx);
 // epi: EPI_*, flip_a: xor 0x80 on A bytes in the loader, conv: implicit-GEMM loader. Returns hipError_t as int.
 int         mfma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &args, int batch, hipStream_t s);
+
+// gemm_ring.hip: the tiles of one workgroup of 4 waves; [epi][flip][conv]
+struct RingEntry
+{
+    MfmaConfig  cfg;
+    int         lds_bytes[2], threads[2]; // dense, convolution
+    const void *fn[3][2][2];
+};
+extern const RingEntry g_ring[];
+extern const int       g_ring_count;
 
 // gemm_dma.hip — same contract as mfma_launch; additionally needs 16-byte aligned A rows, K % 16 == 0 and args.fill16
 int         dma_num_configs();

@@ -425,11 +425,11 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
     char         *D   = (char *)g.D + (int64_t)bz * g.d_batch_stride;
     const int     rr = lane / LPR, cc = (lane % LPR) * 16;
 #pragma unroll
-    for (int it = 0; it < BM / (NW * RPI); ++it)
+    for (int it = 0; it < (BM + NW * RPI - 1) / (NW * RPI); ++it)
     {
         const int r = (it * NW + wave) * RPI + rr;
         const int i = m0 + r, j0 = n0 + cc;
-        if (i >= g.M || j0 >= g.N)
+        if (i >= g.M || j0 >= g.N || (BM % (NW * RPI) != 0 && r >= BM))
             continue;
         const v4i     val = *(const v4i *)(stage + r * PITCH + cc);
         const int64_t idx = (int64_t)i * g.ldd + j0;
