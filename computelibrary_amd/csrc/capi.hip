@@ -195,6 +195,10 @@ struct GemmCore
     bool        writes_recorded = false;
     mi355_requant qp_rq{};
     int     splitk = 1;      // K slices of the pipelined kernel
+    int     byte_idx = -1; // the configuration that takes rows of A on any byte without a copy, and what the model prices it and the other at
+    double  us_bytes = 0, us_dma = 0;
+    bool    byte_lda = false;   // rows or batch entries of A that do not start on dwords, as far as the strides say
+    bool    one_launch = false; // few rows, one launch of the pipelined kernel instead of two of the streaming one's
     int     splitk_plan = 1; // what the cost model chose with the tile shape (create()); prepare() checks it and allocates
     int         patch_c = 0, patch_c_true = 0; // a convolution's channels in the kernels' K, and how many of them count (0: dense)
     int         panels_from = 0; // rows of the output from which the narrow kernel takes several panels of columns
@@ -205,7 +209,7 @@ struct GemmCore
     std::string kname_mfma, kname_dma, kprefix;
     // The names a run can report, composed when the choice is made (create, prepare, update): a run only points at one
     // of them - it must not touch the host heap
-    std::string        kname_narrow, kname_band, kname_dma_full, kname_splitk, kname_mfma_full;
+    std::string        kname_narrow, kname_band, kname_dma_full, kname_bytes, kname_splitk, kname_mfma_full;
     const char        *kname_static = nullptr; // the streaming kernel names its forms itself
     const std::string *kname_run = nullptr; // what the last run took (nullptr: no run yet, kname is what create announced)
     uint8_t fill_byte = 0; // value of the 16 filler bytes (0, or the im2col pad value)
@@ -219,6 +223,7 @@ struct GemmCore
         kname_narrow    = kprefix + "narrow_32x64";
         kname_band      = kprefix + "band_32x64";
         kname_dma_full  = kprefix + kname_dma;
+        kname_bytes     = byte_idx >= 0 ? kprefix + dma_config(byte_idx).name + "_bytes" : std::string();
         kname_splitk    = kname_dma_full + "_splitk" + std::to_string(splitk);
         kname_mfma_full = kprefix + kname_mfma;
     }
@@ -251,7 +256,8 @@ struct GemmCore
         }
         else if (path < 0 || path > MI355_PATH_SKINNY)
             return fail("unknown path %d", path);
-        if (path == MI355_PATH_AUTO)
+        const bool automatic = path == MI355_PATH_AUTO;
+        if (automatic)
             // measured: up to 32 rows the streaming kernel always wins; up to 64 rows only while N is small enough
             // that the pipelined kernel would leave most compute units without a tile
             // (a batch of small products runs the streaming kernel once per entry: the tiled kernels would spend a 64-row
@@ -260,6 +266,61 @@ struct GemmCore
             // kernel that keeps the operand blocks of A in registers for its whole run then applies)
             path = (M <= 32 || (batch == 1 && M <= SKINNY_MAX_M && (N < 8192 || (K <= 4096 && K % 64 == 0)))) ? MI355_PATH_SKINNY
                                                                                                          : MI355_PATH_MFMA;
+        const int cus = num_cus();
+        // The pipelined kernel's tile is chosen with a small cost model in microseconds (the prices and what they were fitted to
+        // stand at g_dma_cost): a tile costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that
+        // fit a compute unit together share all but us_more, plus us_step for every K step, which a full chip slows down
+        // by a share us_load of it (L2, HBM and the power limit are shared by all compute units).
+        // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
+        // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
+        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again. The 0.88: a deep K
+        // under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900: 10.3 us whole, priced
+        // at 8.6, 8.4 as 4 slices; 350 x 126 x 3520: 11.5, 9.2 and 8.4), and with it the choice is no worse on average.
+        auto pick_dma = [&](int loader, int &plan, double &best_cost, int fixed_slices = 0) -> int
+        {
+            int best = -1;
+            for (int i = 0; i < dma_num_configs(); ++i)
+            {
+                const MfmaConfig c = dma_config(i, loader);
+                if (c.us_tile <= 0 || (N <= 64 && c.BN > 64) || Kp % c.BK != 0)
+                    continue;
+                const double tiles   = (double)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN) * batch;
+                const int    occ_lds = (160 * 1024) / c.lds_bytes, occ_wav = 32 / c.waves;
+                const double occ     = std::max(1, std::min(occ_lds, occ_wav));
+                const int    nk      = (K + c.BK - 1) / c.BK;
+                for (int want = fixed_slices ? fixed_slices : 1; want <= (fixed_slices ? fixed_slices : MOST_SLICES); ++want)
+                {
+                    // (slices of equal whole K steps but the last, none of them empty)
+                    const int per = (nk + want - 1) / want, sl = (nk + per - 1) / per;
+                    if (want > 1 && (batch != 1 || per * c.BK < 512))
+                        break;
+                    if (sl != want)
+                        continue;
+                    const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
+                    const double finish = sl > 1 ? 2.4 + 0.1 * sl + 2e-6 * (double)sl * M * N : 0.0;
+                    const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load);
+                    const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 0.88 : 1.0);
+                    if (best < 0 || cost < best_cost)
+                        best = i, best_cost = cost, plan = sl;
+                }
+            }
+            return best;
+        };
+        if (automatic && batch == 1 && path == MI355_PATH_SKINNY && (byte_lda || (b_off_eff() != 0 && K % 64 != 0)) && K >= 16 &&
+            (double)N * K <= 4e6)
+        {
+            // The streaming kernel needs a pass in front here, for a copy of the rows or for their sums; the pipelined one does both
+            // itself and is one launch. Two launches are 8.2 us where the host is what they wait for (3 x 111 x 233: 8.2, one launch
+            // 4.3), in a graph 5.3 us and the stream of B (x 1.5 from 33 rows on; 1 x 600 x 999: 4.4 and 7.0, 1 x 2900 x 2901:
+            // 6.5 and 8.5). From 4 MB of B on the stream counts (50 x 6000 x 6001: 22.9 and 37.6), and rows of
+            // whole 64-byte blocks have the streaming kernel's best forms.
+            int          plan = 1;
+            double       us   = 0;
+            const int    idx  = pick_dma(byte_lda || K % 16 != 0 ? 2 : 0, plan, us, 1);
+            const double two  = std::max(8.2, 5.3 + (double)N * K * (M > 32 ? 1.5 : 1.0) / 4.5e6);
+            if (idx >= 0 && us < two)
+                path = MI355_PATH_MFMA, one_launch = true;
+        }
         if (path == MI355_PATH_SKINNY && M > SKINNY_MAX_M)
             return fail("skinny path needs M <= %d", SKINNY_MAX_M);
         if (path == MI355_PATH_SIMPLE)
@@ -268,8 +329,7 @@ struct GemmCore
             kname = "skinny";
         else
         {
-            const int cus = num_cus();
-            auto      pick = [&](int count, MfmaConfig (*get)(int), const char *env) -> int
+            auto pick = [&](int count, MfmaConfig (*get)(int), const char *env) -> int
             {
                 int  best = -1;
                 long most = -1;
@@ -287,48 +347,11 @@ struct GemmCore
                 (void)env;
                 return best;
             };
-            // The pipelined kernel's tile is chosen with a small cost model in microseconds (the prices and what they were fitted to
-            // stand at g_dma_cost): a tile costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that
-            // fit a compute unit together share all but us_more, plus us_step for every K step, which a full chip slows down
-            // by a share us_load of it (L2, HBM and the power limit are shared by all compute units).
-            // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
-            // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
-            // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again. The 0.88: a deep K
-            // under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900: 10.3 us whole, priced
-            // at 8.6, 8.4 as 4 slices; 350 x 126 x 3520: 11.5, 9.2 and 8.4), and with it the choice is no worse on average.
-            auto pick_dma = [&]() -> int
-            {
-                int    best = -1;
-                double best_cost = 0;
-                for (int i = 0; i < dma_num_configs(); ++i)
-                {
-                    const MfmaConfig c = dma_config(i, patch_c > 0);
-                    if (c.us_tile <= 0 || (N <= 64 && c.BN > 64) || Kp % c.BK != 0)
-                        continue;
-                    const double tiles   = (double)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN) * batch;
-                    const int    occ_lds = (160 * 1024) / c.lds_bytes, occ_wav = 32 / c.waves;
-                    const double occ     = std::max(1, std::min(occ_lds, occ_wav));
-                    const int    nk      = (K + c.BK - 1) / c.BK;
-                    for (int want = 1; want <= MOST_SLICES; ++want)
-                    {
-                        // (slices of equal whole K steps but the last, none of them empty)
-                        const int per = (nk + want - 1) / want, sl = (nk + per - 1) / per;
-                        if (want > 1 && (batch != 1 || per * c.BK < 512))
-                            break;
-                        if (sl != want)
-                            continue;
-                        const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
-                        const double finish = sl > 1 ? 2.4 + 0.1 * sl + 2e-6 * (double)sl * M * N : 0.0;
-                        const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load);
-                        const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 0.88 : 1.0);
-                        if (best < 0 || cost < best_cost)
-                            best = i, best_cost = cost, splitk_plan = sl;
-                    }
-                }
-                return best;
-            };
             cfg_idx = pick(mfma_num_configs(), mfma_config, nullptr);
-            dma_idx = pick_dma();
+            dma_idx = pick_dma(patch_c > 0 ? 1 : 0, splitk_plan, us_dma, one_launch ? 1 : 0);
+            int byte_plan = 1;
+            if (patch_c == 0 && force_tile < 0 && dma_idx >= 0) // (the planes are those of the other's slices)
+                byte_idx = pick_dma(2, byte_plan, us_bytes, splitk_plan);
             if (force_tile >= 0 && Kp % dma_config(force_tile).BK == 0 && dma_idx != force_tile)
             {
                 // a tile shape named by the caller: as many slices as fill the chip once, at least 1024 deep
@@ -343,7 +366,7 @@ struct GemmCore
                 }
             }
             if (K < 16)
-                dma_idx = -1;
+                dma_idx = byte_idx = -1;
             kname_mfma = mfma_config(cfg_idx).name;
             kname_dma  = dma_idx >= 0 ? dma_config(dma_idx).name : "";
             kname      = dma_idx >= 0 ? kname_dma : kname_mfma;
@@ -650,13 +673,19 @@ struct GemmCore
         // through them (dword-aligned rows, K a whole number of 16-byte columns; under K slices every slice its part, which
         // the float epilogue could not take apart again); otherwise one pass over A
         // in front of the GEMM leaves the sums in a vector
-        const bool rowsum_in_kernel = b_off_eff() != 0 && direct && path == MI355_PATH_MFMA && dma_idx >= 0 && K % 16 == 0 && K >= 16 &&
+        // (rows on any byte, or sums that stop inside a 16-byte column, without a pass in front: where the model prices the tile's
+        // own shifting lower than the copy. run_noalloc keeps to the copy and with it to its limits)
+        const double copy_us = 3.3 + (double)M * batch * (direct ? K : K + Kp) * 2.5e-7;
+        const bool   byte_rows = (!direct || (b_off_eff() != 0 && K % 16 != 0)) && ext_ws == nullptr && path == MI355_PATH_MFMA && byte_idx >= 0 &&
+                               !(own_row_terms() && b_off_eff() != 0) && (int64_t)lda * 256 + K < ((int64_t)1 << 32) &&
+                               (one_launch || us_bytes < us_dma + copy_us);
+        const bool rowsum_in_kernel = byte_rows ? b_off_eff() != 0 : b_off_eff() != 0 && direct && path == MI355_PATH_MFMA && dma_idx >= 0 && K % 16 == 0 && K >= 16 &&
                                       (splitk == 1 || epi != EPI_F32) && (int64_t)lda * 256 + K < ((int64_t)1 << 32);
         const bool need_rowvec = b_off_eff() != 0 && !rowsum_in_kernel;
         // the two workspaces of a run: owned by the handle and grown on demand, or carved out of a buffer the caller of
         // this function brings (ext_ws != nullptr: nothing is allocated, sizes beyond ext_ws_bytes are an error)
         const size_t rv_bytes = need_rowvec && !own_row_terms() ? ((sizeof(int32_t) * (size_t)M * batch + 255) & ~(size_t)255) : 0;
-        const size_t ap_bytes = direct ? 0 : (size_t)batch * M * Kp;
+        const size_t ap_bytes = direct || byte_rows ? 0 : (size_t)batch * M * Kp;
         int32_t     *rv       = nullptr;
         int8_t      *ap       = nullptr;
         if (ext_ws != nullptr)
@@ -674,13 +703,14 @@ struct GemmCore
         {
             if (rv_bytes > 0)
                 TRY(rowvec.ensure(rv_bytes));
-            if (!direct)
+            if (ap_bytes > 0)
                 TRY(Ap.ensure(ap_bytes));
             rv = rowvec.as<int32_t>(), ap = Ap.as<int8_t>();
         }
         if (own_row_terms())
             rv = rowvec.as<int32_t>();
-        if (!direct)
+        g.byte_rows = byte_rows ? 1 : 0;
+        if (!direct && !byte_rows)
         {
             // rows not dword aligned: padded, sign-normalised copy (and the row sums in the same pass)
             HIP_TRY(a_prepass_launch(A, lda, a_bs, batch, M, K, flip_a, ap, Kp, need_rowvec ? rv : nullptr, b_off_eff(), s));
@@ -755,9 +785,9 @@ struct GemmCore
         {
             g.fill16 = fill.as<int8_t>();
             // the pipelined kernel moves 16-byte columns of dword-aligned rows straight into LDS
-            const bool aligned =
-                conv ? (g.conv.C % 16 == 0 && ((uintptr_t)g.A & 15) == 0 && g.K % 16 == 0)
-                     : ((((uintptr_t)g.A | (uintptr_t)g.lda | (uintptr_t)g.a_batch_stride) & 3) == 0);
+            const bool aligned = g.byte_rows != 0 ||
+                (conv ? (g.conv.C % 16 == 0 && ((uintptr_t)g.A & 15) == 0 && g.K % 16 == 0)
+                     : ((((uintptr_t)g.A | (uintptr_t)g.lda | (uintptr_t)g.a_batch_stride) & 3) == 0));
             g.a_end = conv ? nullptr : g.A + (int64_t)(batch - 1) * g.a_batch_stride + (int64_t)(g.M - 1) * g.lda + g.K;
             // its producers address a block's A rows (dense) or the whole image batch (convolution) with 32-bit offsets
             const int64_t span = conv ? (int64_t)((g.M + g.conv.OH * g.conv.OW - 1) / (g.conv.OH * g.conv.OW)) *
@@ -775,10 +805,11 @@ struct GemmCore
             }
             else if (dma_idx >= 0 && aligned && g.K >= 16 && span < ((int64_t)1 << 32))
             {
-                const MfmaConfig c = dma_config(dma_idx);
+                const int        idx = g.byte_rows ? byte_idx : dma_idx;
+                const MfmaConfig c   = dma_config(idx);
                 g.tiles_m          = (g.M + c.BM - 1) / c.BM;
                 g.tiles_n          = (g.N + c.BN - 1) / c.BN;
-                kname_run          = &kname_dma_full;
+                kname_run          = g.byte_rows ? &kname_bytes : &kname_dma_full;
                 if (conv)
                     g.conv.pad_word = 0x01010101u * fill_byte; // as in the image: the kernel flips what it loads
                 if (splitk > 1 && batch == 1)
@@ -800,11 +831,11 @@ struct GemmCore
                     // (g.K: K, or K padded to whole steps where the rows of A were copied)
                     gp.a_batch_stride = conv ? 0 : kc, gp.bp_batch_stride = kc, gp.k_slice = (int32_t)kc;
                     kname_run = &kname_splitk;
-                    HIP_TRY(dma_launch(dma_idx, EPI_S32, flip_in_loader, conv, gp, splitk, s));
+                    HIP_TRY(dma_launch(idx, EPI_S32, flip_in_loader, conv, gp, splitk, s));
                     HIP_TRY(splitk_finish_launch(epi, g, parts.as<int32_t>(), (int64_t)M * ldp, ldp, splitk, s));
                     return 0;
                 }
-                HIP_TRY(dma_launch(dma_idx, epi, flip_in_loader, conv, g, batch, s));
+                HIP_TRY(dma_launch(idx, epi, flip_in_loader, conv, g, batch, s));
             }
             else
             {
@@ -984,6 +1015,7 @@ int mi355_gemmlowp_create(const mi355_gemm_desc *desc, mi355_gemm_handle **out)
     c.path     = d.path;
     c.accumulate = (d.flags & MI355_GEMM_ACCUMULATE) != 0, c.act_twice = (d.flags & MI355_GEMM_ACT_TWICE) != 0;
     c.b_shared = d.batch == 1 || d.b_batch_stride == 0;
+    c.byte_lda = ((d.lda | (d.batch > 1 ? d.a_batch_stride : 0)) & 3) != 0;
     if (c.choose_kernel())
     {
         delete h;

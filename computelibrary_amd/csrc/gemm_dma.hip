@@ -850,9 +850,10 @@ struct DmaCost
 {
     double us_tile, us_step, us_load, us_more;
 };
-static const DmaCost g_dma_cost[2][8] = {
+static const DmaCost g_dma_cost[3][8] = {
     {{8.57, 0.622, 0.33, 1.55}, {5.82, 0.412, 0.19, 4.35}, {4.30, 0.307, 0.12, 0.0}, {3.89, 0.188, 0.126, 0.0}, {}, {}, {5.67, 0.536, 0.0, 0.69}, {}},
     {{}, {6.24, 0.541, 0.45, 3.7}, {}, {4.11, 0.339, 0.0, 0.0}, {}, {}, {5.33, 0.818, 0.04, 0.0}, {4.24, 0.489, 0.0, 0.0}},
+    {{}, {}, {}, {3.9, 0.25, 0.126, 0.0}, {}, {}, {}, {}},
 };
 
 // configuration 0 is g_wide, the others are g_ring's
@@ -860,12 +861,13 @@ int dma_num_configs()
 {
     return 1 + g_ring_count;
 }
-MfmaConfig dma_config(int idx, bool conv)
+MfmaConfig dma_config(int idx, int loader)
 {
+    const bool conv = loader == 1;
     MfmaConfig c = idx == 0 ? g_wide.cfg : g_ring[idx - 1].cfg;
     c.waves      = (idx == 0 ? g_wide.threads : g_ring[idx - 1].threads[conv ? 1 : 0]) / 64;
     c.lds_bytes  = idx == 0 ? g_wide.lds_bytes : g_ring[idx - 1].lds_bytes[conv ? 1 : 0];
-    const DmaCost &cost = g_dma_cost[conv ? 1 : 0][idx];
+    const DmaCost &cost = g_dma_cost[loader][idx];
     c.us_tile = cost.us_tile, c.us_step = cost.us_step, c.us_load = cost.us_load, c.us_more = cost.us_more;
     return c;
 }
@@ -874,11 +876,18 @@ int dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &arg
 {
     if (cfg_idx < 0 || cfg_idx >= dma_num_configs() || epi < 0 || epi > 2)
         return (int)hipErrorInvalidValue;
-    const MfmaConfig c       = dma_config(cfg_idx, conv);
+    const MfmaConfig c       = dma_config(cfg_idx, conv ? 1 : 0);
     const int        flip    = flip_a ? 1 : 0;
     int              threads = c.waves * 64, fn_slot = conv ? 1 : 0; // which entry of the once-per-device table below
     const void      *fn      = cfg_idx > 0 ? g_ring[cfg_idx - 1].fn[epi][flip][fn_slot] : conv ? nullptr : g_wide.fn[epi][flip];
-    if (args.epi.rowsum_mul != 0)
+    const bool byte_rows = !conv && args.byte_rows != 0;
+    if (byte_rows)
+    {
+        if (cfg_idx != RING_BYTES_CFG)
+            return (int)hipErrorInvalidValue;
+        fn = g_ring_bytes[epi][flip], fn_slot = 2;
+    }
+    else if (args.epi.rowsum_mul != 0)
     {
         if (args.K % 16 != 0)
             return (int)hipErrorInvalidValue;
@@ -897,7 +906,7 @@ int dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &arg
         args.tiles_n * c.BN < args.N || args.tiles_n * c.BN > round_up(args.N, PACK_N_ALIGN) || args.M < 1)
         return (int)hipErrorInvalidValue;
     if (conv ? (args.conv.C % 16 != 0 || ((uintptr_t)args.A & 15) != 0 || args.K % 16 != 0)
-             : ((((uintptr_t)args.A | (uintptr_t)args.lda | (uintptr_t)args.a_batch_stride) & 3) != 0 || args.a_end == nullptr))
+             : (!byte_rows && ((((uintptr_t)args.A | (uintptr_t)args.lda | (uintptr_t)args.a_batch_stride) & 3) != 0 || args.a_end == nullptr)))
         return (int)hipErrorInvalidValue;
     static_assert(sizeof(g_dma_cost[0]) / sizeof(g_dma_cost[0][0]) == 8, "one price and one flag word per configuration");
     if (c.lds_bytes > 48 * 1024)

@@ -24,7 +24,8 @@ namespace mi355
 enum : int
 {
     RING_DENSE = 0, // dword-aligned rows of A
-    RING_CONV  = 1  // implicit convolution
+    RING_CONV  = 1, // implicit convolution
+    RING_BYTES = 2  // rows of A on any byte
 };
 
 // One wave's loads of a stage: AU / 4 units of A behind BU / 4 units of B
@@ -188,6 +189,136 @@ struct RingLoader
     }
 };
 
+// Rows of A that start on any byte, or whose sums have to stop inside a 16-byte column: direct-to-LDS loads cannot shift bytes,
+// so A and B come into registers (compiler-visible loads) two stages ahead of their write to LDS and four ahead of their use. A
+// lane loads the dwords that hold its 16 bytes - loads off a dword boundary are four times slower - and shifts them into
+// place; bytes beyond K are zero. The copy that a pass in front would make (a_prepass_kernel: 3.3 us and more) is not needed.
+template <int BM, int BN, int BK, int NS, int KG>
+struct RingLoader<BM, BN, BK, NS, KG, RING_BYTES>
+{
+    static constexpr int NW = 4, CPR = BK / 16, RPU = 1024 / BK;
+    static constexpr int AU = BM / RPU, BU = BN / RPU, LA = AU / NW, LB = BU / NW;
+    static constexpr int STAGE = (BM + BN) * BK;
+    static_assert(KG == 1 && BK == 128 && NS == 3, "built for this form");
+    struct Step
+    {
+    };
+    struct Set
+    {
+        v4i a[LA], b[LB];
+        int x[LA]; // the dword behind the four of a[]
+    };
+    const int8_t *a_base, *b_base; // a_base: dword aligned
+    uint32_t      a_off[LA], b_off, b_unit;
+    int           shift[LA]; // bytes from a lane's first dword to its first byte
+    uint32_t      flip;
+    int           c16, K;
+    char         *lds;
+
+    __device__ __forceinline__ void init(const GemmArgs &g, int m0, int n0, int bz, int wave, int lane, char *smem, bool flip_a)
+    {
+        K = g.K, flip = flip_a ? 0x80808080u : 0u;
+        const int ur = lane / CPR;
+        c16          = ((lane % CPR) ^ swz<CPR>(wave * RPU + ur)) * 16;
+        lds          = smem + wave * 1024 + lane * 16;
+        b_base       = g.Bp + (int64_t)bz * g.bp_batch_stride + (int64_t)n0 * g.Kp + (int64_t)wave * RPU * g.Kp;
+        b_off        = (uint32_t)ur * (uint32_t)g.Kp + (uint32_t)c16;
+        b_unit       = (uint32_t)(NW * RPU) * (uint32_t)g.Kp;
+        const int8_t  *a = g.A + (int64_t)bz * g.a_batch_stride + (int64_t)m0 * g.lda;
+        const uint32_t e = (uint32_t)(uintptr_t)a & 3u;
+        a_base           = a - e;
+#pragma unroll
+        for (int i = 0; i < LA; ++i)
+        {
+            // (rows beyond M re-read the last one: their results are never stored)
+            const uint32_t at = e + (uint32_t)min((wave + i * NW) * RPU + ur, g.M - 1 - m0) * (uint32_t)g.lda;
+            a_off[i]          = (at & ~3u) + (uint32_t)c16;
+            shift[i]          = (int)(at & 3u);
+        }
+    }
+    __device__ __forceinline__ void load(Set &s, int kt) const
+    {
+        const int8_t *a_k = a_base + kt * BK, *b_k = b_base + kt * BK;
+        if ((kt + 1) * BK <= K)
+        {
+#pragma unroll
+            for (int i = 0; i < LA; ++i)
+            {
+                // (aligned rows need no fifth dword: it may lie beyond A)
+                s.a[i] = *(const v4i *)__builtin_assume_aligned(a_k + a_off[i], 4);
+                s.x[i] = *(const int *)(a_k + a_off[i] + (shift[i] ? 16u : 0u));
+            }
+        }
+        else
+        {
+            const int rem = min(max(K - kt * BK - c16, 0), 16); // of this lane's 16 bytes; every dword is read that holds one of them
+#pragma unroll
+            for (int i = 0; i < LA; ++i)
+            {
+                const int end = rem ? shift[i] + rem : 0;
+#pragma unroll
+                for (int t = 0; t < 5; ++t)
+                {
+                    int w = 0;
+                    if (4 * t < end)
+                        w = *(const int *)(a_k + a_off[i] + 4 * t);
+                    if (t < 4)
+                        s.a[i][t] = w;
+                    else
+                        s.x[i] = w;
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < LB; ++i)
+            s.b[i] = *(const v4i *)(b_k + (uint32_t)i * (uint64_t)b_unit + b_off);
+    }
+    // stage kt, loaded into s, to its ring slot
+    __device__ __forceinline__ void store(const Set &s, int kt, int slot) const
+    {
+        char *dst = lds + slot * STAGE;
+#pragma unroll
+        for (int i = 0; i < LA; ++i)
+        {
+            v4i v;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                v[t] = (int)(__builtin_amdgcn_alignbyte((uint32_t)(t < 3 ? s.a[i][t < 3 ? t + 1 : 0] : s.x[i]), (uint32_t)s.a[i][t], (uint32_t)shift[i]) ^ flip);
+            if ((kt + 1) * BK > K)
+            {
+                const int rem = K - kt * BK - c16;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                {
+                    const int n = min(max(rem - 4 * t, 0), 4);
+                    v[t] &= n == 4 ? -1 : (1 << (8 * n)) - 1;
+                }
+            }
+            *(v4i *)(dst + i * (NW * 1024)) = v;
+        }
+#pragma unroll
+        for (int i = 0; i < LB; ++i)
+            *(v4i *)(dst + (AU + i * NW) * 1024) = s.b[i];
+    }
+    // (no loads go out between the matrix instructions)
+    __device__ __forceinline__ Step step(int, int) const { return {}; }
+    __device__ __forceinline__ void issue_one(const Step &, int) const {}
+    __device__ __forceinline__ void issue(int, int) const {}
+};
+
+template <typename Loader, int MODE>
+struct ByteSet
+{
+    struct type
+    {
+    };
+};
+template <typename Loader>
+struct ByteSet<Loader, RING_BYTES>
+{
+    using type = typename Loader::Set;
+};
+
 template <int BM, int BN, int BK, int NS, int KG, int EPI, bool FLIP_A, int MODE>
 __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 1 ? 2 : BM * BN <= 64 * 64 ? 4 : 2))) void gemm_ring_kernel(GemmArgs g_in)
 {
@@ -243,8 +374,13 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         qflag = *(const __attribute__((address_space(4))) int32_t *)u_fl;
 
     Loader ld;
-    ld.init(g, m0, n0, bz, wave, lane, lds0);
-    ld.issue(0, 0);
+    if constexpr (MODE == RING_BYTES)
+        ld.init(g, m0, n0, bz, wave, lane, smem, FLIP_A);
+    else
+    {
+        ld.init(g, m0, n0, bz, wave, lane, lds0);
+        ld.issue(0, 0);
+    }
     // per-column epilogue constants: fetched behind the first stage, parked in registers, staged in LDS after the loop
     constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? 1 + QP_COUNT : 0;
     constexpr int PPT  = (NPAR * BN + NW * 64 - 1) / (NW * 64);
@@ -261,10 +397,20 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
                                      : ((global_i32)u_qp)[(int64_t)(par - 1) * g.epi.qp_stride + n0 + col];
         }
     }
+    typename ByteSet<Loader, MODE>::type set_a, set_b; // RING_BYTES: the stages on their way, even and odd ones
+    if constexpr (MODE == RING_BYTES)
+    {
+        ld.load(set_a, 0);
+        if (nk > 1)
+            ld.load(set_b, 1);
+    }
+    else
+    {
 #pragma unroll
-    for (int s = 1; s < NS; ++s)
-        if (s < nk)
-            ld.issue(s, s);
+        for (int s = 1; s < NS; ++s)
+            if (s < nk)
+                ld.issue(s, s);
+    }
     const bool fast = EPI == EPI_FIXEDPOINT && (qflag & 1) == 0;
 
     const int kg    = wave >> 2; // which half of a K step's depth this wave multiplies
@@ -291,7 +437,18 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         rsum[f] = 0;
 
     // this wave's loads of stage 0: behind them NS - 1 stages may still be in flight
-    if (nk < NS)
+    if constexpr (MODE == RING_BYTES)
+    {
+        ld.store(set_a, 0, 0);
+        if (nk > 2)
+            ld.load(set_a, 2);
+        if (nk > 1)
+            ld.store(set_b, 1, 1);
+        if (nk > 3)
+            ld.load(set_b, 3);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    else if (nk < NS)
         wait_vmcnt<0>();
     else
         wait_vmcnt<(NS - 1) * LPW>();
@@ -313,7 +470,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
     {
         constexpr int H = decltype(h_c)::value, CUR = decltype(cur_c)::value;
         constexpr int I0 = decltype(first_c)::value, NI = decltype(count_c)::value;
-        if (FLIP_A)
+        if (FLIP_A && MODE != RING_BYTES)
         {
 #pragma unroll
             for (int f = 0; f < RS; ++f)
@@ -381,33 +538,58 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         read_one(0, 0, smem, f);
     using yes = std::true_type;
     using no  = std::false_type;
-    // steps whose stage kt + NS is whole: [0, lean)
-    const int lean = (ld.whole(nk - 1) ? nk : nk - 1) - NS;
-    int       kt   = 0;
-    if constexpr (SUB == 2)
+    if constexpr (MODE == RING_BYTES)
     {
-        if (lean > 0)
+        // Stage kt + 2 goes to LDS behind the barrier of step kt, stage kt + 4 takes over its registers
+        auto byte_step = [&](int kt, typename Loader::Set &set)
         {
-            k_step(kt++, set0{}, no{}, yes{});
-            for (; kt < lean; ++kt)
-                k_step(kt, set0{}, yes{}, yes{});
-            k_step(kt++, set0{}, yes{}, no{}); // (nk > NS: there is such a step)
+            sub_step(kt, set0{}, set0{}, smem + slot * STAGE, 1, t, set0{}, set0{});
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            block_barrier();
+            slot = slot + 1 == NS ? 0 : slot + 1;
+            if (kt + 2 < nk)
+                ld.store(set, kt + 2, slot + 1 == NS ? 0 : slot + 1);
+            if (kt + 4 < nk)
+                ld.load(set, kt + 4);
+            sub_step(kt, set1{}, set1{}, smem + slot * STAGE, 0, t, set0{}, set0{});
+        };
+        for (int kt = 0; kt < nk; kt += 2)
+        {
+            byte_step(kt, set_a);
+            if (kt + 1 < nk)
+                byte_step(kt + 1, set_b);
         }
-        for (; kt < nk; ++kt)
-            k_step(kt, set0{}, no{}, no{});
     }
     else
     {
-        for (; kt + 1 < lean; kt += 2)
+        // steps whose stage kt + NS is whole: [0, lean)
+        const int lean = (ld.whole(nk - 1) ? nk : nk - 1) - NS;
+        int       kt   = 0;
+        if constexpr (SUB == 2)
         {
-            k_step(kt, set0{}, no{}, yes{});
-            k_step(kt + 1, set1{}, no{}, yes{});
+            if (lean > 0)
+            {
+                k_step(kt++, set0{}, no{}, yes{});
+                for (; kt < lean; ++kt)
+                    k_step(kt, set0{}, yes{}, yes{});
+                k_step(kt++, set0{}, yes{}, no{}); // (nk > NS: there is such a step)
+            }
+            for (; kt < nk; ++kt)
+                k_step(kt, set0{}, no{}, no{});
         }
-        for (; kt < nk; kt += 2)
+        else
         {
-            k_step(kt, set0{}, no{}, no{});
-            if (kt + 1 < nk)
-                k_step(kt + 1, set1{}, no{}, no{});
+            for (; kt + 1 < lean; kt += 2)
+            {
+                k_step(kt, set0{}, no{}, yes{});
+                k_step(kt + 1, set1{}, no{}, yes{});
+            }
+            for (; kt < nk; kt += 2)
+            {
+                k_step(kt, set0{}, no{}, no{});
+                if (kt + 1 < nk)
+                    k_step(kt + 1, set1{}, no{}, no{});
+            }
         }
     }
     // the reads issued last are never used, but must have left the LDS before the epilogue writes there
@@ -471,7 +653,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
     }
     const int row_e = row_w + kg * RE * 16;
     if (rowsum)
-        finish_row_sums<RE>(rfin, g.epi.rowsum_mul, FLIP_A && MODE != RING_CONV ? nk * BK - g.K : 0);
+        finish_row_sums<RE>(rfin, g.epi.rowsum_mul, FLIP_A && MODE == RING_DENSE ? nk * BK - g.K : 0);
 
     if (fast)
     {

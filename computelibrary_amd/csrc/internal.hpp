@@ -59,6 +59,7 @@ struct GemmArgs
     // column of that step could reach beyond a_end. Every other tile may fetch the step whole - the columns at and
     // beyond K then hold whatever follows in memory and meet the zero rows of the packed B. -1: no tile may.
     int32_t  lean_tail_bz;
+    int32_t  byte_rows; // dense: rows of A on any byte, or sums of rows whose K ends inside a 16-byte column (host only: picks the kernel)
 };
 
 struct MfmaConfig
@@ -109,10 +110,13 @@ struct RingEntry
 };
 extern const RingEntry g_ring[];
 extern const int       g_ring_count;
+constexpr int            RING_BYTES_CFG = 3;
+extern const void *const g_ring_bytes[3][2]; // rows on any byte, in that configuration's tiles; [epi][flip]
 
 // gemm_dma.hip — same contract as mfma_launch; additionally needs 16-byte aligned A rows, K % 16 == 0 and args.fill16
 int         dma_num_configs();
-MfmaConfig  dma_config(int idx, bool conv = false); // conv: priced for the implicit convolution's loader
+// loader: 0 dense, 1 the implicit convolution, 2 dense rows on any byte: what the prices are for
+MfmaConfig  dma_config(int idx, int loader = 0);
 int         dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &args, int batch, hipStream_t s);
 
 // gemm_narrow.hip — N <= 64, K <= 1152, 16-byte aligned operands: A straight from global memory into the matrix cores'
