@@ -174,6 +174,7 @@ struct GemmCore
     mi355_requant rq{};
     float   scale = 1.f, act_min = -INFINITY, act_max = INFINITY;
     bool    accumulate = false, act_twice = false;
+    bool    half_out = false; // this run's kernels round to half themselves (set around run_dense)
     int     path = MI355_PATH_AUTO, cfg_idx = 0, dma_idx = -1;
     int     force_tile = -1; // >= 0: the pipelined kernel's tile configuration the caller asked for (MI355_PATH_TILE + n)
     int     Kp = 0, Np = 0;
@@ -651,11 +652,18 @@ struct GemmCore
         p.dst_signed          = dst_dtype == MI355_S8;
         p.accumulate          = accumulate ? 1 : 0;
         p.act_twice           = act_twice ? 1 : 0;
+        p.half_out            = half_out ? 1 : 0;
     }
 
     // K slices to a float destination take the row terms from a pass (see run_dense) that the same product whole would not
     // need: the vector is there from prepare on, so that a first run can be recorded and a run_noalloc needs no workspace
     bool own_row_terms() const { return splitk > 1 && epi == EPI_F32; }
+
+    // Whether the kernel that a run takes can round to half itself: the streaming and the pipelined one, not the fallbacks
+    bool rounds_to_half(int64_t lda) const
+    {
+        return !accumulate && (path == MI355_PATH_SKINNY || (path == MI355_PATH_MFMA && dma_idx >= 0 && K >= 16 && (int64_t)std::max(lda, (int64_t)Kp) * 256 + Kp < ((int64_t)1 << 32)));
+    }
 
     // A, D and bias_f32 are device pointers here
     int run_dense(const int8_t *A, int64_t lda, int64_t a_bs, void *D, int64_t ldd, int64_t d_bs,
@@ -737,7 +745,7 @@ struct GemmCore
     // 4 consecutive outputs of a row may leave as one store when every row start is aligned to 4 elements
     void set_vec_store(GemmArgs &g) const
     {
-        const size_t esz = (epi == EPI_FIXEDPOINT) ? 1 : 4;
+        const size_t esz = (epi == EPI_FIXEDPOINT) ? 1 : half_out ? 2 : 4;
         g.epi.vec_store  = (((uintptr_t)g.D % (4 * esz)) == 0 && g.ldd % 4 == 0 && g.d_batch_stride % 4 == 0) ? 1 : 0;
         g.epi.vec_store16 = (esz == 1 && ((uintptr_t)g.D % 16) == 0 && g.ldd % 16 == 0 && g.d_batch_stride % 16 == 0) ? 1 : 0;
     }
@@ -774,7 +782,7 @@ struct GemmCore
                     GemmArgs ge = gb;
                     ge.A        = gb.A + (int64_t)b * gb.a_batch_stride;
                     ge.Bp       = gb.Bp + (int64_t)b * gb.bp_batch_stride;
-                    ge.D        = (char *)gb.D + (int64_t)b * gb.d_batch_stride * (epi == EPI_FIXEDPOINT ? 1 : 4);
+                    ge.D        = (char *)gb.D + (int64_t)b * gb.d_batch_stride * (epi == EPI_FIXEDPOINT ? 1 : half_out ? 2 : 4);
                     ge.epi.colvec += (int64_t)b * gb.epi.colvec_batch_stride;
                     if (ge.epi.rowvec != nullptr)
                         ge.epi.rowvec += (int64_t)b * gb.epi.rowvec_batch_stride;
@@ -1175,9 +1183,17 @@ int mi355_gemmlowp_run(mi355_gemm_handle *h, const void *A, const float *bias_f3
         if (c.accumulate) // the previous values
             HIP_TRY(restride_nd_launch(Dplanes, Dd, (int)(d.N * esz), d.d_plane_rows, d.M / d.d_plane_rows, d.batch, d_given, d_dense, s));
     }
-    if (f16)
+    if (f16 && c.rounds_to_half(lda))
     {
-        // the kernels write a dense F32 matrix, which is rounded into the half destination afterwards. Accumulating:
+        c.half_out   = true;
+        const int rc = c.run_dense((const int8_t *)Ad, lda, a_bs, Dd, ldd, d_bs, (const float *)bfd, s);
+        c.half_out   = false;
+        if (rc)
+            return rc;
+    }
+    else if (f16)
+    {
+        // Accumulating, and where a fallback kernel runs: a dense F32 matrix, rounded into the half destination afterwards. Accumulating:
         // the addition (and the activation, which has to follow it) happens in that second step, on halfs.
         TRY(h->wsF32.ensure(sizeof(float) * (size_t)d.batch * d.M * d.N));
         float      *ws  = h->wsF32.as<float>();

@@ -330,8 +330,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
         if (fast)
         {
             __syncthreads(); // the consumers' staging of the epilogue constants
-            if (g.epi.vec_store16)
-                __syncthreads(); // ... and of the output tile
+            __syncthreads(); // ... and of the output tile
         }
         return;
     }
@@ -482,20 +481,18 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
         {
             char *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
             const bool rowv = g.epi.rowvec != nullptr || rowsum;
-            if (g.epi.vec_store16 && g.epi.qp_std && qflag == 0 && !rowv)
+            if (g.epi.qp_std && qflag == 0 && !rowv)
                 epilogue_store_staged<true, false, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
                                                                        [] { __syncthreads(); });
-            else if (g.epi.vec_store16 && g.epi.qp_std && qflag == 0)
+            else if (g.epi.qp_std && qflag == 0)
                 epilogue_store_staged<true, true, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
                                                                       [] { __syncthreads(); }, rsum, rowsum);
-            else if (g.epi.vec_store16)
+            else
                 epilogue_store_staged<false, true, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
                                                                        [] { __syncthreads(); }, rsum, rowsum);
-            else
-                epilogue_store_fast<RS, QS, BN>(acc, g, par, m0 + row_w, n0 + col_w, col_w, lane, bz, rsum, rowsum);
         }
     }
-    else if ((EPI == EPI_S32 || EPI == EPI_F32) && g.epi.vec_store && !g.epi.accumulate)
+    else if ((EPI == EPI_S32 || EPI == EPI_F32) && !g.epi.accumulate)
     {
         // the ring is free beyond the last barrier: 16 x (QS*64 + 16) bytes per wave
         if constexpr (EPI != EPI_FIXEDPOINT)
@@ -658,8 +655,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
         if (fast)
         {
             __syncthreads(); // the consumers' staging of the epilogue constants
-            if (g.epi.vec_store16)
-                __syncthreads(); // ... and of the output tile
+            __syncthreads(); // ... and of the output tile
         }
         return;
     }
@@ -792,20 +788,18 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
         {
             char      *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
             const bool rowv  = g.epi.rowvec != nullptr;
-            if (g.epi.vec_store16 && g.epi.qp_std && qflag == 0 && !rowv)
+            if (g.epi.qp_std && qflag == 0 && !rowv)
                 epilogue_store_staged<true, false, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
                                                                        [] { __syncthreads(); });
-            else if (g.epi.vec_store16 && g.epi.qp_std && qflag == 0)
+            else if (g.epi.qp_std && qflag == 0)
                 epilogue_store_staged<true, true, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
                                                                       [] { __syncthreads(); });
-            else if (g.epi.vec_store16)
+            else
                 epilogue_store_staged<false, true, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
                                                                        [] { __syncthreads(); });
-            else
-                epilogue_store_fast<RS, QS, BN>(acc, g, par, m0 + row_w, n0 + col_w, col_w, lane, bz);
         }
     }
-    else if ((EPI == EPI_S32 || EPI == EPI_F32) && g.epi.vec_store && !g.epi.accumulate)
+    else if ((EPI == EPI_S32 || EPI == EPI_F32) && !g.epi.accumulate)
     {
         if constexpr (EPI != EPI_FIXEDPOINT)
             epilogue_store_wave32<EPI, RS, QS>(acc, g, smem + wave * 16 * (QS * 64 + 16), m0 + row_w, n0 + col_w, lane, bz);

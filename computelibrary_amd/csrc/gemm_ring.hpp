@@ -670,20 +670,18 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         {
             char      *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
             const bool rowv  = g.epi.rowvec != nullptr || rowsum;
-            if (g.epi.vec_store16 && g.epi.qp_std && qflag == 0 && !rowv)
+            if (g.epi.qp_std && qflag == 0 && !rowv)
                 epilogue_store_staged<true, false, RE, QS, BM, BN, NW>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
                                                                        [] { __syncthreads(); });
-            else if (g.epi.vec_store16 && g.epi.qp_std && qflag == 0)
+            else if (g.epi.qp_std && qflag == 0)
                 epilogue_store_staged<true, true, RE, QS, BM, BN, NW>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
                                                                       [] { __syncthreads(); }, rfin, rowsum);
-            else if (g.epi.vec_store16)
+            else
                 epilogue_store_staged<false, true, RE, QS, BM, BN, NW>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
                                                                        [] { __syncthreads(); }, rfin, rowsum);
-            else
-                epilogue_store_fast<RE, QS, BN>(fin, g, par, m0 + row_e, n0 + col_w, col_w, lane, bz, rfin, rowsum);
         }
     }
-    else if ((EPI == EPI_S32 || EPI == EPI_F32) && g.epi.vec_store && !g.epi.accumulate)
+    else if ((EPI == EPI_S32 || EPI == EPI_F32) && !g.epi.accumulate)
     {
         if constexpr (EPI != EPI_FIXEDPOINT)
             epilogue_store_wave32<EPI, RE, QS>(fin, g, smem + wave * 16 * (QS * 64 + 16), m0 + row_e, n0 + col_w, lane, bz, rfin, rowsum);

@@ -42,7 +42,7 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(GemmArgs g)
         const int64_t bz = blockIdx.y;
         g.A += bz * g.a_batch_stride;
         g.Bp += bz * g.bp_batch_stride;
-        g.D = (char *)g.D + bz * g.d_batch_stride * (EPI == EPI_FIXEDPOINT ? 1 : 4);
+        g.D = (char *)g.D + bz * g.d_batch_stride * (EPI == EPI_FIXEDPOINT ? 1 : EPI == EPI_F32 && g.epi.half_out ? 2 : 4);
         g.epi.colvec += bz * g.epi.colvec_batch_stride;
         if (g.epi.rowvec)
             g.epi.rowvec += bz * g.epi.rowvec_batch_stride;
@@ -394,8 +394,14 @@ __global__ __launch_bounds__(SK_WAVES * 64) void gemm_skinny_kernel(GemmArgs g)
                 else if (EPI == EPI_FIXEDPOINT)
                     ((int8_t *)g.D)[idx] = (int8_t)epi_fixedpoint(sum[n][r], cv[n], rv, mu[n], sh[n], p);
                 else
-                    ((float *)g.D)[idx] = epi_f32(sum[n][r], (int32_t)((uint32_t)cv[n] + (uint32_t)rv), bf[n],
-                                                  p.bias_f32 != nullptr, p, p.accumulate ? ((float *)g.D)[idx] : 0.f);
+                {
+                    const float f = epi_f32(sum[n][r], (int32_t)((uint32_t)cv[n] + (uint32_t)rv), bf[n], p.bias_f32 != nullptr, p,
+                                            p.accumulate ? ((float *)g.D)[idx] : 0.f);
+                    if (p.half_out)
+                        ((_Float16 *)g.D)[idx] = (_Float16)f;
+                    else
+                        ((float *)g.D)[idx] = f;
+                }
             }
         }
     }
@@ -426,7 +432,7 @@ struct OnceArgs
     int32_t        M, N, KB, grid;
     int32_t        result_offset, stage, lo, hi;
     float          scale, act_min, act_max;
-    int32_t        has_offsets, accumulate, act_twice;
+    int32_t        has_offsets, accumulate, act_twice, half_out;
 };
 // One output of the stage-once kernels: the reduced sum, its column term c, multiplier (or float bias bits) m, shift sh
 // and row term rv through epilogue EPI into element idx of D
@@ -451,8 +457,14 @@ __device__ __forceinline__ void once_store_output(MI355_GLOBAL char *gD, int64_t
         ((MI355_GLOBAL int8_t *)gD)[idx] = (int8_t)q;
     }
     else
-        ((MI355_GLOBAL float *)gD)[idx] = epi_f32(sum, (int32_t)((uint32_t)c + (uint32_t)rv), __int_as_float(m), has_bias, p,
-                                                  p.accumulate ? ((MI355_GLOBAL float *)gD)[idx] : 0.f);
+    {
+        const float f = epi_f32(sum, (int32_t)((uint32_t)c + (uint32_t)rv), __int_as_float(m), has_bias, p,
+                                p.accumulate ? ((MI355_GLOBAL float *)gD)[idx] : 0.f);
+        if (p.half_out)
+            ((MI355_GLOBAL _Float16 *)gD)[idx] = (_Float16)f;
+        else
+            ((MI355_GLOBAL float *)gD)[idx] = f;
+    }
 }
 #undef MI355_GLOBAL
 
@@ -510,7 +522,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
     EpiParams  p{};
     p.result_offset = g.result_offset, p.stage = g.stage, p.lo = g.lo, p.hi = g.hi;
     p.scale = g.scale, p.act_min = g.act_min, p.act_max = g.act_max;
-    p.has_offsets = g.has_offsets, p.accumulate = g.accumulate, p.act_twice = g.act_twice;
+    p.has_offsets = g.has_offsets, p.accumulate = g.accumulate, p.act_twice = g.act_twice, p.half_out = g.half_out;
 
     const int lane = threadIdx.x & 63;
     // (8 k blocks per wave: the wave index as a scalar, so that the addresses of the B blocks are a scalar base plus one
@@ -794,7 +806,7 @@ __global__ __launch_bounds__(ONCE_WAVES * 64) void gemm_skinny_deepk_kernel(Once
     EpiParams  p{};
     p.result_offset = g.result_offset, p.stage = g.stage, p.lo = g.lo, p.hi = g.hi;
     p.scale = g.scale, p.act_min = g.act_min, p.act_max = g.act_max;
-    p.has_offsets = g.has_offsets, p.accumulate = g.accumulate, p.act_twice = g.act_twice;
+    p.has_offsets = g.has_offsets, p.accumulate = g.accumulate, p.act_twice = g.act_twice, p.half_out = g.half_out;
 
     const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
     const int KB = g.KB, NGT = (g.N + 15) / 16, G = g.grid;
@@ -1007,7 +1019,7 @@ static int skinny_once_launch_r(int epi, bool flip_a, const GemmArgs &a, int gri
     const EpiParams &p = a.epi;
     OnceArgs         o{a.A,    a.Bp,   a.D,    p.colvec, p.rowvec,  p.mult,    p.shift,       p.bias_f32,   a.lda,       a.ldd,        a.M,
                a.N,    (int32_t)(a.Kp / 64), grid, p.result_offset, p.stage, p.lo, p.hi, p.scale, p.act_min, p.act_max,
-               p.has_offsets, p.accumulate, p.act_twice};
+               p.has_offsets, p.accumulate, p.act_twice, p.half_out};
     void *kargs[] = {&o};
     return (int)hipLaunchKernel(fn, dim3(grid), dim3(WAVES * 64), kargs, lds, s);
 }
@@ -1035,7 +1047,7 @@ static int skinny_deepk_launch(int epi, bool flip_a, const GemmArgs &a, int grid
     const EpiParams &p = a.epi;
     OnceArgs         o{a.A,    a.Bp,   a.D,    p.colvec, p.rowvec,  p.mult,    p.shift,       p.bias_f32,   a.lda,       a.ldd,        a.M,
                a.N,    (int32_t)(a.Kp / 64), grid, p.result_offset, p.stage, p.lo, p.hi, p.scale, p.act_min, p.act_max,
-               p.has_offsets, p.accumulate, p.act_twice};
+               p.has_offsets, p.accumulate, p.act_twice, p.half_out};
     void *kargs[] = {&o};
     return (int)hipLaunchKernel(fn, dim3(grid), dim3(ONCE_WAVES * 64), kargs, lds, s);
 }

@@ -92,6 +92,17 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const int32_t *__res
             for (int c = 0; c < 4 && j0 + c < g.N; ++c)
                 D[idx + c] = (char)o[c];
     }
+    else if (EPI == EPI_F32 && p.half_out)
+    {
+        typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+        const v4h        h = {(_Float16)__int_as_float(o[0]), (_Float16)__int_as_float(o[1]), (_Float16)__int_as_float(o[2]),
+                              (_Float16)__int_as_float(o[3])};
+        if (vec)
+            *(v4h *)((_Float16 *)D + idx) = h;
+        else
+            for (int c = 0; c < 4 && j0 + c < g.N; ++c)
+                ((_Float16 *)D)[idx + c] = h[c];
+    }
     else
     {
         if (vec)

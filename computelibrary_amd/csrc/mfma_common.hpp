@@ -304,7 +304,7 @@ __device__ __forceinline__ void epilogue_store_t(const v4i (&acc)[RS][QS], const
         }
     }
 }
-// FIXEDPOINT epilogue of the pipelined kernel for multipliers >= 0. The block's per-column constants were staged in LDS
+// FIXEDPOINT epilogue of the narrow kernels for multipliers >= 0, straight to the destination. The block's per-column constants were staged in LDS
 // as par[6][BN]: row 0 the folded offset/bias vector, rows 1..5 the QP_* vectors; col_in_tile is the wave's first
 // column inside the block tile. Same accumulator layout as epilogue_store_t.
 template <int RS, int QS, int BN>
@@ -364,12 +364,13 @@ __device__ __forceinline__ void epilogue_store_fast(const v4i (&acc)[RS][QS], co
         }
     }
 }
-// The same arithmetic as epilogue_store_fast, but the packed 8-bit results of the whole BM x BN block tile are first
-// laid out in LDS (row pitch BN + 16 bytes: the 64 dword writes of a wave instruction - 16 rows by 4 dwords - then hit
-// 64 different banks) and then written with 16 bytes per lane, BN/16 lanes per output row, so a wave instruction writes
-// whole rows of the tile instead of 16-byte pieces of 16 different rows. All NW consumer waves of the block call this
-// together; `barrier` is executed once between the two phases by every wave of the block. Requires p.vec_store16.
-// stage must not overlap par. ROWV: a per-row term exists (b_offset != 0) and is added.
+// FIXEDPOINT epilogue of the pipelined kernel for multipliers >= 0. The block's per-column constants were staged in LDS
+// as par[6][BN]: row 0 the folded offset/bias vector, rows 1..5 the QP_* vectors; col_in_tile is the wave's first
+// column inside the block tile; accumulator layout as in epilogue_store_t. The packed 8-bit results of the whole BM x BN block
+// tile are first laid out in LDS (row pitch BN + 16 bytes: the 64 dword writes of a wave instruction - 16 rows by 4 dwords - then
+// hit 64 different banks) and then written row by row, so a wave instruction writes pieces of rows end to end instead of
+// 16 (or 4 times 1) bytes of 16 different rows. All NW consumer waves of the block call this together; `barrier` is executed
+// once between the two phases by every wave of the block. stage must not overlap par. ROWV: a per-row term exists and is added.
 template <bool STD, bool ROWV, int RS, int QS, int BM, int BN, int NW, typename Barrier>
 __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], const GemmArgs &g, const int32_t *par,
                                                       char *stage, int m0, int n0, int row_in_tile, int col_in_tile,
@@ -420,31 +421,64 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
         }
     }
     barrier();
-    constexpr int LPR = BN / 16;  // lanes per output row
-    constexpr int RPI = 64 / LPR; // rows per wave instruction
-    char         *D   = (char *)g.D + (int64_t)bz * g.d_batch_stride;
-    const int     rr = lane / LPR, cc = (lane % LPR) * 16;
-#pragma unroll
-    for (int it = 0; it < (BM + NW * RPI - 1) / (NW * RPI); ++it)
+    // 16, 4 or 1 byte per lane, as the destination's rows are aligned: a wave instruction writes pieces of rows end to end
+    char *D    = (char *)g.D + (int64_t)bz * g.d_batch_stride;
+    auto  leave = [&](auto bytes_c)
     {
-        const int r = (it * NW + wave) * RPI + rr;
-        const int i = m0 + r, j0 = n0 + cc;
-        if (i >= g.M || j0 >= g.N || (BM % (NW * RPI) != 0 && r >= BM))
-            continue;
-        const v4i     val = *(const v4i *)(stage + r * PITCH + cc);
-        const int64_t idx = (int64_t)i * g.ldd + j0;
-        if (j0 + 16 <= g.N)
-            __builtin_nontemporal_store(val, (v4i *)(D + idx));
-        else
+        constexpr int W = decltype(bytes_c)::value;
+        constexpr int LPR = BN / W > 64 ? 64 : BN / W; // lanes per output row (or per 64 bytes of it)
+        constexpr int PARTS = BN / W / LPR, RPI = 64 / LPR; // ... rows per wave instruction
+        const int     rr = lane / LPR;
+#pragma unroll
+        for (int it = 0; it < (BM + NW * RPI - 1) / (NW * RPI); ++it)
         {
-            for (int t = 0; t < g.N - j0; ++t)
-                D[idx + t] = (char)(val[t >> 2] >> (8 * (t & 3)));
+            const int r = (it * NW + wave) * RPI + rr;
+            const int i = m0 + r;
+#pragma unroll
+            for (int part = 0; part < PARTS; ++part)
+            {
+                const int cc = part * LPR * W + (lane % LPR) * W, j0 = n0 + cc;
+                if (i >= g.M || j0 >= g.N || (BM % (NW * RPI) != 0 && r >= BM))
+                    continue;
+                const int64_t idx = (int64_t)i * g.ldd + j0;
+                if constexpr (W == 16)
+                {
+                    const v4i val = *(const v4i *)(stage + r * PITCH + cc);
+                    if (j0 + 16 <= g.N)
+                        __builtin_nontemporal_store(val, (v4i *)(D + idx));
+                    else
+                    {
+                        for (int t = 0; t < g.N - j0; ++t)
+                            D[idx + t] = (char)(val[t >> 2] >> (8 * (t & 3)));
+                    }
+                }
+                else if constexpr (W == 4)
+                {
+                    const int val = *(const int *)(stage + r * PITCH + cc);
+                    if (j0 + 4 <= g.N)
+                        *(int *)(D + idx) = val;
+                    else
+                    {
+                        for (int t = 0; t < g.N - j0; ++t)
+                            D[idx + t] = (char)(val >> (8 * t));
+                    }
+                }
+                else
+                    D[idx] = stage[r * PITCH + cc];
+            }
         }
-    }
+    };
+    if (p.vec_store16)
+        leave(std::integral_constant<int, 16>{});
+    else if (p.vec_store)
+        leave(std::integral_constant<int, 4>{});
+    else
+        leave(std::integral_constant<int, 1>{});
 }
 // S32 / F32 results of one wave's (RS*16) x (QS*16) sub-tile, 16 rows at a time through a wave-private LDS area
 // (16 rows, pitch QS*64 + 16 bytes) so that they leave as 16 bytes per lane along whole row segments of QS*64 bytes
-// instead of 16-byte pieces of 16 different rows. Needs no synchronisation with other waves. Requires p.vec_store.
+// instead of 16-byte pieces of 16 different rows. Needs no synchronisation with other waves. Halves (EpiParams::half_out) are rounded
+// on the way out: as a pass of its own behind a float workspace that was 5.0 of 21 us at 512 x 4096 x 4096.
 template <int EPI, int RS, int QS>
 __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], const GemmArgs &g, char *stage, int row0,
                                                       int col0, int lane, int bz, const int32_t *rvk = nullptr, bool use_rvk = false)
@@ -458,8 +492,18 @@ __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], 
     const EpiParams &p      = g.epi;
     const int32_t   *colvec = p.colvec + (int64_t)bz * p.colvec_batch_stride;
     const int32_t   *rowvec = p.rowvec ? p.rowvec + (int64_t)bz * p.rowvec_batch_stride : nullptr;
-    char            *D      = (char *)g.D + (int64_t)bz * g.d_batch_stride * 4;
+    typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+    const bool       half   = EPI == EPI_F32 && p.half_out, vec = p.vec_store;
+    const int        esz    = half ? 2 : 4;
+    char            *D      = (char *)g.D + (int64_t)bz * g.d_batch_stride * esz;
     const int        rr = lane / LPR, cc = lane % LPR;
+    auto             store_one = [&](char *to, int32_t v)
+    {
+        if (half)
+            *(_Float16 *)to = (_Float16)__int_as_float(v);
+        else
+            *(int32_t *)to = v;
+    };
     // Everything the loop below needs from global memory is fetched before its first store goes out: a wait for a load
     // issued after a store also waits for that store to reach memory, and one such wait per block of 16 x 16 outputs
     // made the epilogue as slow as its slowest store, sixteen times over.
@@ -491,8 +535,8 @@ __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], 
     {
         constexpr bool BIAS = decltype(bias_c)::value, OFFS = decltype(offs_c)::value, TWICE = decltype(twice_c)::value;
         constexpr bool INSIDE = decltype(inside_c)::value;
-        char         *dp   = D + ((int64_t)(row0 + rr) * g.ldd + col0 + cc * 4) * 4; // this lane's segment of the first row
-        const int64_t step = (int64_t)RPI * g.ldd * 4;
+        char         *dp   = D + ((int64_t)(row0 + rr) * g.ldd + col0 + cc * 4) * esz; // this lane's segment of the first row
+        const int64_t step = (int64_t)RPI * g.ldd * esz;
         const float   scale = p.scale, lo = p.act_min, hi = p.act_max;
 #pragma unroll
         for (int rs = 0; rs < RS; ++rs)
@@ -514,27 +558,45 @@ __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], 
                 }
                 *(v4i *)(stage + lr * PITCH + (qs * 16 + 4 * lh) * 4) = o;
             }
-#pragma unroll
-            for (int it = 0; it < 16 / RPI; ++it)
+            if (vec)
             {
-                const int r   = it * RPI + rr;
-                const v4i val = *(const v4i *)(stage + r * PITCH + cc * 16);
-                if (INSIDE)
+#pragma unroll
+                for (int it = 0; it < 16 / RPI; ++it)
                 {
-                    __builtin_nontemporal_store(val, (v4i *)dp);
-                    dp += step;
-                    continue;
+                    const int r   = it * RPI + rr;
+                    const v4i val = *(const v4i *)(stage + r * PITCH + cc * 16);
+                    const int gi = row0 + rs * 16 + r, j0 = col0 + cc * 4;
+                    if (!INSIDE && (gi >= g.M || j0 >= g.N))
+                        continue;
+                    if (INSIDE || j0 + 3 < g.N)
+                    {
+                        char *to = INSIDE ? dp : D + ((int64_t)gi * g.ldd + j0) * esz;
+                        if (half)
+                            __builtin_nontemporal_store((v4h){(_Float16)__int_as_float(val[0]), (_Float16)__int_as_float(val[1]),
+                                                              (_Float16)__int_as_float(val[2]), (_Float16)__int_as_float(val[3])},
+                                                        (v4h *)to);
+                        else
+                            __builtin_nontemporal_store(val, (v4i *)to);
+                        dp += step;
+                    }
+                    else
+                    {
+                        for (int t = 0; t < g.N - j0; ++t)
+                            store_one(D + ((int64_t)gi * g.ldd + j0 + t) * esz, val[t]);
+                    }
                 }
-                const int gi = row0 + rs * 16 + r, j0 = col0 + cc * 4;
-                if (gi >= g.M || j0 >= g.N)
-                    continue;
-                const int64_t idx = ((int64_t)gi * g.ldd + j0) * 4;
-                if (j0 + 3 < g.N)
-                    __builtin_nontemporal_store(val, (v4i *)(D + idx));
-                else
+            }
+            else
+            {
+                // rows that are not aligned to 4 elements: one element per lane, rows end to end
+#pragma unroll
+                for (int it = 0; it < QS * 4; ++it)
                 {
-                    for (int t = 0; t < g.N - j0; ++t)
-                        *(int32_t *)(D + idx + 4 * t) = val[t];
+                    const int at = it * 64 + lane, r = at / (QS * 16), c = at % (QS * 16);
+                    const int gi = row0 + rs * 16 + r, j = col0 + c;
+                    const int val = *(const int *)(stage + r * PITCH + c * 4);
+                    if (gi < g.M && j < g.N)
+                        store_one(D + ((int64_t)gi * g.ldd + j) * esz, val);
                 }
             }
         }
