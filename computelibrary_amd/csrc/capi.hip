@@ -210,7 +210,7 @@ struct GemmCore
     std::string kname_mfma, kname_dma, kprefix;
     // The names a run can report, composed when the choice is made (create, prepare, update): a run only points at one
     // of them - it must not touch the host heap
-    std::string        kname_narrow, kname_band, kname_dma_full, kname_bytes, kname_splitk, kname_mfma_full;
+    std::string        kname_narrow, kname_band, kname_dma_full, kname_bytes, kname_rows, kname_splitk, kname_mfma_full;
     const char        *kname_static = nullptr; // the streaming kernel names its forms itself
     const std::string *kname_run = nullptr; // what the last run took (nullptr: no run yet, kname is what create announced)
     uint8_t fill_byte = 0; // value of the 16 filler bytes (0, or the im2col pad value)
@@ -224,6 +224,7 @@ struct GemmCore
         kname_narrow    = kprefix + "narrow_32x64";
         kname_band      = kprefix + "band_32x64";
         kname_dma_full  = kprefix + kname_dma;
+        kname_rows      = kprefix + "rows_32x64";
         kname_bytes     = byte_idx >= 0 ? kprefix + dma_config(byte_idx).name + "_bytes" : std::string();
         kname_splitk    = kname_dma_full + "_splitk" + std::to_string(splitk);
         kname_mfma_full = kprefix + kname_mfma;
@@ -934,6 +935,7 @@ struct mi355_conv_handle
     int             c_pad = 0;               // > 0: the kernels see this many channels (source and weights padded, see create)
     ConvGeom        geom_true;               // ... and the geometry with the caller's channel count, for the patches' row sums
     bool            patch_rows = false;      // ... one pixel being the KW taps of a patch row
+    bool            raw_rows = false;        // ... whose kernel takes them from the caller's image where there is no weights offset
     DevBuf          padSrc, padW;
     PtrKind         kindSrc, kindDst; // host or device memory, per argument of run()
 };
@@ -1553,14 +1555,19 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
             const int64_t row_bytes = (int64_t)dr.W * dr.C, pad_bytes = (int64_t)d.W * dp.C, k_row = (int64_t)d.KH * dr.C, k_pad = (int64_t)d.KH * d.KW * dp.C;
             const bool    one_batch_late = d.OFM <= 64 && k_row <= 192 && k_pad > 192 && k_pad <= 384 && (int64_t)d.batch * gp.OH * gp.OW < 8192;
             const bool    large_copy = d.OFM <= 64 && 2 * row_bytes > 3 * pad_bytes && k_pad <= 576;
-            if (h->c_pad && !one_batch_late && !large_copy && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
-                (d.KW * d.C >= 8 || k_pad > 192) &&
+            const bool    pays = !one_batch_late && !large_copy && k_row < k_pad && (2 * row_bytes <= 3 * pad_bytes || 2 * k_row <= k_pad) &&
+                              (d.KW * d.C >= 8 || k_pad > 192);
+            // Without a weights offset nothing is copied at all: see gemm_rows.hip (more than two panels of output channels would
+            // copy the window more often than the pipelined kernel fetches a patch)
+            const bool raw = !f32 && d.requant.stage == MI355_STAGE_FIXEDPOINT && d.OFM <= 128 && d.weights_offset + (d.weights_dtype == MI355_U8 ? 128 : 0) == 0 &&
+                             conv_rows_applies(h->geom_true);
+            if (h->c_pad && (pays || raw) && d.KW > 1 && d.dilation_x == 1 && (int64_t)d.KW * d.C < 1024 &&
                 (int64_t)d.batch * d.H * row_bytes < ((int64_t)1 << 31) &&
                 patch_rows_fit((int64_t)d.batch * d.H, d.W, d.C, dr.W, d.stride_x, d.pad_left, dr.C))
             {
                 conv_geom(dr, gp);
                 if (conv_fast_div_ok(dr, gp))
-                    h->c_pad = dr.C, h->patch_rows = true, gp.c_true = d.KW * d.C, h->geom = gp;
+                    h->c_pad = dr.C, h->patch_rows = true, h->raw_rows = raw, gp.c_true = d.KW * d.C, h->geom = gp;
             }
         }
     }
@@ -1775,7 +1782,8 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         Dd   = h->nhwcDst.p;
     }
     const void *src_true = srcd; // the caller's channel count
-    if (h->c_pad)
+    const bool  raw      = h->raw_rows && c.b_off_eff() == 0 && c.rq.stage == MI355_STAGE_FIXEDPOINT;
+    if (h->c_pad && !raw)
     {
         // pixels of C channels -> pixels of c_pad channels (what the added ones hold meets zero weights; the padding value
         // keeps them in range of the source type)
@@ -1786,7 +1794,19 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
             HIP_TRY(channel_pad_launch(srcd, h->padSrc.p, (int64_t)d.batch * d.H * d.W, d.C, h->c_pad, (uint8_t)(d.pad_value & 0xFF), s));
         srcd = h->padSrc.p;
     }
-    if (h->implicit)
+    if (raw)
+    {
+        GemmArgs g{};
+        c.fill_epi(g.epi, nullptr);
+        g.A = (const int8_t *)src_true, g.Bp = c.Bp.as<int8_t>(), g.Kp = c.Kp;
+        g.D = Dd, g.ldd = c.N, g.M = c.M, g.N = c.N, g.K = c.K;
+        g.conv          = h->geom_true;
+        g.conv.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
+        c.set_vec_store(g);
+        HIP_TRY(conv_rows_launch(c.flip_a, g, d.batch, s));
+        c.kname_run = &c.kname_rows;
+    }
+    else if (h->implicit)
     {
         GemmArgs g{};
         c.fill_epi(g.epi, h->has_bias_f32 ? h->biasF.as<float>() : nullptr);

@@ -1,0 +1,265 @@
+// Convolution of few channels (a first layer: RGB), straight from the caller's NHWC image.
+//
+// The KW taps of an image row are KW * C consecutive bytes, at most 32 here. A workgroup takes a band of output rows of one image and a
+// panel of up to 64 output channels: it copies the window of input rows under the band to LDS byte for byte (padding included, signs
+// normalised), and a lane forms the 16 bytes of its (pixel, k) from the dwords that hold them, shifted into place: in the
+// layout of patch rows (mi355_conv_create), K = KH pieces of 16 or 32 bytes, whose weights are packed the same way; what
+// lies beyond KW * C in a piece are neighbouring pixels, which meet zero weights. The weights of the panel stay in registers.
+//
+// Against patch rows written out in memory and fetched by the narrow kernel (KH / stride times each) the image crosses the chip
+// once: 32 x 224 x 224 x 3 -> 64, 7 x 7, stride 2: 9.4 us of copy and 30 of the narrow kernel, 20.3 in one launch now; 29 x 85 x 85 x 3 -> 32:
+// 10.2, 6.8; 2 x 93 x 93 x 3 -> 32, 5 x 5: 7.6, 4.7. What bounds it: the vector ALU, 10 instructions per output for the
+// requantisation (about 9 us of the 20) and about 60 per 32 pixels for the operands, at 3 waves per SIMD, then the output's bytes.
+#include "mfma_common.hpp"
+
+#include <algorithm>
+
+namespace mi355
+{
+struct RowsArgs
+{
+    GemmArgs g;        // A: the image; conv: its geometry with the caller's channels; K: KH * piece bytes
+    int32_t  pieces;   // 16-byte pieces per window row (1 or 2)
+    int32_t  band, bands, pitch, win_rows; // output rows per workgroup, workgroups per image; LDS bytes per window row, window rows
+    int32_t  row_bytes, left_bytes;        // bytes of an image row, of the padding in front of it
+};
+
+constexpr int ROWS_WAVES = 4;
+
+template <int NKB>
+__global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu(NKB <= 2 ? 4 : 3))) void conv_rows_kernel(RowsArgs a, uint32_t flip)
+{
+    constexpr int    BPITCH = NKB * 64 + 32, OPITCH = 80; // (a panel row 32 bytes past a multiple of 64: see NARROW_PAD_PIECES)
+    constexpr int    NT = ROWS_WAVES * 64, NPAR = 1 + QP_COUNT;
+    const GemmArgs  &g = a.g;
+    const ConvGeom  &c = g.conv;
+    const EpiParams &p = g.epi;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    char    *panel = smem;                                   // 64 rows of BPITCH
+    int32_t *par   = (int32_t *)(smem + 64 * BPITCH);        // [NPAR][64]
+    char    *out   = smem + 64 * BPITCH + NPAR * 256;        // a wave's 32 x 64 results
+    char    *win   = out + ROWS_WAVES * 32 * OPITCH;         // win_rows of a.pitch
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lr = lane & 15, lh = lane >> 4;
+    const int n = (int)blockIdx.x / a.bands, band = (int)blockIdx.x - n * a.bands, n0 = (int)blockIdx.y * 64;
+    const int oy0 = band * a.band, rows = min(a.band, c.OH - oy0), npix = rows * c.OW;
+    const int qflag = p.qp_flag ? *p.qp_flag : 1;
+
+    // the panel of weights: 64 rows of NKB * 64 bytes
+    for (int i = tid; i < 64 * NKB * 4; i += NT)
+    {
+        const int r = i / (NKB * 4), q = i % (NKB * 4);
+        *(v4i *)(panel + r * BPITCH + q * 16) = *(const v4i *)(g.Bp + (int64_t)(n0 + r) * g.Kp + q * 16);
+    }
+    if (p.qp_flag)
+        for (int i = tid; i < NPAR * 64; i += NT)
+            par[i] = i < 64 ? p.colvec[n0 + i] : p.qp[(int64_t)(i / 64 - 1) * p.qp_stride + n0 + i % 64];
+    // the window, a dword per thread and step, four steps of loads at a time
+    {
+        const int      per_row = a.pitch / 4, total = a.win_rows * per_row;
+        const int      iy0 = oy0 * c.stride_y - c.pad_top;
+        const int8_t  *image = g.A + (int64_t)n * c.H * a.row_bytes;
+        for (int i0 = tid; i0 < total; i0 += 4 * NT)
+        {
+            uint32_t lo[4], hi[4], keep[4], sh[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+            {
+                const int i = i0 + u * NT, r = i / per_row, x = (i - r * per_row) * 4 - a.left_bytes, iy = iy0 + r;
+                lo[u] = hi[u] = keep[u] = sh[u] = 0;
+                if (i < total && iy >= 0 && iy < c.H && x > -4 && x < a.row_bytes)
+                {
+                    // bytes x .. x + 3 of the row, those in [0, row_bytes) count; only dwords that hold one of them are read
+                    const int8_t   *at = image + (int64_t)iy * a.row_bytes + max(x, 0);
+                    const uint32_t  m  = (uint32_t)(uintptr_t)at & 3u;
+                    const int       skip = max(-x, 0), left = min(a.row_bytes - max(x, 0), 4 - skip); // valid bytes from `at` on
+                    const int8_t   *lp = at - m;
+                    lo[u]   = *(const uint32_t *)lp;
+                    hi[u]   = m + (uint32_t)left > 4u ? *(const uint32_t *)(lp + 4) : 0u;
+                    sh[u]   = m | ((uint32_t)skip << 8);
+                    keep[u] = (left >= 4 ? ~0u : (1u << (8 * left)) - 1u) << (8 * skip);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+            {
+                const int i = i0 + u * NT;
+                if (i < total)
+                {
+                    const uint32_t v = __builtin_amdgcn_alignbyte(hi[u], lo[u], sh[u] & 3u) << (8 * (sh[u] >> 8));
+                    *(uint32_t *)(win + (int64_t)i * 4) = ((v & keep[u]) | (c.pad_word & ~keep[u])) ^ flip;
+                }
+            }
+        }
+    }
+    __syncthreads();
+
+    v4i fb[NKB][4];
+    int koff[NKB];
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+    {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            fb[kb][q] = *(const v4i *)(panel + (q * 16 + lr) * BPITCH + (kb * 4 + lh) * 16);
+        const int piece = kb * 4 + lh, ky = a.pieces == 2 ? piece >> 1 : piece;
+        // (pieces beyond the last row meet zero weights: any bytes of the window do)
+        koff[kb] = min(ky, c.KH - 1) * c.dil_y * a.pitch + (a.pieces == 2 ? (piece & 1) * 16 : 0);
+    }
+    const int     cols = min(g.N - n0, 64);
+    char         *mine = out + wave * 32 * OPITCH;
+    char         *D    = (char *)g.D + ((int64_t)n * c.OH + oy0) * c.OW * g.ldd + n0;
+    const int32_t off2p1 = 2 * p.result_offset + 1;
+    for (int t = wave; t * 32 < npix; t += ROWS_WAVES)
+    {
+        v4i acc[2][4];
+#pragma unroll
+        for (int rb = 0; rb < 2; ++rb)
+        {
+            const int   pix = min(t * 32 + rb * 16 + lr, npix - 1);
+            const int   r = fast_div(pix, c.magic_OW), x = pix - r * c.OW;
+            const int   at = r * c.stride_y * a.pitch + x * c.stride_x * c.C;
+            const char *from = win + (at & ~3);
+            const int   m    = at & 3;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                acc[rb][q] = (v4i){0, 0, 0, 0};
+#pragma unroll
+            for (int kb = 0; kb < NKB; ++kb)
+            {
+                uint32_t w[5];
+#pragma unroll
+                for (int d = 0; d < 5; ++d)
+                    w[d] = *(const uint32_t *)(from + koff[kb] + 4 * d);
+                v4i fa;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    fa[d] = (int)__builtin_amdgcn_alignbyte(w[d + 1], w[d], (uint32_t)m);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc[rb][q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[kb][q], fa, acc[rb][q], 0, 0, 0);
+            }
+        }
+        // requantise into the wave's own 32 x 64 bytes of LDS (accumulator layout as in epilogue_store_t)
+        auto each = [&](auto requant)
+        {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+            {
+                if (q * 16 >= cols)
+                    continue;
+                const int col = q * 16 + 4 * lh;
+                const v4i cv = *(const v4i *)(par + col);
+#pragma unroll
+                for (int rb = 0; rb < 2; ++rb)
+                {
+                    int32_t o[4];
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        o[d] = requant(acc[rb][q][d], cv[d], col + d);
+                    const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
+                    const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
+                    *(uint32_t *)(mine + (rb * 16 + lr) * OPITCH + col) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+                }
+            }
+        };
+        if (qflag == 0 && p.qp_std)
+            each([&](int32_t v, int32_t cv, int col) {
+                return std_requant((int32_t)((uint32_t)v + (uint32_t)cv), par[(1 + QP_S2) * 64 + col], par[(1 + QP_RSM1) * 64 + col], off2p1, p.lo, p.hi);
+            });
+        else if ((qflag & 1) == 0)
+            each([&](int32_t v, int32_t cv, int col) {
+                return fast_requant((int32_t)((uint32_t)v + (uint32_t)cv), par[(1 + QP_S2) * 64 + col], par[(1 + QP_CMASK) * 64 + col],
+                                    par[(1 + QP_LS) * 64 + col], par[(1 + QP_RSM1) * 64 + col], par[(1 + QP_RMASK) * 64 + col], p.result_offset, p.lo, p.hi);
+            });
+        else
+            each([&](int32_t v, int32_t, int col) {
+                int first = n0; // (hidden: the addresses of 16 columns in three vectors, kept over the loop, were 100 registers)
+                asm volatile("" : "+s"(first));
+                const int j = min(first + col, g.N - 1);
+                return epi_fixedpoint(v, p.colvec[j], 0, p.mult ? p.mult[j] : p.mult_s, p.shift ? p.shift[j] : p.shift_s, p);
+            });
+        // ... and out, 16, 4 or 1 byte per lane
+        auto leave = [&](auto bytes_c)
+        {
+            constexpr int W = decltype(bytes_c)::value, LPR = 64 / W, RPI = 64 / LPR;
+#pragma unroll
+            for (int it = 0; it < 32 / RPI; ++it)
+            {
+                const int r = it * RPI + lane / LPR, cc = (lane % LPR) * W, pix = t * 32 + r;
+                if (pix >= npix || cc >= cols)
+                    continue;
+                char       *to = D + (int64_t)pix * g.ldd + cc;
+                const char *at = mine + r * OPITCH + cc;
+                if constexpr (W == 16)
+                    __builtin_nontemporal_store(*(const v4i *)at, (v4i *)to); // (N % 16 == 0 where this form is taken)
+                else if constexpr (W == 4)
+                    *(int *)to = *(const int *)at;
+                else
+                    *to = *at;
+            }
+        };
+        if (p.vec_store16 && g.N % 16 == 0)
+            leave(std::integral_constant<int, 16>{});
+        else if (p.vec_store && g.N % 4 == 0)
+            leave(std::integral_constant<int, 4>{});
+        else
+            leave(std::integral_constant<int, 1>{});
+    }
+}
+
+// pieces per window row for this geometry (the caller's channels), 0: not for this kernel. K is KH of them.
+int conv_rows_pieces(const ConvGeom &c)
+{
+    const int row = c.KW * c.C, pieces = (row + 15) / 16;
+    return c.dil_x == 1 && pieces <= 2 && c.KH * pieces <= 16 ? pieces : 0;
+}
+
+// conv: the caller's geometry, pad_word the raw padding byte replicated. The band is chosen here: as many output rows as give a
+// wave about 4 tiles of 32 pixels, fewer where that leaves the chip without two workgroups per compute unit, within 40 KiB of window
+int conv_rows_launch(bool flip_a, const GemmArgs &args, int batch, hipStream_t s)
+{
+    RowsArgs a{};
+    a.g              = args;
+    const ConvGeom &c = args.conv;
+    a.pieces         = conv_rows_pieces(c);
+    if (a.pieces == 0 || args.N < 1 || batch < 1 || args.epi.rowsum_mul != 0 || args.epi.rowvec != nullptr || args.epi.stage != 0)
+        return (int)hipErrorInvalidValue;
+    const int nkb = (c.KH * a.pieces + 3) / 4, panels = (args.N + 63) / 64;
+    if (args.Kp < nkb * 64 || round_up(args.N, PACK_N_ALIGN) < panels * 64)
+        return (int)hipErrorInvalidValue;
+    a.row_bytes  = c.W * c.C;
+    a.left_bytes = c.pad_left * c.C;
+    // the last pixel's pieces and the dword behind them end inside the window row
+    a.pitch = round_up(((c.OW - 1) * c.stride_x) * c.C + a.pieces * 16 + 8, 16) + 16;
+    auto window = [&](int rows) { return (rows - 1) * c.stride_y + (c.KH - 1) * c.dil_y + 1; };
+    const int most = std::max(1, (ROWS_WAVES * 32 * 4 + c.OW - 1) / c.OW);
+    int       band = std::min(c.OH, most);
+    while (band > 1 && ((int64_t)window(band) * a.pitch > 40 * 1024 || (int64_t)batch * ((c.OH + band - 1) / band) * panels < 512))
+        --band;
+    a.band = band, a.bands = (c.OH + band - 1) / band, a.win_rows = window(band);
+    const int64_t lds = 64 * (nkb * 64 + 32) + (1 + QP_COUNT) * 256 + ROWS_WAVES * 32 * 80 + (int64_t)a.win_rows * a.pitch;
+    if (lds > 64 * 1024 || (int64_t)batch * a.bands > INT32_MAX || panels > 65535)
+        return (int)hipErrorInvalidValue;
+    const dim3 grid((unsigned)(batch * a.bands), (unsigned)panels), block(ROWS_WAVES * 64);
+    const uint32_t flip = flip_a ? 0x80808080u : 0u;
+    switch (nkb)
+    {
+        case 1: conv_rows_kernel<1><<<grid, block, lds, s>>>(a, flip); break;
+        case 2: conv_rows_kernel<2><<<grid, block, lds, s>>>(a, flip); break;
+        case 3: conv_rows_kernel<3><<<grid, block, lds, s>>>(a, flip); break;
+        case 4: conv_rows_kernel<4><<<grid, block, lds, s>>>(a, flip); break;
+        default: return (int)hipErrorInvalidValue;
+    }
+    return (int)hipGetLastError();
+}
+// whether the launch above would take it: the window of one output row has to fit
+bool conv_rows_applies(const ConvGeom &c)
+{
+    const int pieces = conv_rows_pieces(c);
+    if (pieces == 0)
+        return false;
+    const int64_t pitch = ((int64_t)(c.OW - 1) * c.stride_x) * c.C + pieces * 16 + 40;
+    return pitch * ((int64_t)(c.KH - 1) * c.dil_y + 1) <= 30 * 1024 && (int64_t)c.OH * c.OW < (1 << 24);
+}
+} // namespace mi355
