@@ -275,7 +275,8 @@ struct GemmCore
         // by a share us_load of it (L2, HBM and the power limit are shared by all compute units).
         // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
         // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
-        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again. The 0.88: a deep K
+        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again (convolutions: 0.2, 15x9x10x480
+        // -> 144, 5x5: 18.0 us as 5 slices, 16.7 as 8). The 0.88: a deep K
         // under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900: 10.3 us whole, priced
         // at 8.6, 8.4 as 4 slices; 350 x 126 x 3520: 11.5, 9.2 and 8.4), and with it the choice is no worse on average.
         auto pick_dma = [&](int loader, int &plan, double &best_cost, int fixed_slices = 0) -> int
@@ -299,7 +300,7 @@ struct GemmCore
                     if (sl != want)
                         continue;
                     const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
-                    const double finish = sl > 1 ? 2.4 + 0.1 * sl + 2e-6 * (double)sl * M * N : 0.0;
+                    const double finish = sl > 1 ? 2.4 + 0.1 * sl + (loader == 1 ? 0.8e-6 : 2e-6) * (double)sl * M * N : 0.0;
                     const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load);
                     const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 0.88 : 1.0);
                     if (best < 0 || cost < best_cost)
@@ -759,6 +760,16 @@ struct GemmCore
         HIP_TRY(conv_rowsum_launch(rs_src, rs_geom, M, flip_a, g.epi.rowsum_mul, rowvec.as<int32_t>(), s));
         g.epi.rowvec = rowvec.as<int32_t>(), g.epi.rowsum_mul = 0;
         return 0;
+    }
+
+    // Whether the kernel that launch() gives this convolution writes its 8-bit results as planes (EpiParams::planes) on request: the
+    // pipelined one's tiles, whole K
+    bool stores_planes(const GemmArgs &g) const
+    {
+        const int64_t span = (int64_t)((g.M + g.conv.OH * g.conv.OW - 1) / (g.conv.OH * g.conv.OW)) * g.conv.H * g.conv.W * g.conv.C;
+        const bool    narrow = has_narrow && span < ((int64_t)1 << 31) && narrow_applies(g);
+        return epi == EPI_FIXEDPOINT && path == MI355_PATH_MFMA && splitk == 1 && dma_idx > 0 && !narrow && g.conv.C % 16 == 0 &&
+               ((uintptr_t)g.A & 15) == 0 && g.K % 16 == 0 && g.K >= 16 && span < ((int64_t)1 << 32);
     }
 
     int launch(GemmArgs &g, bool flip_in_loader, bool conv, hipStream_t s)
@@ -1772,6 +1783,7 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
     }
     const bool nchw   = d.layout == MI355_NCHW;
     void      *Dfinal = Dd;
+    bool       planes = false; // the kernel writes NCHW itself
     if (nchw)
     {
         // every image [C][H*W] -> [H*W][C]; the kernels write [OH*OW][OFM] per image into a buffer of their own
@@ -1820,6 +1832,11 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         g.D = Dd, g.ldd = c.N, g.d_batch_stride = 0;
         g.M = c.M, g.N = c.N, g.K = c.K;
         g.conv = h->geom;
+        if (nchw && c.stores_planes(g))
+        {
+            // straight into the caller's planes
+            g.D = Dfinal, g.epi.planes = h->geom.OH * h->geom.OW, planes = true;
+        }
         c.set_vec_store(g);
         TRY(c.launch(g, c.flip_a, true, s));
     }
@@ -1833,7 +1850,9 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         HIP_TRY(im2col_nhwc_launch(srcd, h->cols.p, d.batch, g2, ldc, s));
         TRY(c.run_dense(h->cols.as<int8_t>(), ldc, 0, Dd, c.N, 0, h->has_bias_f32 ? h->biasF.as<float>() : nullptr, s));
     }
-    if (nchw)
+    if (planes)
+        Dd = Dfinal;
+    else if (nchw)
     {
         HIP_TRY((c.epi == EPI_F32 ? transpose_words_launch : transpose_bytes_launch)(Dd, Dfinal, d.batch, h->geom.OH * h->geom.OW, c.N, s));
         Dd = Dfinal;

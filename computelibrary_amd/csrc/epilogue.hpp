@@ -46,6 +46,7 @@ struct EpiParams
     // (std_requant applies), bit 0 set when some multiplier is negative (then only the general formula applies)
     const int32_t *qp_flag;
     int32_t        accumulate; // EPI_S32 / EPI_F32: add the destination's previous contents (GEMMInfo::accumulate)
+    int32_t        planes;     // 8-bit results of a convolution's tiles as [image][column][planes pixels] (NCHW); 0: rows
     int32_t        half_out;   // EPI_F32: the result is rounded to half (nearest even) and stored as such (not when accumulating)
     int32_t        act_twice;  // EPI_F32: the activation clamp is also applied before the offset term is added
     // != 0: the pipelined kernels sum the rows of A themselves while its tiles pass through their registers (what

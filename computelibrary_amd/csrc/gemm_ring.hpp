@@ -670,15 +670,23 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         {
             char      *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
             const bool rowv  = g.epi.rowvec != nullptr || rowsum;
-            if (g.epi.qp_std && qflag == 0 && !rowv)
-                epilogue_store_staged<true, false, RE, QS, BM, BN, NW>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
-                                                                       [] { __syncthreads(); });
-            else if (g.epi.qp_std && qflag == 0)
-                epilogue_store_staged<true, true, RE, QS, BM, BN, NW>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
-                                                                      [] { __syncthreads(); }, rfin, rowsum);
+            auto       store = [&](auto planes_c)
+            {
+                constexpr bool PL = decltype(planes_c)::value;
+                if (g.epi.qp_std && qflag == 0 && !rowv)
+                    epilogue_store_staged<true, false, RE, QS, BM, BN, NW, PL>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
+                                                                               [] { __syncthreads(); });
+                else if (g.epi.qp_std && qflag == 0)
+                    epilogue_store_staged<true, true, RE, QS, BM, BN, NW, PL>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
+                                                                              [] { __syncthreads(); }, rfin, rowsum);
+                else
+                    epilogue_store_staged<false, true, RE, QS, BM, BN, NW, PL>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
+                                                                               [] { __syncthreads(); }, rfin, rowsum);
+            };
+            if (MODE == RING_CONV && g.epi.planes != 0)
+                store(integral_constant<bool, MODE == RING_CONV>{});
             else
-                epilogue_store_staged<false, true, RE, QS, BM, BN, NW>(fin, g, par, stage, m0, n0, row_e, col_w, wave, lane, bz,
-                                                                       [] { __syncthreads(); }, rfin, rowsum);
+                store(no{});
         }
     }
     else if ((EPI == EPI_S32 || EPI == EPI_F32) && !g.epi.accumulate)
@@ -686,6 +694,8 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         if constexpr (EPI != EPI_FIXEDPOINT)
             epilogue_store_wave32<EPI, RE, QS>(fin, g, smem + wave * 16 * (QS * 64 + 16), m0 + row_e, n0 + col_w, lane, bz, rfin, rowsum);
     }
+    else if (MODE == RING_CONV && EPI == EPI_FIXEDPOINT && g.epi.planes != 0)
+        epilogue_store_t<EPI, RE, QS, MODE == RING_CONV>(fin, g, m0 + row_e, n0 + col_w, lane, bz, rfin, rowsum);
     else
         epilogue_store_t<EPI, RE, QS>(fin, g, m0 + row_e, n0 + col_w, lane, bz, rfin, rowsum);
 }

@@ -183,7 +183,7 @@ __device__ __forceinline__ void epilogue_store(const v16i (&acc)[FM][FN], const 
 // holds, for every (rs, qs), output row rs*16 + l%16 and the 4 consecutive output columns qs*16 + 4*(l/16) + {0..3}
 // in the 4 registers of acc[rs][qs]: per-column parameters are read as 16-byte vectors and 4 results leave in one store.
 // (row0, col0) is the wave's top-left output coordinate.
-template <int EPI, int RS, int QS>
+template <int EPI, int RS, int QS, bool PLANES = false>
 __device__ __forceinline__ void epilogue_store_t(const v4i (&acc)[RS][QS], const GemmArgs &g, int row0, int col0,
                                                  int lane, int bz, const int32_t *rvk = nullptr, bool use_rvk = false)
 {
@@ -233,7 +233,15 @@ __device__ __forceinline__ void epilogue_store_t(const v4i (&acc)[RS][QS], const
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
                     packed |= ((uint32_t)epi_fixedpoint(acc[rs][qs][t], cv[t], rv[rs], mu[t], sh[t], p) & 0xFFu) << (8 * t);
-                if (vec)
+                if (PLANES)
+                {
+                    const int n = fast_div(fast_div(i, g.conv.magic_OW), g.conv.magic_OH);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (j0 + t < g.N)
+                            D[((int64_t)n * g.N + j0 + t) * p.planes + i - n * p.planes] = (char)(packed >> (8 * t));
+                }
+                else if (vec)
                     *(uint32_t *)(D + idx) = packed;
                 else
                 {
@@ -371,13 +379,14 @@ __device__ __forceinline__ void epilogue_store_fast(const v4i (&acc)[RS][QS], co
 // hit 64 different banks) and then written row by row, so a wave instruction writes pieces of rows end to end instead of
 // 16 (or 4 times 1) bytes of 16 different rows. All NW consumer waves of the block call this together; `barrier` is executed
 // once between the two phases by every wave of the block. stage must not overlap par. ROWV: a per-row term exists and is added.
-template <bool STD, bool ROWV, int RS, int QS, int BM, int BN, int NW, typename Barrier>
+// PLANES (a convolution): laid out column by column instead, and written as runs of a plane's pixels (EpiParams::planes).
+template <bool STD, bool ROWV, int RS, int QS, int BM, int BN, int NW, bool PLANES = false, typename Barrier>
 __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], const GemmArgs &g, const int32_t *par,
                                                       char *stage, int m0, int n0, int row_in_tile, int col_in_tile,
                                                       int wave, int lane, int bz, Barrier barrier,
                                                       const int32_t *rvk = nullptr, bool use_rvk = false)
 {
-    constexpr int    PITCH = BN + 16;
+    constexpr int    PITCH = PLANES ? BM + 16 : BN + 16;
     const int        lr = lane & 15, lh = lane >> 4;
     const EpiParams &p      = g.epi;
     const int32_t   *rowvec = p.rowvec ? p.rowvec + (int64_t)bz * p.rowvec_batch_stride : nullptr;
@@ -417,10 +426,51 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
             }
             const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
             const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
-            *(uint32_t *)(stage + (row_in_tile + rs * 16 + lr) * PITCH + c) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+            if constexpr (PLANES)
+            {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    stage[(c + t) * PITCH + row_in_tile + rs * 16 + lr] = (char)o[t];
+                (void)p01, (void)p23;
+            }
+            else
+                *(uint32_t *)(stage + (row_in_tile + rs * 16 + lr) * PITCH + c) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
         }
     }
     barrier();
+    if constexpr (PLANES)
+    {
+        char *D     = (char *)g.D;
+        auto  leave = [&](auto bytes_c)
+        {
+            constexpr int W = decltype(bytes_c)::value, TOTAL = BM * BN / W;
+#pragma unroll
+            for (int it = 0; it < (TOTAL + NW * 64 - 1) / (NW * 64); ++it)
+            {
+                const int at = (it * NW + wave) * 64 + lane, c = at / (BM / W), r = at % (BM / W) * W;
+                const int i = m0 + r, j = n0 + c;
+                if (i >= g.M || j >= g.N || (TOTAL % (NW * 64) != 0 && c >= BN))
+                    continue;
+                // (pieces of W pixels do not cross images: W divides the plane, M and i)
+                const int   n  = fast_div(fast_div(i, g.conv.magic_OW), g.conv.magic_OH);
+                char       *to = D + ((int64_t)n * g.N + j) * p.planes + i - n * p.planes;
+                const char *from = stage + c * PITCH + r;
+                if constexpr (W == 16)
+                    __builtin_nontemporal_store(*(const v4i *)from, (v4i *)to);
+                else if constexpr (W == 4)
+                    *(int *)to = *(const int *)from;
+                else
+                    *to = *from;
+            }
+        };
+        if (p.planes % 16 == 0 && ((uintptr_t)D & 15) == 0)
+            leave(std::integral_constant<int, 16>{});
+        else if (p.planes % 4 == 0 && ((uintptr_t)D & 3) == 0)
+            leave(std::integral_constant<int, 4>{});
+        else
+            leave(std::integral_constant<int, 1>{});
+        return;
+    }
     // 16, 4 or 1 byte per lane, as the destination's rows are aligned: a wave instruction writes pieces of rows end to end
     char *D    = (char *)g.D + (int64_t)bz * g.d_batch_stride;
     auto  leave = [&](auto bytes_c)
