@@ -275,8 +275,8 @@ struct GemmCore
         // by a share us_load of it (L2, HBM and the power limit are shared by all compute units).
         // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
         // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
-        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again (convolutions: 0.2, 15x9x10x480
-        // -> 144, 5x5: 18.0 us as 5 slices, 16.7 as 8). The 0.88: a deep K
+        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again (convolutions: 0.3, and a
+        // tile that has its compute unit to itself waits for its addresses alone, 1.15: 15x9x10x480 -> 144, 5x5: 20.8 us as 3 slices, 17.1 as 6). The 0.88: a deep K
         // under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900: 10.3 us whole, priced
         // at 8.6, 8.4 as 4 slices; 350 x 126 x 3520: 11.5, 9.2 and 8.4), and with it the choice is no worse on average.
         auto pick_dma = [&](int loader, int &plan, double &best_cost, int fixed_slices = 0) -> int
@@ -300,8 +300,8 @@ struct GemmCore
                     if (sl != want)
                         continue;
                     const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
-                    const double finish = sl > 1 ? 2.4 + 0.1 * sl + (loader == 1 ? 0.8e-6 : 2e-6) * (double)sl * M * N : 0.0;
-                    const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load);
+                    const double finish = sl > 1 ? 2.4 + 0.1 * sl + (loader == 1 ? 1.2e-6 : 2e-6) * (double)sl * M * N : 0.0;
+                    const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load) * (loader == 1 && per_cu == 1 ? 1.15 : 1.0);
                     const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 0.88 : 1.0);
                     if (best < 0 || cost < best_cost)
                         best = i, best_cost = cost, plan = sl;
