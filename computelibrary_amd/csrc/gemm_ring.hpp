@@ -452,6 +452,8 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         wait_vmcnt<0>();
     else
         wait_vmcnt<(NS - 1) * LPW>();
+    if constexpr (MODE == RING_CONV) // ... and the padding it wrote there itself: the other waves read that too
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     block_barrier(); // stage 0 is in LDS
 
     v4i  fa[2][RS], fb[2][QS];
