@@ -1,5 +1,6 @@
 // Direct-to-LDS loads and the waits that go with them, issued by hand: the compiler cannot tell which LDS bytes such a load
-// writes and would wait for all of them in front of every LDS read.
+// writes and would wait for all of them in front of every LDS read. Nor does it keep the distances that the hardware asks for inside such a
+// block: one instruction between a write of M0 and a load to LDS (what it puts there itself for its own builtin).
 #pragma once
 #include "mfma_common.hpp"
 
@@ -8,13 +9,13 @@ namespace mi355
 // one wave instruction: 64 lanes x 16 bytes from the lanes' addresses to 1 KiB of LDS at lds_addr
 __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_addr)
 {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
 }
 
 // scalar-base form: address = sbase (SGPR pair, wave-uniform) + zero-extended per-lane 32-bit offset
 __device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_addr)
 {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 
 // ... for the lanes in `lanes` (not none), while those in `others` write `pad` to LDS at slot + off. All 64 lanes are active.

@@ -31,12 +31,12 @@ namespace mi355
 // (scalar base + one 32-bit offset per lane)
 __device__ __forceinline__ void narrow_dma16(const void *sbase, uint32_t voff, uint32_t lds_addr)
 {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 // (one 64-bit address per lane)
 __device__ __forceinline__ void narrow_dma16_at(const void *from, uint32_t lds_addr)
 {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(from), "s"(lds_addr) : "memory");
 }
 
 // x / d with the reciprocal of ConvGeom::magic_* (0 stands for d == 1), without a branch on the reciprocal
@@ -489,9 +489,9 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
                 asm volatile("s_lshl_b32 s92, %[wv], 10\n\t"
                              "s_mov_b32 s93, %[wv]\n"
                              "1:\n\t"
+                             "s_mov_b32 m0, s92\n\t"
                              "s_add_u32 s90, %[blo], s92\n\t"
                              "s_addc_u32 s91, %[bhi], 0\n\t"
-                             "s_mov_b32 m0, s92\n\t"
                              "global_load_lds_dwordx4 %[v16], s[90:91]\n\t"
                              "s_add_u32 s93, s93, %[step]\n\t"
                              "s_add_u32 s92, s92, %[stepb]\n\t"
@@ -504,9 +504,9 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
                 asm volatile("s_lshl_b32 s92, %[wv], 10\n\t"
                              "s_mov_b32 s93, %[wv]\n"
                              "1:\n\t"
+                             "s_mov_b32 m0, s92\n\t"
                              "s_add_u32 s90, %[blo], s92\n\t"
                              "s_addc_u32 s91, %[bhi], 0\n\t"
-                             "s_mov_b32 m0, s92\n\t"
                              "global_load_lds_dwordx4 %[v16], s[90:91]\n\t"
                              "s_add_u32 s93, s93, %[step]\n\t"
                              "s_add_u32 s92, s92, %[stepb]\n\t"

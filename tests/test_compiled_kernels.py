@@ -13,24 +13,27 @@ from computelibrary_amd import capi
 OBJDUMP = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
 
 
+KEEP = re.compile(r"^\s*(ds_write|s_barrier|s_waitcnt|global_load_lds|\S+\s+m0,)")
+
+
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
-    """{symbol: [(opcode, operands), ...]}"""
+    """{symbol: [(position, opcode, operands), ...]}, the instructions that the tests below ask for"""
     if not os.path.exists(OBJDUMP):
         pytest.skip("no llvm-objdump")
-    d = tmp_path_factory.mktemp("code")
-    lib = shutil.copy(capi.LIB_PATH, d)
-    subprocess.run([OBJDUMP, "--offloading", lib], check=True, stdout=subprocess.DEVNULL)
-    out, code = {}, None
-    for obj in sorted(glob.glob(lib + ".*gfx950")):
-        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", obj], check=True, stdout=subprocess.PIPE, text=True).stdout
-        for line in text.splitlines():
-            line = line.split("//")[0]
-            if line.startswith("<"):
-                code = out.setdefault(line.strip("<>: \n"), [])
-            elif code is not None and line.strip():
-                op, _, rest = line.strip().partition(" ")
-                code.append((op, [a.strip() for a in rest.split(",")]))
+    out = {}
+    for which in (capi.LIB_PATH, os.path.join(os.path.dirname(capi.LIB_PATH), "libmi355ceilings.so")):
+        lib = shutil.copy(which, tmp_path_factory.mktemp("code"))
+        subprocess.run([OBJDUMP, "--offloading", lib], check=True, stdout=subprocess.DEVNULL)
+        for obj in sorted(glob.glob(lib + ".*gfx950")):
+            text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", obj], check=True, stdout=subprocess.PIPE, text=True).stdout
+            code = None
+            for at, line in enumerate(text.splitlines()):
+                if line.startswith("<"):
+                    code = out.setdefault(line.strip("<>: \n"), [])
+                elif code is not None and KEEP.match(line):
+                    op, _, rest = line.split("//")[0].strip().partition(" ")
+                    code.append((at, op, [a.strip() for a in rest.split(",")]))
     assert out
     return out
 
@@ -43,9 +46,19 @@ def test_convolutions_wait_for_their_padding_before_they_publish_it(kernels):
         if not re.search(r"gemm_ring_kernel.*Li1EEEv", name):  # (the last template argument: RING_CONV)
             continue
         seen += 1
-        at = next(i for i, (op, _) in enumerate(code) if op == "s_barrier")
-        writes = [i for i in range(at) if code[i][0].startswith("ds_write")]
+        barrier = next(i for i, (_, op, _) in enumerate(code) if op == "s_barrier")
+        writes = [i for i in range(barrier) if code[i][1].startswith("ds_write")]
         assert writes, name
-        waits = [i for i in range(writes[-1], at) if code[i][0] == "s_waitcnt" and "lgkmcnt(0)" in " ".join(code[i][1])]
-        assert waits and not any(code[i][0].startswith("ds_write") for i in range(waits[-1], at)), name
+        assert any(op == "s_waitcnt" and "lgkmcnt(0)" in " ".join(args) for _, op, args in code[writes[-1]:barrier]), name
     assert seen >= 3
+
+
+def test_a_load_to_lds_keeps_its_distance_from_the_write_of_m0(kernels):
+    """Loads to LDS take their destination from M0 and need one instruction between its write and themselves."""
+    seen = 0
+    for name, code in kernels.items():
+        for (a, _, args), (b, op, _) in zip(code, code[1:]):
+            if op.startswith("global_load_lds"):
+                seen += 1
+                assert not (args[0] == "m0" and b == a + 1), name
+    assert seen > 1000
