@@ -13,7 +13,8 @@ from computelibrary_amd import capi
 OBJDUMP = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "llvm-objdump")
 
 
-KEEP = re.compile(r"^\s*(ds_write|s_barrier|s_waitcnt|global_load_lds|\S+\s+m0,)")
+KEEP = re.compile(r"^\s*(ds_write|s_barrier|s_waitcnt|s_nop|global_|buffer_|flat_|v_readlane|v_readfirstlane|v_cmp_\S+\s+s\[|\S+\s+m0,)")
+MOST = 5  # wait states that a load needs behind a vector instruction which wrote its scalar address
 
 
 @pytest.fixture(scope="module")
@@ -62,3 +63,25 @@ def test_a_load_to_lds_keeps_its_distance_from_the_write_of_m0(kernels):
                 seen += 1
                 assert not (args[0] == "m0" and b == a + 1), name
     assert seen > 1000
+
+
+def scalars(operand):
+    m = re.match(r"s\[(\d+):(\d+)\]$|s(\d+)$", operand.split(" ")[0])
+    return set() if m is None else {int(m[3])} if m[3] else set(range(int(m[1]), int(m[2]) + 1))
+
+
+def test_a_load_keeps_its_distance_from_a_vector_write_of_its_address(kernels):
+    """v_readlane (a spilled scalar that comes back), v_readfirstlane and compares write scalar registers; a memory instruction that reads
+    one needs five wait states in between (an instruction is one, s_nop n is n + 1)."""
+    for name, code in kernels.items():
+        written = []  # (position, wait states that s_nop adds up to there, registers)
+        nops = 0
+        for at, op, args in code:
+            if op == "s_nop":
+                nops += int(args[0])
+            elif op.startswith(("v_read", "v_cmp")):
+                written = [w for w in written if at - w[0] <= MOST] + [(at, nops, scalars(args[0]))]
+            elif op.startswith(("global_", "buffer_", "flat_")):
+                read = set().union(*(scalars(a) for a in args))
+                for pos, n, regs in written:
+                    assert not (regs & read) or at - pos - 1 + nops - n >= MOST, (name, op, args)
