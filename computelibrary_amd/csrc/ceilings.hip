@@ -378,8 +378,7 @@ __global__ __launch_bounds__(1024) void lds_read_kernel(int steps, int *sink, in
 
 __device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_addr)
 {
-    uint64_t base; // (see direct_lds.hpp)
-    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0" : "=&s"(base) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 
 // The 256 x 128 x 128 tile's stream: workgroup (tm, tn) of an 8 x 32 tile grid (XCD-major order as in the GEMM) moves 48

@@ -109,9 +109,9 @@ struct PanelProducer
             const int      u   = pw + i * NP; // wave-uniform
             const uint32_t dst = base + (uint32_t)u * 1024u;
             if (i >= AU / NP)
-                dma16s(b_k + (int64_t)(u - AU) * RPU * Kp, lane_b, dst);
+                dma16s_copied(b_k + (int64_t)(u - AU) * RPU * Kp, lane_b, dst);
             else
-                dma16s(a_k + (int64_t)u * RPU * lda, lane_a, dst);
+                dma16s_copied(a_k + (int64_t)u * RPU * lda, lane_a, dst);
         }
     }
 
@@ -130,7 +130,7 @@ struct PanelProducer
             const int      u   = pw + i * NP; // wave-uniform
             const uint32_t dst = base + (uint32_t)u * 1024u;
             if (u >= AU)
-                dma16s(b_k + (int64_t)(u - AU) * RPU * Kp, lane_b, dst);
+                dma16s_copied(b_k + (int64_t)(u - AU) * RPU * Kp, lane_b, dst);
             else
             {
                 // rows beyond M re-read row M-1 (their results are never stored): only the last row tile has any
@@ -138,7 +138,7 @@ struct PanelProducer
                 const int8_t  *ub   = edge ? a_k : a_k + (int64_t)u * RPU * lda;
                 const uint32_t o    = edge ? (uint32_t)min(u * RPU + ur, rows_left - 1) * (uint32_t)lda + (uint32_t)c16 : lane_a;
                 if (full)
-                    dma16s(ub, o, dst);
+                    dma16s_copied(ub, o, dst);
                 else
                 {
                     // last K step. Columns at or beyond K read the fill bytes. A column that straddles K reads on into
@@ -413,7 +413,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
             const int st = kt + NS - 1;
 #pragma unroll
             for (int i = 0; i < CBU; ++i)
-                dma16s(cb_base + (int64_t)st * BK + (int64_t)i * NW * RPU * g.Kp, cb_lane,
+                dma16s_copied(cb_base + (int64_t)st * BK + (int64_t)i * NW * RPU * g.Kp, cb_lane,
                        cb_lds + (uint32_t)(st % NS) * STAGE + (uint32_t)(i * NW) * 1024u);
         }
         if (FLIP_A)

@@ -31,8 +31,7 @@ namespace mi355
 // (scalar base + one 32-bit offset per lane)
 __device__ __forceinline__ void narrow_dma16(const void *sbase, uint32_t voff, uint32_t lds_addr)
 {
-    uint64_t base; // (see direct_lds.hpp)
-    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0" : "=&s"(base) : "v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
 }
 // (one 64-bit address per lane)
 __device__ __forceinline__ void narrow_dma16_at(const void *from, uint32_t lds_addr)
