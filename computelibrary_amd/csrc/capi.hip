@@ -667,6 +667,14 @@ struct GemmCore
         return !accumulate && (path == MI355_PATH_SKINNY || (path == MI355_PATH_MFMA && dma_idx >= 0 && K >= 16 && (int64_t)std::max(lda, (int64_t)Kp) * 256 + Kp < ((int64_t)1 << 32)));
     }
 
+    // (behind choose_kernel) the register-staged kernel runs what is not the narrow one's
+    void no_pipelined_kernel()
+    {
+        dma_idx = byte_idx = -1, splitk_plan = 1;
+        kname_dma.clear();
+        kname = kname_mfma;
+    }
+
     // A, D and bias_f32 are device pointers here
     int run_dense(const int8_t *A, int64_t lda, int64_t a_bs, void *D, int64_t ldd, int64_t d_bs,
                   const float *bias_f32, hipStream_t s)
@@ -1424,6 +1432,15 @@ static bool conv_fast_div_ok(const mi355_conv_desc &d, const ConvGeom &g)
     return M * g.OW < lim && (M / g.OW + 1) * g.OH < lim && (K + 256) * d.C < lim && ((int64_t)d.KH * d.KW + 256) * d.KW < lim;
 }
 
+// The ring kernel's loader works a tap's offset out with 24-bit factors (an image row's bytes and a dilated filter's extent among them)
+// and puts what lies beyond K 2^30 rows down, outside any image.
+static bool conv_taps_ok(const ConvGeom &g)
+{
+    const int64_t lim = (int64_t)1 << 24;
+    return (int64_t)g.KH * g.KW < lim && g.C < lim && (int64_t)(g.KH - 1) * g.dil_y < lim && (int64_t)(g.KW - 1) * g.dil_x < lim &&
+           (g.KH == 1 || (int64_t)g.W * g.C < lim) && g.H < (1 << 29) && g.pad_top < (1 << 29);
+}
+
 void mi355_conv_out_dims(const mi355_conv_desc *desc, int32_t *OH, int32_t *OW)
 {
     ConvGeom g{};
@@ -1620,6 +1637,8 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
     h->geom.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
     if (h->implicit)
         c.fill_byte = (uint8_t)(d.pad_value & 0xFF);
+    if (h->implicit && !conv_taps_ok(h->geom))
+        c.no_pipelined_kernel();
     c.kprefix = h->implicit ? "implicit_" : "im2col+";
     c.kname   = c.kprefix + c.kname;
     c.refresh_names();

@@ -49,6 +49,7 @@ struct RingLoader
     uint32_t      spare; // convolution: LDS address of 1 KiB that nothing reads
     uint32_t      lds0, b_unit; // b_unit: bytes of the packed B between two units of this wave
     int           c16, K, k_base, lane_id;
+    int           row_c;     // convolution: bytes of an image row
     bool          never_out; // convolution: no tap of any pixel lies outside the image
     bool          tail_whole; // a last step that K ends in may be fetched whole
     ConvGeom      conv;
@@ -67,6 +68,7 @@ struct RingLoader
         if (MODE == RING_CONV)
         {
             conv   = g.conv;
+            row_c  = conv.W * conv.C;
             pad    = (v4i){(int)conv.pad_word, (int)conv.pad_word, (int)conv.pad_word, (int)conv.pad_word};
             asm volatile("" : "+v"(pad)); // (stays in its registers)
             never_out = conv.pad_top == 0 && conv.pad_left == 0 && (conv.OH - 1) * conv.stride_y + (conv.KH - 1) * conv.dil_y < conv.H &&
@@ -117,14 +119,14 @@ struct RingLoader
         t.b_k = b_base + t.k0; // inside the zero-padded packed panel
         if (MODE == RING_CONV)
         {
-            // one tap per lane and step: the lane's column is the same in every unit
+            // one tap per lane and step: the lane's column is the same in every unit (24-bit factors: see conv_taps_ok)
             const int k   = k_base + t.k0 + c16;
             const int tap = (int)__umulhi((uint32_t)k, conv.magic_C) + (conv.magic_C ? 0 : k);
             const int c0  = k - (int)__umul24(tap, conv.C);
             const int ky  = (int)__umulhi((uint32_t)tap, conv.magic_KW) + (conv.magic_KW ? 0 : tap);
             const int kx  = tap - (int)__umul24(ky, conv.KW);
             t.dy = (int)__umul24(ky, conv.dil_y), t.dx = (int)__umul24(kx, conv.dil_x);
-            t.off  = __umul24(__umul24(t.dy, conv.W) + t.dx, conv.C) + c0;
+            t.off  = __umul24(t.dy, row_c) + __umul24(t.dx, conv.C) + c0;
             t.dy   = t.k0 + c16 < K ? t.dy : (1 << 30); // nothing beyond K
             t.slot = t.dst + (uint32_t)lane_id * 16u;
             t.inside = never_out && t.k0 + BK <= K;
