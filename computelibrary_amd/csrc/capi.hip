@@ -1,6 +1,7 @@
 // Implementation of the C ABI declared in include/mi355_gemmlowp.h: descriptor checks, kernel selection, device
 // workspace ownership, host <-> device staging, and the launches. No arithmetic lives here.
 #include "../../include/mi355_gemmlowp.h"
+#include "conv_rows_plan.hpp"
 #include "internal.hpp"
 
 #include <algorithm>

@@ -10,9 +10,8 @@
 // once: 32 x 224 x 224 x 3 -> 64, 7 x 7, stride 2: 9.4 us of copy and 30 of the narrow kernel, 20.3 in one launch now; 29 x 85 x 85 x 3 -> 32:
 // 10.2, 6.8; 2 x 93 x 93 x 3 -> 32, 5 x 5: 7.6, 4.7. What bounds it: the vector ALU, 10 instructions per output for the
 // requantisation (about 9 us of the 20) and about 60 per 32 pixels for the operands, at 3 waves per SIMD, then the output's bytes.
+#include "conv_rows_plan.hpp"
 #include "mfma_common.hpp"
-
-#include <algorithm>
 
 namespace mi355
 {
@@ -24,13 +23,12 @@ struct RowsArgs
     int32_t  row_bytes, left_bytes;        // bytes of an image row, of the padding in front of it
 };
 
-constexpr int ROWS_WAVES = 4;
-
 template <int NKB>
 __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu(NKB <= 2 ? 4 : 3))) void conv_rows_kernel(RowsArgs a, uint32_t flip)
 {
-    constexpr int    BPITCH = NKB * 64 + 32, OPITCH = 80; // (a panel row 32 bytes past a multiple of 64: see NARROW_PAD_PIECES)
+    constexpr int    BPITCH = NKB * 64 + 32, OPITCH = ROWS_OPITCH; // (a panel row 32 bytes past a multiple of 64: see NARROW_PAD_PIECES)
     constexpr int    NT = ROWS_WAVES * 64, NPAR = 1 + QP_COUNT;
+    static_assert(NPAR == ROWS_NPAR, "conv_rows_fixed_lds counts them");
     const GemmArgs  &g = a.g;
     const ConvGeom  &c = g.conv;
     const EpiParams &p = g.epi;
@@ -208,58 +206,31 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
     }
 }
 
-// pieces per window row for this geometry (the caller's channels), 0: not for this kernel. K is KH of them.
-int conv_rows_pieces(const ConvGeom &c)
-{
-    const int row = c.KW * c.C, pieces = (row + 15) / 16;
-    return c.dil_x == 1 && pieces <= 2 && c.KH * pieces <= 16 ? pieces : 0;
-}
-
-// conv: the caller's geometry, pad_word the raw padding byte replicated. The band is chosen here: as many output rows as give a
-// wave about 4 tiles of 32 pixels, fewer where that leaves the chip without two workgroups per compute unit, within 40 KiB of window
+// conv: the caller's geometry, pad_word the raw padding byte replicated
 int conv_rows_launch(bool flip_a, const GemmArgs &args, int batch, hipStream_t s)
 {
-    RowsArgs a{};
-    a.g              = args;
-    const ConvGeom &c = args.conv;
-    a.pieces         = conv_rows_pieces(c);
-    if (a.pieces == 0 || args.N < 1 || batch < 1 || args.epi.rowsum_mul != 0 || args.epi.rowvec != nullptr || args.epi.stage != 0)
+    RowsArgs        a{};
+    const ConvGeom &c      = args.conv;
+    const int       panels = (args.N + 63) / 64;
+    RowsPlan        p;
+    if (args.N < 1 || !conv_rows_plan(c, batch, panels, p) || args.epi.rowsum_mul != 0 || args.epi.rowvec != nullptr || args.epi.stage != 0)
         return (int)hipErrorInvalidValue;
-    const int nkb = (c.KH * a.pieces + 3) / 4, panels = (args.N + 63) / 64;
-    if (args.Kp < nkb * 64 || round_up(args.N, PACK_N_ALIGN) < panels * 64)
+    if (args.Kp < p.nkb * 64 || round_up(args.N, PACK_N_ALIGN) < panels * 64)
         return (int)hipErrorInvalidValue;
+    a.g      = args;
+    a.pieces = p.pieces, a.band = p.band, a.bands = p.bands, a.pitch = p.pitch, a.win_rows = p.win_rows;
     a.row_bytes  = c.W * c.C;
     a.left_bytes = c.pad_left * c.C;
-    // the last pixel's pieces and the dword behind them end inside the window row
-    a.pitch = round_up(((c.OW - 1) * c.stride_x) * c.C + a.pieces * 16 + 8, 16) + 16;
-    auto window = [&](int rows) { return (rows - 1) * c.stride_y + (c.KH - 1) * c.dil_y + 1; };
-    const int most = std::max(1, (ROWS_WAVES * 32 * 4 + c.OW - 1) / c.OW);
-    int       band = std::min(c.OH, most);
-    while (band > 1 && ((int64_t)window(band) * a.pitch > 40 * 1024 || (int64_t)batch * ((c.OH + band - 1) / band) * panels < 512))
-        --band;
-    a.band = band, a.bands = (c.OH + band - 1) / band, a.win_rows = window(band);
-    const int64_t lds = 64 * (nkb * 64 + 32) + (1 + QP_COUNT) * 256 + ROWS_WAVES * 32 * 80 + (int64_t)a.win_rows * a.pitch;
-    if (lds > 64 * 1024 || (int64_t)batch * a.bands > INT32_MAX || panels > 65535)
-        return (int)hipErrorInvalidValue;
-    const dim3 grid((unsigned)(batch * a.bands), (unsigned)panels), block(ROWS_WAVES * 64);
+    const dim3 grid((unsigned)(batch * p.bands), (unsigned)panels), block(ROWS_WAVES * 64);
     const uint32_t flip = flip_a ? 0x80808080u : 0u;
-    switch (nkb)
+    switch (p.nkb)
     {
-        case 1: conv_rows_kernel<1><<<grid, block, lds, s>>>(a, flip); break;
-        case 2: conv_rows_kernel<2><<<grid, block, lds, s>>>(a, flip); break;
-        case 3: conv_rows_kernel<3><<<grid, block, lds, s>>>(a, flip); break;
-        case 4: conv_rows_kernel<4><<<grid, block, lds, s>>>(a, flip); break;
+        case 1: conv_rows_kernel<1><<<grid, block, p.lds, s>>>(a, flip); break;
+        case 2: conv_rows_kernel<2><<<grid, block, p.lds, s>>>(a, flip); break;
+        case 3: conv_rows_kernel<3><<<grid, block, p.lds, s>>>(a, flip); break;
+        case 4: conv_rows_kernel<4><<<grid, block, p.lds, s>>>(a, flip); break;
         default: return (int)hipErrorInvalidValue;
     }
     return (int)hipGetLastError();
-}
-// whether the launch above would take it: the window of one output row has to fit
-bool conv_rows_applies(const ConvGeom &c)
-{
-    const int pieces = conv_rows_pieces(c);
-    if (pieces == 0)
-        return false;
-    const int64_t pitch = ((int64_t)(c.OW - 1) * c.stride_x) * c.C + pieces * 16 + 40;
-    return pitch * ((int64_t)(c.KH - 1) * c.dil_y + 1) <= 30 * 1024 && (int64_t)c.OH * c.OW < (1 << 24);
 }
 } // namespace mi355

@@ -133,8 +133,7 @@ bool narrow_applies(const GemmArgs &args);
 int  narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, bool *band = nullptr);
 
 // gemm_rows.hip — convolutions of few channels straight from the caller's image (window rows of KW * C <= 32 bytes, 8-bit destinations by the
-// fixed-point stage, no weights offset). args: Bp packed with K = KH pieces of 16 or 32 bytes, conv the caller's geometry
-bool conv_rows_applies(const ConvGeom &c);
+// fixed-point stage, no weights offset; conv_rows_plan.hpp says which). args: Bp packed with K = KH pieces of 16 or 32 bytes, conv the caller's geometry
 int  conv_rows_launch(bool flip_a, const GemmArgs &args, int batch, hipStream_t s);
 
 // gemm_skinny.hip — M <= 64, B packed in matrix-core operand order (see pack_b_launch)
