@@ -13,10 +13,12 @@ __device__ __forceinline__ void dma16(const void *gptr, uint32_t lds_addr)
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "s"(lds_addr) : "memory");
 }
 
-// scalar-base form: address = sbase (SGPR pair, wave-uniform) + zero-extended per-lane 32-bit offset. For kernels that spill no scalars
-__device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_addr)
+// scalar-base form: address = sbase (SGPR pair, wave-uniform) + zero-extended per-lane 32-bit offset; to LDS at lds_addr + off, added up on
+// the way into M0 (with the s_nop that is one instruction, the K step of a 64 x 64 tile is as long as without either). For kernels that
+// spill no scalars
+__device__ __forceinline__ void dma16s(const void *sbase, uint32_t voff, uint32_t lds_addr, int off)
 {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr) : "memory");
+    asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(lds_addr), "n"(off) : "memory", "scc");
 }
 
 // ... and for those that do: the base goes through a scalar copy, which the hardware does hold back, in the place of the s_nop. (Used

@@ -137,7 +137,7 @@ struct RingLoader
     __device__ __forceinline__ void issue_one(const Step &t, int i) const
     {
         if (i >= LA)
-            dma16s(t.b_k + (uint32_t)(i - LA) * (uint64_t)b_unit, b_off, t.dst + (uint32_t)(AU + (i - LA) * NW) * 1024u);
+            dma16s(t.b_k + (uint32_t)(i - LA) * (uint64_t)b_unit, b_off, t.dst, (AU + (i - LA) * NW) * 1024);
         else if (MODE == RING_CONV)
         {
             const uint32_t d = t.dst + (uint32_t)i * (NW * 1024u);
@@ -149,12 +149,12 @@ struct RingLoader
                 in = __builtin_amdgcn_ballot_w64((unsigned)(iy0[i] + t.dy) < (unsigned)conv.H) &
                      __builtin_amdgcn_ballot_w64((unsigned)(ix0[i] + t.dx) < (unsigned)conv.W);
             if (in == ~0ull)
-                dma16s(t.a_k, a_off[i] + t.off, d);
+                dma16s(t.a_k, a_off[i] + t.off, t.dst, i * (NW * 1024));
             else
                 dma16s_or_pad(t.a_k, in ? a_off[i] + t.off : 0u, in ? d : spare, in ? in : ~0ull, ~in, t.slot, i * (NW * 1024), pad);
         }
         else
-            dma16s(t.a_k, a_off[i], t.dst + (uint32_t)i * (NW * 1024u));
+            dma16s(t.a_k, a_off[i], t.dst, i * (NW * 1024));
     }
     // all of a stage's
     __device__ __forceinline__ void issue(int kt, int slot) const
