@@ -61,6 +61,6 @@ bool conv_rows_plan(const G &c, int batch, int panels, RowsPlan &p)
                           (int64_t)batch * ((c.OH + p.band - 1) / p.band) * panels < 512))
         --p.band;
     p.bands = (c.OH + p.band - 1) / p.band, p.win_rows = (int)conv_rows_window(c, p.band), p.lds = lds(p.band);
-    return p.lds <= ROWS_MAX_LDS && (int64_t)batch * p.bands <= INT32_MAX && panels <= 65535;
+    return p.lds <= ROWS_MAX_LDS && ((int64_t)batch * p.bands + 7) * panels <= INT32_MAX; // (workgroups)
 }
 } // namespace mi355

@@ -21,6 +21,7 @@ struct RowsArgs
     int32_t  pieces;   // 16-byte pieces per window row (1 or 2)
     int32_t  band, bands, pitch, win_rows; // output rows per workgroup, workgroups per image; LDS bytes per window row, window rows
     int32_t  row_bytes, left_bytes;        // bytes of an image row, of the padding in front of it
+    int32_t  batch, panels;                // panels: 0 where they run one after the other
 };
 
 template <int NKB>
@@ -39,7 +40,15 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
     char    *win   = out + ROWS_WAVES * 32 * OPITCH;         // win_rows of a.pitch
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lr = lane & 15, lh = lane >> 4;
-    const int n = (int)blockIdx.x / a.bands, band = (int)blockIdx.x - n * a.bands, n0 = (int)blockIdx.y * 64;
+    int wg = (int)blockIdx.x, n0 = (int)blockIdx.y * 64;
+    if (a.panels > 1) // panels of one band side by side (see conv_rows_launch), 8 workgroups apart: on the same die
+    {
+        const int at = wg / (8 * a.panels), in = wg - at * 8 * a.panels;
+        wg = at * 8 + (in & 7), n0 = (in >> 3) * 64;
+        if (wg >= a.bands * a.batch)
+            return;
+    }
+    const int n = wg / a.bands, band = wg - n * a.bands;
     const int oy0 = band * a.band, rows = min(a.band, c.OH - oy0), npix = rows * c.OW;
     const int qflag = p.qp_flag ? *p.qp_flag : 1;
 
@@ -221,7 +230,13 @@ int conv_rows_launch(bool flip_a, const GemmArgs &args, int batch, hipStream_t s
     a.pieces = p.pieces, a.band = p.band, a.bands = p.bands, a.pitch = p.pitch, a.win_rows = p.win_rows;
     a.row_bytes  = c.W * c.C;
     a.left_bytes = c.pad_left * c.C;
-    const dim3 grid((unsigned)(batch * p.bands), (unsigned)panels), block(ROWS_WAVES * 64);
+    // The panels of a band write different parts of the same lines. One panel after the other over the whole image batch, a large
+    // destination's lines leave the caches in between and go out twice: in pieces of 16 bytes and from 24 MB on the panels
+    // go side by side (16 x 186 x 189 x 3 -> 112, 5 x 5: 55.3 and 46.1 us, by patch rows 51.0; 30 x 192 x 192 x 3 -> 96, 3 x 3: 91.3, 80.0,
+    // 88.2; not 2 x 408 x 408 x 4 -> 65, 3 x 3: 28.8, 33.7, nor 19 MB of 96 columns, 7 x 7: 18.7, 20.8; 128 columns: no difference)
+    const bool side = panels > 1 && args.epi.vec_store16 && args.N % 16 == 0 && args.N % 64 != 0 && (int64_t)batch * c.OH * c.OW * args.N > 24000000;
+    a.batch = batch, a.panels = side ? panels : 0;
+    const dim3 grid(side ? (unsigned)(((int64_t)batch * p.bands + 7) / 8 * 8 * panels) : (unsigned)(batch * p.bands), side ? 1u : (unsigned)panels), block(ROWS_WAVES * 64);
     const uint32_t flip = flip_a ? 0x80808080u : 0u;
     switch (p.nkb)
     {

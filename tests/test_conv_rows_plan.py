@@ -77,3 +77,13 @@ def _check(shape, wshape, stride, pad, dt=np.uint8, mult_sign=1, layout=capi.NHW
     ((128, 25, 1057, 3), (16, 7, 7, 3), (4, 4), (3, 3, 3, 3))])
 def test_window_near_the_limit(shape, wshape, stride, pad):
     _check(shape, wshape, stride, pad)
+
+
+# the panels of a large destination side by side: two of them, bands not a multiple of 8, a last band that is shorter
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,wshape,layout", [
+    ((5, 233, 230, 3), (96, 3, 3, 3), capi.NHWC),
+    ((3, 301, 299, 3), (112, 4, 4, 3), capi.NCHW),
+    ((4, 250, 253, 4), (80, 7, 7, 4), capi.NHWC)])
+def test_panels_side_by_side(shape, wshape, layout):
+    _check(shape, wshape, (1, 1), (wshape[1] // 2,) * 4, np.int8, layout=layout)
