@@ -273,13 +273,14 @@ struct GemmCore
         // The pipelined kernel's tile is chosen with a small cost model in microseconds (the prices and what they were fitted to
         // stand at g_dma_cost): a tile costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that
         // fit a compute unit together share all but us_more, plus us_step for every K step, which a full chip slows down
-        // by a share us_load of it (L2, HBM and the power limit are shared by all compute units).
+        // by a share us_load of it (L2, HBM and the power limit are shared by all compute units); the tiles that share a compute unit
+        // take at least us_lone for a K step together.
         // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
         // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
-        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again (convolutions: 0.3, and a
-        // tile that has its compute unit to itself waits for its addresses alone, 1.15: 15x9x10x480 -> 144, 5x5: 20.8 us as 3 slices, 17.1 as 6). The 0.88: a deep K
-        // under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900: 10.3 us whole, priced
-        // at 8.6, 8.4 as 4 slices; 350 x 126 x 3520: 11.5, 9.2 and 8.4), and with it the choice is no worse on average.
+        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again (convolutions, fitted with their tiles:
+        // 3.2, 0.18 and 0.22). The 0.88 of dense products: a deep K under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900:
+        // 10.3 us whole, priced at 8.6, 8.4 as 4 slices). Over 816 products the choice is 1.43 % slower than the best with it, 1.31 %
+        // with 1, over 327 with rows on any byte 2.1 % and more than 2.7 %: both together are even from 0.85 to 0.95.
         auto pick_dma = [&](int loader, int &plan, double &best_cost, int fixed_slices = 0) -> int
         {
             int best = -1;
@@ -301,9 +302,10 @@ struct GemmCore
                     if (sl != want)
                         continue;
                     const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
-                    const double finish = sl > 1 ? 2.4 + 0.1 * sl + (loader == 1 ? 1.2e-6 : 2e-6) * (double)sl * M * N : 0.0;
-                    const double rounds = std::ceil(per_cu / occ), steps = per_cu * per * c.us_step * (1.0 + c.us_load * load) * (loader == 1 && per_cu == 1 ? 1.15 : 1.0);
-                    const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 ? 0.88 : 1.0);
+                    const double finish = sl <= 1 ? 0.0 : loader == 1 ? 3.2 + 0.18 * sl + 0.88e-6 * (double)sl * M * N : 2.4 + 0.1 * sl + 2e-6 * (double)sl * M * N;
+                    const double rounds = std::ceil(per_cu / occ), full = std::floor(per_cu / occ), rest = per_cu - full * occ, step = c.us_step * (1.0 + c.us_load * load);
+                    const double steps  = per * (full * std::max(c.us_lone, occ * step) + (rest > 0 ? std::max(c.us_lone, rest * step) : 0.0));
+                    const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 && loader != 1 ? 0.88 : 1.0);
                     if (best < 0 || cost < best_cost)
                         best = i, best_cost = cost, plan = sl;
                 }
@@ -314,15 +316,16 @@ struct GemmCore
             (double)N * K <= 4e6)
         {
             // The streaming kernel needs a pass in front here, for a copy of the rows or for their sums; the pipelined one does both
-            // itself and is one launch. Two launches are 8.2 us where the host is what they wait for (3 x 111 x 233: 8.2, one launch
-            // 4.3), in a graph 5.3 us and the stream of B (x 1.5 from 33 rows on; 1 x 600 x 999: 4.4 and 7.0, 1 x 2900 x 2901:
-            // 6.5 and 8.5). From 4 MB of B on the stream counts (50 x 6000 x 6001: 22.9 and 37.6), and rows of
-            // whole 64-byte blocks have the streaming kernel's best forms.
+            // itself and is one launch. Launched one by one from the host two launches take 6.2 us at least and one 4.3, so it may gain there what
+            // it loses in a graph: taken where it gains more than it loses (in a graph and one by one: 1 x 94 x 489: 3.7 -> 4.7 and 6.2 -> 5.2;
+            // not 3 x 384 x 745: 4.2 -> 5.7 and 6.2 -> 6.1; 1 x 27 x 1327: 4.3 -> 8.1, 7.8 -> 8.2). The two launches in a graph: fitted
+            // to 159 products (8 %); over these the choice is 5 % faster than two launches in a graph and 17 % one by one. From 4 MB of B on the stream
+            // counts (50 x 6000 x 6001: 22.9 and 37.6), and rows of whole 64-byte blocks have the streaming kernel's best forms.
             int          plan = 1;
             double       us   = 0;
             const int    idx  = pick_dma(byte_lda || K % 16 != 0 ? 2 : 0, plan, us, 1);
-            const double two  = std::max(8.2, 5.3 + (double)N * K * (M > 32 ? 1.5 : 1.0) / 4.5e6);
-            if (idx >= 0 && us < two)
+            const double two  = M > 32 ? 4.2 + 2.0e-3 * K + 0.36e-6 * N * K : 3.9 + 0.64e-3 * K + 0.25e-6 * N * K;
+            if (idx >= 0 && std::max(4.3, us) < (std::max(6.2, two) + two) / 2)
                 path = MI355_PATH_MFMA, one_launch = true;
         }
         if (path == MI355_PATH_SKINNY && M > SKINNY_MAX_M)
@@ -694,7 +697,8 @@ struct GemmCore
         // in front of the GEMM leaves the sums in a vector
         // (rows on any byte, or sums that stop inside a 16-byte column, without a pass in front: where the model prices the tile's
         // own shifting lower than the copy. run_noalloc keeps to the copy and with it to its limits)
-        const double copy_us = 3.3 + (double)M * batch * (direct ? K : K + Kp) * 2.5e-7;
+        // (the pass: fitted to 4000 runs with it in front. A workgroup walks along one row, hence the term in K)
+        const double copy_us = std::max(2.5, 1.05 + (double)M * batch * (direct ? K : K + Kp) * 4.5e-7 + K * 0.49e-3);
         const bool   byte_rows = (!direct || (b_off_eff() != 0 && K % 16 != 0)) && ext_ws == nullptr && path == MI355_PATH_MFMA && byte_idx >= 0 &&
                                !(own_row_terms() && b_off_eff() != 0) && (int64_t)lda * 256 + K < ((int64_t)1 << 32) &&
                                (one_launch || us_bytes < us_dma + copy_us);

@@ -835,19 +835,22 @@ static const WideEntry g_wide = {
      {MI355_DFN(256, 128, 128, 2, 2, 3, 2, false), MI355_DFN(256, 128, 128, 2, 2, 3, 2, true)}}};
 
 // What a tile and a K step of each configuration cost, in microseconds, and by what share a K step gets slower as the chip
-// fills (us_more: what of the start-up and the epilogue a tile does not share with the tile beside it on its compute unit): fitted
-// to every tile shape at up to 9 slice counts over 215 dense products (33 to 8192 rows, 16 to 11008 columns, K 16 to 11008) and 154
-// convolutions (16 to 2048 channels, 1 x 1 to 5 x 5); over those the choice is 1.5 % slower than the best of the sweep on average.
-// us_tile 0: not chosen, runs where a caller names it. In the sweep the 6-stage ring and the 256-deep 128 x 64 tile were the best
-// of a shape by 0.2 % on average, 128 x 64 tiles in convolutions by 0.3 %.
+// fills (us_more: what of the start-up and the epilogue a tile does not share with the tile beside it on its compute unit; us_lone: the
+// least that a K step takes however few tiles share the compute unit, where addresses or loads through registers are what it waits
+// for). Dense: fitted to every tile shape at up to 9 slice counts over 215 products (33 to 8192 rows, 16 to 11008 columns, K 16 to
+// 11008); over 816 others the choice is 1.4 % slower than the best of the sweep on average, 39 of them by more than a tenth.
+// Convolutions: fitted to every tile at up to 12 slice counts over 800 (16 to 512 channels, 1 x 1 to 5 x 5, up to 82k rows): 0.8 % and 10.
+// (Without us_lone, and without 128 x 64 tiles, one in 15 was over 3 % slower than in the tiles before the ring kernel: 10 x 51 x 51 x 160 -> 304, 3 x 3:
+// 27.5 us then, 31.6, 27.3 now; of 701 there are 9.) Rows on any byte: 1000 runs over 534 products, mean error 9 %.
+// us_tile 0: not chosen, runs where a caller names it.
 struct DmaCost
 {
-    double us_tile, us_step, us_load, us_more;
+    double us_tile, us_step, us_load, us_more, us_lone;
 };
 static const DmaCost g_dma_cost[3][8] = {
     {{8.57, 0.622, 0.33, 1.55}, {5.82, 0.412, 0.19, 4.35}, {4.30, 0.307, 0.12, 0.0}, {3.89, 0.188, 0.126, 0.0}, {}, {}, {5.67, 0.536, 0.0, 0.69}, {}},
-    {{}, {6.24, 0.541, 0.45, 3.7}, {}, {4.11, 0.339, 0.0, 0.0}, {}, {}, {5.33, 0.818, 0.04, 0.0}, {4.24, 0.489, 0.0, 0.0}},
-    {{}, {}, {}, {3.9, 0.25, 0.126, 0.0}, {}, {}, {}, {}},
+    {{}, {5.36, 0.807, 0.0, 0.0}, {4.29, 0.426, 0.191, 0.263, 0.746}, {3.91, 0.258, 0.112, 0.0, 0.480}, {}, {}, {4.41, 0.603, 0.212, 2.40, 1.079}, {4.27, 0.429, 0.178, 0.334, 0.696}},
+    {{}, {}, {}, {3.20, 0.245, 0.212, 0.287, 0.474}, {}, {}, {}, {}},
 };
 
 // configuration 0 is g_wide, the others are g_ring's
@@ -862,7 +865,7 @@ MfmaConfig dma_config(int idx, int loader)
     c.waves      = (idx == 0 ? g_wide.threads : g_ring[idx - 1].threads[conv ? 1 : 0]) / 64;
     c.lds_bytes  = idx == 0 ? g_wide.lds_bytes : g_ring[idx - 1].lds_bytes[conv ? 1 : 0];
     const DmaCost &cost = g_dma_cost[loader][idx];
-    c.us_tile = cost.us_tile, c.us_step = cost.us_step, c.us_load = cost.us_load, c.us_more = cost.us_more;
+    c.us_tile = cost.us_tile, c.us_step = cost.us_step, c.us_load = cost.us_load, c.us_more = cost.us_more, c.us_lone = cost.us_lone;
     return c;
 }
 

@@ -67,7 +67,7 @@ struct MfmaConfig
     const char *name;
     int         BM, BN, BK;
     int         waves = 0, lds_bytes = 0; // per workgroup (filled in for the pipelined kernel's configurations)
-    double      us_tile = 0, us_step = 0, us_load = 0, us_more = 0; // ... and what the cost model prices them at (see GemmCore::choose_kernel; us_tile 0: not chosen)
+    double      us_tile = 0, us_step = 0, us_load = 0, us_more = 0, us_lone = 0; // ... and what the cost model prices them at (see GemmCore::choose_kernel; us_tile 0: not chosen)
 };
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
