@@ -962,6 +962,8 @@ struct mi355_conv_handle
     bool            raw_rows = false;        // ... whose kernel takes them from the caller's image where there is no weights offset
     DevBuf          padSrc, padW;
     PtrKind         kindSrc, kindDst; // host or device memory, per argument of run()
+    bool   from_image() const { return raw_rows && core.b_off_eff() == 0 && core.rq.stage == MI355_STAGE_FIXEDPOINT; }
+    size_t pad_bytes() const { return (size_t)d.batch * d.H * geom.W * c_pad; }
 };
 
 extern "C"
@@ -1727,6 +1729,9 @@ int mi355_conv_update_quant(mi355_conv_handle *h, int32_t src_offset, int32_t we
     c.refresh_names();
     if (!c.prepared)
         return 0;
+    // a run that went straight from the image has made no patch rows: the next one may be recorded and could not make room for them
+    if (h->raw_rows && !h->from_image())
+        TRY(h->padSrc.ensure(h->pad_bytes()));
     if (c.rq.per_channel)
     {
         if (!mult || !shift)
@@ -1818,12 +1823,12 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         Dd   = h->nhwcDst.p;
     }
     const void *src_true = srcd; // the caller's channel count
-    const bool  raw      = h->raw_rows && c.b_off_eff() == 0 && c.rq.stage == MI355_STAGE_FIXEDPOINT;
+    const bool  raw      = h->from_image();
     if (h->c_pad && !raw)
     {
         // pixels of C channels -> pixels of c_pad channels (what the added ones hold meets zero weights; the padding value
         // keeps them in range of the source type)
-        TRY(h->padSrc.ensure((size_t)d.batch * d.H * h->geom.W * h->c_pad));
+        TRY(h->padSrc.ensure(h->pad_bytes()));
         if (h->patch_rows)
             HIP_TRY(patch_rows_launch(srcd, h->padSrc.p, (int64_t)d.batch * d.H, d.W, d.C, h->geom.W, d.stride_x, d.pad_left, h->c_pad, (uint8_t)(d.pad_value & 0xFF), s));
         else
