@@ -707,7 +707,8 @@ struct GemmCore
         const bool need_rowvec = b_off_eff() != 0 && !rowsum_in_kernel;
         // the two workspaces of a run: owned by the handle and grown on demand, or carved out of a buffer the caller of
         // this function brings (ext_ws != nullptr: nothing is allocated, sizes beyond ext_ws_bytes are an error)
-        const size_t rv_bytes = need_rowvec && !own_row_terms() ? ((sizeof(int32_t) * (size_t)M * batch + 255) & ~(size_t)255) : 0;
+        const size_t rv_size  = (sizeof(int32_t) * (size_t)M * batch + 255) & ~(size_t)255;
+        const size_t rv_bytes = need_rowvec && !own_row_terms() ? rv_size : 0;
         const size_t ap_bytes = direct || byte_rows ? 0 : (size_t)batch * M * Kp;
         int32_t     *rv       = nullptr;
         int8_t      *ap       = nullptr;
@@ -728,6 +729,9 @@ struct GemmCore
                 TRY(rowvec.ensure(rv_bytes));
             if (ap_bytes > 0)
                 TRY(Ap.ensure(ap_bytes));
+            // (sums inside the kernel now, by a pass where another A's rows start on dwords: a run that is recorded later finds the vector)
+            if (byte_rows && b_off_eff() != 0 && rowvec.cap < rv_size && !capturing(s))
+                TRY(rowvec.ensure(rv_size));
             rv = rowvec.as<int32_t>(), ap = Ap.as<int8_t>();
         }
         if (own_row_terms())

@@ -44,3 +44,35 @@ def test_a_convolution_whose_update_takes_it_off_the_image():
             check(w_zp)
         graph.close()
     conv.close()
+
+
+def test_rows_of_another_alignment():
+    """Sums of rows whose K ends inside a 16-byte column: inside the kernel for rows on any byte, by a pass into a vector of the handle's
+    where the rows start on dwords (1500 x 40 x 2052: the copy that the first would need is what makes the difference)."""
+    torch = torch_dev()
+    M, N, K = 1500, 40, 2052
+    rng = np.random.default_rng(52)
+    A, B = rng.integers(-128, 128, size=(M, K), dtype=np.int8), rng.integers(-128, 128, size=(K, N), dtype=np.int8)
+    want = oracle.gemmlowp_s32(A, B, -3, 5)
+    buf = torch.zeros(M * K + 1, dtype=torch.int8, device="cuda")
+    buf[1:] = to_dev(A).flatten()
+    odd, even = buf[1:], to_dev(A)
+    D = torch.zeros((M, N), dtype=torch.int32, device="cuda")
+    g = capi.Gemm(M, N, K, capi.S8, capi.S8, capi.S32, capi.EPI_S32, -3, 5)
+    g.prepare(to_dev(B))
+    announce("recorded run on rows of another alignment", M, N, K)
+    g.run(odd, D)
+    torch.cuda.synchronize()
+    first = g.kernel_name
+    np.testing.assert_array_equal(D.cpu().numpy(), want)
+    side = torch.cuda.Stream()
+    graph = _Graph(lambda stream: g.run(even, D, None, stream), side)
+    assert first.endswith("_bytes") and not g.kernel_name.endswith("_bytes"), (first, g.kernel_name)
+    for _ in range(2):
+        D.zero_()
+        torch.cuda.synchronize()
+        graph.launch(side)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(D.cpu().numpy(), want)
+    graph.close()
+    g.close()
