@@ -101,7 +101,7 @@ MfmaConfig  mfma_config(int idx);
 // epi: EPI_*, flip_a: xor 0x80 on A bytes in the loader, conv: implicit-GEMM loader. Returns hipError_t as int.
 int         mfma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &args, int batch, hipStream_t s);
 
-// gemm_ring.hip: the tiles of one workgroup of 4 waves; [epi][flip][conv]
+// gemm_ring.hip: tiles whose waves (4, or 8 in two groups) all load and all multiply; [epi][flip][conv], null where not built
 struct RingEntry
 {
     MfmaConfig  cfg;
@@ -113,7 +113,8 @@ extern const int       g_ring_count;
 constexpr int            RING_BYTES_CFG = 3;
 extern const void *const g_ring_bytes[3][2]; // rows on any byte, in that configuration's tiles; [epi][flip]
 
-// gemm_dma.hip — same contract as mfma_launch; additionally needs 16-byte aligned A rows, K % 16 == 0 and args.fill16
+// gemm_dma.hip — same contract as mfma_launch; additionally needs args.fill16, K >= 16 and rows of A that start on dwords (any byte with
+// args.byte_rows); K % 16 == 0 where the kernel sums the rows of A, and for convolutions C % 16 == 0 and a 16-byte aligned image
 int         dma_num_configs();
 // loader: 0 dense, 1 the implicit convolution, 2 dense rows on any byte: what the prices are for
 MfmaConfig  dma_config(int idx, int loader = 0);
