@@ -1306,7 +1306,7 @@ int mi355_gemmlowp_run_noalloc(mi355_gemm_handle *h, const void *A, const float 
     if (bias_f32 && c.epi != EPI_F32)
         return fail("float bias is only valid with the F32 epilogue");
     if (d.dst_dtype == MI355_F16)
-        return fail("mi355_gemmlowp_run_noalloc does not write F16 destinations (they need a float matrix as workspace)");
+        return fail("mi355_gemmlowp_run_noalloc does not write F16 destinations (some need a float matrix as workspace)");
     if (h->a_planes() || h->d_planes())
         return fail("mi355_gemmlowp_run_noalloc does not take planes with gaps between them (they need dense copies)");
     if (!h->kindA.is_device(A) || !h->kindD.is_device(D) || (bias_f32 && !h->kindBiasF.is_device(bias_f32)))
@@ -1817,14 +1817,22 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
     const bool nchw   = d.layout == MI355_NCHW;
     void      *Dfinal = Dd;
     bool       planes = false; // the kernel writes NCHW itself
+    // ... or [OH*OW][OFM] per image into a buffer of its own
+    auto own_dst = [&]() -> int
+    {
+        TRY(h->nhwcDst.ensure(dst_bytes));
+        Dd = h->nhwcDst.p;
+        return 0;
+    };
     if (nchw)
     {
-        // every image [C][H*W] -> [H*W][C]; the kernels write [OH*OW][OFM] per image into a buffer of their own
+        // every image [C][H*W] -> [H*W][C]
         TRY(h->nhwcSrc.ensure(src_bytes));
-        TRY(h->nhwcDst.ensure(dst_bytes));
         HIP_TRY(transpose_bytes_launch(srcd, h->nhwcSrc.p, d.batch, d.C, d.H * d.W, s));
         srcd = h->nhwcSrc.p;
-        Dd   = h->nhwcDst.p;
+        // (an update moves a convolution of few channels between a kernel that writes planes and one that does not: made by either run)
+        if (!h->implicit || h->raw_rows)
+            TRY(own_dst());
     }
     const void *src_true = srcd; // the caller's channel count
     const bool  raw      = h->from_image();
@@ -1862,14 +1870,14 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         c.rs_geom.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
         g.A = (const int8_t *)srcd, g.lda = 0, g.a_batch_stride = 0;
         g.Bp = c.Bp.as<int8_t>(), g.Kp = c.Kp, g.bp_batch_stride = 0;
-        g.D = Dd, g.ldd = c.N, g.d_batch_stride = 0;
+        g.ldd = c.N, g.d_batch_stride = 0;
         g.M = c.M, g.N = c.N, g.K = c.K;
         g.conv = h->geom;
         if (nchw && c.stores_planes(g))
-        {
-            // straight into the caller's planes
-            g.D = Dfinal, g.epi.planes = h->geom.OH * h->geom.OW, planes = true;
-        }
+            Dd = Dfinal, g.epi.planes = h->geom.OH * h->geom.OW, planes = true; // straight into the caller's planes
+        else if (nchw)
+            TRY(own_dst());
+        g.D = Dd;
         c.set_vec_store(g);
         TRY(c.launch(g, c.flip_a, true, s));
     }
@@ -1883,9 +1891,7 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         HIP_TRY(im2col_nhwc_launch(srcd, h->cols.p, d.batch, g2, ldc, s));
         TRY(c.run_dense(h->cols.as<int8_t>(), ldc, 0, Dd, c.N, 0, h->has_bias_f32 ? h->biasF.as<float>() : nullptr, s));
     }
-    if (planes)
-        Dd = Dfinal;
-    else if (nchw)
+    if (nchw && !planes)
     {
         HIP_TRY((c.epi == EPI_F32 ? transpose_words_launch : transpose_bytes_launch)(Dd, Dfinal, d.batch, h->geom.OH * h->geom.OW, c.N, s));
         Dd = Dfinal;

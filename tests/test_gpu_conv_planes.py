@@ -35,3 +35,24 @@ def test_planes(shape, wshape, stride, pad, dt, w_dt, negative):
     got, name = run_conv(src, w, bias, zp, w_zp, mult, shift, 5, info.min, info.max, stride, pad, (1, 1), layout=capi.NCHW)
     assert name.startswith("implicit_pp") and "splitk" not in name, name
     np.testing.assert_array_equal(got, oracle.conv_nhwc_direct(src, w, bias, zp, w_zp, mult, shift, 5, info.min, info.max, stride, pad, (1, 1)))
+
+
+def test_planes_take_no_second_destination():
+    """A run whose kernel writes the planes itself holds no buffer of the destination's size in another layout (51 MB here)."""
+    import torch
+    rng = np.random.default_rng(77)
+    conv = capi.Conv(capi.conv_desc(32, 56, 56, 16, 512, 1, 1, (1, 1), (0, 0, 0, 0), (1, 1), capi.S8, capi.S8, capi.S8, 0, 0, 0,
+                                    capi.requant(1 << 30, 8, 0, -128, 127, False), layout=capi.NCHW))
+    src = torch.from_numpy(rng.integers(-128, 128, size=(32, 16, 56, 56), dtype=np.int8)).cuda()
+    w = torch.from_numpy(rng.integers(-128, 128, size=(512, 16, 1, 1), dtype=np.int8)).cuda()
+    out = torch.zeros((32, 512, 56, 56), dtype=torch.int8, device="cuda")
+    conv.prepare(w)
+    torch.cuda.synchronize()
+    announce("conv planes, memory of the first run")
+    before = torch.cuda.mem_get_info()[0]
+    conv.run(src, out)
+    torch.cuda.synchronize()
+    taken, name = before - torch.cuda.mem_get_info()[0], conv.kernel_name
+    conv.close()
+    assert name.startswith("implicit_pp") and "splitk" not in name, name
+    assert taken < out.numel() // 2, taken
