@@ -32,7 +32,7 @@
 // Accumulators are kept transposed (the B panel is fed as the first matrix operand), so each lane ends up with 4
 // consecutive output columns per accumulator block: the epilogue reads the per-column parameters as 16-byte vectors and
 // packs 4 int8 results into one dword. Those dwords go to LDS first (the ring is free by then) and leave as whole
-// 128-byte tile rows, 16 bytes per lane; where the destination is not 16-byte aligned they are stored directly.
+// 128-byte tile rows, 16, 4 or 1 byte per lane as the destination's alignment allows.
 #include "direct_lds.hpp"
 
 #include <atomic>
@@ -47,8 +47,8 @@ namespace mi355
 // that column is the same for every unit of a wave (see SAME_COL), so a dense producer keeps ONE offset register for A
 // and one for B and moves from unit to unit and from K step to K step by scalar additions to the base: no vector
 // registers per load (arrays of per-load offsets were spilled to scratch memory, and every reload waited for all the
-// loads in flight). Lanes that must read padding instead (K tail of A, out-of-image taps of the implicit convolution)
-// need a different base: a wave with any such lane falls back to per-lane addresses for that one load.
+// loads in flight). Lanes that must read padding instead (the K tail of A) need a different base: such a load goes out with
+// per-lane addresses.
 template <int BM, int BN, int BK, int NP, int NS>
 struct PanelProducer
 {
