@@ -323,7 +323,11 @@ struct GemmCore
             // counts (50 x 6000 x 6001: 22.9 and 37.6), and rows of whole 64-byte blocks have the streaming kernel's best forms.
             int          plan = 1;
             double       us   = 0;
-            const int    idx  = pick_dma(byte_lda || K % 16 != 0 ? 2 : 0, plan, us, 1);
+            const bool   bytes = byte_lda || K % 16 != 0;
+            const int    idx  = pick_dma(bytes ? 2 : 0, plan, us, 1);
+            if (bytes)
+                us *= 0.82; // (a single row of tiles takes 0.90 of the price, over 222 products of up to 64 rows. The factor weighs the gain one by
+                            // one against the loss in a graph: with 1 49 of them lose over 5 % one by one and 4 over 10 % in a graph, with 0.8 7 and 23)
             const double two  = M > 32 ? 4.2 + 2.0e-3 * K + 0.36e-6 * N * K : 3.9 + 0.64e-3 * K + 0.25e-6 * N * K;
             if (idx >= 0 && std::max(4.3, us) < (std::max(6.2, two) + two) / 2)
                 path = MI355_PATH_MFMA, one_launch = true;
@@ -697,11 +701,14 @@ struct GemmCore
         // in front of the GEMM leaves the sums in a vector
         // (rows on any byte, or sums that stop inside a 16-byte column, without a pass in front: where the model prices the tile's
         // own shifting lower than the copy. run_noalloc keeps to the copy and with it to its limits)
-        // (the pass: fitted to 4000 runs with it in front. A workgroup walks along one row, hence the term in K)
-        const double copy_us = std::max(2.5, 1.05 + (double)M * batch * (direct ? K : K + Kp) * 4.5e-7 + K * 0.49e-3);
+        // (the pass: what 370 products took more than their tiles' price, mean error of both together 8 %. A workgroup walks along one row,
+        // hence the term in K)
+        // (sums alone, which copy nothing: the older fit of both sides, whose price of the tiles is about 0.82 of the present one)
+        const double copy_us = direct ? std::max(2.5, 1.05 + (double)M * batch * K * 4.5e-7 + K * 0.49e-3)
+                                      : 2.15 + (double)M * batch * (K + Kp) * 5.17e-7 + K * 0.46e-3;
         const bool   byte_rows = (!direct || (b_off_eff() != 0 && K % 16 != 0)) && ext_ws == nullptr && path == MI355_PATH_MFMA && byte_idx >= 0 &&
                                !(own_row_terms() && b_off_eff() != 0) && (int64_t)lda * 256 + K < ((int64_t)1 << 32) &&
-                               (one_launch || us_bytes < us_dma + copy_us);
+                               (one_launch || us_bytes * (direct ? 0.82 : 1.0) < us_dma + copy_us);
         const bool rowsum_in_kernel = byte_rows ? b_off_eff() != 0 : b_off_eff() != 0 && direct && path == MI355_PATH_MFMA && dma_idx >= 0 && K % 16 == 0 && K >= 16 &&
                                       (splitk == 1 || epi != EPI_F32) && (int64_t)lda * 256 + K < ((int64_t)1 << 32);
         const bool need_rowvec = b_off_eff() != 0 && !rowsum_in_kernel;

@@ -841,7 +841,9 @@ static const WideEntry g_wide = {
 // 11008); over 816 others the choice is 1.4 % slower than the best of the sweep on average, 39 of them by more than a tenth.
 // Convolutions: fitted to every tile at up to 12 slice counts over 800 (16 to 512 channels, 1 x 1 to 5 x 5, up to 82k rows): 0.8 % and 10.
 // (Without us_lone, and without 128 x 64 tiles, one in 15 was over 3 % slower than in the tiles before the ring kernel: 10 x 51 x 51 x 160 -> 304, 3 x 3:
-// 27.5 us then, 31.6, 27.3 now; of 701 there are 9.) Rows on any byte: 1000 runs over 534 products, mean error 9 %.
+// 27.5 us then, 31.6, 27.3 now; of 701 there are 9.) Rows on any byte: 370 products of more than 64 rows, mean error 9 %; between these tiles and
+// the pass in front with its tiles the choice is 0.9 % slower than the better one, 14 % faster than always the pass, slower than that by over 5 %
+// for 5 of them (with prices a fifth too low 1.0 % and 13: 6737 x 640 x 4659 65.1 us, by the pass 56.9).
 // us_tile 0: not chosen, runs where a caller names it.
 struct DmaCost
 {
@@ -850,7 +852,7 @@ struct DmaCost
 static const DmaCost g_dma_cost[3][8] = {
     {{8.57, 0.622, 0.33, 1.55}, {5.82, 0.412, 0.19, 4.35}, {4.30, 0.307, 0.12, 0.0}, {3.89, 0.188, 0.126, 0.0}, {}, {}, {5.67, 0.536, 0.0, 0.69}, {}},
     {{}, {5.36, 0.807, 0.0, 0.0}, {4.29, 0.426, 0.191, 0.263, 0.746}, {3.91, 0.258, 0.112, 0.0, 0.480}, {}, {}, {4.41, 0.603, 0.212, 2.40, 1.079}, {4.27, 0.429, 0.178, 0.334, 0.696}},
-    {{}, {}, {}, {3.20, 0.245, 0.212, 0.287, 0.474}, {}, {}, {}, {}},
+    {{}, {}, {}, {4.07, 0.245, 0.329, 0.0, 0.529}, {}, {}, {}, {}},
 };
 
 // configuration 0 is g_wide, the others are g_ring's
