@@ -12,9 +12,11 @@
 // loads are what a wave's time goes into: in convolutions (14x14x256 -> 256, 3x3, batch 32: 64 x 64 tiles of a 256-deep step
 // 12.1 us with two groups).
 //
-// What bounds it: the LDS of a compute unit, 128 bytes a clock for the loads' writes and the operand reads together - 64 x 64 tiles
-// 48 KiB a step (384 clocks; 380 measured with one workgroup per compute unit), 128 x 128 96 KiB (768; 850 measured). With
-// loading waves apart, two barriers a step and a wave of loads behind each, those were 800 to 1000 clocks whatever the tile
+// What bounds it: the loads. A compute unit takes a KiB to LDS every 16 to 18 clocks, so the 16, 24 and 32 KiB of a 64 x 64, 128 x 64
+// and 128 x 128 step are 270, 410 and 540 of the 380, 660 and 850 clocks that one takes with one workgroup per compute unit. Operand reads
+// keep the LDS busy 0.17 to 0.20 of the time and the matrix cores are 0.16 to 0.31 (counters: 128 x 4096 x 4096, 512 x 4096 x 4096,
+// 2048 x 2048 x 2048); the rest is the barrier's wait for the last wave. With
+// loading waves apart, two barriers a step and a wave of loads behind each, a step was 800 to 1000 clocks whatever the tile
 // (128 x 4096 x 4096: 17.7 us in 128 x 64 tiles, now 8.8 in 64 x 64; 2048 x 2048 x 2048: 15.9 to 11.3; 14x14x256 -> 256: 15.2 to 12.1).
 #pragma once
 #include "direct_lds.hpp"
