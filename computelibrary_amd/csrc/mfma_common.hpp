@@ -7,6 +7,12 @@ namespace mi355
 {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+// Four dwords, or four halves, at an address of any alignment that their elements have (v4i_any: on any byte): gfx950 stores them with one
+// instruction all the same
+typedef int      v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef int      int_any __attribute__((aligned(1)));
+typedef int      v4i_word __attribute__((ext_vector_type(4), aligned(4)));
+typedef _Float16 v4h_half __attribute__((ext_vector_type(4), aligned(2)));
 
 // LDS tiles are rows of CPR 16-byte columns. Column c of row r is stored at column c ^ swz(r). The LDS serves a 16-byte
 // access 16 lanes (256 bytes, all 64 banks) per clock: 16 consecutive rows reading the same logical column must land in
@@ -471,11 +477,18 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
             leave(std::integral_constant<int, 1>{});
         return;
     }
-    // 16, 4 or 1 byte per lane, as the destination's rows are aligned: a wave instruction writes pieces of rows end to end
+    // 16 bytes per lane whatever the destination's alignment (a store of 16 bytes may start on any byte): a wave instruction writes
+    // pieces of rows end to end. In a tile on the right edge the last piece of a row moves back to end where the row does; the bytes
+    // it shares with the piece before it are written twice, with the same values. A byte or a dword per lane where rows are not
+    // aligned to 16 made the stores as many instructions as the tile has bytes per lane: 2048 x 4095 x 512 12.1 us, now 9.0, 4000 x 1001
+    // x 64 6.9 and 5.1, 2774 x 2406 x 227 14.2 and 10.8. Rows on 16 bytes go past the caches (a write is exactly the output then);
+    // others share cache lines with the next tile's, which the L2 has to put together.
     char *D    = (char *)g.D + (int64_t)bz * g.d_batch_stride;
-    auto  leave = [&](auto bytes_c)
+    const int ncols = min(BN, g.N - n0);
+    auto  leave = [&](auto bytes_c, auto edge_c, auto nt_c)
     {
-        constexpr int W = decltype(bytes_c)::value;
+        constexpr int  W    = decltype(bytes_c)::value;
+        constexpr bool EDGE = decltype(edge_c)::value;
         constexpr int LPR = BN / W > 64 ? 64 : BN / W; // lanes per output row (or per 64 bytes of it)
         constexpr int PARTS = BN / W / LPR, RPI = 64 / LPR; // ... rows per wave instruction
         const int     rr = lane / LPR;
@@ -487,43 +500,52 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
 #pragma unroll
             for (int part = 0; part < PARTS; ++part)
             {
-                const int cc = part * LPR * W + (lane % LPR) * W, j0 = n0 + cc;
-                if (i >= g.M || j0 >= g.N || (BM % (NW * RPI) != 0 && r >= BM))
+                const int cc = part * LPR * W + (lane % LPR) * W;
+                if (i >= g.M || (EDGE && cc >= ncols) || (BM % (NW * RPI) != 0 && r >= BM))
                     continue;
-                const int64_t idx = (int64_t)i * g.ldd + j0;
+                const int   c0   = EDGE ? min(cc, ncols - W) : cc;
+                char       *to   = D + (int64_t)i * g.ldd + n0 + c0;
+                const char *from = stage + r * PITCH + c0;
                 if constexpr (W == 16)
                 {
-                    const v4i val = *(const v4i *)(stage + r * PITCH + cc);
-                    if (j0 + 16 <= g.N)
-                        __builtin_nontemporal_store(val, (v4i *)(D + idx));
-                    else
+                    v4i val;
+                    if constexpr (EDGE)
                     {
-                        for (int t = 0; t < g.N - j0; ++t)
-                            D[idx + t] = (char)(val[t >> 2] >> (8 * (t & 3)));
+                        const int      *w  = (const int *)(stage + r * PITCH + (c0 & ~3)); // (a fifth dword: the pitch has 16 bytes to spare)
+                        const uint32_t  by = (uint32_t)c0 & 3u;
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            val[t] = (int)__builtin_amdgcn_alignbyte((uint32_t)w[t + 1], (uint32_t)w[t], by);
                     }
+                    else
+                        val = *(const v4i *)from;
+                    if constexpr (decltype(nt_c)::value)
+                        __builtin_nontemporal_store(val, (v4i *)to);
+                    else
+                        *(v4i_any *)to = val;
                 }
                 else if constexpr (W == 4)
                 {
-                    const int val = *(const int *)(stage + r * PITCH + cc);
-                    if (j0 + 4 <= g.N)
-                        *(int *)(D + idx) = val;
-                    else
-                    {
-                        for (int t = 0; t < g.N - j0; ++t)
-                            D[idx + t] = (char)(val >> (8 * t));
-                    }
+                    const uint32_t *w = (const uint32_t *)(stage + r * PITCH + (c0 & ~3));
+                    *(int_any *)to    = (int)__builtin_amdgcn_alignbyte(w[1], w[0], (uint32_t)c0 & 3u);
                 }
                 else
-                    D[idx] = stage[r * PITCH + cc];
+                    *to = *from;
             }
         }
     };
-    if (p.vec_store16)
-        leave(std::integral_constant<int, 16>{});
-    else if (p.vec_store)
-        leave(std::integral_constant<int, 4>{});
+    using yes = std::true_type;
+    using no  = std::false_type;
+    if (ncols == BN && p.vec_store16)
+        leave(std::integral_constant<int, 16>{}, no{}, yes{});
+    else if (ncols == BN)
+        leave(std::integral_constant<int, 16>{}, no{}, no{});
+    else if (ncols >= 16)
+        leave(std::integral_constant<int, 16>{}, yes{}, no{});
+    else if (ncols >= 4)
+        leave(std::integral_constant<int, 4>{}, yes{}, no{});
     else
-        leave(std::integral_constant<int, 1>{});
+        leave(std::integral_constant<int, 1>{}, yes{}, no{});
 }
 // S32 / F32 results of one wave's (RS*16) x (QS*16) sub-tile, 16 rows at a time through a wave-private LDS area
 // (16 rows, pitch QS*64 + 16 bytes) so that they leave as 16 bytes per lane along whole row segments of QS*64 bytes
@@ -543,17 +565,10 @@ __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], 
     const int32_t   *colvec = p.colvec + (int64_t)bz * p.colvec_batch_stride;
     const int32_t   *rowvec = p.rowvec ? p.rowvec + (int64_t)bz * p.rowvec_batch_stride : nullptr;
     typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-    const bool       half   = EPI == EPI_F32 && p.half_out, vec = p.vec_store;
+    const bool       half   = EPI == EPI_F32 && p.half_out, nt = p.vec_store;
     const int        esz    = half ? 2 : 4;
     char            *D      = (char *)g.D + (int64_t)bz * g.d_batch_stride * esz;
     const int        rr = lane / LPR, cc = lane % LPR;
-    auto             store_one = [&](char *to, int32_t v)
-    {
-        if (half)
-            *(_Float16 *)to = (_Float16)__int_as_float(v);
-        else
-            *(int32_t *)to = v;
-    };
     // Everything the loop below needs from global memory is fetched before its first store goes out: a wait for a load
     // issued after a store also waits for that store to reach memory, and one such wait per block of 16 x 16 outputs
     // made the epilogue as slow as its slowest store, sixteen times over.
@@ -585,7 +600,12 @@ __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], 
     {
         constexpr bool BIAS = decltype(bias_c)::value, OFFS = decltype(offs_c)::value, TWICE = decltype(twice_c)::value;
         constexpr bool INSIDE = decltype(inside_c)::value;
-        char         *dp   = D + ((int64_t)(row0 + rr) * g.ldd + col0 + cc * 4) * esz; // this lane's segment of the first row
+        // This lane's 4 columns: on the right edge the last ones of a row move back to end where the row does, and share columns with
+        // the ones before, which both write with the same values. Rows may start on any element (see v4i_word)
+        const int     ncols = INSIDE ? QS * 16 : min(QS * 16, __builtin_amdgcn_readfirstlane(g.N - col0));
+        const bool    few   = !INSIDE && ncols < 4, mine = cc * 4 < ncols;
+        const int     c0    = INSIDE ? cc * 4 : max(min(cc * 4, ncols - 4), 0);
+        char         *dp   = D + ((int64_t)(row0 + rr) * g.ldd + col0 + c0) * esz; // ... of the first row
         const int64_t step = (int64_t)RPI * g.ldd * esz;
         const float   scale = p.scale, lo = p.act_min, hi = p.act_max;
 #pragma unroll
@@ -608,59 +628,70 @@ __device__ __forceinline__ void epilogue_store_wave32(const v4i (&acc)[RS][QS], 
                 }
                 *(v4i *)(stage + lr * PITCH + (qs * 16 + 4 * lh) * 4) = o;
             }
-            if (vec)
+            if (!few)
             {
-                // (all reads, then all stores, with no condition between them but the edge's own; the rarer forms below in loops that are
-                // not unrolled. With halves and last pieces of under 4 columns tested at every store and all of it written out, the float
-                // kernel of 256 x 128 tiles was 2.4 times as long: 30 x 450 x 1008 x 1408 38.4 us, now 34.3)
+                // (all reads, then all stores, with no condition between them but the edge's own. With halves and last pieces of under 4
+                // columns tested at every store and all of it written out, the float kernel of 256 x 128 tiles was 2.4 times as long:
+                // 30 x 450 x 1008 x 1408 38.4 us, then 34.3. Rows that are not aligned to 16 bytes share cache lines between tiles and are
+                // left to the L2: 47 x 678 x 734 x 24 to float 37.2 us one element per lane, 36 past the caches, 25.6 like this; 25 x
+                // 320 x 977 x 23 17.0, 14.5 and 13.3)
                 v4i val[16 / RPI];
 #pragma unroll
                 for (int it = 0; it < 16 / RPI; ++it)
-                    val[it] = *(const v4i *)(stage + (it * RPI + rr) * PITCH + cc * 16);
-                const int  rows = g.M - (row0 + rs * 16 + rr), j0 = col0 + cc * 4;
-                const bool whole = j0 + 3 < g.N;
-                char      *first = dp;
-                auto       leave = [&](auto half_c)
                 {
+                    const char *from = stage + (it * RPI + rr) * PITCH + c0 * 4;
+                    val[it]          = INSIDE ? *(const v4i *)from : (v4i)*(const v4i_word *)from;
+                }
+                const int  rows = mine ? g.M - (row0 + rs * 16 + rr) : 0;
+                auto       leave = [&](auto half_c, auto nt_c)
+                {
+                    constexpr bool NT = decltype(nt_c)::value;
 #pragma unroll
                     for (int it = 0; it < 16 / RPI; ++it)
                     {
-                        if (INSIDE || (whole && it * RPI < rows))
+                        if (INSIDE || it * RPI < rows)
                         {
                             if constexpr (decltype(half_c)::value)
-                                __builtin_nontemporal_store((v4h){(_Float16)__int_as_float(val[it][0]), (_Float16)__int_as_float(val[it][1]),
-                                                                  (_Float16)__int_as_float(val[it][2]), (_Float16)__int_as_float(val[it][3])},
-                                                            (v4h *)dp);
+                            {
+                                const v4h h = {(_Float16)__int_as_float(val[it][0]), (_Float16)__int_as_float(val[it][1]),
+                                               (_Float16)__int_as_float(val[it][2]), (_Float16)__int_as_float(val[it][3])};
+                                if constexpr (NT)
+                                    __builtin_nontemporal_store(h, (v4h_half *)dp);
+                                else
+                                    *(v4h_half *)dp = h;
+                            }
+                            else if constexpr (NT)
+                                __builtin_nontemporal_store(val[it], (v4i_word *)dp);
                             else
-                                __builtin_nontemporal_store(val[it], (v4i *)dp);
+                                *(v4i_word *)dp = val[it];
                         }
                         dp += step;
                     }
                 };
-                if (half)
-                    leave(std::true_type{});
-                else
-                    leave(std::false_type{});
-                if (!INSIDE && (g.N & 3) != 0 && !whole && j0 < g.N)
+                if (nt)
                 {
-#pragma unroll 1
-                    for (int it = 0; it < 16 / RPI; ++it)
-#pragma unroll 1
-                        for (int t = 0; t < g.N - j0 && it * RPI < rows; ++t)
-                            store_one(first + it * step + t * esz, *(const int *)(stage + (it * RPI + rr) * PITCH + cc * 16 + t * 4));
+                    if (half)
+                        leave(std::true_type{}, std::true_type{});
+                    else
+                        leave(std::false_type{}, std::true_type{});
                 }
+                else if (half)
+                    leave(std::true_type{}, std::false_type{});
+                else
+                    leave(std::false_type{}, std::false_type{});
             }
             else
             {
-                // rows that are not aligned to 4 elements: one element per lane, rows end to end
-#pragma unroll 1
-                for (int it = 0; it < QS * 4; ++it)
+                // under 4 columns: one element per lane
+                const int at = lane / 4, c = lane % 4;
+                const int val = *(const int *)(stage + at * PITCH + c * 4);
+                if (c < ncols && row0 + rs * 16 + at < g.M)
                 {
-                    const int at = it * 64 + lane, r = at / (QS * 16), c = at % (QS * 16);
-                    const int gi = row0 + rs * 16 + r, j = col0 + c;
-                    const int val = *(const int *)(stage + r * PITCH + c * 4);
-                    if (gi < g.M && j < g.N)
-                        store_one(D + ((int64_t)gi * g.ldd + j) * esz, val);
+                    char *to = D + ((int64_t)(row0 + rs * 16 + at) * g.ldd + col0 + c) * esz;
+                    if (half)
+                        *(_Float16 *)to = (_Float16)__int_as_float(val);
+                    else
+                        *(int32_t *)to = val;
                 }
             }
         }

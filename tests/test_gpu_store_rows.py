@@ -35,6 +35,31 @@ def test_pipelined(path, M, N, K):
         np.testing.assert_array_equal(got.view(np.uint16), wantf.astype(np.float16).view(np.uint16))
 
 
+# tiles on the right edge with 1 to 3, 4 to 15 and 16 or more columns left, whose last pieces move back to the end of the row; rows that start on
+# any element, as the caller's own row stride or as the previous row ends
+@pytest.mark.parametrize("N", [2, 5, 17, 30, 63, 70, 77, 93, 141, 255])
+@pytest.mark.parametrize("path,M", [(capi.PATH_TILE + 0, 257), (capi.PATH_TILE + 3, 70), (capi.PATH_TILE + 6, 129)])
+def test_right_edge(path, M, N):
+    K = 132
+    rng = np.random.default_rng(M + N)
+    A, B = (rng.integers(-128, 128, size=s, dtype=np.int8) for s in ((2, M, K), (K, N)))
+    bias = rng.integers(-20000, 20000, size=N, dtype=np.int32)
+    mult, shift = oracle.calculate_quantized_multipliers(1.0, rng.uniform(0.5, 2.0, size=N) * 40.0 / (K ** 0.5 * 74.0 * 74.0), 1.0)
+    for ldd in (N, N + 1, (N + 15) // 16 * 16):
+        announce("right edge", path, (M, N, K), "ldd", ldd)
+        how = dict(path=path, device=True, ldd=ldd)
+        got8, _ = run_gemm(A, B, capi.EPI_FIXEDPOINT, np.int8, 3, 0, bias, mult, shift, 7, -128, 127, **how)
+        got32, _ = run_gemm(A, B, capi.EPI_S32, np.int32, -5, 9, **how)
+        gotf, _ = run_gemm(A, B, capi.EPI_F32, np.float32, scale=3e-4, **how)
+        goth, _ = run_gemm(A, B, capi.EPI_F32, np.float16, scale=3e-4, **how)
+        for z in range(2):
+            np.testing.assert_array_equal(got8[z], oracle.gemmlowp_fixedpoint(A[z], B, bias, 3, 0, mult, shift, 7, -128, 127, np.int8))
+            np.testing.assert_array_equal(got32[z], oracle.gemmlowp_s32(A[z], B, -5, 9))
+            wantf = np.asarray(oracle.gemmlowp_f32(A[z], B, None, 0, 0, 3e-4))
+            np.testing.assert_array_equal(gotf[z].view(np.uint32), wantf.view(np.uint32))
+            np.testing.assert_array_equal(goth[z].view(np.uint16), wantf.astype(np.float16).view(np.uint16))
+
+
 # streaming forms (staged, per step, stage-once of 8, 16, 32 and 64 rows, deep K, a batch on the grid), slices, rows on any byte
 @pytest.mark.parametrize("batch,M,N,K", [(1, 5, 70, 200), (1, 8, 4099, 256), (1, 16, 300, 1024), (1, 30, 129, 640), (1, 60, 65, 512),
                                          (1, 8, 33, 9000), (1, 8, 48, 8320), (3, 7, 29, 64), (1, 100, 64, 4096), (1, 70, 61, 513)])
