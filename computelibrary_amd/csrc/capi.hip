@@ -638,7 +638,7 @@ struct GemmCore
     {
         p.qp                  = qp_on ? qp.as<int32_t>() : nullptr;
         p.qp_flag             = qp_on ? qp.as<int32_t>() + (size_t)QP_COUNT * Np : nullptr;
-        p.qp_std              = (qp_on && rq.result_offset > -(1 << 28) && rq.result_offset < (1 << 28)) ? 1 : 0;
+        p.qp_std              = (qp_on && rq.result_offset >= -STD_MAX_OFFSET && rq.result_offset <= STD_MAX_OFFSET) ? 1 : 0;
         p.qp_stride           = Np;
         p.colvec              = colvec.as<int32_t>();
         p.rowvec              = nullptr;
@@ -654,7 +654,6 @@ struct GemmCore
         const int32_t tlo = dst_dtype == MI355_S8 ? -128 : 0, thi = dst_dtype == MI355_S8 ? 127 : 255;
         p.lo                  = rq.min_bound > tlo ? rq.min_bound : tlo;
         p.hi                  = rq.max_bound < thi ? rq.max_bound : thi;
-        p.qp_pk16             = (p.qp_std && rq.result_offset >= -1024 && rq.result_offset <= 1024 && p.lo >= -1024 && p.hi <= 1024) ? 1 : 0;
         p.scale               = scale;
         p.act_min             = act_min;
         p.act_max             = act_max;

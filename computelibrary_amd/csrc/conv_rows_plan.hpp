@@ -6,7 +6,7 @@
 namespace mi355
 {
 constexpr int ROWS_WAVES = 4, ROWS_MAX_LDS = 64 * 1024; // (two workgroups per compute unit)
-constexpr int ROWS_OPITCH = 80, ROWS_NPAR = 6;          // LDS bytes of a wave's row of 64 results; words of constants per column
+constexpr int ROWS_OPITCH = 80, ROWS_NPAR = 4;          // LDS bytes of a wave's row of 64 results; words of constants per column
 
 struct RowsPlan
 {

@@ -36,13 +36,12 @@ struct EpiParams
     int32_t        dst_signed;
     int32_t        vec_store; // destination rows / base / batch stride allow 4-element vector stores
     int32_t        vec_store16; // ... and 16-byte stores of 8-bit results
-    // Pre-digested per-column requantisation vectors qp[5][qp_stride] (see fast_requant below), or nullptr when some
+    // Digested per-column requantisation vectors qp[QP_COUNT][qp_stride] (see fast_requant below), or nullptr when some
     // multiplier is negative and the general formula has to be used
     const int32_t *qp;
     int64_t        qp_stride;
-    int32_t        qp_std; // |result_offset| < 2^28: std_requant may be used where the flag word allows it
-    int32_t        qp_pk16; // ... and |result_offset|, |lo|, |hi| <= 1024: std_requant4_pk16 may be used instead
-    // One word written together with qp: 0 when every column has a multiplier >= 2^30 and a shift in [2, 31]
+    int32_t        qp_std; // |result_offset| <= STD_MAX_OFFSET: std_requant may be used where the flag word allows it
+    // One word written together with qp: 0 when every column has a multiplier >= 2^30 and a shift in [2, STD_MAX_SHIFT]
     // (std_requant applies), bit 0 set when some multiplier is negative (then only the general formula applies)
     const int32_t *qp_flag;
     int32_t        accumulate; // EPI_S32 / EPI_F32: add the destination's previous contents (GEMMInfo::accumulate)
@@ -55,21 +54,33 @@ struct EpiParams
     int32_t        rowsum_mul;
 };
 
-// Per-column constants of the branch-free requantisation used by the pipelined kernel's epilogue, valid for
-// multipliers >= 0 (everything calculate_quantized_multiplier produces):
-//   s2    = (int32)(2*mult mod 2^32), cmask = (2*mult >= 2^31) ? -1 : 0   so that  sqdmulh(a, mult) = mulhi(a, s2) + (a & cmask)
-//   ls    = max(-shift, 0)                                              left shift before the multiply
-//   rsm1  = max(shift - 1, 0), rmask = shift > 0 ? 1 : 0                 so that  rshr(x) = ((x >> rsm1) + rmask) >> rmask
-// Shifts of 32 or more in either direction give 0 in the reference arithmetic: encoded as a zero multiplier.
+// Per-column constants of the branch-free requantisation used by the matrix-core kernels' epilogues, valid for multipliers >= 0
+// (everything calculate_quantized_multiplier produces): the multiplier and the shift less one. Shifts of 32 or more in either
+// direction give 0 in the reference arithmetic: encoded as a zero multiplier.
 enum : int
 {
-    QP_S2 = 0,
-    QP_CMASK,
-    QP_LS,
-    QP_RSM1,
-    QP_RMASK,
+    QP_M = 0,
+    QP_SM1,
     QP_COUNT
 };
+// A block's constants in LDS: rows of the column terms, the two vectors above and std_requant's addend, which is made from the
+// launch's result offset where the others are parked
+enum : int
+{
+    PAR_CV = 0,
+    PAR_M,
+    PAR_SM1,
+    PAR_ADD,
+    PAR_ROWS
+};
+constexpr int PAR_LOADS = 1 + QP_COUNT; // rows that come from memory
+// word idx of the PAR_LOADS rows of `pitch` words each
+__device__ __forceinline__ void park_constant(int32_t *par, int idx, int pitch, int32_t w, int32_t result_offset)
+{
+    par[idx] = w;
+    if (idx >= PAR_SM1 * pitch)
+        par[idx + pitch] = (int32_t)((uint32_t)(2 * result_offset + 1) << ((w - 1) & 31));
+}
 
 // min(max(x, lo), hi) for lo <= hi as one instruction (the compiler keeps min and max apart: it cannot know lo <= hi)
 __device__ __forceinline__ int32_t clamp_med3(int32_t x, int32_t lo, int32_t hi)
@@ -79,40 +90,40 @@ __device__ __forceinline__ int32_t clamp_med3(int32_t x, int32_t lo, int32_t hi)
     return r;
 }
 
-__device__ __forceinline__ int32_t fast_requant(int32_t v, int32_t s2, int32_t cmask, int32_t ls, int32_t rsm1,
-                                                int32_t rmask, int32_t result_offset, int32_t lo, int32_t hi)
+// sqdmulh(a, m) = mulhi(a, (int32)(2m)) + (2m >= 2^31 ? a : 0); a left shift by -shift in front of it or a rounding right shift behind
+__device__ __forceinline__ int32_t fast_requant(int32_t v, int32_t m, int32_t sm1, int32_t result_offset, int32_t lo, int32_t hi)
 {
+    const int32_t ls = sm1 < -1 ? -1 - sm1 : 0, rsm1 = sm1 > 0 ? sm1 : 0, rmask = sm1 >= 0 ? 1 : 0;
     const int32_t pre = (int32_t)((uint32_t)v << ls);
-    const int32_t h   = __mulhi(pre, s2) + (pre & cmask);
+    const int32_t h   = __mulhi(pre, (int32_t)((uint32_t)m << 1)) + (m >= 0x40000000 ? pre : 0);
     const int32_t r   = ((h >> rsm1) + rmask) >> rmask;
     return clamp_med3((int32_t)((uint32_t)r + (uint32_t)result_offset), lo, hi);
 }
 
-// The common case of fast_requant (cmask = -1, ls = 0, rmask = 1, rsm1 >= 1): the rounding increment and the result
-// offset are one constant, off2p1 = 2*result_offset + 1, added before the last shift:
-// ((x + 1) >> 1) + off == (x + 1 + 2*off) >> 1, and |x| <= 2^30 here, so nothing overflows.
-__device__ __forceinline__ int32_t std_requant(int32_t v, int32_t s2, int32_t rsm1, int32_t off2p1, int32_t lo, int32_t hi)
+// The common case (multiplier m >= 2^30, shift s of 2 to STD_MAX_SHIFT, result offset within STD_MAX_OFFSET): rounding increment and result
+// offset go in as one addend behind the multiplication. floor((floor(v m / 2^31) + 2^(s-1)) / 2^s) + off is
+// floor((v m + (2 off + 1) 2^(30+s)) / 2^(31+s)), and of that 2^32 comes off first: add = (2 off + 1) 2^(s-2) meets mulhi(v, m) there
+// (below 2^30 each: no overflow). 5.75 vector instructions per output with the column term and the packing, 7.75 before (the
+// multiplication by 2m, v added once more, the increment behind the first shift and a second shift by one): 32 x 224 x 224 x 3 -> 64, 7 x 7
+// stride 2, 20.6 -> 18.4 us; 2048 x 4096 x 4096 31.1 -> 30.3, 8192 x 11008 x 4096 318 -> 311 (two builds in turn on one machine). Larger
+// shifts and offsets take fast_requant. Two constants per column come from memory instead of five.
+constexpr int STD_MAX_SHIFT = 22, STD_MAX_OFFSET = 511;
+__device__ __forceinline__ int32_t std_requant(int32_t v, int32_t m, int32_t sm1, int32_t add, int32_t lo, int32_t hi)
 {
-    const int32_t h = __mulhi(v, s2) + v;
-    return clamp_med3(((h >> rsm1) + off2p1) >> 1, lo, hi);
+    return clamp_med3((__mulhi(v, m) + add) >> sm1, lo, hi);
 }
 
-// std_requant of 4 values at once, the 4 results' low bytes packed into one word. After the per-column shift the
-// values are narrowed to 16 bits with saturation and the constant, the halving and the clamp work on pairs
-// (2.75 vector-ALU slots per value instead of 3.75). Same results as std_requant while |off2p1| <= 2049 and
-// -1024 <= lo <= hi <= 1024: a value the narrowing saturates ends beyond +-15359 after the halving and is clamped
-// to lo or hi either way.
+// std_requant of 4 values at once, the 4 results' low bytes packed into one word. The values are narrowed to 16 bits with saturation
+// and clamped in pairs: what the narrowing saturates is outside the bounds of an 8-bit type either way.
 typedef short pk16_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t std_requant4_pk16(const int32_t (&v)[4], const int32_t (&s2)[4], const int32_t (&rsm1)[4],
-                                                      pk16_t off2p1, pk16_t lo, pk16_t hi)
+typedef int   v4i_par __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint32_t std_requant4(const int32_t (&v)[4], v4i_par m, v4i_par sm1, v4i_par add, pk16_t lo, pk16_t hi)
 {
     int32_t x[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t)
-        x[t] = (__mulhi(v[t], s2[t]) + v[t]) >> rsm1[t];
+        x[t] = (__mulhi(v[t], m[t]) + add[t]) >> sm1[t];
     pk16_t a = __builtin_amdgcn_cvt_pk_i16(x[0], x[1]), b = __builtin_amdgcn_cvt_pk_i16(x[2], x[3]);
-    a = __builtin_elementwise_add_sat(a, off2p1) >> (pk16_t){1, 1};
-    b = __builtin_elementwise_add_sat(b, off2p1) >> (pk16_t){1, 1};
     a = __builtin_elementwise_min(__builtin_elementwise_max(a, lo), hi);
     b = __builtin_elementwise_min(__builtin_elementwise_max(b, lo), hi);
     return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a), 0x06040200u);

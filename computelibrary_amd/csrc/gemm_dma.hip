@@ -256,7 +256,7 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
 
     // per-column epilogue constants of this block: fetched now by the consumer waves (before their share of the start-up
     // loads, so that waiting for those covers these too), parked in registers, staged in LDS after the loop
-    constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? 1 + QP_COUNT : 0;
+    constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? PAR_LOADS : 0;
     constexpr int PPT  = (NPAR * BN + NW * 64 - 1) / (NW * 64);
     int32_t       par_reg[PPT > 0 ? PPT : 1];
     if (fast && wave < NW)
@@ -474,12 +474,12 @@ __global__ __launch_bounds__(GWM *GWN * 192) __attribute__((amdgpu_waves_per_eu(
         {
             const int idx = tid + t * NW * 64;
             if (idx < NPAR * BN)
-                par[idx] = par_reg[t];
+                park_constant(par, idx, BN, par_reg[t], g.epi.result_offset);
         }
         __syncthreads();
         if (EPI == EPI_FIXEDPOINT)
         {
-            char *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
+            char *stage = smem + PAR_ROWS * BN * 4;
             const bool rowv = g.epi.rowvec != nullptr || rowsum;
             if (g.epi.qp_std && qflag == 0 && !rowv)
                 epilogue_store_staged<true, false, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,
@@ -589,7 +589,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
 
     // per-column epilogue constants: fetched by the consumer waves behind their share of the start-up loads, parked in
     // registers, staged in LDS after the loop
-    constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? 1 + QP_COUNT : 0;
+    constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? PAR_LOADS : 0;
     constexpr int PPT  = (NPAR * BN + NW * 64 - 1) / (NW * 64);
     static_assert((NS - 2) * LPW + PPT < 64, "vmcnt range");
     int32_t       par_reg[PPT > 0 ? PPT : 1];
@@ -781,12 +781,12 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(GemmArgs g_in)
         {
             const int idx = tid + t * NW * 64;
             if (idx < NPAR * BN)
-                par[idx] = par_reg[t];
+                park_constant(par, idx, BN, par_reg[t], g.epi.result_offset);
         }
         __syncthreads();
         if (EPI == EPI_FIXEDPOINT)
         {
-            char      *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
+            char      *stage = smem + PAR_ROWS * BN * 4;
             const bool rowv  = g.epi.rowvec != nullptr;
             if (g.epi.qp_std && qflag == 0 && !rowv)
                 epilogue_store_staged<true, false, RS, QS, BM, BN, NW>(acc, g, par, stage, m0, n0, row_w, col_w, wave, lane, bz,

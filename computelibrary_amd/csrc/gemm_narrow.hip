@@ -86,8 +86,8 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     constexpr int RS = NARROW_ROWS / 16, QS = NARROW_BN / 16;
     constexpr int KBLK  = NB * 3;         // k blocks the loop covers (the B panel is zero beyond K)
     constexpr int PITCH = KBLK * 64 + NARROW_PAD_PIECES * 16; // bytes per B row in LDS
-    constexpr int NPAR  = 1 + QP_COUNT;
-    extern __shared__ __attribute__((aligned(16))) char smem[]; // B panel [npan * 64][PITCH], then par[NPAR][npan * 64]
+    constexpr int NPAR  = PAR_LOADS;
+    extern __shared__ __attribute__((aligned(16))) char smem[]; // B panel [npan * 64][PITCH], then par[PAR_ROWS][npan * 64]
 
     // Everything the main part uses is fetched here in one batch of scalar loads and pinned in registers (left alone, the
     // compiler fetches kernel arguments where they are first used: a round trip to memory each time). Pointers go
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
                                  : tail_start * (NARROW_WAVES * NARROW_ROWS) + (tail * tail_waves + wave) * NARROW_ROWS;
     const bool active = (tail < 0 || wave < tail_waves) && row0 < a_M;
 
-    // the epilogue's per-column constants (column term + the digested requantisation vectors), where they exist: 6 x 64
+    // the epilogue's per-column constants (column term + the digested requantisation vectors), where they exist: 3 x 64
     // dwords, one or two per thread, fetched first and parked in LDS with the B panel
     const bool    have_qp = EPI == EPI_FIXEDPOINT && u_qp != 0;
     constexpr int TPN     = NB == 1 ? (NPAR * NARROW_BN * NARROW_MAX_PANELS + NARROW_WAVES * 64 - 1) / (NARROW_WAVES * 64) : 2; // dwords per thread
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int i = 0; i < TPN; ++i)
             if (tid + i * NARROW_WAVES * 64 < NPAR * BNT)
-                par[tid + i * NARROW_WAVES * 64] = tp[i];
+                park_constant(par, tid + i * NARROW_WAVES * 64, BNT, tp[i], g.epi.result_offset);
     };
     int qflag = 1;
     if (have_qp && u_fl != 0)
@@ -364,10 +364,11 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
     }
     if (fast && g.epi.qp_std && (qflag & 3) == 0 && g.epi.vec_store && (g.N & 3) == 0)
     {
-        // every column has a normalised multiplier and a right shift of 2..31: the short form of the requantisation.
+        // every column has a normalised multiplier and a right shift of 2 to STD_MAX_SHIFT: the short form of the requantisation.
         // Lane l holds, for row rb * 16 + l % 16, the 4 consecutive columns q * 16 + 4 * (l / 16) + {0..3}: one dword
         // (N is a multiple of 4 here, so a lane's four columns exist together or not at all).
-        const int32_t  off2p1 = 2 * g.epi.result_offset + 1, lo = g.epi.lo, hi = g.epi.hi;
+        const int16_t  lo16 = (int16_t)g.epi.lo, hi16 = (int16_t)g.epi.hi;
+        const pk16_t   lo = {lo16, lo16}, hi = {hi16, hi16};
         const int      a_N    = g.N;
         int32_t        rv[RS];
         char          *drow[RS]; // this lane's row of D at column 4 * (l / 16)
@@ -382,24 +383,18 @@ __global__ __launch_bounds__(NARROW_WAVES * 64) __attribute__((amdgpu_waves_per_
         for (int q = 0; q < QS; ++q)
         {
             const int c  = q * 16 + 4 * lh;
-            const v4i s2 = *(const v4i *)(par + (1 + QP_S2) * BNT + col0 + c), r1 = *(const v4i *)(par + (1 + QP_RSM1) * BNT + col0 + c);
-            const v4i cv = *(const v4i *)(par + col0 + c);
+            const v4i cv = *(const v4i *)(par + PAR_CV * BNT + col0 + c), m = *(const v4i *)(par + PAR_M * BNT + col0 + c);
+            const v4i sm1 = *(const v4i *)(par + PAR_SM1 * BNT + col0 + c), add = *(const v4i *)(par + PAR_ADD * BNT + col0 + c);
 #pragma unroll
             for (int rb = 0; rb < RS; ++rb)
             {
-                int32_t o[4];
+                int32_t v[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
-                {
-                    // std_requant with the clamp as one median instruction (lo <= hi)
-                    const int32_t v = (int32_t)((uint32_t)acc[rb][q][t] + (uint32_t)cv[t] + (uint32_t)rv[rb]);
-                    const int32_t h = __mulhi(v, s2[t]) + v;
-                    asm("v_med3_i32 %0, %1, %2, %3" : "=v"(o[t]) : "v"(((h >> r1[t]) + off2p1) >> 1), "s"(lo), "v"(hi));
-                }
-                const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
-                const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
+                    v[t] = (int32_t)((uint32_t)acc[rb][q][t] + (uint32_t)cv[t] + (uint32_t)rv[rb]);
+                const uint32_t w = std_requant4(v, m, sm1, add, lo, hi);
                 if (row0 + rb * 16 + lr < a_M && col0 + c < a_N)
-                    *(uint32_t *)(drow[rb] + q * 16) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+                    *(uint32_t *)(drow[rb] + q * 16) = w;
             }
         }
     }
@@ -466,9 +461,9 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
     constexpr int RS = NARROW_ROWS / 16, QS = NARROW_BN / 16;
     constexpr int KBLK  = NB * 3;
     constexpr int PITCH = KBLK * 64 + NARROW_PAD_PIECES * 16;
-    constexpr int NPAR  = 1 + QP_COUNT;
+    constexpr int NPAR  = PAR_LOADS;
     constexpr int NDMA  = KBLK * 4 + NARROW_PAD_PIECES; // transfers of 1 KiB that make up a panel
-    // LDS: B panels [npan * 64][PITCH] | par[NPAR][npan * 64], the flag word | (from the next KiB) the staged window
+    // LDS: B panels [npan * 64][PITCH] | par[PAR_ROWS][npan * 64], the flag word | (from the next KiB) the staged window
     extern __shared__ __attribute__((aligned(1024))) char smem[];
 #define MI355_GLOBAL __attribute__((address_space(1)))
 #ifdef MI355_PHASE_CLOCKS
@@ -568,11 +563,11 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
     // ((x >> sw_r) & sw_mask) - the bits of x below the pixel size land below the mask
     const int sw_mask = sw_m << 5, sw_r = lc - (5 - sw_sh);
     const uint32_t lds0    = (uint32_t)(size_t)(__attribute__((address_space(3))) char *)smem;
-    const int      img_off = (ncols * PITCH + NPAR * ncols * 4 + 4 + 1023) & ~1023; // (+ 4: the flag word)
+    const int      img_off = (ncols * PITCH + PAR_ROWS * ncols * 4 + 4 + 1023) & ~1023; // (+ 4: the flag word)
     const int      s_img   = img_off >> lc; // LDS pixel index of the window's first pixel
 
-    // epilogue constants (one dword per thread: 6 x 64 of them per panel), the flag word of the requantisation
-    // (fetched by the waves that start first - with one panel the threads of waves 0 to 5 hold one constant each, wave 0
+    // epilogue constants (one dword per thread: 3 x 64 of them per panel), the flag word of the requantisation
+    // (fetched by the waves that start first - with one panel the threads of waves 0 to 2 hold one constant each, wave 0
     // the flag word - and handed on through LDS: the waves that start last then have nothing to wait for before the barrier)
     const bool    have_qp = EPI == EPI_FIXEDPOINT && u_qp != 0;
     constexpr int TPN     = MULTI ? (NPAR * NARROW_BN * NARROW_MAX_PANELS + HALO_WAVES * 64 - 1) / (HALO_WAVES * 64) : 1;
@@ -635,16 +630,16 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int i = 0; i < TPN; ++i)
         if (have_qp && tid + i * HALO_WAVES * 64 < NPAR * ncols)
-            par[tid + i * HALO_WAVES * 64] = tp[i];
+            park_constant(par, tid + i * HALO_WAVES * 64, ncols, tp[i], g.epi.result_offset);
     if (tid == 0)
-        par[NPAR * ncols] = qflag;
+        par[PAR_ROWS * ncols] = qflag;
     __syncthreads();
     MI355_BAND_PHASE(3); // everybody's transfers have landed
     if (!active)
         return;
     if (wave >= HALO_DMA_WAVES)
         tile_setup();
-    const int  qflag_u = __builtin_amdgcn_readfirstlane(par[NPAR * ncols]);
+    const int  qflag_u = __builtin_amdgcn_readfirstlane(par[PAR_ROWS * ncols]);
     const bool fast    = have_qp && (qflag_u & 1) == 0;
 
     // Weights with an offset: the row sums of the tile's patches, by matrix instructions of their own against ones (here and
@@ -749,12 +744,12 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
         MI355_BAND_PHASE(4); // matrix instructions issued
 
         const int row0 = m_base + wave * NARROW_ROWS, a_M = m_base + P; // rows of the GEMM this tile covers, and where the band ends
-        if (fast && g.epi.qp_pk16 && (qflag_u & 3) == 0 && g.epi.vec_store && (g.N & 3) == 0)
+        if (fast && g.epi.qp_std && (qflag_u & 3) == 0 && g.epi.vec_store && (g.N & 3) == 0)
         {
             // the short form of the requantisation, 4 columns at a time: lane l holds, for row rb * 16 + l % 16, the 4
             // consecutive columns pc0 + q * 16 + 4 * (l / 16) + {0..3}
-            const int16_t  o16 = (int16_t)(2 * g.epi.result_offset + 1), lo16 = (int16_t)g.epi.lo, hi16 = (int16_t)g.epi.hi;
-            const pk16_t   off2p1 = {o16, o16}, lo = {lo16, lo16}, hi = {hi16, hi16};
+            const int16_t  lo16 = (int16_t)g.epi.lo, hi16 = (int16_t)g.epi.hi;
+            const pk16_t   lo = {lo16, lo16}, hi = {hi16, hi16};
             const int      a_N    = g.N;
             int32_t        rv[RSX];
             char          *drow[RSX];
@@ -769,9 +764,8 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
             for (int q = 0; q < QS; ++q)
             {
                 const int c  = pc0 + q * 16 + 4 * lh;
-                const v4i s2 = *(const v4i *)(par + (1 + QP_S2) * ncols + c), r1 = *(const v4i *)(par + (1 + QP_RSM1) * ncols + c);
-                const v4i cv = *(const v4i *)(par + c);
-                const int32_t s2a[4] = {s2[0], s2[1], s2[2], s2[3]}, r1a[4] = {r1[0], r1[1], r1[2], r1[3]};
+                const v4i cv = *(const v4i *)(par + PAR_CV * ncols + c), m = *(const v4i *)(par + PAR_M * ncols + c);
+                const v4i sm1 = *(const v4i *)(par + PAR_SM1 * ncols + c), add = *(const v4i *)(par + PAR_ADD * ncols + c);
 #pragma unroll
                 for (int rb = 0; rb < RSX; ++rb)
                 {
@@ -779,7 +773,7 @@ __global__ __launch_bounds__(HALO_WAVES * 64) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
                         v[t] = (int32_t)((uint32_t)acc[rb][q][t] + (uint32_t)cv[t] + (uint32_t)rv[rb]);
-                    const uint32_t w = std_requant4_pk16(v, s2a, r1a, off2p1, lo, hi);
+                    const uint32_t w = std_requant4(v, m, sm1, add, lo, hi);
                     if (row0 + rb * 16 + lr < a_M && c < a_N)
                         *(uint32_t *)(drow[rb] + q * 16) = w;
                 }
@@ -864,7 +858,7 @@ static bool halo_plan(const GemmArgs &a, int epi, int cus, int &rpw, int &wpi, s
     // the staged window: band + halo + padding (see the kernel)
     const int64_t in_rows = (int64_t)(rpw - 1) * c.stride_y + (int64_t)(c.KH - 1) * c.dil_y + 1;
     const int64_t wp      = (int64_t)(c.OW - 1) * c.stride_x + (int64_t)(c.KW - 1) * c.dil_x + 1;
-    const int64_t img_off = (ncols * (nb * 192 + NARROW_PAD_PIECES * 16) + (1 + QP_COUNT) * ncols * 4 + 4 + 1023) & ~(int64_t)1023;
+    const int64_t img_off = (ncols * (nb * 192 + NARROW_PAD_PIECES * 16) + PAR_ROWS * ncols * 4 + 4 + 1023) & ~(int64_t)1023;
     const int64_t bytes   = img_off + ((in_rows * wp * c.C + 1023) & ~(int64_t)1023);
     if (bytes > 160 * 1024 || images * wpi > (int64_t)INT32_MAX)
         return false;
@@ -963,7 +957,7 @@ int narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, boo
     if (fn == nullptr)
         return (int)hipErrorInvalidValue;
     const int    npan = (args.N + NARROW_BN - 1) / NARROW_BN;
-    const size_t lds  = (size_t)npan * NARROW_BN * (nb * 192 + NARROW_PAD_PIECES * 16) + (size_t)(1 + QP_COUNT) * npan * NARROW_BN * sizeof(int32_t);
+    const size_t lds  = (size_t)npan * NARROW_BN * (nb * 192 + NARROW_PAD_PIECES * 16) + (size_t)PAR_ROWS * npan * NARROW_BN * sizeof(int32_t);
     if (lds > 48 * 1024)
     {
         // once per kernel and device (for the largest panel count the kernel may meet)
@@ -974,7 +968,7 @@ int narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, boo
             return (int)hipErrorInvalidDevice;
         if ((done.load(std::memory_order_acquire) & (1u << dev)) == 0)
         {
-            const size_t most = nb == 1 ? (size_t)NARROW_MAX_PANELS * NARROW_BN * (192 + 16 + (1 + QP_COUNT) * sizeof(int32_t)) : lds;
+            const size_t most = nb == 1 ? (size_t)NARROW_MAX_PANELS * NARROW_BN * (192 + 16 + PAR_ROWS * sizeof(int32_t)) : lds;
             const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
             if (e != hipSuccess)
                 return (int)e;

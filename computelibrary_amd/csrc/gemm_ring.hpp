@@ -386,7 +386,7 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         ld.issue(0, 0);
     }
     // per-column epilogue constants: fetched behind the first stage, parked in registers, staged in LDS after the loop
-    constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? 1 + QP_COUNT : 0;
+    constexpr int NPAR = (EPI == EPI_FIXEDPOINT) ? PAR_LOADS : 0;
     constexpr int PPT  = (NPAR * BN + NW * 64 - 1) / (NW * 64);
     int32_t       par_reg[PPT > 0 ? PPT : 1];
     if (EPI == EPI_FIXEDPOINT && u_fl != 0)
@@ -669,12 +669,12 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
         {
             const int idx = tid + t * NW * 64;
             if (idx < NPAR * BN)
-                par[idx] = par_reg[t];
+                park_constant(par, idx, BN, par_reg[t], g.epi.result_offset);
         }
         __syncthreads();
         if (EPI == EPI_FIXEDPOINT)
         {
-            char      *stage = smem + ((NPAR * BN * 4 + 15) & ~15);
+            char      *stage = smem + PAR_ROWS * BN * 4;
             const bool rowv  = g.epi.rowvec != nullptr || rowsum;
             auto       store = [&](auto planes_c)
             {

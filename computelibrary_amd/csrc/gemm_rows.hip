@@ -7,9 +7,9 @@
 // lies beyond KW * C in a piece are neighbouring pixels, which meet zero weights. The weights of the panel stay in registers.
 //
 // Against patch rows written out in memory and fetched by the narrow kernel (KH / stride times each) the image crosses the chip
-// once: 32 x 224 x 224 x 3 -> 64, 7 x 7, stride 2: 9.4 us of copy and 30 of the narrow kernel, 20.3 in one launch now; 29 x 85 x 85 x 3 -> 32:
-// 10.2, 6.8; 2 x 93 x 93 x 3 -> 32, 5 x 5: 7.6, 4.7. What bounds it: the vector ALU, 10 instructions per output for the
-// requantisation (about 9 us of the 20) and about 60 per 32 pixels for the operands, at 3 waves per SIMD, then the output's bytes.
+// once: 32 x 224 x 224 x 3 -> 64, 7 x 7, stride 2: 9.4 us of copy and 30 of the narrow kernel, 20.6 in one launch, 18.4 with two vector instructions less per output; 29 x 85 x 85 x 3 -> 32:
+// 10.2, 6.8; 2 x 93 x 93 x 3 -> 32, 5 x 5: 7.6, 4.7. What bounds it: the vector ALU, 5.75 instructions per output for the
+// requantisation and about 60 per 32 pixels for the operands, at 3 waves per SIMD, then the output's bytes.
 #include "conv_rows_plan.hpp"
 #include "mfma_common.hpp"
 
@@ -28,7 +28,7 @@ template <int NKB>
 __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu(NKB <= 2 ? 4 : 3))) void conv_rows_kernel(RowsArgs a, uint32_t flip)
 {
     constexpr int    BPITCH = NKB * 64 + 32, OPITCH = ROWS_OPITCH; // (a panel row 32 bytes past a multiple of 64: see NARROW_PAD_PIECES)
-    constexpr int    NT = ROWS_WAVES * 64, NPAR = 1 + QP_COUNT;
+    constexpr int    NT = ROWS_WAVES * 64, NPAR = PAR_ROWS;
     static_assert(NPAR == ROWS_NPAR, "conv_rows_fixed_lds counts them");
     const GemmArgs  &g = a.g;
     const ConvGeom  &c = g.conv;
@@ -59,8 +59,8 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
         *(v4i *)(panel + r * BPITCH + q * 16) = *(const v4i *)(g.Bp + (int64_t)(n0 + r) * g.Kp + q * 16);
     }
     if (p.qp_flag)
-        for (int i = tid; i < NPAR * 64; i += NT)
-            par[i] = i < 64 ? p.colvec[n0 + i] : p.qp[(int64_t)(i / 64 - 1) * p.qp_stride + n0 + i % 64];
+        for (int i = tid; i < PAR_LOADS * 64; i += NT)
+            park_constant(par, i, 64, i < 64 ? p.colvec[n0 + i] : p.qp[(int64_t)(i / 64 - 1) * p.qp_stride + n0 + i % 64], p.result_offset);
     // the window, a dword per thread and step, four steps of loads at a time
     {
         const int      per_row = a.pitch / 4, total = a.win_rows * per_row;
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
     const int     cols = min(g.N - n0, 64);
     char         *mine = out + wave * 32 * OPITCH;
     char         *D    = (char *)g.D + ((int64_t)n * c.OH + oy0) * c.OW * g.ldd + n0;
-    const int32_t off2p1 = 2 * p.result_offset + 1;
+    const pk16_t  lo16 = {(int16_t)p.lo, (int16_t)p.lo}, hi16 = {(int16_t)p.hi, (int16_t)p.hi};
     for (int t = wave; t * 32 < npix; t += ROWS_WAVES)
     {
         v4i acc[2][4];
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
             }
         }
         // requantise into the wave's own 32 x 64 bytes of LDS (accumulator layout as in epilogue_store_t)
-        auto each = [&](auto requant)
+        auto each = [&](auto requant4)
         {
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -156,31 +156,40 @@ __global__ __launch_bounds__(ROWS_WAVES * 64) __attribute__((amdgpu_waves_per_eu
                 if (q * 16 >= cols)
                     continue;
                 const int col = q * 16 + 4 * lh;
-                const v4i cv = *(const v4i *)(par + col);
 #pragma unroll
                 for (int rb = 0; rb < 2; ++rb)
-                {
-                    int32_t o[4];
-#pragma unroll
-                    for (int d = 0; d < 4; ++d)
-                        o[d] = requant(acc[rb][q][d], cv[d], col + d);
-                    const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
-                    const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
-                    *(uint32_t *)(mine + (rb * 16 + lr) * OPITCH + col) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
-                }
+                    *(uint32_t *)(mine + (rb * 16 + lr) * OPITCH + col) = requant4(acc[rb][q], col);
             }
         };
+        auto one_by_one = [&](auto requant)
+        {
+            each([&](v4i v, int col) {
+                int32_t o[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    o[d] = requant(v[d], col + d);
+                const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
+                const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
+                return __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+            });
+        };
         if (qflag == 0 && p.qp_std)
-            each([&](int32_t v, int32_t cv, int col) {
-                return std_requant((int32_t)((uint32_t)v + (uint32_t)cv), par[(1 + QP_S2) * 64 + col], par[(1 + QP_RSM1) * 64 + col], off2p1, p.lo, p.hi);
+            each([&](v4i v, int col) {
+                const v4i cv = *(const v4i *)(par + PAR_CV * 64 + col);
+                int32_t   x[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    x[d] = (int32_t)((uint32_t)v[d] + (uint32_t)cv[d]);
+                return std_requant4(x, *(const v4i *)(par + PAR_M * 64 + col), *(const v4i *)(par + PAR_SM1 * 64 + col),
+                                    *(const v4i *)(par + PAR_ADD * 64 + col), lo16, hi16);
             });
         else if ((qflag & 1) == 0)
-            each([&](int32_t v, int32_t cv, int col) {
-                return fast_requant((int32_t)((uint32_t)v + (uint32_t)cv), par[(1 + QP_S2) * 64 + col], par[(1 + QP_CMASK) * 64 + col],
-                                    par[(1 + QP_LS) * 64 + col], par[(1 + QP_RSM1) * 64 + col], par[(1 + QP_RMASK) * 64 + col], p.result_offset, p.lo, p.hi);
+            one_by_one([&](int32_t v, int col) {
+                return fast_requant((int32_t)((uint32_t)v + (uint32_t)par[PAR_CV * 64 + col]), par[PAR_M * 64 + col], par[PAR_SM1 * 64 + col],
+                                    p.result_offset, p.lo, p.hi);
             });
         else
-            each([&](int32_t v, int32_t, int col) {
+            one_by_one([&](int32_t v, int col) {
                 int first = n0; // (hidden: the addresses of 16 columns in three vectors, kept over the loop, were 100 registers)
                 asm volatile("" : "+s"(first));
                 const int j = min(first + col, g.N - 1);

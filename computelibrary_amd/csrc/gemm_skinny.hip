@@ -449,9 +449,8 @@ __device__ __forceinline__ void once_store_output(MI355_GLOBAL char *gD, int64_t
         const int32_t v = (int32_t)((uint32_t)sum + (uint32_t)c + (uint32_t)rv);
         int32_t       q;
         if (p.stage == 0 && m >= 0 && sh > -32 && sh < 32)
-            // the branch-free form of the same arithmetic (see fast_requant), its constants derived here
-            q = fast_requant(v, (int32_t)((uint32_t)m << 1), (uint32_t)m >= 0x40000000u ? -1 : 0, sh < 0 ? -sh : 0, sh > 1 ? sh - 1 : 0,
-                             sh > 0 ? 1 : 0, p.result_offset, p.lo, p.hi);
+            // the branch-free form of the same arithmetic
+            q = fast_requant(v, m, sh - 1, p.result_offset, p.lo, p.hi);
         else
             q = epi_fixedpoint(sum, c, rv, m, sh, p);
         ((MI355_GLOBAL int8_t *)gD)[idx] = (int8_t)q;

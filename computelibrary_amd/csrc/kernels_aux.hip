@@ -458,16 +458,12 @@ __global__ void qparams_kernel(const int32_t *__restrict__ mult, const int32_t *
     }
     if (m < 0)
         atomicOr(neg, 1);
-    if (j < N && !(m >= 0x40000000 && s >= 2 && s < 32))
-        atomicOr(neg, 2); // not the common case (normalised multiplier, right shift by 2 or more)
+    if (j < N && !(m >= 0x40000000 && s >= 2 && s <= STD_MAX_SHIFT))
+        atomicOr(neg, 2); // not the common case (see std_requant)
     if (s >= 32 || s <= -32)
         m = 0, s = 0; // the reference arithmetic yields 0 for these
-    const uint32_t m2          = (uint32_t)m << 1;
-    qp[QP_S2 * (int64_t)Np + j]    = (int32_t)m2;
-    qp[QP_CMASK * (int64_t)Np + j] = ((uint32_t)m >= 0x40000000u) ? -1 : 0;
-    qp[QP_LS * (int64_t)Np + j]    = s < 0 ? -s : 0;
-    qp[QP_RSM1 * (int64_t)Np + j]  = s > 1 ? s - 1 : 0;
-    qp[QP_RMASK * (int64_t)Np + j] = s > 0 ? 1 : 0;
+    qp[QP_M * (int64_t)Np + j]   = m;
+    qp[QP_SM1 * (int64_t)Np + j] = s - 1;
 }
 
 int qparams_launch(const int32_t *mult, const int32_t *shift, int32_t mult_s, int32_t shift_s, int N, int Np,

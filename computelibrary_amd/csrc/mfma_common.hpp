@@ -319,7 +319,7 @@ __device__ __forceinline__ void epilogue_store_t(const v4i (&acc)[RS][QS], const
     }
 }
 // FIXEDPOINT epilogue of the narrow kernels for multipliers >= 0, straight to the destination. The block's per-column constants were staged in LDS
-// as par[6][BN]: row 0 the folded offset/bias vector, rows 1..5 the QP_* vectors; col_in_tile is the wave's first
+// as par[PAR_ROWS][BN]; col_in_tile is the wave's first
 // column inside the block tile. Same accumulator layout as epilogue_store_t.
 template <int RS, int QS, int BN>
 __device__ __forceinline__ void epilogue_store_fast(const v4i (&acc)[RS][QS], const GemmArgs &g, const int32_t *par,
@@ -342,12 +342,8 @@ __device__ __forceinline__ void epilogue_store_fast(const v4i (&acc)[RS][QS], co
     {
         const int c  = col_in_tile + qs * 16 + 4 * lh;
         const int j0 = col0 + qs * 16 + 4 * lh;
-        const v4i cv = *(const v4i *)(par + 0 * BN + c);
-        const v4i s2 = *(const v4i *)(par + (1 + QP_S2) * BN + c);
-        const v4i cm = *(const v4i *)(par + (1 + QP_CMASK) * BN + c);
-        const v4i ls = *(const v4i *)(par + (1 + QP_LS) * BN + c);
-        const v4i r1 = *(const v4i *)(par + (1 + QP_RSM1) * BN + c);
-        const v4i rm = *(const v4i *)(par + (1 + QP_RMASK) * BN + c);
+        const v4i cv = *(const v4i *)(par + PAR_CV * BN + c), mu = *(const v4i *)(par + PAR_M * BN + c);
+        const v4i sm1 = *(const v4i *)(par + PAR_SM1 * BN + c);
 #pragma unroll
         for (int rs = 0; rs < RS; ++rs)
         {
@@ -357,7 +353,7 @@ __device__ __forceinline__ void epilogue_store_fast(const v4i (&acc)[RS][QS], co
             for (int t = 0; t < 4; ++t)
             {
                 const int32_t v = (int32_t)((uint32_t)acc[rs][qs][t] + (uint32_t)cv[t] + (uint32_t)rv[rs]);
-                o[t]            = fast_requant(v, s2[t], cm[t], ls[t], r1[t], rm[t], p.result_offset, p.lo, p.hi);
+                o[t]            = fast_requant(v, mu[t], sm1[t], p.result_offset, p.lo, p.hi);
             }
             // low bytes of o[0..3] -> one dword
             const uint32_t p01    = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
@@ -379,7 +375,7 @@ __device__ __forceinline__ void epilogue_store_fast(const v4i (&acc)[RS][QS], co
     }
 }
 // FIXEDPOINT epilogue of the pipelined kernel for multipliers >= 0. The block's per-column constants were staged in LDS
-// as par[6][BN]: row 0 the folded offset/bias vector, rows 1..5 the QP_* vectors; col_in_tile is the wave's first
+// as par[PAR_ROWS][BN]; col_in_tile is the wave's first
 // column inside the block tile; accumulator layout as in epilogue_store_t. The packed 8-bit results of the whole BM x BN block
 // tile are first laid out in LDS (row pitch BN + 16 bytes: the 64 dword writes of a wave instruction - 16 rows by 4 dwords - then
 // hit 64 different banks) and then written row by row, so a wave instruction writes pieces of rows end to end instead of
@@ -397,7 +393,7 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
     const EpiParams &p      = g.epi;
     const int32_t   *rowvec = p.rowvec ? p.rowvec + (int64_t)bz * p.rowvec_batch_stride : nullptr;
     int32_t          rv[RS];
-    const int32_t    off2p1 = 2 * p.result_offset + 1;
+    const pk16_t     lo16 = {(int16_t)p.lo, (int16_t)p.lo}, hi16 = {(int16_t)p.hi, (int16_t)p.hi};
 #pragma unroll
     for (int rs = 0; rs < RS; ++rs)
     {
@@ -408,39 +404,39 @@ __device__ __forceinline__ void epilogue_store_staged(const v4i (&acc)[RS][QS], 
     for (int qs = 0; qs < QS; ++qs)
     {
         const int c  = col_in_tile + qs * 16 + 4 * lh;
-        const v4i cv = *(const v4i *)(par + 0 * BN + c);
-        const v4i s2 = *(const v4i *)(par + (1 + QP_S2) * BN + c);
-        const v4i r1 = *(const v4i *)(par + (1 + QP_RSM1) * BN + c);
-        v4i       cm = {0, 0, 0, 0}, ls = cm, rm = cm;
-        if (!STD)
-        {
-            cm = *(const v4i *)(par + (1 + QP_CMASK) * BN + c);
-            ls = *(const v4i *)(par + (1 + QP_LS) * BN + c);
-            rm = *(const v4i *)(par + (1 + QP_RMASK) * BN + c);
-        }
+        const v4i cv = *(const v4i *)(par + PAR_CV * BN + c), mu = *(const v4i *)(par + PAR_M * BN + c);
+        const v4i sm1 = *(const v4i *)(par + PAR_SM1 * BN + c);
+        v4i       add = {0, 0, 0, 0};
+        if (STD)
+            add = *(const v4i *)(par + PAR_ADD * BN + c);
 #pragma unroll
         for (int rs = 0; rs < RS; ++rs)
         {
-            int32_t o[4];
+            int32_t v[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t)
+                v[t] = ROWV ? (int32_t)((uint32_t)acc[rs][qs][t] + (uint32_t)cv[t] + (uint32_t)rv[rs]) : (int32_t)((uint32_t)acc[rs][qs][t] + (uint32_t)cv[t]);
+            if constexpr (STD && !PLANES)
+                *(uint32_t *)(stage + (row_in_tile + rs * 16 + lr) * PITCH + c) = std_requant4(v, mu, sm1, add, lo16, hi16);
+            else
             {
-                const int32_t v = ROWV ? (int32_t)((uint32_t)acc[rs][qs][t] + (uint32_t)cv[t] + (uint32_t)rv[rs])
-                                       : (int32_t)((uint32_t)acc[rs][qs][t] + (uint32_t)cv[t]);
-                o[t] = STD ? std_requant(v, s2[t], r1[t], off2p1, p.lo, p.hi)
-                           : fast_requant(v, s2[t], cm[t], ls[t], r1[t], rm[t], p.result_offset, p.lo, p.hi);
-            }
-            const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
-            const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
-            if constexpr (PLANES)
-            {
+                int32_t o[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
-                    stage[(c + t) * PITCH + row_in_tile + rs * 16 + lr] = (char)o[t];
-                (void)p01, (void)p23;
+                    o[t] = STD ? std_requant(v[t], mu[t], sm1[t], add[t], p.lo, p.hi) : fast_requant(v[t], mu[t], sm1[t], p.result_offset, p.lo, p.hi);
+                if constexpr (PLANES)
+                {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        stage[(c + t) * PITCH + row_in_tile + rs * 16 + lr] = (char)o[t];
+                }
+                else
+                {
+                    const uint32_t p01 = __builtin_amdgcn_perm((uint32_t)o[1], (uint32_t)o[0], 0x0c0c0400u);
+                    const uint32_t p23 = __builtin_amdgcn_perm((uint32_t)o[3], (uint32_t)o[2], 0x0c0c0400u);
+                    *(uint32_t *)(stage + (row_in_tile + rs * 16 + lr) * PITCH + c) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
+                }
             }
-            else
-                *(uint32_t *)(stage + (row_in_tile + rs * 16 + lr) * PITCH + c) = __builtin_amdgcn_perm(p23, p01, 0x05040100u);
         }
     }
     barrier();
