@@ -20,7 +20,7 @@ CEILINGS_SOURCES = ["ceilings.hip"]
 # the product library once more with the pipelined kernel compiled to leave clock readings at the ends of its parts
 # (`bench.py --phase-clocks`); also a library of its own
 PHASES_LIB = os.path.join(LIBDIR, "libmi355phases.so")
-SOURCES = ["gemm_dma.hip", "gemm_ring.hip", "gemm_mfma.hip", "gemm_skinny.hip", "gemm_narrow.hip", "gemm_rows.hip", "kernels_aux.hip", "capi.hip"]
+SOURCES = ["gemm_dma.hip", "gemm_ring.hip", "gemm_mfma.hip", "gemm_skinny.hip", "gemm_narrow.hip", "gemm_rows.hip", "gemm_window.hip", "kernels_aux.hip", "capi.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

@@ -2,6 +2,7 @@
 // workspace ownership, host <-> device staging, and the launches. No arithmetic lives here.
 #include "../../include/mi355_gemmlowp.h"
 #include "conv_rows_plan.hpp"
+#include "conv_window_plan.hpp"
 #include "internal.hpp"
 
 #include <algorithm>
@@ -211,7 +212,7 @@ struct GemmCore
     std::string kname_mfma, kname_dma, kprefix;
     // The names a run can report, composed when the choice is made (create, prepare, update): a run only points at one
     // of them - it must not touch the host heap
-    std::string        kname_narrow, kname_band, kname_dma_full, kname_bytes, kname_rows, kname_splitk, kname_mfma_full;
+    std::string        kname_window, kname_narrow, kname_band, kname_dma_full, kname_bytes, kname_rows, kname_splitk, kname_mfma_full;
     const char        *kname_static = nullptr; // the streaming kernel names its forms itself
     const std::string *kname_run = nullptr; // what the last run took (nullptr: no run yet, kname is what create announced)
     uint8_t fill_byte = 0; // value of the 16 filler bytes (0, or the im2col pad value)
@@ -222,6 +223,7 @@ struct GemmCore
 
     void refresh_names()
     {
+        kname_window    = kprefix + "pp_window_64";
         kname_narrow    = kprefix + "narrow_32x64";
         kname_band      = kprefix + "band_32x64";
         kname_dma_full  = kprefix + kname_dma;
@@ -394,13 +396,14 @@ struct GemmCore
 
     // B (device memory; N rows of K elements when transposed) -> the packed image the chosen kernel reads, the columns' sums
     // and the per-column terms of the epilogue. bias_in: device memory, or null
-    int pack(const void *B, int64_t ldb, int64_t b_bs, bool transposed, int kf, const int32_t *bias_in, hipStream_t s)
+    // (both: one transposed B once more in operand order, behind the other image)
+    int pack(const void *B, int64_t ldb, int64_t b_bs, bool transposed, int kf, const int32_t *bias_in, hipStream_t s, bool both = false)
     {
         const bool   skinny = path == MI355_PATH_SKINNY;
         DevBuf      &dst    = skinny ? Bs : Bp;
         const size_t image  = (size_t)Np * Kp;
         has_bias            = bias_in != nullptr;
-        TRY(dst.ensure(image * nb()));
+        TRY(dst.ensure(image * (both ? 2 : nb())));
         TRY(colsum.ensure(sizeof(int32_t) * (size_t)Np * nb()));
         TRY(colvec.ensure(sizeof(int32_t) * (size_t)Np * nb()));
         if (has_bias)
@@ -418,7 +421,7 @@ struct GemmCore
             ColumnFinish   f   = column_finish(epi == EPI_FIXEDPOINT ? bias_in : nullptr);
             f.colsum += (int64_t)b * Np, f.colvec += (int64_t)b * Np;
             if (transposed)
-                HIP_TRY(pack_bt_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, out, f, s));
+                HIP_TRY(pack_bt_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, out, f, s, both ? out + image : nullptr));
             else
                 HIP_TRY(pack_b_launch(src, ldb, b_bs, n, K, N, Kp, Np, flip_b, kf, skinny, splits, out, colpart.as<int32_t>(), f, s));
         }
@@ -503,6 +506,12 @@ struct GemmCore
         return e != hipSuccess ? e : got;
     }
 
+    // whether the narrow kernel's image of B is made
+    bool narrow_form() const
+    {
+        return path == MI355_PATH_MFMA && patch_c > 0 && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192 && M >= panels_from)) && narrow_panel_chunks(K) > 0;
+    }
+
     // after pack(): everything else a run reads
     int finish_prepare(const int32_t *mult_in, const int32_t *shift_in, hipStream_t s)
     {
@@ -521,7 +530,7 @@ struct GemmCore
             HIP_TRY(hipMemcpyAsync(shift.p, shift_in, sizeof(int32_t) * (size_t)N, hipMemcpyDefault, s));
         }
         // few output columns and a short K: the image of the B panel the narrow kernel copies into LDS
-        has_narrow = path == MI355_PATH_MFMA && patch_c > 0 && nb() == 1 && (N <= 64 || (N <= 256 && K <= 192 && M >= panels_from)) && narrow_panel_chunks(K) > 0;
+        has_narrow = narrow_form();
         if (has_narrow)
         {
             const int chunks = narrow_panel_chunks(K);
@@ -972,6 +981,28 @@ struct mi355_conv_handle
     bool            raw_rows = false;        // ... whose kernel takes them from the caller's image where there is no weights offset
     DevBuf          padSrc, padW;
     PtrKind         kindSrc, kindDst; // host or device memory, per argument of run()
+    bool       window_made = false, window = false; // gemm_window.hip runs it: decided at create; with the present offsets
+    WindowPlan window_plan;
+    bool       from_window() const { return window && core.rq.stage == MI355_STAGE_FIXEDPOINT; }
+    // how it is divided (which depends on whether there is a weights offset)
+    bool divide_window()
+    {
+        return conv_window_plan(geom_true, d.batch, d.OFM, d.layout == MI355_NCHW, core.b_off_eff() != 0, num_cus(), window_plan);
+    }
+    bool choose_window()
+    {
+        const bool planes = d.layout == MI355_NCHW;
+        if (d.path != MI355_CONV_AUTO || core.epi != EPI_FIXEDPOINT || raw_rows || !divide_window())
+            return false;
+        // (the narrow kernel needs no copy and starts half a microsecond earlier: 18 x 18 x 48 -> 24, 1 x 1: 3.6 us, 4.3 here. Several of its panels are up
+        // to a fifth slower: 21 x 24 x 24 x 16 -> 88, 3 x 3 stride 2: 5.4, 4.6)
+        if (!planes && (c_pad == 0 || patch_rows) && core.narrow_form())
+            return false;
+        // (register-staged tiles, which run what the pipelined kernel does not take, look every byte up)
+        const double tiles_us = core.dma_idx >= 0 ? core.us_dma : 1e9;
+        return conv_window_pays(window_plan.us, conv_other_us(geom_true, d.batch, d.OFM, core.K, planes, core.b_off_eff() != 0, c_pad > 0, core.narrow_form(), tiles_us, num_cus()),
+                                !planes && c_pad == 0 && core.splitk_plan > 1);
+    }
     bool   from_image() const { return raw_rows && core.b_off_eff() == 0 && core.rq.stage == MI355_STAGE_FIXEDPOINT; }
     size_t pad_bytes() const { return (size_t)d.batch * d.H * geom.W * c_pad; }
 };
@@ -1573,6 +1604,8 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
     // and the constant a_offset * b_offset * K uses the unpadded K.
     h->geom_true = h->geom;
     h->geom.c_true = h->geom_true.c_true = d.C;
+    int      taps_c = 0; // under patch rows: the padded channels of single taps, and their geometry
+    ConvGeom taps_geom{};
     {
         if (d.path == MI355_CONV_AUTO && d.C % 16 != 0)
         {
@@ -1610,22 +1643,29 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
                 (int64_t)d.batch * d.H * row_bytes < ((int64_t)1 << 31) &&
                 patch_rows_fit((int64_t)d.batch * d.H, d.W, d.C, dr.W, d.stride_x, d.pad_left, dr.C))
             {
+                taps_c = h->c_pad, taps_geom = h->geom;
                 conv_geom(dr, gp);
                 if (conv_fast_div_ok(dr, gp))
                     h->c_pad = dr.C, h->patch_rows = true, h->raw_rows = raw, gp.c_true = d.KW * d.C, h->geom = gp;
             }
         }
     }
-    const int64_t M64 = (int64_t)d.batch * h->geom.OH * h->geom.OW;
-    const int64_t K64 = (int64_t)d.KH * h->geom.KW * h->geom.C;
-    if (M64 > INT32_MAX || K64 > INT32_MAX)
+    auto set_sizes = [&]() -> int
+    {
+        const int64_t M64 = (int64_t)d.batch * h->geom.OH * h->geom.OW;
+        const int64_t K64 = (int64_t)d.KH * h->geom.KW * h->geom.C;
+        if (M64 > INT32_MAX || K64 > INT32_MAX)
+            return fail("convolution too large");
+        c.M = (int)M64, c.N = d.OFM, c.K = (int)K64, c.batch = 1;
+        c.k_const = h->c_pad ? d.KH * d.KW * d.C : 0;
+        c.patch_c = h->geom.C, c.patch_c_true = h->geom.c_true;
+        return 0;
+    };
+    if (set_sizes())
     {
         delete h;
-        return fail("convolution too large");
+        return 1;
     }
-    c.M = (int)M64, c.N = d.OFM, c.K = (int)K64, c.batch = 1;
-    c.k_const = h->c_pad ? d.KH * d.KW * d.C : 0;
-    c.patch_c = h->geom.C, c.patch_c_true = h->geom.c_true;
     // Patch rows bring a short K to convolutions of few channels whatever their size; one panel after the other pays from some
     // rows per compute unit on (us, panels against the pipelined kernel, 128 and 256 columns, 3 channels, 5 x 5, stride 2: 1568
     // rows 8.0 / 5.9 and 11.1 / 5.9; 12544: 8.3 / 6.9 and 11.7 / 8.4; 25088: 9.0 / 8.7 and 12.5 / 10.6; 18 channels, 3 x 3, 12544: 8.7 / 8.5
@@ -1645,6 +1685,17 @@ int mi355_conv_create(const mi355_conv_desc *desc, mi355_conv_handle **out)
     {
         delete h;
         return 1;
+    }
+    h->window_made = h->window = h->choose_window();
+    if (h->window && h->patch_rows)
+    {
+        // its weights are those of single taps
+        h->patch_rows = false, h->c_pad = taps_c, h->geom = taps_geom, c.panels_from = 0;
+        if (set_sizes() || c.choose_kernel())
+        {
+            delete h;
+            return 1;
+        }
     }
     // The patch matrix is only materialised on request (path 1) or where the loaders' reciprocal divisions would not be
     // exact. Channel counts that are not a multiple of 16 and are not padded (see above: a request for the caller's tensor as
@@ -1711,7 +1762,7 @@ int mi355_conv_prepare(mi355_conv_handle *h, const void *weights, const void *bi
     TRY(to_device(c.rq.per_channel ? shift : nullptr, sizeof(int32_t) * c.N, h->stageShift, s, &shiftd));
     // weights [OFM][KH][KW][C] are already the K-contiguous layout with k = c + kx*C + ky*C*KW
     // (src/cpu/kernels/CpuWeightsReshapeKernel.cpp:150-166)
-    TRY(c.pack(wd, c.K, 0, true, 0, (const int32_t *)biasd, s));
+    TRY(c.pack(wd, c.K, 0, true, 0, (const int32_t *)biasd, s, h->window_made));
     TRY(c.finish_prepare((const int32_t *)multd, (const int32_t *)shiftd, s));
     HIP_TRY(hipStreamSynchronize(s));
     c.prepared = true;
@@ -1737,8 +1788,23 @@ int mi355_conv_update_quant(mi355_conv_handle *h, int32_t src_offset, int32_t we
     c.fill_byte      = (uint8_t)(pad_value & 0xFF);
     c.kprefix        = h->implicit ? "implicit_" : "im2col+";
     c.refresh_names();
+    h->window = h->window_made && h->divide_window();
     if (!c.prepared)
         return 0;
+    // a run that kept its window in LDS has neither padded channels nor turned a layout round: the next one may be recorded and could not make room
+    if (h->window_made && !h->from_window())
+    {
+        if (h->c_pad)
+            TRY(h->padSrc.ensure(h->pad_bytes()));
+        if (h->d.layout == MI355_NCHW)
+        {
+            ConvTensorSteps st, dt;
+            TRY(conv_src_steps(h->d, st));
+            TRY(conv_dst_steps(h->d, dt));
+            TRY(h->nhwcSrc.ensure(st.bytes));
+            TRY(h->nhwcDst.ensure(dt.bytes));
+        }
+    }
     // a run that went straight from the image has made no patch rows: the next one may be recorded and could not make room for them
     if (h->raw_rows && !h->from_image())
         TRY(h->padSrc.ensure(h->pad_bytes()));
@@ -1830,7 +1896,20 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
         Dd = h->nhwcDst.p;
         return 0;
     };
-    if (nchw)
+    if (h->from_window())
+    {
+        GemmArgs g{};
+        c.fill_epi(g.epi, nullptr);
+        g.epi.rowsum_mul = c.b_off_eff(), g.epi.planes = nchw ? h->geom.OH * h->geom.OW : 0;
+        g.A = (const int8_t *)srcd, g.Bp = c.Bp.as<int8_t>() + (size_t)c.Np * c.Kp, g.Kp = c.Kp;
+        g.D = Dd, g.ldd = c.N, g.M = c.M, g.N = c.N, g.K = c.K;
+        g.conv          = h->geom_true;
+        g.conv.pad_word = ((uint32_t)d.pad_value & 0xFFu) * 0x01010101u;
+        HIP_TRY(conv_window_launch(h->window_plan, c.flip_a, g, d.batch, s));
+        c.kname_run = &c.kname_window;
+        planes      = nchw;
+    }
+    else if (nchw)
     {
         // every image [C][H*W] -> [H*W][C]
         TRY(h->nhwcSrc.ensure(src_bytes));
@@ -1842,7 +1921,7 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
     }
     const void *src_true = srcd; // the caller's channel count
     const bool  raw      = h->from_image();
-    if (h->c_pad && !raw)
+    if (h->c_pad && !raw && !h->from_window())
     {
         // pixels of C channels -> pixels of c_pad channels (what the added ones hold meets zero weights; the padding value
         // keeps them in range of the source type)
@@ -1853,7 +1932,9 @@ int mi355_conv_run(mi355_conv_handle *h, const void *src, void *dst, void *strea
             HIP_TRY(channel_pad_launch(srcd, h->padSrc.p, (int64_t)d.batch * d.H * d.W, d.C, h->c_pad, (uint8_t)(d.pad_value & 0xFF), s));
         srcd = h->padSrc.p;
     }
-    if (raw)
+    if (h->from_window())
+        ; // (done)
+    else if (raw)
     {
         GemmArgs g{};
         c.fill_epi(g.epi, nullptr);

@@ -188,6 +188,14 @@ __device__ __forceinline__ int32_t clamp_i32(int32_t v, int32_t lo, int32_t hi)
     return min(max(v, lo), hi);
 }
 
+// requant_fixedpoint and the clamp without a branch, for any multiplier, from the digested constants
+__device__ __forceinline__ int32_t any_requant(int32_t v, int32_t m, int32_t sm1, int32_t result_offset, int32_t lo, int32_t hi)
+{
+    const int32_t ls = sm1 < -1 ? -1 - sm1 : 0, rsm1 = sm1 > 0 ? sm1 : 0, rmask = sm1 >= 0 ? 1 : 0;
+    const int32_t h  = sqdmulh((int32_t)((uint32_t)v << ls), m);
+    return clamp_med3((int32_t)((uint32_t)(((h >> rsm1) + rmask) >> rmask) + (uint32_t)result_offset), lo, hi);
+}
+
 // One element of the FIXEDPOINT epilogue: acc (raw dot product) -> 8-bit value as int32
 __device__ __forceinline__ int32_t epi_fixedpoint(int32_t acc, int32_t colv, int32_t rowv, int32_t mult, int32_t shift,
                                                   const EpiParams &p)

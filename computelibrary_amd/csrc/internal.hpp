@@ -137,6 +137,11 @@ int  narrow_launch(int epi, bool flip_a, const GemmArgs &args, hipStream_t s, bo
 // fixed-point stage, no weights offset; conv_rows_plan.hpp says which). args: Bp packed with K = KH pieces of 16 or 32 bytes, conv the caller's geometry
 int  conv_rows_launch(bool flip_a, const GemmArgs &args, int batch, hipStream_t s);
 
+// gemm_window.hip — convolutions whose input window lies in LDS, in the caller's layout (conv_window_plan.hpp says which and how). args: Bp the
+// weights in operand order, conv the caller's geometry with the raw padding byte, epi.planes != 0: NCHW on both sides
+struct WindowPlan;
+int  conv_window_launch(const WindowPlan &plan, bool flip_a, const GemmArgs &args, int batch, hipStream_t s);
+
 // gemm_skinny.hip — M <= 64, B packed in matrix-core operand order (see pack_b_launch)
 constexpr int SKINNY_MAX_M = 64;
 // *variant (when given): a static string naming the form of the kernel that ran
@@ -160,9 +165,9 @@ struct ColumnFinish
 int pack_b_splits(int Kp, int Np, int nb);
 int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny, int splits,
                   int8_t *out, int32_t *partial, const ColumnFinish &f, hipStream_t s);
-// the same from B given as [N][ldk] with K contiguous (conv weights [OFM][KH*KW*C])
+// the same from B given as [N][ldk] with K contiguous (conv weights [OFM][KH*KW*C]). operands: the image in operand order as well (one matrix)
 int pack_bt_launch(const void *Bt, int64_t ldk, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
-                   int8_t *out, const ColumnFinish &f, hipStream_t s);
+                   int8_t *out, const ColumnFinish &f, hipStream_t s, int8_t *operands = nullptr);
 // the first rows of Bp -> [rows][chunks + NARROW_PAD_PIECES] pieces of 16 bytes, zero beyond Kp; the padding: a row of ones (zeros
 // for what does not count of a patch of K with c_true of C channels)
 int pack_b_narrow_launch(const int8_t *Bp, int Kp, int Np, int chunks, int rows, int K, int C, int c_true, int8_t *Bn, hipStream_t s);

@@ -301,7 +301,8 @@ int pack_b_launch(const void *B, int64_t ldb, int64_t b_bs, int nb, int K, int N
 // no other wave.
 template <bool SKINNY>
 __global__ __launch_bounds__(256) void pack_bt_kernel(const uint8_t *__restrict__ Bt, int64_t ldk, int64_t b_bs, int K, int N, int Kp,
-                                                      int Np, uint32_t flip4, int kf, int8_t *__restrict__ out, ColumnFinish f)
+                                                      int Np, uint32_t flip4, int kf, int8_t *__restrict__ out, ColumnFinish f,
+                                                      int8_t *__restrict__ operands)
 {
     const int b = blockIdx.y, n = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     out += (int64_t)b * Np * Kp;
@@ -326,6 +327,8 @@ __global__ __launch_bounds__(256) void pack_bt_kernel(const uint8_t *__restrict_
         }
         s += sum4_i8((int)w[0]) + sum4_i8((int)w[1]) + sum4_i8((int)w[2]) + sum4_i8((int)w[3]);
         *(v4i *)(out + packed_offset<SKINNY>(n, kc, Kp)) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+        if (!SKINNY && operands)
+            *(v4i *)(operands + packed_offset<true>(n, kc, Kp)) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
@@ -335,15 +338,15 @@ __global__ __launch_bounds__(256) void pack_bt_kernel(const uint8_t *__restrict_
 }
 
 int pack_bt_launch(const void *Bt, int64_t ldk, int64_t b_bs, int nb, int K, int N, int Kp, int Np, bool flip, int kf, bool skinny,
-                   int8_t *out, const ColumnFinish &f, hipStream_t s)
+                   int8_t *out, const ColumnFinish &f, hipStream_t s, int8_t *operands)
 {
-    if (Np % 4 || Kp % 64 || Np < N || Kp < K || nb < 1 || nb > 65535 || (kf > 1 && K % kf != 0))
+    if (Np % 4 || Kp % 64 || (operands && (nb != 1 || skinny)) || Np < N || Kp < K || nb < 1 || nb > 65535 || (kf > 1 && K % kf != 0))
         return (int)hipErrorInvalidValue;
     const dim3 grid(Np / 4, nb), block(256);
     if (skinny)
-        pack_bt_kernel<true><<<grid, block, 0, s>>>((const uint8_t *)Bt, ldk, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, out, f);
+        pack_bt_kernel<true><<<grid, block, 0, s>>>((const uint8_t *)Bt, ldk, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, out, f, nullptr);
     else
-        pack_bt_kernel<false><<<grid, block, 0, s>>>((const uint8_t *)Bt, ldk, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, out, f);
+        pack_bt_kernel<false><<<grid, block, 0, s>>>((const uint8_t *)Bt, ldk, b_bs, K, N, Kp, Np, flip ? 0x80808080u : 0u, kf, out, f, operands);
     return launch_status();
 }
 
