@@ -185,7 +185,7 @@ struct GemmCore
     bool    has_narrow = false; // Bn holds the narrow kernel's image of B
     bool    pt_vectors = false; // streaming path, per-tensor requantisation: mult / shift hold the scalars, replicated
     std::string kname;
-    DevBuf  Bp, Bs, Bn, colsum, colvec, colpart, rowvec, mult, shift, bias, Ap, fill, qp, zeros, parts, zerocol;
+    DevBuf  Bp, Bs, Bn, colsum, colvec, colpart, rowvec, mult, shift, bias, Ap, fill, qp, zeros, parts, zerocol, arrived;
     // A prepare that only enqueues (on the legacy default stream, every operand in device memory, nothing left to set up): an
     // event behind it, which runs on other streams wait for
     hipEvent_t  prep_done    = nullptr;
@@ -193,7 +193,8 @@ struct GemmCore
     bool        recorded = false; // a run was recorded into a graph, which may be launched at any time
     // What is known of buffers that are written once and then kept (see keep_flags)
     int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not known)
-    bool        zeros_set = false, zerocol_set = false;
+    bool        zeros_set = false, zerocol_set = false, arrived_set = false;
+    SkinnySlices sk_plan; // the streaming kernel's K slices and their memory (prepare() fills it in)
     bool        qp_scalar_set = false; // the per-tensor requantisation vectors hold qp_rq
     bool        writes_recorded = false;
     mi355_requant qp_rq{};
@@ -244,7 +245,7 @@ struct GemmCore
             (void)hipEventDestroy(prep_done);
         prep_done = nullptr, prep_pending = false;
         Bp.release(), Bs.release(), Bn.release(), colsum.release(), colvec.release(), colpart.release(), rowvec.release(), mult.release();
-        shift.release(), bias.release(), Ap.release(), fill.release(), qp.release(), zeros.release(), parts.release(), zerocol.release();
+        shift.release(), bias.release(), Ap.release(), fill.release(), qp.release(), zeros.release(), parts.release(), zerocol.release(), arrived.release();
     }
 
     static constexpr int MOST_SLICES = 32;
@@ -263,14 +264,10 @@ struct GemmCore
             return fail("unknown path %d", path);
         const bool automatic = path == MI355_PATH_AUTO;
         if (automatic)
-            // measured: up to 32 rows the streaming kernel always wins; up to 64 rows only while N is small enough
-            // that the pipelined kernel would leave most compute units without a tile
+            // measured: up to 32 rows the streaming kernel always wins, up to 64 rows sometimes (below)
             // (a batch of small products runs the streaming kernel once per entry: the tiled kernels would spend a 64-row
             // tile, mostly padding, on each)
-            // (and up to 64 rows whenever K <= 4096 is a whole number of 64-byte blocks: the form of the streaming
-            // kernel that keeps the operand blocks of A in registers for its whole run then applies)
-            path = (M <= 32 || (batch == 1 && M <= SKINNY_MAX_M && (N < 8192 || (K <= 4096 && K % 64 == 0)))) ? MI355_PATH_SKINNY
-                                                                                                         : MI355_PATH_MFMA;
+            path = (M <= 32 || (batch == 1 && M <= SKINNY_MAX_M)) ? MI355_PATH_SKINNY : MI355_PATH_MFMA;
         const int cus = num_cus();
         // The pipelined kernel's tile is chosen with a small cost model in microseconds (the prices and what they were fitted to
         // stand at g_dma_cost): a tile costs MfmaConfig::us_tile for its start-up and epilogue, of which the workgroups that
@@ -314,6 +311,21 @@ struct GemmCore
             }
             return best;
         };
+        if (automatic && path == MI355_PATH_SKINNY && M > 32 && K >= 16)
+        {
+            // 33 to 64 rows: the tiles, or up to a K of 4096 the streaming kernel, whose operand blocks of A then stay in registers (its
+            // forms beyond are slower than the tiles everywhere: 60 rows, 3072 x 12128 23.8 us, tiles 17.6; 2880 x 7936 17.9 and 11.1), whichever
+            // is priced lower. The tiles' prices come from a B that stays in the caches; weights that come from memory add what B is over
+            // 20 MB at 3.3 TB/s (15 products of 0.8 to 78 MB: 0.9 to 17.4 us, off by 1). 60 rows, tiles and stream: 8640 x 2880 9.1 and
+            // 13.0, 9792 x 3264 12.7 and 13.6; 3264 x 3264 9.8 and 8.7, 11008 x 4096 17.8 and 16.6, 768 x 2064 8.3 and 6.1.
+            // (Whole 64-byte blocks with an offset on B, whose row sums take the streaming kernel a pass, were not measured and stay there.)
+            int          plan = 1;
+            double       tiles = 0;
+            const double pass = byte_lda || b_off_eff() != 0 ? 2.5 : 0.0, cold = std::max(1.0, 0.3 * ((double)N * K * 1e-6 - 20.0));
+            if (pick_dma(byte_lda || (b_off_eff() != 0 && K % 16 != 0) ? 2 : 0, plan, tiles) >= 0 &&
+                (K > 4096 || ((b_off_eff() == 0 || K % 64 != 0) && tiles + cold < skinny_64rows_us(M, N, K, cus) + pass)))
+                path = MI355_PATH_MFMA;
+        }
         if (automatic && batch == 1 && path == MI355_PATH_SKINNY && (byte_lda || (b_off_eff() != 0 && K % 64 != 0)) && K >= 16 &&
             (double)N * K <= 4e6)
         {
@@ -546,6 +558,21 @@ struct GemmCore
             HIP_TRY(fill_i32_launch(zeros.as<int32_t>(), 0, SKINNY_MAX_M, s));
             zeros_set = true;
         }
+        if (path == MI355_PATH_SKINNY && batch == 1)
+        {
+            sk_plan = skinny_slices(M, N, K, num_cus());
+            if (sk_plan.slices > 1)
+            {
+                TRY(parts.ensure(sizeof(int32_t) * sk_plan.words));
+                if (!arrived_set)
+                {
+                    TRY(arrived.ensure(sizeof(int32_t) * (size_t)sk_plan.grid));
+                    HIP_TRY(fill_i32_launch(arrived.as<int32_t>(), 0, sk_plan.grid, s));
+                    arrived_set = true;
+                }
+                sk_plan.parts = parts.as<int32_t>(), sk_plan.arrived = arrived.as<int32_t>();
+            }
+        }
         // A deep K under few output tiles: the pipelined kernel would leave most compute units idle, each of the others
         // walking the whole K. The K range is cut into slices that run as the batch entries of one S32 launch (the slice
         // offset is the batch stride of A and of the packed B alike), and a second kernel sums the planes and applies the
@@ -580,7 +607,7 @@ struct GemmCore
         if (!writes_recorded && s != nullptr && capturing(s))
             writes_recorded = true;
         if (writes_recorded)
-            fill_set = -1, zeros_set = zerocol_set = qp_scalar_set = false;
+            fill_set = -1, zeros_set = zerocol_set = arrived_set = qp_scalar_set = false;
     }
 
     int set_fill(hipStream_t s)
@@ -830,7 +857,7 @@ struct GemmCore
                     ge.epi.colvec += (int64_t)b * gb.epi.colvec_batch_stride;
                     if (ge.epi.rowvec != nullptr)
                         ge.epi.rowvec += (int64_t)b * gb.epi.rowvec_batch_stride;
-                    HIP_TRY(skinny_launch(epi, flip_in_loader, ge, 1, s, &kname_static));
+                    HIP_TRY(skinny_launch(epi, flip_in_loader, ge, 1, s, &kname_static, batch == 1 ? &sk_plan : nullptr));
                 }
         }
         else

@@ -429,10 +429,15 @@ struct OnceArgs
     const int32_t *colvec, *rowvec, *mult, *shift;
     const float   *bias_f32;
     int64_t        lda, ldd;
-    int32_t        M, N, KB, grid;
+    int32_t        M, N, KB, grid; // KB: k blocks that hold any of K
     int32_t        result_offset, stage, lo, hi;
     float          scale, act_min, act_max;
     int32_t        has_offsets, accumulate, act_twice, half_out;
+    int32_t        KBS, K; // k blocks from one column group of the packed B to the next; K, a multiple of 16
+    // K slices (the stage-once kernel's SLICED form): k blocks per slice, slices, their partial sums [slice][column group][row * 16 + column]
+    // and one counter for each workgroup of a slice, zero between launches
+    int32_t        KS, slices;
+    int32_t       *parts, *arrived;
 };
 // One output of the stage-once kernels: the reduced sum, its column term c, multiplier (or float bias bits) m, shift sh
 // and row term rv through epilogue EPI into element idx of D
@@ -479,7 +484,9 @@ __host__ __device__ constexpr int once_pitch(int rows, int per)
 // its K slice of A in LDS; 64 rows x 4096 bytes would not fit there, and need not: the operand blocks of A stay in
 // registers for the whole kernel, so with 64 rows a workgroup has 8 waves (256 registers each: 128 of them hold A) and
 // gathers the blocks straight from global memory, once.
-template <int EPI, bool FLIP_A, int PER, bool MULTI, int ROWS, int WAVES = ONCE_WAVES>
+// SLICED: blockIdx.y is a slice of K. Every workgroup of a slice leaves its partial sums in memory and counts itself in;
+// the last of those that share its columns adds the others' to its own and writes the outputs. Nobody waits for anybody.
+template <int EPI, bool FLIP_A, int PER, bool MULTI, int ROWS, int WAVES = ONCE_WAVES, bool SLICED = false>
 __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g)
 {
     static_assert(ROWS == 8 || ROWS == 16 || ROWS == 32 || ROWS == 64, "rows");
@@ -495,6 +502,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
     // has its operands of A in registers (the two together would not fit)
     constexpr bool RED_IN_STAGE = RB > 1 || (ROWS == 16 && PER == 8); // (16 rows of 8 k blocks per wave fill LDS as well)
     __shared__ __attribute__((aligned(16))) int32_t red_own[RED_IN_STAGE ? 1 : 2 * WAVES * RB * RL * 4];
+    __shared__ int32_t                              last; // SLICED: whether this workgroup is the last of its columns
     __shared__ int32_t                              par[4][64]; // [vector][group * 16 + column]; row vector: [3][row]
     extern __shared__ __attribute__((aligned(16))) char a_stage[]; // [WAVES][ROWS][PITCH] (nothing staged with 64 rows)
     // (the launch sizes the dynamic area for the larger of the two)
@@ -512,7 +520,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
                    "+s"(g.has_offsets), "+s"(g.accumulate), "+s"(g.act_twice), "+s"(g.lda), "+s"(g.ldd), "+s"(g.M), "+s"(g.N),
                    "+s"(g.KB), "+s"(g.grid), "+s"(u_a), "+s"(u_b), "+s"(u_d), "+s"(u_cv), "+s"(u_rv), "+s"(u_mu), "+s"(u_sh),
                    "+s"(u_bf));
-    const MI355_GLOBAL int8_t *const  gA = (const MI355_GLOBAL int8_t *)u_a, *const gB = (const MI355_GLOBAL int8_t *)u_b;
+    asm volatile("" : "+s"(g.KBS), "+s"(g.K));
+    const int slice0 = SLICED ? (int)blockIdx.y * g.KS : 0; // the slice's first k block
+    const MI355_GLOBAL int8_t *const gA = (const MI355_GLOBAL int8_t *)u_a + (int64_t)slice0 * 64, *const gB = (const MI355_GLOBAL int8_t *)u_b + (int64_t)slice0 * 1024;
     MI355_GLOBAL char *const          gD = (MI355_GLOBAL char *)u_d;
     const MI355_GLOBAL int32_t *const g_colvec = (const MI355_GLOBAL int32_t *)u_cv, *const g_rowvec = (const MI355_GLOBAL int32_t *)u_rv,
                                      *const g_mult = (const MI355_GLOBAL int32_t *)u_mu, *const g_shift = (const MI355_GLOBAL int32_t *)u_sh,
@@ -527,7 +537,9 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
     // (8 k blocks per wave: the wave index as a scalar, so that the addresses of the B blocks are a scalar base plus one
     // per-lane offset - as per-lane 64-bit addresses, all computed ahead, they pushed the B blocks out of the registers)
     const int wave = (PER == 8 && ROWS < 64) ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : (int)(threadIdx.x >> 6);
-    const int KB   = g.KB;
+    const int KB   = SLICED ? min(g.KS, g.KB - slice0) : g.KB;
+    const int kend = min(KB * 64, g.K - slice0 * 64); // (a multiple of 16: the last k block may end early, where B is zero)
+    const int KBS  = g.KBS;
     const int NGT  = (g.N + 15) / 16;
     const int G    = g.grid; // == gridDim.x
     const int mine = (NGT - (int)blockIdx.x + G - 1) / G; // column groups of this workgroup, 1..ONCE_MAX_GROUPS
@@ -563,7 +575,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
     {
         // lanes past the end of K (last busy wave) re-read the slice's first 16 bytes into columns nobody reads; waves
         // without k blocks re-read the last k block
-        const int col = a_sc < min(PER, KB - kb0) * 64 ? a_sc : 0;
+        const int col = a_sc < kend - kb0 * 64 ? a_sc : 0;
 #pragma unroll
         for (int i = 0; i < NA; ++i)
             ta[i] = *(const MI355_GLOBAL v4i *)(gA + (int64_t)min(i * RPL + a_sr, g.M - 1) * g.lda + (int64_t)min(kb0, KB - 1) * 64 + col);
@@ -582,14 +594,14 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
         const int grp = min((int)blockIdx.x + gi * G, NGT - 1);
 #pragma unroll
         for (int u = decltype(u0c)::value; u < decltype(u1c)::value; ++u) // k blocks past KB (last busy wave) re-read the last one
-            fb[slot][u] = __builtin_nontemporal_load((const MI355_GLOBAL v4i *)(bp + ((int64_t)grp * KB + max(min(u, KB - 1 - kb0), 0)) * 1024));
+            fb[slot][u] = __builtin_nontemporal_load((const MI355_GLOBAL v4i *)(bp + ((int64_t)grp * KBS + max(min(u, KB - 1 - kb0), 0)) * 1024));
     };
     auto load_b = [&](int slot, int gi)
     {
         const int grp = min((int)blockIdx.x + gi * G, NGT - 1);
 #pragma unroll
         for (int u = 0; u < PER; ++u)
-            fb[slot][u] = __builtin_nontemporal_load((const MI355_GLOBAL v4i *)(bp + ((int64_t)grp * KB + max(min(u, KB - 1 - kb0), 0)) * 1024));
+            fb[slot][u] = __builtin_nontemporal_load((const MI355_GLOBAL v4i *)(bp + ((int64_t)grp * KBS + max(min(u, KB - 1 - kb0), 0)) * 1024));
     };
     // MULTI: every workgroup has at least two groups. Nothing between here and the wait for A may sit behind a branch:
     // the compiler would no longer know how many loads are in flight and would make the wait for A wait for B as well
@@ -607,8 +619,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
             for (int u = 0; u < PER; ++u)
-                fa[rb][u] = *(const MI355_GLOBAL v4i *)(gA + (int64_t)min(rb * 16 + arow, g.M - 1) * g.lda +
-                                                        (int64_t)min(kb0 + u, KB - 1) * 64 + akc);
+            {
+                const int k = min(kb0 + u, KB - 1) * 64;
+                fa[rb][u] = *(const MI355_GLOBAL v4i *)(gA + (int64_t)min(rb * 16 + arow, g.M - 1) * g.lda + k + (akc < kend - k ? akc : 0));
+            }
     }
     if constexpr (A_GLOBAL)
     {
@@ -654,7 +668,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
     // of group gi + 1 wait for the loads of group gi + 2 as well.
     auto groups = [&](auto count)
     {
-        constexpr int MINE = decltype(count)::value;
+        constexpr int MINE = decltype(count)::value, OUTS = SLICED ? (ROWS * 16 + WAVES * 64 - 1) / (WAVES * 64) : 1;
+        int32_t       part[SLICED ? MINE : 1][OUTS];
 #pragma unroll
         for (int gi = 0; gi < MINE; ++gi)
         {
@@ -752,10 +767,71 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_once_kernel(OnceArgs g
 #pragma unroll
                 for (int w = 0; w < WAVES; ++w)
                     sum += r[w * RB * RL * 4];
+                if constexpr (SLICED)
+                {
+                    part[gi][o / (WAVES * 64)] = sum;
+                    continue;
+                }
                 const int32_t c = par[0][gi * 16 + ecol], m = par[1][gi * 16 + ecol], sh = par[2][gi * 16 + ecol], rv = par[3][erow & (ROWS - 1)];
                 if (j < g.N && erow < g.M)
                     once_store_output<EPI>(gD, (int64_t)erow * g.ldd + j, sum, c, m, sh, rv, has_bias, p);
             }
+        }
+        if constexpr (SLICED)
+        {
+            // Stores and loads of device scope, which go past the caches that dies do not share: a wave's are where all can see them when
+            // its count of stores in flight is zero, so the barrier and the counter need no fence. (A release fence writes the whole
+            // L2 back, once per wave: 42 us instead of 12 at 25 x 3072 x 12128.) 1.4 us behind the last group.
+            auto place = [&](int z, int gi, int o) { return g.parts + ((int64_t)z * NGT + (int)blockIdx.x + gi * G) * (ROWS * 16) + o; };
+#pragma unroll
+            for (int gi = 0; gi < MINE; ++gi)
+#pragma unroll
+                for (int q = 0; q < OUTS; ++q)
+                    if (t + q * WAVES * 64 < ROWS * 16)
+                        __hip_atomic_store(place(blockIdx.y, gi, t + q * WAVES * 64), part[gi][q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (t == 0)
+                last = __hip_atomic_fetch_add(g.arrived + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.slices - 1;
+            __syncthreads();
+            if (!last)
+                return;
+            asm volatile("" ::: "memory");
+            if (t == 0)
+                __hip_atomic_store(g.arrived + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // (three slices' sums in flight together)
+            for (int z0 = 1; z0 < g.slices; z0 += 3)
+            {
+                int32_t other[3][MINE][OUTS];
+#pragma unroll
+                for (int y = 0; y < 3; ++y)
+                {
+                    int z = (int)blockIdx.y + min(z0 + y, g.slices - 1);
+                    z     = z >= g.slices ? z - g.slices : z;
+#pragma unroll
+                    for (int gi = 0; gi < MINE; ++gi)
+#pragma unroll
+                        for (int q = 0; q < OUTS; ++q)
+                            other[y][gi][q] = __hip_atomic_load(place(z, gi, min(t + q * WAVES * 64, ROWS * 16 - 1)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int y = 0; y < 3; ++y)
+#pragma unroll
+                    for (int gi = 0; gi < MINE; ++gi)
+#pragma unroll
+                        for (int q = 0; q < OUTS; ++q)
+                            part[gi][q] += z0 + y < g.slices ? other[y][gi][q] : 0;
+            }
+#pragma unroll
+            for (int gi = 0; gi < MINE; ++gi)
+#pragma unroll
+                for (int q = 0; q < OUTS; ++q)
+                {
+                    const int o = t + q * WAVES * 64, erow = o >> 4, ecol = o & 15, j = ((int)blockIdx.x + gi * G) * 16 + ecol;
+                    if (o < ROWS * 16 && j < g.N && erow < g.M)
+                        once_store_output<EPI>(gD, (int64_t)erow * g.ldd + j, part[gi][q], par[0][gi * 16 + ecol], par[1][gi * 16 + ecol],
+                                               par[2][gi * 16 + ecol], par[3][erow & (ROWS - 1)], has_bias, p);
+                }
         }
     };
     if (!MULTI || mine == 1)
@@ -808,7 +884,7 @@ __global__ __launch_bounds__(ONCE_WAVES * 64) void gemm_skinny_deepk_kernel(Once
     p.has_offsets = g.has_offsets, p.accumulate = g.accumulate, p.act_twice = g.act_twice, p.half_out = g.half_out;
 
     const int t = (int)threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int KB = g.KB, NGT = (g.N + 15) / 16, G = g.grid;
+    const int KB = g.KB, KBS = g.KBS, NGT = (g.N + 15) / 16, G = g.grid;
     const int mine = (NGT - (int)blockIdx.x + G - 1) / G; // column groups of this workgroup, 1..ONCE_MAX_GROUPS
     const int kb0  = wave * PER;
     const int nb   = min(max(KB - kb0, 0), PER); // k blocks of this wave (the last busy wave may be short, later ones have none)
@@ -825,7 +901,7 @@ __global__ __launch_bounds__(ONCE_WAVES * 64) void gemm_skinny_deepk_kernel(Once
         par_v                           = vec[v == 3 ? min(lane & 7, g.M - 1) : j];
     }
     // this wave's slice of A, piece by piece: piece q of the slice is row q / PPR, 16-byte column q % PPR. Rows past M
-    // re-read row M-1, columns past the wave's k blocks its first column (neither is ever used)
+    // re-read row M-1, columns past the wave's share of K its first column (neither is ever used)
     char     *a_lds = a_stage + wave * 8 * PITCH;
     v4i       ta[NA];
     const int kbase = min(kb0, KB - 1) * 64;
@@ -833,7 +909,7 @@ __global__ __launch_bounds__(ONCE_WAVES * 64) void gemm_skinny_deepk_kernel(Once
     for (int i = 0; i < NA; ++i)
     {
         const int q = i * 64 + lane, row = q / PPR, pc = q - row * PPR;
-        ta[i]       = *(const MI355_GLOBAL v4i *)(gA + (int64_t)min(row, g.M - 1) * g.lda + kbase + (pc < nb * 4 ? pc * 16 : 0));
+        ta[i]       = *(const MI355_GLOBAL v4i *)(gA + (int64_t)min(row, g.M - 1) * g.lda + kbase + (pc * 16 < min(PER * 64, g.K - kb0 * 64) ? pc * 16 : 0));
     }
     // B in units of one chunk of one group: unit c of group gi
     const MI355_GLOBAL int8_t *bp = gB + ((int64_t)min(kb0, KB - 1) * 64 + lane) * 16;
@@ -848,7 +924,7 @@ __global__ __launch_bounds__(ONCE_WAVES * 64) void gemm_skinny_deepk_kernel(Once
 #pragma unroll
         for (int u = 0; u < CH; ++u) // k blocks past the wave's last re-read it
             fb[slot][u] = __builtin_nontemporal_load(
-                (const MI355_GLOBAL v4i *)((const MI355_GLOBAL int8_t *)b + ((int64_t)grp * KB + max(min(c * CH + u, KB - 1 - kb0), 0)) * 1024));
+                (const MI355_GLOBAL v4i *)((const MI355_GLOBAL int8_t *)b + ((int64_t)grp * KBS + max(min(c * CH + u, KB - 1 - kb0), 0)) * 1024));
     };
     load_unit(0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -992,17 +1068,17 @@ int device_cus()
     return n;
 }
 
-template <int PER, bool MULTI, int ROWS>
-static int skinny_once_launch_r(int epi, bool flip_a, const GemmArgs &a, int grid, hipStream_t s)
+template <int PER, bool MULTI, int ROWS, bool SLICED = false>
+static int skinny_once_launch_r(int epi, bool flip_a, const GemmArgs &a, int grid, hipStream_t s, const SkinnySlices *plan = nullptr)
 {
     constexpr int WAVES = ROWS == 64 ? 8 : ONCE_WAVES;
     static const void *const fns[3][2] = {
-        {(const void *)gemm_skinny_once_kernel<EPI_S32, false, PER, MULTI, ROWS, WAVES>,
-         (const void *)gemm_skinny_once_kernel<EPI_S32, true, PER, MULTI, ROWS, WAVES>},
-        {(const void *)gemm_skinny_once_kernel<EPI_FIXEDPOINT, false, PER, MULTI, ROWS, WAVES>,
-         (const void *)gemm_skinny_once_kernel<EPI_FIXEDPOINT, true, PER, MULTI, ROWS, WAVES>},
-        {(const void *)gemm_skinny_once_kernel<EPI_F32, false, PER, MULTI, ROWS, WAVES>,
-         (const void *)gemm_skinny_once_kernel<EPI_F32, true, PER, MULTI, ROWS, WAVES>}};
+        {(const void *)gemm_skinny_once_kernel<EPI_S32, false, PER, MULTI, ROWS, WAVES, SLICED>,
+         (const void *)gemm_skinny_once_kernel<EPI_S32, true, PER, MULTI, ROWS, WAVES, SLICED>},
+        {(const void *)gemm_skinny_once_kernel<EPI_FIXEDPOINT, false, PER, MULTI, ROWS, WAVES, SLICED>,
+         (const void *)gemm_skinny_once_kernel<EPI_FIXEDPOINT, true, PER, MULTI, ROWS, WAVES, SLICED>},
+        {(const void *)gemm_skinny_once_kernel<EPI_F32, false, PER, MULTI, ROWS, WAVES, SLICED>,
+         (const void *)gemm_skinny_once_kernel<EPI_F32, true, PER, MULTI, ROWS, WAVES, SLICED>}};
     // the kernel fetches these without asking
     if (a.epi.colvec == nullptr || a.epi.rowvec == nullptr || (epi == EPI_FIXEDPOINT && (a.epi.mult == nullptr || a.epi.shift == nullptr)))
         return (int)hipErrorInvalidValue;
@@ -1017,10 +1093,17 @@ static int skinny_once_launch_r(int epi, bool flip_a, const GemmArgs &a, int gri
         return e;
     const EpiParams &p = a.epi;
     OnceArgs         o{a.A,    a.Bp,   a.D,    p.colvec, p.rowvec,  p.mult,    p.shift,       p.bias_f32,   a.lda,       a.ldd,        a.M,
-               a.N,    (int32_t)(a.Kp / 64), grid, p.result_offset, p.stage, p.lo, p.hi, p.scale, p.act_min, p.act_max,
-               p.has_offsets, p.accumulate, p.act_twice, p.half_out};
+               a.N,    (a.K + 63) / 64, grid, p.result_offset, p.stage, p.lo, p.hi, p.scale, p.act_min, p.act_max,
+               p.has_offsets, p.accumulate, p.act_twice, p.half_out, (int32_t)(a.Kp / 64), a.K};
+    int   slices  = 1;
+    if (SLICED)
+    {
+        if (plan == nullptr || plan->parts == nullptr || plan->arrived == nullptr)
+            return (int)hipErrorInvalidValue;
+        o.KS = plan->blocks, o.slices = slices = plan->slices, o.parts = plan->parts, o.arrived = plan->arrived;
+    }
     void *kargs[] = {&o};
-    return (int)hipLaunchKernel(fn, dim3(grid), dim3(WAVES * 64), kargs, lds, s);
+    return (int)hipLaunchKernel(fn, dim3(grid, slices), dim3(WAVES * 64), kargs, lds, s);
 }
 
 // (built for one column group per workgroup only: with the group loop written out for 2 to 4 groups as well, the
@@ -1045,8 +1128,8 @@ static int skinny_deepk_launch(int epi, bool flip_a, const GemmArgs &a, int grid
         return e;
     const EpiParams &p = a.epi;
     OnceArgs         o{a.A,    a.Bp,   a.D,    p.colvec, p.rowvec,  p.mult,    p.shift,       p.bias_f32,   a.lda,       a.ldd,        a.M,
-               a.N,    (int32_t)(a.Kp / 64), grid, p.result_offset, p.stage, p.lo, p.hi, p.scale, p.act_min, p.act_max,
-               p.has_offsets, p.accumulate, p.act_twice, p.half_out};
+               a.N,    (a.K + 63) / 64, grid, p.result_offset, p.stage, p.lo, p.hi, p.scale, p.act_min, p.act_max,
+               p.has_offsets, p.accumulate, p.act_twice, p.half_out, (int32_t)(a.Kp / 64), a.K};
     void *kargs[] = {&o};
     return (int)hipLaunchKernel(fn, dim3(grid), dim3(ONCE_WAVES * 64), kargs, lds, s);
 }
@@ -1085,7 +1168,61 @@ static int once_grid(int groups, int cus)
     return cus * ((groups + ONCE_MAX_GROUPS * cus - 1) / (ONCE_MAX_GROUPS * cus));
 }
 
-int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStream_t s, const char **variant)
+// What the stage-once form takes for 33 to 64 rows and a K of up to 4096, in us: its start, its share of A, and the k blocks of every column
+// group. (60 rows, off by at most 12 %: 768 x 2064 6.1, 3264 x 3264 8.7, 4096 x 4096 11.7, 9792 x 3264 13.6, 12288 x 4096 17.2; 42 rows: 0.88 of that.)
+double skinny_64rows_us(int M, int N, int K, int cus)
+{
+    const int groups = (N + 15) / 16, KB = (K + 63) / 64, grid = once_grid(groups, cus);
+    const int each = (groups + grid - 1) / grid, rounds = (grid + cus - 1) / cus;
+    return rounds * (2.2 + 0.077 * KB + 0.05 * KB * each) * (0.85 + 0.15 * (M - 32) / 32);
+}
+
+// 17 to 32 rows take slices where K is over 4096, the most that the stage-once form has room for in registers and LDS, 9 to 16 rows where
+// it is over 8192. What a workgroup costs beside its start: its share of A, PER k blocks for each of 16 waves, and PER blocks of every
+// column group. At 32 rows slices of 2 and 4 blocks with 1 to 4 groups took 3.7 + PER * (0.4 + 0.5 * groups) us, within 10 %.
+// Before (the streaming form) and with slices, us: 25 rows, 3072 x 12128: 15.9, 12.0; 4096 x 11008: 15.6, 13.2; 2880 x 7936: 11.4, 9.4;
+// 1472 x 5424: 8.4, 7.1; 8589 x 9113 (two rounds of workgroups): 41, 29. 12 rows, 3264 x 11072: 11.7, 10.9; 3072 x 12128: 12.4, 10.8; with two
+// rounds no faster (27.4, 27.9), so only where one suffices. Up to 8 rows the form for deep K is the faster one (9.2 and 10.5 at
+// 3264 x 11072); whole K where that fits: 25 rows, 4096 x 4096: 6.7, in slices 8.0.
+SkinnySlices skinny_slices(int M, int N, int K, int cus)
+{
+    SkinnySlices best{};
+    const int    groups = (N + 15) / 16, KB = (K + 63) / 64;
+    if (M <= 8 || M > 32 || cus < 1 || KB <= (M > 16 ? 4 : 8) * ONCE_WAVES)
+        return best;
+    double    least  = 0;
+    const int rounds = M > 16 ? 8 : 1;
+    for (int want = 2; want <= 16; ++want)
+    {
+        const int blocks = (KB + want - 1) / want, slices = (KB + blocks - 1) / blocks;
+        if (blocks > 4 * ONCE_WAVES || slices != want || slices > cus)
+            continue;
+        for (int round = 1; round <= rounds; ++round)
+        {
+            const int at_once = std::min(groups, round * cus / slices), each = (groups + at_once - 1) / at_once;
+            if (each > ONCE_MAX_GROUPS)
+                continue;
+            const double us = round * (3.7 + (blocks > 2 * ONCE_WAVES ? 4 : 2) * (0.4 + 0.5 * each)) + 0.1 * slices;
+            if (best.slices == 0 || us < least)
+            {
+                least       = us;
+                best.slices = slices, best.blocks = blocks, best.grid = (groups + each - 1) / each, best.rows = M > 16 ? 32 : 16;
+                best.words = (size_t)slices * groups * best.rows * 16;
+            }
+            break;
+        }
+    }
+    return best;
+}
+
+template <int ROWS>
+static int skinny_sliced_launch(int epi, bool flip_a, const GemmArgs &a, hipStream_t s, const SkinnySlices &plan)
+{
+    return plan.blocks <= 2 * ONCE_WAVES ? skinny_once_launch_r<2, true, ROWS, true>(epi, flip_a, a, plan.grid, s, &plan)
+                                         : skinny_once_launch_r<4, true, ROWS, true>(epi, flip_a, a, plan.grid, s, &plan);
+}
+
+int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStream_t s, const char **variant, const SkinnySlices *plan)
 {
     const char *unused;
     const char *&form = variant ? *variant : unused;
@@ -1093,10 +1230,10 @@ int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStre
     if (args.M < 1 || args.M > SKINNY_MAX_M || args.Kp % 64 != 0 || args.K > args.Kp || batch < 1 || batch > 65535)
         return (int)hipErrorInvalidValue;
     const int groups = (args.N + 15) / 16;
-    const int KB     = (int)(args.Kp / 64);
+    const int KB     = (args.K + 63) / 64;
     // Up to 8 rows every wave copies its K slice of A (at most 1 KiB per row) into LDS once and takes its operands
     // from there; that needs nothing to guard
-    const bool align_ok = args.K == args.Kp && args.K % 64 == 0 && args.lda % 16 == 0 && ((uintptr_t)args.A & 15) == 0 &&
+    const bool align_ok = args.K % 16 == 0 && args.lda % 16 == 0 && ((uintptr_t)args.A & 15) == 0 &&
                           (batch == 1 || args.a_batch_stride % 16 == 0);
     // (a batch along the grid: the streaming form, whose workgroups need nothing from each other)
     const bool align_ok1 = align_ok && batch == 1;
@@ -1106,6 +1243,11 @@ int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStre
     // up to 16 rows it also takes 4096 < K <= 8192 with 8 k blocks per wave (one group's worth of B in flight per wave,
     // refilled half by half - the same bytes as two groups of 4 k blocks).
     // up to 8 rows and 8192 < K <= 16384: the stage-once form for deep K (3 or 4 chunks of 4 k blocks per wave)
+    if (plan != nullptr && plan->slices > 1 && align_ok1 && args.M <= plan->rows && epi >= EPI_S32 && epi <= EPI_F32)
+    {
+        form = "skinny_slices";
+        return plan->rows == 16 ? skinny_sliced_launch<16>(epi, flip_a, args, s, *plan) : skinny_sliced_launch<32>(epi, flip_a, args, s, *plan);
+    }
     if (stage_ok && batch == 1 && KB > 8 * ONCE_WAVES && KB <= 16 * ONCE_WAVES && epi >= EPI_S32 && epi <= EPI_F32)
     {
         const int cus = device_cus();
@@ -1157,7 +1299,7 @@ int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStre
     // step of 8 k blocks and all workgroups are resident together (24 waves of this size per compute unit), 4 otherwise
     int waves = (groups >= 512 && !(stage_ok && KB >= 64 && (int64_t)groups * 8 <= 24 * 256)) ? 4 : 8;
     const int  per   = (KB + waves - 1) / waves;
-    const bool stage = stage_ok && per * 64 <= sk_a_slice(waves);
+    const bool stage = stage_ok && args.K == args.Kp && per * 64 <= sk_a_slice(waves);
     // more than 8 rows: per-step staging (dword-aligned rows are enough: the staging loads are plain 16-byte loads)
     const bool step = args.M > 8 && args.lda % 4 == 0 && ((uintptr_t)args.A & 3) == 0;
     // (17..24 rows: the gathers of the unstaged variants below re-read row M-1 for the missing rows of the second

@@ -144,8 +144,19 @@ int  conv_window_launch(const WindowPlan &plan, bool flip_a, const GemmArgs &arg
 
 // gemm_skinny.hip — M <= 64, B packed in matrix-core operand order (see pack_b_launch)
 constexpr int SKINNY_MAX_M = 64;
-// *variant (when given): a static string naming the form of the kernel that ran
-int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStream_t s, const char **variant = nullptr);
+// K in slices that run side by side (slices < 2: none): k blocks of 64 per slice, workgroups per slice, rows the kernel is built for;
+// what it needs beside the operands: `words` for partial sums, and `grid` counters that are zero (and are left zero)
+struct SkinnySlices
+{
+    int      slices = 0, blocks = 0, grid = 0, rows = 0;
+    size_t   words  = 0;
+    int32_t *parts = nullptr, *arrived = nullptr;
+};
+double       skinny_64rows_us(int M, int N, int K, int cus);
+SkinnySlices skinny_slices(int M, int N, int K, int cus);
+// *variant (when given): a static string naming the form of the kernel that ran; plan: the slices, with their memory, or null
+int skinny_launch(int epi, bool flip_a, const GemmArgs &args, int batch, hipStream_t s, const char **variant = nullptr,
+                  const SkinnySlices *plan = nullptr);
 
 // kernels_aux.hip
 // What the packing kernels make of a column's sum: colsum[b][Np] and colvec[b][j] = a_off*colsum + a_off*b_off*K (+ bias[j]);

@@ -75,7 +75,7 @@ typedef enum mi355_epilogue
 typedef enum mi355_path
 {
     MI355_PATH_AUTO   = 0, /* pipelined matrix-core kernel, or the streaming kernel for small M (<= 32; <= 64 with
-                            * N < 8192 or with K <= 4096 a multiple of 64) */
+                            * K <= 4096 where it is priced lower) */
     MI355_PATH_SIMPLE = 1, /* one thread per output, no matrix cores: the plain fallback (any alignment, any shape) */
     MI355_PATH_MFMA   = 2, /* a tiled matrix-core kernel whatever M is */
     MI355_PATH_SKINNY = 3, /* the streaming kernel (M <= 64) */
