@@ -194,13 +194,14 @@ struct GemmCore
     // What is known of buffers that are written once and then kept (see keep_flags)
     int         fill_set = -1; // the byte the 16 filler bytes hold (-1: not known)
     bool        zeros_set = false, zerocol_set = false, arrived_set = false;
+    ptrdiff_t    sums_at = -1; // where the sums of many slices lie in `arrived`, behind the counters (-1: in `parts`)
     SkinnySlices sk_plan; // the streaming kernel's K slices and their memory (prepare() fills it in)
     bool        qp_scalar_set = false; // the per-tensor requantisation vectors hold qp_rq
     bool        writes_recorded = false;
     mi355_requant qp_rq{};
     int     splitk = 1;      // K slices of the pipelined kernel
     int     byte_idx = -1; // the configuration that takes rows of A on any byte without a copy, and what the model prices it and the other at
-    double  us_bytes = 0, us_dma = 0;
+    double  us_bytes = 0, us_dma = 0, us_copied = 0;
     bool    byte_lda = false;   // rows or batch entries of A that do not start on dwords, as far as the strides say
     bool    one_launch = false; // few rows, one launch of the pipelined kernel instead of two of the streaming one's
     int     splitk_plan = 1; // what the cost model chose with the tile shape (create()); prepare() checks it and allocates
@@ -275,11 +276,21 @@ struct GemmCore
         // by a share us_load of it (L2, HBM and the power limit are shared by all compute units); the tiles that share a compute unit
         // take at least us_lone for a K step together.
         // A single GEMM may also run its K range as slices (see finish_prepare()): the tiles of all slices share the
-        // chip, every slice has its share of the K steps, and a second kernel sums the planes: 2.4 us for the launch
-        // and its latency, 0.1 us per plane one thread walks over and 0.5 us per MB written and read again (convolutions, fitted with their tiles:
-        // 3.2, 0.18 and 0.22). The 0.88 of dense products: a deep K under few tiles is slower than its price, which comes from fuller chips (256 x 221 x 2900:
-        // 10.3 us whole, priced at 8.6, 8.4 as 4 slices). Over 816 products the choice is 1.43 % slower than the best with it, 1.31 %
-        // with 1, over 327 with rows on any byte 2.1 % and more than 2.7 %: both together are even from 0.85 to 0.95.
+        // chip, every slice has its share of the K steps, and the last workgroup of a tile adds up the others' sums: 0.7 us, 0.3 us per
+        // slice and 0.6 us per million sums written and read again, beyond JOIN_PLANES slices 0.9 us and 4 us
+        // per million additions, fitted to 14 products of 64 to 1162 rows with 2 to 16 slices, off by 0.4 on average (convolutions, fitted with
+        // their tiles and a second launch for the sums, which took 1 us more: 3.2, 0.18 and 0.88; rows on any byte, which keep that launch: 2.4,
+        // 0.1 and 2, and 0.88 of it all). The 1.06 of dense products: where both are priced alike whole tiles are the faster ones more often
+        // (100 x 1000 x 2000: 6.3 us whole, 6.7 as 2 slices; 256 x 1024 x 2048: 6.0 and 7.0).
+        auto finish_us = [&](int loader, int sl) -> double
+        {
+            const double sums = (double)sl * M * N;
+            return sl <= 1           ? 0.0
+                   : loader == 1     ? 3.2 + 0.18 * sl + 0.88e-6 * sums
+                   : loader == 2     ? 2.4 + 0.1 * sl + 2e-6 * sums
+                   : sl <= JOIN_PLANES ? 0.7 + 0.3 * sl + 0.6e-6 * sums
+                                     : 0.9 + 4e-6 * sums;
+        };
         auto pick_dma = [&](int loader, int &plan, double &best_cost, int fixed_slices = 0) -> int
         {
             int best = -1;
@@ -296,15 +307,15 @@ struct GemmCore
                 {
                     // (slices of equal whole K steps but the last, none of them empty)
                     const int per = (nk + want - 1) / want, sl = (nk + per - 1) / per;
-                    if (want > 1 && (batch != 1 || per * c.BK < 512))
+                    if (want > 1 && (batch != 1 || per * c.BK < 512 || (i == 0 && fixed_slices == 0)))
                         break;
                     if (sl != want)
                         continue;
                     const double per_cu = std::ceil(tiles * sl / cus), load = std::min(1.0, tiles * sl / cus);
-                    const double finish = sl <= 1 ? 0.0 : loader == 1 ? 3.2 + 0.18 * sl + 0.88e-6 * (double)sl * M * N : 2.4 + 0.1 * sl + 2e-6 * (double)sl * M * N;
+                    const double finish = finish_us(loader, sl);
                     const double rounds = std::ceil(per_cu / occ), full = std::floor(per_cu / occ), rest = per_cu - full * occ, step = c.us_step * (1.0 + c.us_load * load);
                     const double steps  = per * (full * std::max(c.us_lone, occ * step) + (rest > 0 ? std::max(c.us_lone, rest * step) : 0.0));
-                    const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl > 1 && loader != 1 ? 0.88 : 1.0);
+                    const double cost   = (rounds * c.us_tile + (per_cu - rounds) * c.us_more + steps + finish) * (sl <= 1 || loader == 1 ? 1.0 : loader == 2 ? 0.88 : 1.06);
                     if (best < 0 || cost < best_cost)
                         best = i, best_cost = cost, plan = sl;
                 }
@@ -376,7 +387,11 @@ struct GemmCore
             dma_idx = pick_dma(patch_c > 0 ? 1 : 0, splitk_plan, us_dma, one_launch ? 1 : 0);
             int byte_plan = 1;
             if (patch_c == 0 && force_tile < 0 && dma_idx >= 0) // (the planes are those of the other's slices)
+            {
                 byte_idx = pick_dma(2, byte_plan, us_bytes, splitk_plan);
+                // (against rows on any byte, whose slices take the second launch: fitted with that launch and its prices on both sides)
+                us_copied = splitk_plan > 1 ? 0.83 * us_dma + 0.88 * (finish_us(2, splitk_plan) - finish_us(0, splitk_plan)) : us_dma;
+            }
             if (force_tile >= 0 && Kp % dma_config(force_tile).BK == 0 && dma_idx != force_tile)
             {
                 // a tile shape named by the caller: as many slices as fill the chip once, at least 1024 deep
@@ -564,26 +579,33 @@ struct GemmCore
             if (sk_plan.slices > 1)
             {
                 TRY(parts.ensure(sizeof(int32_t) * sk_plan.words));
-                if (!arrived_set)
-                {
-                    TRY(arrived.ensure(sizeof(int32_t) * (size_t)sk_plan.grid));
-                    HIP_TRY(fill_i32_launch(arrived.as<int32_t>(), 0, sk_plan.grid, s));
-                    arrived_set = true;
-                }
+                TRY(clear_arrived(sk_plan.grid, s));
                 sk_plan.parts = parts.as<int32_t>(), sk_plan.arrived = arrived.as<int32_t>();
             }
         }
         // A deep K under few output tiles: the pipelined kernel would leave most compute units idle, each of the others
-        // walking the whole K. The K range is cut into slices that run as the batch entries of one S32 launch (the slice
-        // offset is the batch stride of A and of the packed B alike), and a second kernel sums the planes and applies the
+        // walking the whole K. The K range is cut into slices that run as the batch entries of one launch (the slice
+        // offset is the batch stride of A and of the packed B alike); a tile's last workgroup sums its slices and applies the
         // epilogue. Slices are whole K steps of the tile shape, the last one as many as are left.
         splitk = 1;
         if (path == MI355_PATH_MFMA && dma_idx >= 0 && batch == 1)
             splitk = splitk_plan;
         if (splitk > 1)
         {
+            size_t words = 0, tiles = 0;
+            if (dma_idx > 0)
+            {
+                const MfmaConfig c = dma_config(dma_idx);
+                tiles = (size_t)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN);
+                words = tiles * (size_t)ring_slice_words(c.BM, c.BN);
+            }
             const size_t ldp = ((size_t)N + 3) & ~(size_t)3;
-            TRY(parts.ensure(sizeof(int32_t) * (size_t)splitk * M * ldp));
+            // (many slices: one place for the sums of a tile, behind the counters. 256 x 128 tiles, rows on any byte: planes of sums)
+            const bool added = splitk > JOIN_PLANES;
+            tiles            = (tiles + 1) & ~(size_t)1;
+            sums_at          = added ? (ptrdiff_t)tiles : -1;
+            TRY(clear_arrived(tiles + (added ? words : 0), s));
+            TRY(parts.ensure(sizeof(int32_t) * (size_t)splitk * std::max(added ? (size_t)0 : words, dma_idx == 0 || byte_idx >= 0 ? (size_t)M * ldp : (size_t)0)));
             if (own_row_terms())
                 TRY(rowvec.ensure(sizeof(int32_t) * (size_t)M));
             if (!zerocol_set)
@@ -608,6 +630,18 @@ struct GemmCore
             writes_recorded = true;
         if (writes_recorded)
             fill_set = -1, zeros_set = zerocol_set = arrived_set = qp_scalar_set = false;
+    }
+
+    // the counters of workgroups that finish a slice of K (each run leaves them zero)
+    int clear_arrived(size_t n, hipStream_t s)
+    {
+        if (n == 0 || (arrived_set && arrived.cap >= sizeof(int32_t) * n))
+            return 0;
+        arrived_set = false;
+        TRY(arrived.ensure(sizeof(int32_t) * n));
+        HIP_TRY(fill_i32_launch(arrived.as<int32_t>(), 0, (int64_t)n, s));
+        arrived_set = true;
+        return 0;
     }
 
     int set_fill(hipStream_t s)
@@ -743,7 +777,7 @@ struct GemmCore
                                       : 2.15 + (double)M * batch * (K + Kp) * 5.17e-7 + K * 0.46e-3;
         const bool   byte_rows = (!direct || (b_off_eff() != 0 && K % 16 != 0)) && ext_ws == nullptr && path == MI355_PATH_MFMA && byte_idx >= 0 &&
                                !(own_row_terms() && b_off_eff() != 0) && (int64_t)lda * 256 + K < ((int64_t)1 << 32) &&
-                               (one_launch || us_bytes * (direct ? 0.82 : 1.0) < us_dma + copy_us);
+                               (one_launch || us_bytes * (direct ? 0.82 : 1.0) < us_copied + copy_us);
         const bool rowsum_in_kernel = byte_rows ? b_off_eff() != 0 : b_off_eff() != 0 && direct && path == MI355_PATH_MFMA && dma_idx >= 0 && K % 16 == 0 && K >= 16 &&
                                       (splitk == 1 || epi != EPI_F32) && (int64_t)lda * 256 + K < ((int64_t)1 << 32);
         const bool need_rowvec = b_off_eff() != 0 && !rowsum_in_kernel;
@@ -896,20 +930,27 @@ struct GemmCore
                     // the float epilogue rounds the product and the offset terms apart: they must not meet in the planes
                     if (conv && epi == EPI_F32 && g.epi.rowsum_mul != 0)
                         TRY(conv_row_terms(g, s));
-                    const int     ldp = (N + 3) & ~3;
-                    const int64_t kc  = (int64_t)(((K + c.BK - 1) / c.BK + splitk - 1) / splitk) * c.BK;
-                    GemmArgs      gp  = g;
-                    gp.epi                     = EpiParams{};
-                    gp.epi.colvec              = zerocol.as<int32_t>();
-                    gp.epi.colvec_batch_stride = 0;
-                    gp.epi.vec_store           = 1;
-                    gp.epi.rowsum_mul          = g.epi.rowsum_mul; // every slice adds its own part of the row terms
-                    gp.D = parts.as<int32_t>(), gp.ldd = ldp, gp.d_batch_stride = (int64_t)M * ldp;
+                    const int64_t kc = (int64_t)(((K + c.BK - 1) / c.BK + splitk - 1) / splitk) * c.BK;
+                    GemmArgs      gp = g;
                     // (dense: a slice starts kc bytes into every row of A; convolution: kc values into every patch,
                     // which the loader adds to the k it decodes)
                     // (g.K: K, or K padded to whole steps where the rows of A were copied)
                     gp.a_batch_stride = conv ? 0 : kc, gp.bp_batch_stride = kc, gp.k_slice = (int32_t)kc;
+                    gp.epi.colvec_batch_stride = gp.epi.rowvec_batch_stride = 0, gp.d_batch_stride = 0;
                     kname_run = &kname_splitk;
+                    if (idx > 0 && !g.byte_rows)
+                    {
+                        gp.slices = splitk, gp.arrived = arrived.as<int32_t>(), gp.parts = sums_at >= 0 ? gp.arrived + sums_at : parts.as<int32_t>();
+                        HIP_TRY(dma_launch(idx, epi, flip_in_loader, conv, gp, splitk, s));
+                        return 0;
+                    }
+                    // 256 x 128 tiles, where the caller names them, and rows on any byte: a second launch sums the slices' planes
+                    const int ldp              = (N + 3) & ~3;
+                    gp.epi                     = EpiParams{};
+                    gp.epi.colvec              = zerocol.as<int32_t>();
+                    gp.epi.vec_store           = 1;
+                    gp.epi.rowsum_mul          = g.epi.rowsum_mul; // every slice adds its own part of the row terms
+                    gp.D = parts.as<int32_t>(), gp.ldd = ldp, gp.d_batch_stride = (int64_t)M * ldp;
                     HIP_TRY(dma_launch(idx, EPI_S32, flip_in_loader, conv, gp, splitk, s));
                     HIP_TRY(splitk_finish_launch(epi, g, parts.as<int32_t>(), (int64_t)M * ldp, ldp, splitk, s));
                     return 0;

@@ -899,6 +899,8 @@ int dma_launch(int cfg_idx, int epi, bool flip_a, bool conv, const GemmArgs &arg
     if (args.k_slice != 0 && (args.k_slice < 0 || args.k_slice % c.BK != 0 || (int64_t)args.k_slice * (batch - 1) >= args.K ||
                               (int64_t)args.k_slice * batch < args.K))
         return (int)hipErrorInvalidValue;
+    if (args.slices > 1 && (cfg_idx == 0 || byte_rows || args.slices != batch || args.parts == nullptr || args.arrived == nullptr))
+        return (int)hipErrorInvalidValue;
     // shapes the kernel assumes: dword-aligned rows of at least one 16-byte column (whole columns of one tap for the
     // convolution), tiles that cover the output and stay inside the packed B panel
     if (args.K < 16 || args.K > args.Kp || args.Kp % c.BK != 0 || args.tiles_m * c.BM < args.M ||

@@ -323,6 +323,122 @@ struct ByteSet<Loader, RING_BYTES>
     using type = typename Loader::Set;
 };
 
+// K slices (GemmArgs::slices): the workgroups of a tile leave their sums in memory and count themselves in; the last one takes the counter
+// back to zero, fetches the tile's sums and goes on to the epilogue. False for the others. Nobody waits for anybody. Up to JOIN_PLANES
+// slices each has a place of its own, whose sums the last workgroup has in flight together; more of them add theirs up in one place,
+// which the last one leaves zero (64 x 64 x 16384 as 8 slices 9.0 and 7.8 us, as 16 10.0 and 6.8; 256 x 256 x 8192 as 8 9.1 and 8.7; but 592 x 182 x 3856
+// as 4 7.4 and 8.0, 500 x 500 x 5000 9.0 and 10.3: every addition is one to memory).
+// All of it is of device scope, past the caches that dies do not share: when a wave's count of stores in flight is zero all can see
+// them, so the barrier and the counter need no fence (a release fence writes back the whole L2).
+// What it took the place of, a second launch over planes of sums, and this, us: 592 x 182 x 3856 9.3, 7.4 as 4 slices; 130 x 2048 x 4096 10.8, 8.9
+// as 2; 48 x 548 x 3583 10.4, 7.6 as 6; 60 x 4096 x 11008 17.1, 16.1 as 4.
+template <int RE, int QS, int NT>
+__device__ __forceinline__ bool join_slices(v4i (&fin)[RE][QS], int32_t (&rfin)[RE], bool rowsum, const GemmArgs &g, int tile, int slice, int tid, int *flag)
+{
+    typedef unsigned long long                     u64;
+    typedef __attribute__((address_space(1))) u64 *g64;
+    typedef __attribute__((address_space(1))) int *g32;
+    constexpr int SUMS = RE * QS * 2, ALL = SUMS + (RE + 1) / 2; // pairs of words of a thread: sums, then row terms
+    constexpr int AT_ONCE = SUMS >= 32 ? 1 : 32 / SUMS;           // slices whose sums are in flight together
+    const int     tiles = g.tiles_m * g.tiles_n;
+    const bool    added = g.slices > JOIN_PLANES;
+    auto          place = [&](int z) { return (g64)(uintptr_t)g.parts + ((int64_t)z * tiles + tile) * (ALL * NT) + tid; };
+    auto          pair  = [](int lo, int hi) { return (u64)(uint32_t)lo | ((u64)(uint32_t)hi << 32); };
+    // (one place: the words of a thread as single words, NT apart)
+    const g32 sum_at = (g32)(uintptr_t)g.parts + (int64_t)tile * (ALL * 2 * NT) + tid;
+    if (added)
+    {
+#pragma unroll
+        for (int u = 0; u < SUMS * 2; ++u)
+            __hip_atomic_fetch_add(sum_at + u * NT, fin[u / 4 / QS][u / 4 % QS][u % 4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (rowsum)
+#pragma unroll
+            for (int i = 0; i < RE; ++i)
+                __hip_atomic_fetch_add(sum_at + (SUMS * 2 + i) * NT, rfin[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    else
+    {
+        const g64 own = place(slice);
+#pragma unroll
+        for (int u = 0; u < SUMS; ++u)
+            __hip_atomic_store(own + u * NT, pair(fin[u / 2 / QS][u / 2 % QS][u % 2 * 2], fin[u / 2 / QS][u / 2 % QS][u % 2 * 2 + 1]),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (rowsum)
+#pragma unroll
+            for (int i = 0; i < RE; i += 2)
+                __hip_atomic_store(own + (SUMS + i / 2) * NT, pair(rfin[i], rfin[i + 1 < RE ? i + 1 : i]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    const g32 count = (g32)(uintptr_t)g.arrived + tile;
+    if (tid == 0)
+        *flag = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == g.slices - 1;
+    __syncthreads();
+    if (*flag == 0)
+        return false;
+    if (tid == 0)
+        __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::: "memory");
+    if (added)
+    {
+#pragma unroll
+        for (int u = 0; u < SUMS * 2; ++u)
+            fin[u / 4 / QS][u / 4 % QS][u % 4] = __hip_atomic_load(sum_at + u * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (rowsum)
+#pragma unroll
+            for (int i = 0; i < RE; ++i)
+                rfin[i] = __hip_atomic_load(sum_at + (SUMS * 2 + i) * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int u = 0; u < SUMS * 2; ++u)
+            __hip_atomic_store(sum_at + u * NT, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (rowsum)
+#pragma unroll
+            for (int i = 0; i < RE; ++i)
+                __hip_atomic_store(sum_at + (SUMS * 2 + i) * NT, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads(); // the flag's place is the epilogue's
+        return true;
+    }
+    for (int z0 = 1; z0 < g.slices; z0 += AT_ONCE)
+    {
+        u64 sums[AT_ONCE][SUMS], rows[AT_ONCE][(RE + 1) / 2];
+#pragma unroll
+        for (int y = 0; y < AT_ONCE; ++y)
+        {
+            const int z   = slice + z0 + y;
+            const g64 its = place(z >= g.slices ? z - g.slices : z);
+            if (z0 + y < g.slices)
+            {
+#pragma unroll
+                for (int u = 0; u < SUMS; ++u)
+                    sums[y][u] = __hip_atomic_load(its + u * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (rowsum)
+#pragma unroll
+                    for (int i = 0; i < (RE + 1) / 2; ++i)
+                        rows[y][i] = __hip_atomic_load(its + (SUMS + i) * NT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+#pragma unroll
+        for (int y = 0; y < AT_ONCE; ++y)
+        {
+            if (z0 + y < g.slices)
+            {
+#pragma unroll
+                for (int u = 0; u < SUMS; ++u)
+                {
+                    fin[u / 2 / QS][u / 2 % QS][u % 2 * 2] += (int)(uint32_t)sums[y][u];
+                    fin[u / 2 / QS][u / 2 % QS][u % 2 * 2 + 1] += (int)(uint32_t)(sums[y][u] >> 32);
+                }
+                if (rowsum)
+#pragma unroll
+                    for (int i = 0; i < RE; ++i)
+                        rfin[i] += (int)(uint32_t)(rows[y][i / 2] >> (i % 2 * 32));
+            }
+        }
+    }
+    __syncthreads(); // the flag's place is the epilogue's
+    return true;
+}
+
 template <int BM, int BN, int BK, int NS, int KG, int EPI, bool FLIP_A, int MODE>
 __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 1 ? 2 : BM * BN <= 64 * 64 ? 4 : 2))) void gemm_ring_kernel(GemmArgs g_in)
 {
@@ -660,6 +776,14 @@ __global__ __launch_bounds__(256 * KG) __attribute__((amdgpu_waves_per_eu(KG == 
     const int row_e = row_w + kg * RE * 16;
     if (rowsum)
         finish_row_sums<RE>(rfin, g.epi.rowsum_mul, FLIP_A && MODE == RING_DENSE ? nk * BK - g.K : 0);
+    // (rows on any byte: slices as planes and a second launch. With this behind their loop they were 3 to 5 % slower whole and 12 to 17 % in slices)
+    if constexpr (MODE != RING_BYTES)
+        if (g.slices > 1)
+        {
+            if (!join_slices<RE, QS, NW * 64>(fin, rfin, rowsum, g, tm * g.tiles_n + tn, bz, tid, (int *)smem))
+                return;
+            bz = 0;
+        }
 
     if (fast)
     {

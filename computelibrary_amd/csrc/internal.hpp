@@ -59,6 +59,10 @@ struct GemmArgs
     // column of that step could reach beyond a_end. Every other tile may fetch the step whole - the columns at and
     // beyond K then hold whatever follows in memory and meet the zero rows of the packed B. -1: no tile may.
     int32_t  lean_tail_bz;
+    // slices > 1 (join_slices() in gemm_ring.hpp): the batch entries are slices of one product, whose sums meet in `parts`: up to JOIN_PLANES slices
+    // ring_slice_words() per tile and slice, else per tile and zero between launches. One counter per tile, zero between launches
+    int32_t  slices;
+    int32_t *parts, *arrived;
     int32_t  byte_rows; // dense: rows of A on any byte, or sums of rows whose K ends inside a 16-byte column (host only: picks the kernel)
 };
 
@@ -108,6 +112,9 @@ struct RingEntry
     int         lds_bytes[2], threads[2]; // dense, convolution
     const void *fn[3][2][2];
 };
+constexpr int JOIN_PLANES = 5;
+// words of a tile's sums and row terms, for any of the configurations
+constexpr int64_t ring_slice_words(int BM, int BN) { return (int64_t)BM * BN * 5 / 4; }
 extern const RingEntry g_ring[];
 extern const int       g_ring_count;
 constexpr int            RING_BYTES_CFG = 3;
